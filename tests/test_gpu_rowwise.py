@@ -128,6 +128,22 @@ def test_layer_norm_modulation_bf16(shape):
     torch.testing.assert_close(y, oracle.layer_norm_modulation_ref(x, scale, shift, eps=1e-6), atol=1e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,vectors", [(2, 9, 513), (3, 4, 640), (1, 5, 767), (2, 8, 768), (2, 3, 769)])
+def test_layer_norm_modulation_wide_rows(dtype, B, L, vectors):
+    """Rows of 513 to 768 sixteen-byte vectors stay in registers, twelve vectors per lane; one more vector
+    takes the block-per-row kernel. Tolerances as for the narrower rows of the same type."""
+    n = vectors * (4 if dtype == torch.float32 else 8)
+    g = seeded(B + L + vectors)
+    x = randn(g, B, L, n, dtype=dtype).to(DEV)
+    scale, shift = (randn(g, B, 1, n, dtype=dtype, std=0.1).to(DEV) for _ in range(2))
+    y = tk.layer_norm_modulation(x, scale, shift)
+    tol = dict(atol=1e-5, rtol=0) if dtype == torch.float32 else dict(atol=1e-2, rtol=1e-2)
+    torch.testing.assert_close(y, oracle.layer_norm_modulation_ref(x, scale, shift), **tol)
+    w = (torch.rand(n, generator=g) + 0.5).to(dtype).to(DEV)
+    torch.testing.assert_close(tk.rms_norm(x, w), oracle.rms_norm_ref(x, w), **tol)
+
+
 def test_layer_norm_modulation_config2_cpu_oracle():
     x, scale, shift = cfg.config2("cpu", scale=0.25)
     want = oracle.layer_norm_modulation_ref(x, scale, shift, eps=1e-6)

@@ -184,6 +184,14 @@ typedef struct flux_linear_args {
 
 int flux_linear_bf16(const flux_linear_args* args, void* stream);
 
+/* The same with a workspace of device memory (16-byte aligned, the launch's own until it has run), which
+ * lets the library cut K over several workgroups where M and N alone give too few tiles: the fp32
+ * partial sums go through it and are added in a fixed order. flux_linear_workspace_bytes says how much
+ * the launch can use (0 = none; flux_linear_bf16 is then the same call); with less, the product runs
+ * with fewer parts or in one. */
+int64_t flux_linear_workspace_bytes(const flux_linear_args* args);
+int flux_linear_bf16_ws(const flux_linear_args* args, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Non-causal attention forward: O = softmax(Q K^T * sm_scale) V, bf16 in/out, fp32 online softmax.
  * Replaces scaled_dot_product_attention / _attn_fwd (kernels/attention.py:173-221, 70-170).

@@ -307,3 +307,41 @@ def test_linear_head_and_tail_launches(gated):
     want32 = x.float() + gy
     bound = 2.0 ** -8 * 1.01 * (2 * gy.abs() + want32.abs()) + 2e-3
     assert ((out.float() - want32).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("B,L,N,K,splits", [
+    (1, 9, 64, 64, 1), (1, 65, 96, 128, 1),          # one slab, two slabs; a row past the smallest tile
+    (3, 43, 200, 4096, 2), (1, 320, 384, 3072, 2),   # few tiles, long K: K over several workgroups (batch elements inside a tile)
+    (7, 19, 1000, 520, 1),                           # K tail, columns past the last tile, seven batch elements in two tiles
+    (1, 333, 9216, 192, 1), (2, 640, 3072, 640, 1),  # eight-wave tiles, ragged and exact
+    (1, 2700, 3072, 192, 1), (3, 1445, 3072, 128, 1), (1, 2049, 9224, 72, 1),   # four-wave rectangles with rows and columns to spare
+])
+def test_linear_tile_edges(B, L, N, K, splits):
+    """Every tile family where it can go wrong: row, column and K remainders, several batch elements in a
+    tile, K split over workgroups. Plain, GELU and gated-residual epilogues against the fp32 product, at
+    half a bf16 ulp per rounding plus the spread of an fp32 sum in another order."""
+    from triton_kernels import _native as nv
+    g = seeded(B + L + N + K)
+    M = B * L
+    a = randn(g, M, K, dtype=torch.bfloat16).to(DEV)
+    w = randn(g, N, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV)
+    b = randn(g, N, dtype=torch.bfloat16, std=0.5).to(DEV)
+    args = nv.LinearArgs()
+    y0 = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    args.A, args.W, args.Y, args.M, args.N, args.K = a.data_ptr(), w.data_ptr(), y0.data_ptr(), M, N, K
+    args.lda, args.ldw, args.ldy, args.split_n = K, K, N, N
+    assert (nv.lib().flux_linear_workspace_bytes(nv.byref(args)) > 0) == (splits > 1)
+    for act in ("", "GELU"):
+        ref32 = oracle.linear_ref_fp32(a, w, b, act)
+        y = tk.linear(a, w, b, activation=act)
+        assert ((y.float() - ref32).abs() <= half_ulp_bound(ref32)).all(), act
+    x = randn(g, B, L, N, dtype=torch.bfloat16).to(DEV)
+    gate = randn(g, B, 1, N, dtype=torch.bfloat16).to(DEV)
+    out = torch.full((B, L, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    tk.linear_into(a, w, b, out=out.view(M, N), resid=x.view(M, N), gate=gate)
+    assert torch.equal(out, oracle.gated_residual_ref(x, gate, tk.linear(a, w, b).view(B, L, N)))
+    # without a workspace the same product runs unsplit
+    args.bias = b.data_ptr()
+    nv.check(nv.lib().flux_linear_bf16(nv.byref(args), nv.stream_ptr(a.device)), "flux_linear_bf16")
+    ref32 = oracle.linear_ref_fp32(a, w, b)
+    assert ((y0.float() - ref32).abs() <= half_ulp_bound(ref32)).all()

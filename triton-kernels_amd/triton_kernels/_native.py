@@ -88,6 +88,8 @@ SIGNATURES = {
                                              c_int64, c_int32, c_float, c_void_p]),
     "flux_qkv_prep": (c_int32, [POINTER(QkvPrepArgs), c_void_p]),
     "flux_linear_bf16": (c_int32, [POINTER(LinearArgs), c_void_p]),
+    "flux_linear_workspace_bytes": (c_int64, [POINTER(LinearArgs)]),
+    "flux_linear_bf16_ws": (c_int32, [POINTER(LinearArgs), c_void_p, c_int64, c_void_p]),
     "flux_attention_fwd_bf16": (c_int32, [POINTER(AttnArgs), c_void_p]),
     "flux_silu": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
     "flux_gelu_tanh": (c_int32, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int32, c_void_p]),

@@ -123,7 +123,12 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
                  qk is not None and "qk-norm-rope", in_activation and f"in:{in_activation}"]
         launch_hook(linear_launch_metadata(M, N, K, x.element_size(), "+".join(p for p in parts if p)))
     with nv.on_device(dev):
-        rc = nv.lib().flux_linear_bf16(nv.byref(a), nv.stream_ptr(dev))
+        need = nv.lib().flux_linear_workspace_bytes(nv.byref(a))
+        if need:   # K cut over several workgroups: partial sums in memory of this launch's stream
+            ws = torch.empty((need,), dtype=torch.uint8, device=dev)
+            rc = nv.lib().flux_linear_bf16_ws(nv.byref(a), ws.data_ptr(), need, nv.stream_ptr(dev))
+        else:
+            rc = nv.lib().flux_linear_bf16(nv.byref(a), nv.stream_ptr(dev))
     nv.check(rc, "flux_linear_bf16")
     del keep
     return out

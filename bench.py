@@ -416,8 +416,8 @@ def cpu_baseline(torch):
 
 
 def double_block(torch, steps):
-    """The fused double-stream block (4096 img + 512 txt tokens, same hidden size, the txt chain on the
-    block's side stream), timed like the headline: an extra key, not the metric."""
+    """The fused double-stream block (4096 img + 512 txt tokens, same hidden size), timed like the
+    headline: an extra key, not the metric."""
     import triton_kernels as tk
     from triton_kernels.testing import flux_pe
     dev = "cuda"

@@ -77,6 +77,15 @@ int flux_layer_norm_modulation(const void* x, const void* scale, const void* shi
                                int64_t batch, int64_t seq, int32_t n, int64_t mod_batch_stride,
                                int32_t dtype, float eps, void* stream);
 
+/* The same on two tensors of the same width and type in one launch (the text and the image rows of a
+ * double-stream block). */
+typedef struct flux_layer_norm_args {
+    const void* x; const void* scale; const void* shift; void* y;
+    int64_t batch, seq, mod_batch_stride;
+} flux_layer_norm_args;
+int flux_layer_norm_modulation_pair(const flux_layer_norm_args* first, const flux_layer_norm_args* second, int32_t n,
+                                    int32_t dtype, float eps, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Q/K/V preparation: the fused gather behind RoPE apply and QKV split/concat.
  *
@@ -174,12 +183,10 @@ typedef struct flux_linear_args {
     int64_t flags;                             /* FLUX_LINEAR_* bits, 0 = none */
 } flux_linear_args;
 
-/* flags: the launch will run beside work of another stream (the txt chain beside the img chain of
- * the double-stream block). The library then keeps the tile shape whose last round leaves CUs free
- * for that work instead of the one that fills every round of the 256 CUs exactly, and gives a
- * small problem few, larger workgroups instead of one or two on every CU; both other choices are
- * the faster ones only when the launch has the GPU to itself. The result is the same bits either
- * way. */
+/* flags: the launch will run beside work of another stream. The library then keeps the tile shape whose
+ * last round leaves CUs free for that work instead of the one that fills every round of the 256 CUs
+ * exactly, which is the faster one only when the launch has the GPU to itself. The result is the same
+ * bits either way. */
 #define FLUX_LINEAR_SHARED_GPU 1
 
 int flux_linear_bf16(const flux_linear_args* args, void* stream);
@@ -191,6 +198,20 @@ int flux_linear_bf16(const flux_linear_args* args, void* stream);
  * with fewer parts or in one. */
 int64_t flux_linear_workspace_bytes(const flux_linear_args* args);
 int flux_linear_bf16_ws(const flux_linear_args* args, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Two products in one call, e.g. the text and the image rows of a double-stream block through their own
+ * weights. With the same N, K and form of epilogue they share one launch whose tiles are those of both;
+ * otherwise they run one after the other on the stream. a_rows[i] > 0: rows of A come in batches of that
+ * many rows with row stride lda and a_batch_stride elements from one batch to the next (a slice of a longer
+ * sequence); the stride is a multiple of 8 and at least a_rows * lda, all batches span less
+ * than 2 GiB, and M > 8 (else FLUX_E_UNSUPPORTED). */
+typedef struct flux_linear_pair_args {
+    flux_linear_args product[2];
+    int64_t a_rows[2], a_batch_stride[2];      /* 0 = evenly strided */
+} flux_linear_pair_args;
+
+int64_t flux_linear_pair_workspace_bytes(const flux_linear_pair_args* args);
+int flux_linear_bf16_pair(const flux_linear_pair_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Non-causal attention forward: O = softmax(Q K^T * sm_scale) V, bf16 in/out, fp32 online softmax.

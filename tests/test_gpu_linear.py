@@ -15,6 +15,7 @@ import triton_kernels as tk
 from oracle import flux_oracle as oracle
 from triton_kernels import testing as cfg
 from triton_kernels.kernels import qk_fusable
+from triton_kernels.kernels.linear import linear_pair_into
 from util import DEV, randn, seeded
 
 pytestmark = pytest.mark.gpu
@@ -345,3 +346,49 @@ def test_linear_tile_edges(B, L, N, K, splits):
     nv.check(nv.lib().flux_linear_bf16(nv.byref(args), nv.stream_ptr(a.device)), "flux_linear_bf16")
     ref32 = oracle.linear_ref_fp32(a, w, b)
     assert ((y0.float() - ref32).abs() <= half_ulp_bound(ref32)).all()
+
+
+@pytest.mark.parametrize("B,L0,L1,N,K", [
+    (1, 65, 9, 96, 128),          # one tile row each, the smallest tiles
+    (3, 43, 21, 3072, 4096),      # K over several workgroups, batch elements inside a tile
+    (2, 300, 77, 200, 520),       # K tail, columns past the last tile
+    (2, 1445, 256, 3072, 192),    # four-wave rectangles, ragged rows in both products
+    (1, 4096, 512, 1024, 64),     # square tiles or exact rectangles
+])
+def test_linear_pair(B, L0, L1, N, K):
+    """Two products in one launch against each product in fp32 (half a bf16 ulp plus the spread of another
+    order of summation): plain, GELU, and the gated residual with x as slices of one longer sequence, whose
+    batch elements are not evenly strided."""
+    g = seeded(B + L0 + L1 + N + K)
+    whole = randn(g, B, L0 + L1, K, dtype=torch.bfloat16).to(DEV)
+    xs = [whole[:, :L0], whole[:, L0:]]
+    ws = [randn(g, N, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV) for _ in xs]
+    bs = [randn(g, N, dtype=torch.bfloat16, std=0.5).to(DEV) for _ in xs]
+    refs = [oracle.linear_ref_fp32(x.reshape(-1, K), w, b) for x, w, b in zip(xs, ws, bs)]
+    for act in ("", "GELU"):
+        ys = linear_pair_into(*(dict(x=x, w=w, b=b, activation=act) for x, w, b in zip(xs, ws, bs)))
+        for y, x, w, b in zip(ys, xs, ws, bs):
+            ref32 = oracle.linear_ref_fp32(x.reshape(-1, K), w, b, act)
+            assert ((y.float() - ref32).abs() <= half_ulp_bound(ref32)).all(), act
+    rs = [randn(g, B, n, N, dtype=torch.bfloat16).to(DEV) for n in (L0, L1)]
+    gates = [randn(g, B, 1, N, dtype=torch.bfloat16).to(DEV) for _ in xs]
+    outs = linear_pair_into(*(dict(x=x, w=w, b=b, resid=r, gate=gt) for x, w, b, r, gt in zip(xs, ws, bs, rs, gates)))
+    plain = linear_pair_into(*(dict(x=x, w=w, b=b) for x, w, b in zip(xs, ws, bs)))
+    for out, y, r, gt, ref in zip(outs, plain, rs, gates, refs):
+        assert torch.equal(out.view(r.shape), oracle.gated_residual_ref(r, gt, y.view(r.shape)))
+    # products that cannot share a launch run one after the other
+    ys = linear_pair_into(dict(x=xs[0], w=ws[0], b=bs[0]), dict(x=xs[1], w=ws[1][:8], b=None))
+    assert ((ys[0].float() - refs[0]).abs() <= half_ulp_bound(refs[0])).all()
+    ref32 = oracle.linear_ref_fp32(xs[1].reshape(-1, K), ws[1][:8], None)
+    assert ((ys[1].float() - ref32).abs() <= half_ulp_bound(ref32)).all()
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_linear_pair_of_row_vectors(rows):
+    """The two modulation projections of a double-stream block in one launch: the bits of two launches."""
+    g = seeded(rows)
+    x = randn(g, rows, 3072, dtype=torch.bfloat16).to(DEV)
+    calls = [dict(x=x, w=randn(g, 1026, 3072, dtype=torch.bfloat16, std=0.02).to(DEV), b=randn(g, 1026, dtype=torch.bfloat16).to(DEV), in_activation="SiLU")
+             for _ in range(2)]
+    for y, call in zip(linear_pair_into(*calls), calls):
+        assert torch.equal(y, tk.linear_into(**call))

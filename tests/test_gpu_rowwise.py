@@ -144,6 +144,20 @@ def test_layer_norm_modulation_wide_rows(dtype, B, L, vectors):
     torch.testing.assert_close(tk.rms_norm(x, w), oracle.rms_norm_ref(x, w), **tol)
 
 
+@pytest.mark.parametrize("dtype,B,L0,L1,N", [
+    (torch.bfloat16, 1, 4, 1, 3072), (torch.bfloat16, 3, 20, 7, 3072),   # modulation in LDS; seven rows to a batch element: read per row
+    (torch.float32, 2, 5, 8, 1000), (torch.bfloat16, 2, 3, 2, 9001),     # masked columns; a block per row, unaligned
+])
+def test_layer_norm_modulation_pair(dtype, B, L0, L1, N):
+    """Two tensors in one launch give the bits of two launches."""
+    from triton_kernels.kernels.normalization import layer_norm_modulation_pair
+    g = seeded(B + L0 + L1 + N)
+    calls = [tuple(randn(g, B, n, N, dtype=dtype).to(DEV) for n in (L, 1, 1)) for L in (L0, L1)]
+    for y, call in zip(layer_norm_modulation_pair(*calls), calls):
+        assert torch.equal(y, tk.layer_norm_modulation(*call))
+
+
+
 def test_layer_norm_modulation_config2_cpu_oracle():
     x, scale, shift = cfg.config2("cpu", scale=0.25)
     want = oracle.layer_norm_modulation_ref(x, scale, shift, eps=1e-6)

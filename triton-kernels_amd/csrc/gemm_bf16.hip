@@ -329,15 +329,16 @@ __device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, 
     const int lrow = tid >> 3;
     const int lchunk = (tid & 7) ^ ((lrow >> 1) & 7);
     const int rows_a = min(p.M - m0, BM), rows_b = min(p.N - n0, BN);
-    bf16_t* const base_a = const_cast<bf16_t*>(p.A + static_cast<int64_t>(m0) * p.lda);
+    const int64_t a0 = row_of_a(p, m0);
+    bf16_t* const base_a = const_cast<bf16_t*>(p.A + a0);
     bf16_t* const base_b = const_cast<bf16_t*>(p.W + static_cast<int64_t>(n0) * p.ldw);
-    const int bytes_a = static_cast<int>(((rows_a - 1) * p.lda + p.K) * 2);
+    const int bytes_a = static_cast<int>((row_of_a(p, m0 + rows_a - 1) - a0 + p.K) * 2);
     const int bytes_b = static_cast<int>(((rows_b - 1) * p.ldw + p.K) * 2);
     uint32_t voff_a[PU], voff_b[PU];
 #pragma unroll
     for (int i = 0; i < PU; ++i) {
         const int r = i * 32 + lrow;
-        voff_a[i] = r < rows_a ? static_cast<uint32_t>((r * p.lda + lchunk * 8) * 2) : kOutOfRange;
+        voff_a[i] = r < rows_a ? static_cast<uint32_t>((row_of_a(p, m0 + r) - a0 + lchunk * 8) * 2) : kOutOfRange;
         voff_b[i] = r < rows_b ? static_cast<uint32_t>((r * p.ldw + lchunk * 8) * 2) : kOutOfRange;
     }
     // the slab range ends at ke: everything from there on reads as zeros, like the K tail
@@ -496,9 +497,9 @@ template <int MI, bool KTAIL>
 __global__ __launch_bounds__(kGemmThreads) void gemm_nt_ring_kernel(GemmLaunch L) {
     constexpr int BM = 64 * MI, BK = 64, NU = 5, UNIT = BM * BK * 2;
     __shared__ __attribute__((aligned(1024))) char lds[NU * UNIT];
-    const GemmParams& p = L.p;
     int tm, tn;
-    if (p.qk_cols > 0 ? !tile_of_block_qk(L, BM, tm, tn) : !tile_of_block(L, tm, tn)) return;
+    if (L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BM, tm, tn) : !tile_of_block(L, tm, tn)) return;
+    const GemmParams& p = product_of_tile(L, tm);
     const int m0 = tm * BM, n0 = tn * BM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -544,13 +545,14 @@ __device__ __forceinline__ void gemm_rect_slabs(const GemmParams& p, char* lds, 
     const int lrow = tid >> 3;
     const int lchunk = (tid & 7) ^ ((lrow >> 1) & 7);
     const int rows_a = min(p.M - m0, BM), rows_b = min(p.N - n0, BN);
-    bf16_t* const base_a = const_cast<bf16_t*>(p.A + static_cast<int64_t>(m0) * p.lda);
+    const int64_t a0 = row_of_a(p, m0);
+    bf16_t* const base_a = const_cast<bf16_t*>(p.A + a0);
     bf16_t* const base_b = const_cast<bf16_t*>(p.W + static_cast<int64_t>(n0) * p.ldw);
-    const int bytes_a = static_cast<int>(((rows_a - 1) * p.lda + p.K) * 2);
+    const int bytes_a = static_cast<int>((row_of_a(p, m0 + rows_a - 1) - a0 + p.K) * 2);
     const int bytes_b = static_cast<int>(((rows_b - 1) * p.ldw + p.K) * 2);
     uint32_t voff_a[PA], voff_b[PW];
 #pragma unroll
-    for (int i = 0; i < PA; ++i) voff_a[i] = i * 32 + lrow < rows_a ? static_cast<uint32_t>(((i * 32 + lrow) * p.lda + lchunk * 8) * 2) : kOutOfRange;
+    for (int i = 0; i < PA; ++i) voff_a[i] = i * 32 + lrow < rows_a ? static_cast<uint32_t>((row_of_a(p, m0 + i * 32 + lrow) - a0 + lchunk * 8) * 2) : kOutOfRange;
 #pragma unroll
     for (int i = 0; i < PW; ++i) voff_b[i] = i * 32 + lrow >= rows_b ? kOutOfRange : static_cast<uint32_t>(((i * 32 + lrow) * p.ldw + lchunk * 8) * 2);
     const int k_end = min(p.K, ke * BK);
@@ -681,9 +683,9 @@ template <int FM, int FN, bool KTAIL>
 __global__ __launch_bounds__(kGemmThreads) void gemm_nt_rect_kernel(GemmLaunch L) {
     constexpr int BM = 32 * FM, BN = 32 * FN, BK = 64;
     __shared__ __attribute__((aligned(1024))) char lds[(3 * BM + 2 * BN) * BK * 2];
-    const GemmParams& p = L.p;
     int tm, tn;
-    if (FN == 8 && p.qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
+    if (FN == 8 && L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
+    const GemmParams& p = product_of_tile(L, tm);
     const int m0 = tm * BM, n0 = tn * BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -712,7 +714,8 @@ constexpr int gemv_depth(int rows) { return rows <= 2 ? 6 : 3; }
 // from memory as they are needed.
 // EXACT: K = 512 * U, so every lane has exactly U vectors per row and the K loop runs once, without tests.
 template <int MM, bool SILU_LDS, bool EXACT>
-__global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmParams p) {
+__global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
+    const GemmParams& p = g.p[blockIdx.y];
     constexpr int CPW = kGemvCols, U = gemv_depth(MM);  // CPW * U 16-byte loads of W in flight per lane: a whole row of 3072
     extern __shared__ __attribute__((aligned(16))) char act_lds[];
     const int lane = threadIdx.x & 63;
@@ -813,14 +816,15 @@ __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmParams p) {
 }
 
 template <int MM>
-static void launch_gemv(const GemmParams& p, hipStream_t st) {
-    const unsigned grid = (unsigned)((p.N + 4 * kGemvCols - 1) / (4 * kGemvCols));
+static void launch_gemv(const GemmSet& g, hipStream_t st) {
+    const GemmParams& p = g.p[0];
+    const dim3 grid((unsigned)((p.N + 4 * kGemvCols - 1) / (4 * kGemvCols)), (unsigned)g.n);
     const size_t act_bytes = static_cast<size_t>(MM) * p.K * 2;
     const bool lds = act_bytes <= kGemvSiluLds, exact = p.K == 512 * gemv_depth(MM);
-    if (lds && exact) hipLaunchKernelGGL((gemv_small_m_kernel<MM, true, true>), dim3(grid), dim3(256), act_bytes, st, p);
-    else if (lds) hipLaunchKernelGGL((gemv_small_m_kernel<MM, true, false>), dim3(grid), dim3(256), act_bytes, st, p);
-    else if (exact) hipLaunchKernelGGL((gemv_small_m_kernel<MM, false, true>), dim3(grid), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((gemv_small_m_kernel<MM, false, false>), dim3(grid), dim3(256), 0, st, p);
+    if (lds && exact) hipLaunchKernelGGL((gemv_small_m_kernel<MM, true, true>), grid, dim3(256), act_bytes, st, g);
+    else if (lds) hipLaunchKernelGGL((gemv_small_m_kernel<MM, true, false>), grid, dim3(256), act_bytes, st, g);
+    else if (exact) hipLaunchKernelGGL((gemv_small_m_kernel<MM, false, true>), grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((gemv_small_m_kernel<MM, false, false>), grid, dim3(256), 0, st, g);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -853,16 +857,16 @@ __global__ __launch_bounds__(256) void gemm_nt_scalar_kernel(GemmParams p) {
 }
 
 template <int MI>
-static void launch_tiled(const GemmParams& p, hipStream_t st) {
-    const GemmLaunch L = make_launch(p, 64 * MI, 64 * MI);
-    if (p.K % 64 == 0) hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, false>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+static void launch_tiled(const GemmSet& g, hipStream_t st) {
+    const GemmLaunch L = make_launch(g, 64 * MI, 64 * MI);
+    if (g.p[0].K % 64 == 0) hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, false>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
     else hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, true>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
 }
 
 template <int FM, int FN>
-static void launch_rect(const GemmParams& p, hipStream_t st) {
-    const GemmLaunch L = make_launch(p, 32 * FM, 32 * FN);
-    if (p.K % 64 == 0) hipLaunchKernelGGL((gemm_nt_rect_kernel<FM, FN, false>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+static void launch_rect(const GemmSet& g, hipStream_t st) {
+    const GemmLaunch L = make_launch(g, 32 * FM, 32 * FN);
+    if (g.p[0].K % 64 == 0) hipLaunchKernelGGL((gemm_nt_rect_kernel<FM, FN, false>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
     else hipLaunchKernelGGL((gemm_nt_rect_kernel<FM, FN, true>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
 }
 
@@ -906,36 +910,45 @@ static const TileShape kTileShapes[] = {
     {kPair, 3, 3, 0.325}, {kPair, 2, 3, 0.287}, {kPair, 2, 2, 0.183}, {kPair, 4, 8, 0.900},
 };
 
-static int64_t tile_count(const GemmParams& p, const TileShape& t) {
-    return static_cast<int64_t>((p.M + 32 * t.fm - 1) / (32 * t.fm)) * ((p.N + 32 * t.fn - 1) / (32 * t.fn));
+static int64_t tile_count(const GemmSet& g, const TileShape& t) {
+    int64_t rows = 0;
+    for (int i = 0; i < g.n; ++i) rows += (g.p[i].M + 32 * t.fm - 1) / (32 * t.fm);
+    return rows * ((g.p[0].N + 32 * t.fn - 1) / (32 * t.fn));
 }
-static int64_t split_bytes(const GemmParams& p, const TileShape& t, int splits) {
-    return tile_count(p, t) * splits * (32 * t.fm) * (32 * t.fn) * 4;
+static int64_t split_bytes(const GemmSet& g, const TileShape& t, int splits) {
+    return tile_count(g, t) * splits * (32 * t.fm) * (32 * t.fn) * 4;
 }
 
-static double tile_cost_us(const GemmParams& p, const TileShape& t, int splits) {
+static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
     const double kLaunch = 4.6, kTileLarge = 4.3, kTilePair = 2.7, kReduce = 1.7, kSplitGBs = 5970.0, kWeightGBs = 4500.0;
     const double kIdleShare = 0.31;   // a workgroup runs up to this much faster the emptier the GPU is
-    const int64_t tiles = tile_count(p, t) * splits;
+    const int64_t tiles = tile_count(g, t) * splits;
     const int64_t rounds = (tiles + kGemmCUs - 1) / kGemmCUs;
     const double fill = static_cast<double>(tiles) / (rounds * kGemmCUs);
-    const int slabs = ((p.K + 63) / 64 + splits - 1) / splits;
+    const int slabs = ((g.p[0].K + 63) / 64 + splits - 1) / splits;
     const double us = rounds * ((t.family == kPair ? kTilePair : kTileLarge) + slabs * t.slab_us * (1.0 - kIdleShare * (1.0 - fill)));
-    return kLaunch + std::max(us, 2e-3 * p.N * p.K / kWeightGBs) + (splits > 1 ? kReduce + 2e-3 * split_bytes(p, t, splits) / kSplitGBs : 0.0);
+    return kLaunch + std::max(us, 2e-3 * g.n * g.p[0].N * g.p[0].K / kWeightGBs) + (splits > 1 ? kReduce + 2e-3 * split_bytes(g, t, splits) / kSplitGBs : 0.0);
 }
 
-static TilePlan plan_tiles(const GemmParams& p, bool shared_gpu, int64_t workspace_bytes) {
+static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_bytes) {
     // The rectangular and eight-wave tiles have one epilogue: 16-byte outputs, a wave's columns on one side of
     // split_n and act_begin, no GELU in front of a gate. Anything else takes the square tiles' checked one.
-    const bool form = p.vec_io && p.N % 8 == 0 && (p.bias == nullptr || p.bias_vec) && !(p.gate != nullptr && p.act != FLUX_ACT_NONE) &&
-                      p.lda * 2 * 288 < 0x7fffffffLL && p.ldw * 2 * 256 < 0x7fffffffLL && p.ldy * 2 * 288 < 0x7fffffffLL &&
-                      p.ldy2 * 2 * 288 < 0x7fffffffLL;   // 32-bit byte offsets inside a tile's rows
+    const GemmParams& p = g.p[0];
+    bool form = true;
+    int64_t square_tiles = 0;
+    for (int i = 0; i < g.n; ++i) {
+        const GemmParams& q = g.p[i];
+        form = form && q.vec_io && q.N % 8 == 0 && (q.bias == nullptr || q.bias_vec) && !(q.gate != nullptr && q.act != FLUX_ACT_NONE) &&
+               q.lda * 2 * 288 < 0x7fffffffLL && q.ldw * 2 * 256 < 0x7fffffffLL && q.ldy * 2 * 288 < 0x7fffffffLL &&
+               q.ldy2 * 2 * 288 < 0x7fffffffLL;   // 32-bit byte offsets inside a tile's rows
+        square_tiles += static_cast<int64_t>((q.M + 255) / 256) * ((q.N + 255) / 256);
+    }
     auto columns_ok = [&](int fn) {
         const int w = 16 * fn;
         return (p.split_n >= p.N || p.split_n % w == 0) && (p.act == FLUX_ACT_NONE || p.act_begin >= p.N || p.act_begin % w == 0);
     };
     if (!form) {   // 256-wide tiles once they fill most of the chip, else 128-wide ones, two workgroups per CU
-        const bool big = static_cast<int64_t>((p.M + 255) / 256) * ((p.N + 255) / 256) >= 160;
+        const bool big = square_tiles >= 160;
         return {kSquare, big ? 8 : 4, big ? 8 : 4, 1, 0.0};
     }
     TilePlan best = {kSquare, 8, 8, 1, 1e30};
@@ -947,8 +960,8 @@ static TilePlan plan_tiles(const GemmParams& p, bool shared_gpu, int64_t workspa
         if (t.family != kSquare && !columns_ok(t.fn)) continue;
         const int most = t.family == kPair && p.K % 64 == 0 && p.qk_cols == 0 ? 10 : 1;
         for (int s = 1; s <= most; ++s) {
-            if (s > 1 && (tile_count(p, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(p, t, s) > workspace_bytes)) break;
-            const double us = tile_cost_us(p, t, s);
+            if (s > 1 && (tile_count(g, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(g, t, s) > workspace_bytes)) break;
+            const double us = tile_cost_us(g, t, s);
             if (us < best.us) best = {t.family, t.fm, t.fn, s, us};
         }
     }
@@ -959,15 +972,19 @@ static TilePlan plan_tiles(const GemmParams& p, bool shared_gpu, int64_t workspa
         best = {kSquare, 8, 8, 1, 1e30};
         for (const TileShape& t : kTileShapes) {
             if (t.fn != 8 || (t.family == kPair) != pair || (t.family != kSquare && !columns_ok(8))) continue;
-            const double us = tile_cost_us(p, t, 1);
+            const double us = tile_cost_us(g, t, 1);
             if (us < best.us) best = {t.family, t.fm, t.fn, 1, us};
         }
     }
     return best;
 }
 
-// With `need` nothing is launched: it receives the workspace the launch would like to have.
-static int linear_launch(const flux_linear_args* a, void* workspace, int64_t workspace_bytes, int64_t* need, hipStream_t st) {
+// How a call can be served.
+enum LinearRoute { kNothing, kScalar, kRows, kTiles };
+
+// Checks a call and turns it into the kernels' parameters.
+static int read_linear_args(const flux_linear_args* a, GemmParams& p, LinearRoute& route) {
+    route = kNothing;
     if (!a) return fail(FLUX_E_NULL, "flux_linear_bf16: null args");
     if (!a->A || !a->W || !a->Y) return fail(FLUX_E_NULL, "flux_linear_bf16: null operand");
     if (a->M < 0 || a->N < 0 || a->K < 0) return fail(FLUX_E_SHAPE, "flux_linear_bf16: negative size");
@@ -983,11 +1000,11 @@ static int linear_launch(const flux_linear_args* a, void* workspace, int64_t wor
     if ((a->gate == nullptr) != (a->resid == nullptr)) return fail(FLUX_E_NULL, "flux_linear_bf16: gate and resid go together");
     if (a->gate && a->rows_per_batch <= 0) return fail(FLUX_E_SHAPE, "flux_linear_bf16: rows_per_batch must be positive with a gate");
 
-    GemmParams p;
     p.A = static_cast<const bf16_t*>(a->A); p.W = static_cast<const bf16_t*>(a->W); p.bias = static_cast<const bf16_t*>(a->bias);
     p.Y = static_cast<bf16_t*>(a->Y); p.Y2 = split ? static_cast<bf16_t*>(a->Y2) : nullptr;
     p.resid = static_cast<const bf16_t*>(a->resid); p.gate = static_cast<const bf16_t*>(a->gate);
     p.M = (int)a->M; p.N = (int)a->N; p.K = (int)a->K;
+    p.a_rows = 1; p.a_skip = 0;
     p.lda = a->lda; p.ldw = a->ldw; p.ldy = a->ldy; p.ldy2 = a->ldy2; p.ldresid = a->ldresid;
     p.gate_stride = a->gate_batch_stride;
     p.split_n = split ? (int)a->split_n : p.N;
@@ -1025,49 +1042,115 @@ static int linear_launch(const flux_linear_args* a, void* workspace, int64_t wor
         p.qk_cols = (int)cols; p.qk_heads = (int)f->heads; p.qk_seq_len = (int)f->seq_len; p.qk_out_len = (int)f->out_len;
         p.qk_pos0 = (int)f->pos0; p.qk_eps = f->eps;
     }
-    if (need != nullptr && (p.K == 0 || (p.M <= 8 && p.qk_cols == 0))) return FLUX_OK;
-    if (p.K == 0) {
-        // Degenerate contraction: the scalar kernel's empty K loop leaves bias/epilogue only.
-        hipLaunchKernelGGL(gemm_nt_scalar_kernel, dim3((unsigned)(((int64_t)p.M * p.N + 255) / 256)), dim3(256), 0, st, p);
-        return check_launch("flux_linear_bf16");
-    }
     const bool vec_in = aligned16(a->A) && aligned16(a->W) && a->K % 8 == 0 && a->lda % 8 == 0 && a->ldw % 8 == 0;
     // 32-bit byte offsets inside one tile's rows
     const bool off_ok = a->lda * 2 * 256 < 0x7fffffffLL && a->ldw * 2 * 256 < 0x7fffffffLL;
-    if (!vec_in || !off_ok) {
-        if (need != nullptr) return FLUX_OK;
-        hipLaunchKernelGGL(gemm_nt_scalar_kernel, dim3((unsigned)(((int64_t)p.M * p.N + 255) / 256)), dim3(256), 0, st, p);
-        return check_launch("flux_linear_bf16");
+    // (degenerate contraction, K = 0: the scalar kernel's empty K loop leaves bias and epilogue only)
+    route = p.K == 0 || !vec_in || !off_ok ? kScalar : (p.M <= 8 && p.qk_cols == 0 ? kRows : kTiles);
+    return FLUX_OK;
+}
+
+static int launch_rows(const GemmSet& g, hipStream_t st) {
+    switch (g.p[0].M) {
+        case 1: launch_gemv<1>(g, st); break;
+        case 2: launch_gemv<2>(g, st); break;
+        case 3: launch_gemv<3>(g, st); break;
+        case 4: launch_gemv<4>(g, st); break;
+        case 5: launch_gemv<5>(g, st); break;
+        case 6: launch_gemv<6>(g, st); break;
+        case 7: launch_gemv<7>(g, st); break;
+        default: launch_gemv<8>(g, st); break;
     }
-    if (p.M <= 8 && p.qk_cols == 0) {
-        switch (p.M) {
-            case 1: launch_gemv<1>(p, st); break;
-            case 2: launch_gemv<2>(p, st); break;
-            case 3: launch_gemv<3>(p, st); break;
-            case 4: launch_gemv<4>(p, st); break;
-            case 5: launch_gemv<5>(p, st); break;
-            case 6: launch_gemv<6>(p, st); break;
-            case 7: launch_gemv<7>(p, st); break;
-            default: launch_gemv<8>(p, st); break;
-        }
-        return check_launch("flux_linear_bf16");
-    }
-    const TilePlan plan = plan_tiles(p, (a->flags & FLUX_LINEAR_SHARED_GPU) != 0, need != nullptr ? INT64_MAX : workspace_bytes);
+    return check_launch("flux_linear_bf16");
+}
+
+// With `need` nothing is launched: it receives the workspace the launch would like to have.
+static int launch_tiles(const GemmSet& g, bool shared_gpu, void* workspace, int64_t workspace_bytes, int64_t* need, hipStream_t st) {
+    const TilePlan plan = plan_tiles(g, shared_gpu, need != nullptr ? INT64_MAX : workspace_bytes);
     if (need != nullptr) {
-        if (plan.splits > 1) *need = split_bytes(p, {plan.family, plan.fm, plan.fn, 0.0}, plan.splits);
+        if (plan.splits > 1) *need = split_bytes(g, {plan.family, plan.fm, plan.fn, 0.0}, plan.splits);
         return FLUX_OK;
     }
     switch (plan.family) {
-        case kSquare: if (plan.fm == 8) launch_tiled<4>(p, st); else launch_tiled<2>(p, st); break;
+        case kSquare: if (plan.fm == 8) launch_tiled<4>(g, st); else launch_tiled<2>(g, st); break;
         case kRect:
-            if (plan.fm == 9) launch_rect<9, 6>(p, st);
-            else if (plan.fm == 8) launch_rect<8, 6>(p, st);
-            else if (plan.fn == 6) launch_rect<7, 6>(p, st);
-            else launch_rect<7, 8>(p, st);
+            if (plan.fm == 9) launch_rect<9, 6>(g, st);
+            else if (plan.fm == 8) launch_rect<8, 6>(g, st);
+            else if (plan.fn == 6) launch_rect<7, 6>(g, st);
+            else launch_rect<7, 8>(g, st);
             break;
-        case kPair: launch_pair_tiles(plan.fm, plan.fn, p, plan.splits, static_cast<float*>(workspace), st); break;
+        case kPair: launch_pair_tiles(plan.fm, plan.fn, g, plan.splits, static_cast<float*>(workspace), st); break;
     }
     return check_launch("flux_linear_bf16");
+}
+
+static int linear_launch(const flux_linear_args* a, void* workspace, int64_t workspace_bytes, int64_t* need, hipStream_t st) {
+    GemmSet g;
+    LinearRoute route;
+    g.n = 1;
+    const int rc = read_linear_args(a, g.p[0], route);
+    if (rc != FLUX_OK || route == kNothing) return rc;
+    if (route == kTiles) return launch_tiles(g, (a->flags & FLUX_LINEAR_SHARED_GPU) != 0, workspace, workspace_bytes, need, st);
+    if (need != nullptr) return FLUX_OK;
+    if (route == kRows) { g.p[1] = g.p[0]; return launch_rows(g, st); }
+    const GemmParams& p = g.p[0];
+    hipLaunchKernelGGL(gemm_nt_scalar_kernel, dim3((unsigned)(((int64_t)p.M * p.N + 255) / 256)), dim3(256), 0, st, p);
+    return check_launch("flux_linear_bf16");
+}
+
+// Rows of A in batches whose distance is not rows x lda (a slice of a longer sequence).
+static int set_a_batches(GemmParams& p, int64_t rows, int64_t stride, LinearRoute route, const char* what) {
+    if (rows == 0) return FLUX_OK;
+    if (rows < 0 || stride < 0) return fail(FLUX_E_SHAPE, "%s: negative rows or stride of A's batches", what);
+    if (route == kNothing || p.M <= rows || stride == rows * p.lda) return FLUX_OK;
+    if (route != kTiles || stride % 8 != 0 || stride < rows * p.lda || ((p.M - 1) / rows + 1) * stride * 2 >= 0x7fffffffLL)
+        return fail(FLUX_E_UNSUPPORTED, "%s: batches of A need more than 8 rows in all, a stride of a multiple of 8 and less than 2 GiB in all", what);
+    p.a_rows = (int)rows;
+    p.a_skip = stride - rows * p.lda;
+    return FLUX_OK;
+}
+
+// One launch for both products where they have the same N, K and form of epilogue, so that the tile grid is
+// that of their rows together; else one after the other through the same workspace (the stream orders them).
+// 1024 + 256 rows of the double-stream block, one launch against two on two streams: 3072 x 9216 weights 59 us
+// (55 and 31 side by side), 12288 x 3072 81 (66, 33), 3072 x 12288 101 (85, 36); the pass 567 -> 371 us.
+static int linear_pair_launch(const flux_linear_pair_args* a, void* workspace, int64_t workspace_bytes, int64_t* need, hipStream_t st) {
+    if (!a) return fail(FLUX_E_NULL, "flux_linear_bf16_pair: null args");
+    GemmSet g;
+    LinearRoute route[2];
+    for (int i = 0; i < 2; ++i) {
+        int rc = read_linear_args(&a->product[i], g.p[i], route[i]);
+        if (rc == FLUX_OK) rc = set_a_batches(g.p[i], a->a_rows[i], a->a_batch_stride[i], route[i], "flux_linear_bf16_pair");
+        if (rc != FLUX_OK) return rc;
+    }
+    const GemmParams &p = g.p[0], &q = g.p[1];
+    const bool same = route[0] == route[1] && p.N == q.N && p.K == q.K && p.act == q.act && p.act_begin == q.act_begin && p.split_n == q.split_n &&
+                      p.in_silu == q.in_silu && (p.gate != nullptr) == (q.gate != nullptr) && p.qk_cols == q.qk_cols;
+    const bool shared_gpu = ((a->product[0].flags | a->product[1].flags) & FLUX_LINEAR_SHARED_GPU) != 0;
+    if (need != nullptr) *need = 0;
+    if (same && route[0] == kTiles) {
+        g.n = 2;
+        return launch_tiles(g, shared_gpu, workspace, workspace_bytes, need, st);
+    }
+    if (same && route[0] == kRows && p.M == q.M) {
+        g.n = 2;
+        return need != nullptr ? FLUX_OK : launch_rows(g, st);
+    }
+    for (int i = 0; i < 2; ++i) {
+        int64_t part = 0;
+        int rc;
+        if (route[i] == kTiles) {
+            GemmSet one;
+            one.n = 1;
+            one.p[0] = g.p[i];
+            rc = launch_tiles(one, shared_gpu, workspace, workspace_bytes, need != nullptr ? &part : nullptr, st);
+        } else {
+            rc = linear_launch(&a->product[i], workspace, workspace_bytes, need != nullptr ? &part : nullptr, st);
+        }
+        if (rc != FLUX_OK) return rc;
+        if (need != nullptr) *need = std::max(*need, part);
+    }
+    return FLUX_OK;
 }
 
 extern "C" int flux_linear_bf16(const flux_linear_args* a, void* stream) {
@@ -1082,4 +1165,14 @@ extern "C" int64_t flux_linear_workspace_bytes(const flux_linear_args* a) {
 extern "C" int flux_linear_bf16_ws(const flux_linear_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
     if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace)))) return fail(FLUX_E_NULL, "flux_linear_bf16_ws: workspace must be 16-byte aligned memory");
     return linear_launch(a, workspace, workspace_bytes, nullptr, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t flux_linear_pair_workspace_bytes(const flux_linear_pair_args* a) {
+    int64_t need = 0;
+    return linear_pair_launch(a, nullptr, 0, &need, nullptr) == FLUX_OK ? need : 0;
+}
+
+extern "C" int flux_linear_bf16_pair(const flux_linear_pair_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace)))) return fail(FLUX_E_NULL, "flux_linear_bf16_pair: workspace must be 16-byte aligned memory");
+    return linear_pair_launch(a, workspace, workspace_bytes, nullptr, static_cast<hipStream_t>(stream));
 }

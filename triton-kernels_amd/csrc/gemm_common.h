@@ -17,6 +17,8 @@ struct GemmParams {
     bf16_t* Y; bf16_t* Y2;
     const bf16_t* resid; const bf16_t* gate;
     int M, N, K;
+    int a_rows;          // A's rows come in batches of this many ...
+    int64_t a_skip;      // ... with this many elements beyond lda between two batches (0: evenly strided)
     int64_t lda, ldw, ldy, ldy2, ldresid, gate_stride;
     int split_n, y2_col0, rows_per_batch;
     int act, act_begin;
@@ -32,10 +34,18 @@ struct GemmParams {
     float qk_eps;
 };
 
-// One launch of a tiled kernel over the tile grid of a product.
+// One or two products of the same N and K (and the same epilogue form) that share a launch.
+struct GemmSet {
+    GemmParams p[2];
+    int n;
+};
+
+// One launch of a tiled kernel over the tile grid of a set: the tile rows of the second product follow
+// those of the first, so the tile orders below see one grid of tiles_m x tiles_n.
 struct GemmLaunch {
-    GemmParams p;
+    GemmParams p[2];
     int tiles_m, tiles_n, group_m;
+    int tiles_m0;               // tile rows of the first product
     int splits;                 // > 1: every tile's K range is cut into this many parts, each a workgroup of its own
     int slabs_per_split;
     float* partial;             // splits > 1: fp32 accumulators, [splits][tiles][4 waves][fragments][64 lanes][4]
@@ -75,7 +85,7 @@ __device__ __forceinline__ u32x2 pack4_bf16(float a, float b, float c, float d) 
 // resident on an XCD still share panels, and the q/k tiles of a patch the same rows of the rotation
 // table), and every XCD takes its eighth of the first followed by its eighth of the second.
 __device__ __forceinline__ bool tile_of_block_qk(const GemmLaunch& L, int bn, int& tm, int& tn) {
-    const int nq = L.p.qk_cols / bn;
+    const int nq = L.p[0].qk_cols / bn;
     const int Q = L.tiles_m * nq, R = L.tiles_m * (L.tiles_n - nq);
     const int per_xcd = gridDim.x / 8;
     const int x = blockIdx.x % 8, i = blockIdx.x / 8;
@@ -111,6 +121,21 @@ __device__ __forceinline__ bool tile_of_block(const GemmLaunch& L, int& tm, int&
     if (t >= L.tiles_m * L.tiles_n) return false;
     tile_at(L, t, tm, tn);
     return true;
+}
+
+// The product that tile row tm belongs to; tm becomes the row inside it. The index is uniform, so the fields
+// are scalar loads from the kernel arguments either way.
+__device__ __forceinline__ const GemmParams& product_of_tile(const GemmLaunch& L, int& tm) {
+    const int second = tm >= L.tiles_m0 ? 1 : 0;
+    tm -= second ? L.tiles_m0 : 0;
+    return L.p[second];
+}
+
+// Element offset of row m of A.
+__device__ __forceinline__ int64_t row_of_a(const GemmParams& p, int m) {
+    int64_t o = m * p.lda;
+    if (p.a_skip != 0) o += (static_cast<uint32_t>(m) / static_cast<uint32_t>(p.a_rows)) * p.a_skip;
+    return o;
 }
 
 // One buffer load of 64 x 16 bytes, written by the memory pipeline straight into LDS at dst
@@ -439,10 +464,13 @@ __device__ __forceinline__ void gemm_finish_rect(const GemmParams& p, f32x4 (&ac
     }
 }
 
-inline GemmLaunch make_launch(const GemmParams& p, int bm, int bn) {
+inline GemmLaunch make_launch(const GemmSet& g, int bm, int bn) {
     GemmLaunch L;
-    L.p = p;
-    L.tiles_m = (p.M + bm - 1) / bm;
+    const GemmParams& p = g.p[0];
+    L.p[0] = p;
+    L.p[1] = g.p[g.n - 1];
+    L.tiles_m0 = L.tiles_m = (p.M + bm - 1) / bm;
+    if (g.n > 1) L.tiles_m += (g.p[1].M + bm - 1) / bm;
     L.tiles_n = (p.N + bn - 1) / bn;
     L.group_m = 4;
     L.splits = 1;
@@ -453,6 +481,6 @@ inline GemmLaunch make_launch(const GemmParams& p, int bm, int bn) {
 inline unsigned grid_of(const GemmLaunch& L) { return static_cast<unsigned>((L.tiles_m * L.tiles_n * L.splits + 7) / 8 * 8); }
 
 // Eight-wave tiles (gemm_pair.hip). K range in `splits` parts, which then need `partial`.
-void launch_pair_tiles(int fm, int fn, const GemmParams& p, int splits, float* partial, hipStream_t st);
+void launch_pair_tiles(int fm, int fn, const GemmSet& g, int splits, float* partial, hipStream_t st);
 
 }  // namespace flux

@@ -37,9 +37,10 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
     const int lrow = w4 * 8 + (lane >> 3);
     const int lchunk = (lane & 7) ^ ((lrow >> 1) & 7);
     const int rows_a = min(p.M - m0, BM), rows_b = min(p.N - n0, BN);
-    bf16_t* const base_a = const_cast<bf16_t*>(p.A + static_cast<int64_t>(m0) * p.lda);
+    const int64_t a0 = row_of_a(p, m0);
+    bf16_t* const base_a = const_cast<bf16_t*>(p.A + a0);
     bf16_t* const base_b = const_cast<bf16_t*>(p.W + static_cast<int64_t>(n0) * p.ldw);
-    const int bytes_a = static_cast<int>(((rows_a - 1) * p.lda + p.K) * 2);
+    const int bytes_a = static_cast<int>((row_of_a(p, m0 + rows_a - 1) - a0 + p.K) * 2);
     const int bytes_b = static_cast<int>(((rows_b - 1) * p.ldw + p.K) * 2);
     uint32_t voff[NL];
 #pragma unroll
@@ -47,7 +48,7 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
         const int pass = 2 * j + G;
         if (pass < FM) {
             const int r = pass * 32 + lrow;
-            voff[j] = r < rows_a ? static_cast<uint32_t>((r * p.lda + lchunk * 8) * 2) : kOutOfRange;
+            voff[j] = r < rows_a ? static_cast<uint32_t>((row_of_a(p, m0 + r) - a0 + lchunk * 8) * 2) : kOutOfRange;
         } else {
             const int r = (pass - FM) * 32 + lrow;
             voff[j] = r < rows_b ? static_cast<uint32_t>((r * p.ldw + lchunk * 8) * 2) : kOutOfRange;
@@ -132,7 +133,6 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
     constexpr int R0 = (FM + 1) / 2, R1 = FM - R0;   // fragment rows that group 0 / group 1 finishes
     __shared__ __attribute__((aligned(1024))) char lds[ST * (BM + BN) * BK * 2];
     static_assert(4 * FM * FN * 1024 <= ST * (BM + BN) * BK * 2 && 2 * rect_epilogue_lds(FN) <= ST * (BM + BN) * BK * 2, "exchange and epilogue must fit the ring");
-    const GemmParams& p = L.p;
     int t = 0, split = 0, tm, tn;
     if constexpr (SPLIT) {   // the parts of a tile are `tiles` places apart in the sequence
         t = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
@@ -141,8 +141,9 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
         t -= split * (L.tiles_m * L.tiles_n);
         tile_at(L, t, tm, tn);
     } else {
-        if (FN == 8 && p.qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
+        if (FN == 8 && L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
     }
+    const GemmParams& p = product_of_tile(L, tm);
     const int m0 = tm * BM, n0 = tn * BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_reduce_kernel(GemmLaunch L)
     const int t = blockIdx.x / FM, row = blockIdx.x - t * FM;
     int tm, tn;
     tile_at(L, t, tm, tn);
-    const GemmParams& p = L.p;
+    const GemmParams& p = product_of_tile(L, tm);
     const int m0 = tm * BM, n0 = tn * BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -211,25 +212,26 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_reduce_kernel(GemmLaunch L)
 }
 
 template <int FM, int FN, int ST>
-static void launch_pair(const GemmParams& p, int splits, float* partial, hipStream_t st) {
-    GemmLaunch L = make_launch(p, 32 * FM, 32 * FN);
+static void launch_pair(const GemmSet& g, int splits, float* partial, hipStream_t st) {
+    const int K = g.p[0].K;
+    GemmLaunch L = make_launch(g, 32 * FM, 32 * FN);
     if (splits > 1) {   // (whole slabs only)
-        L.slabs_per_split = (p.K / 64 + splits - 1) / splits;
-        L.splits = (p.K / 64 + L.slabs_per_split - 1) / L.slabs_per_split;
+        L.slabs_per_split = (K / 64 + splits - 1) / splits;
+        L.splits = (K / 64 + L.slabs_per_split - 1) / L.slabs_per_split;
         L.partial = partial;
     }
     if (L.splits > 1) {
         hipLaunchKernelGGL((gemm_nt_pair_kernel<FM, FN, ST, false, true>), dim3(grid_of(L)), dim3(kPairThreads), 0, st, L);
         hipLaunchKernelGGL((gemm_reduce_kernel<FM, FN>), dim3((unsigned)(L.tiles_m * L.tiles_n * FM)), dim3(kGemmThreads), 0, st, L);
-    } else if (p.K % 64 == 0) {
+    } else if (K % 64 == 0) {
         hipLaunchKernelGGL((gemm_nt_pair_kernel<FM, FN, ST, false, false>), dim3(grid_of(L)), dim3(kPairThreads), 0, st, L);
     } else {
         hipLaunchKernelGGL((gemm_nt_pair_kernel<FM, FN, ST, true, false>), dim3(grid_of(L)), dim3(kPairThreads), 0, st, L);
     }
 }
 
-void launch_pair_tiles(int fm, int fn, const GemmParams& p, int splits, float* partial, hipStream_t st) {
-#define FLUX_PAIR(FM, FN, ST) if (fm == FM && fn == FN) return launch_pair<FM, FN, ST>(p, splits, partial, st)
+void launch_pair_tiles(int fm, int fn, const GemmSet& g, int splits, float* partial, hipStream_t st) {
+#define FLUX_PAIR(FM, FN, ST) if (fm == FM && fn == FN) return launch_pair<FM, FN, ST>(g, splits, partial, st)
     FLUX_PAIR(5, 6, 3); FLUX_PAIR(6, 6, 3); FLUX_PAIR(4, 6, 3); FLUX_PAIR(8, 4, 3); FLUX_PAIR(7, 4, 3); FLUX_PAIR(6, 4, 4);
     FLUX_PAIR(5, 4, 4); FLUX_PAIR(4, 4, 4); FLUX_PAIR(5, 3, 4); FLUX_PAIR(4, 3, 4); FLUX_PAIR(3, 3, 4); FLUX_PAIR(2, 3, 4);
     FLUX_PAIR(2, 2, 6); FLUX_PAIR(4, 8, 3);

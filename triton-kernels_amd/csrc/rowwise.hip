@@ -294,6 +294,22 @@ __global__ __launch_bounds__(kBlock) void rms_norm_bwd_block(
 // For bf16 storage the normalised value, (1+scale) and the product are each rounded to bf16 before
 // the next step, the evaluation order of functional/normalization.py:6-12 on bf16 tensors.
 // ------------------------------------------------------------------------------------------------
+// One or two tensors of the same width per launch (t[1]'s blocks follow the blocks0 of t[0]): the text
+// and the image rows of a double-stream block, whose text part is a few microseconds of work behind a
+// launch of its own.
+template <typename T>
+struct LnMod {
+    const T* x; const T* scale; const T* shift; T* y;
+    int64_t rows, seq, mod_stride;
+};
+template <typename T>
+struct LnModSet {
+    LnMod<T> t[2];
+    unsigned blocks0;
+    int n;
+    float eps;
+};
+
 // Straight-line: rows past the end and columns past n are clamped for the loads (x, scale and shift
 // vectors all go out before the first reduction) and masked in the sums; only the stores are
 // predicated. FULL = the row fills the lanes exactly (n == G * ITER * VEC), no column masks at all.
@@ -302,15 +318,23 @@ __global__ __launch_bounds__(kBlock) void rms_norm_bwd_block(
 // row needs all of both vectors; loaded and converted by each wave for itself (MODLDS = false, the
 // general form) that is as many loads as the row itself has and a fifth of the kernel's arithmetic.
 template <typename T, int G, int ITER, bool FULL, bool MODLDS>
-__global__ __launch_bounds__(kBlock) void ln_mod_fwd_regs(
-    const T* __restrict__ x, const T* __restrict__ scale, const T* __restrict__ shift, T* __restrict__ y,
-    int64_t rows, int64_t seq, int n, int64_t mod_stride, float eps) {
+__global__ __launch_bounds__(kBlock) void ln_mod_fwd_regs(LnModSet<T> set) {
+    const bool second = blockIdx.x >= set.blocks0;
+    const LnMod<T>& t = set.t[second];
+    const unsigned block = blockIdx.x - (second ? set.blocks0 : 0u);
+    const T* __restrict__ const x = t.x;
+    const T* __restrict__ const scale = t.scale;
+    const T* __restrict__ const shift = t.shift;
+    T* __restrict__ const y = t.y;
+    const int64_t rows = t.rows, seq = t.seq, mod_stride = t.mod_stride;
+    const int n = set.n;
+    const float eps = set.eps;
     constexpr int VEC = Elem<T>::VEC;
     constexpr int ROWS_PER_BLOCK = kBlock / G;
     constexpr int NMAX = MODLDS ? G * ITER * VEC : 1;
     __shared__ __attribute__((aligned(16))) float g_lds[NMAX], d_lds[NMAX];
     const int lane = threadIdx.x % G;
-    const int64_t row_raw = static_cast<int64_t>(blockIdx.x) * ROWS_PER_BLOCK + threadIdx.x / G;
+    const int64_t row_raw = static_cast<int64_t>(block) * ROWS_PER_BLOCK + threadIdx.x / G;
     const bool row_ok = row_raw < rows;
     const int64_t row = row_ok ? row_raw : rows - 1;
     const int64_t b = row / seq;
@@ -333,7 +357,7 @@ __global__ __launch_bounds__(kBlock) void ln_mod_fwd_regs(
     }
     if (MODLDS) {
         // the first row's batch element is every row's (the host checks that a block does not span two)
-        const int64_t b0 = (static_cast<int64_t>(blockIdx.x) * ROWS_PER_BLOCK) / seq;
+        const int64_t b0 = (static_cast<int64_t>(block) * ROWS_PER_BLOCK) / seq;
         for (int c = threadIdx.x * VEC; c < n; c += kBlock * VEC) {
             const Vec16<T> a = ld16(scale + b0 * mod_stride + c), d = ld16(shift + b0 * mod_stride + c);
 #pragma unroll
@@ -515,37 +539,50 @@ static int rms_bwd_launch(const void* dy, const void* x, const void* scale, cons
 }
 
 template <typename T>
-static int ln_mod_launch(const void* x, const void* scale, const void* shift, void* y, int64_t batch, int64_t seq, int n,
-                         int64_t mod_stride, float eps, hipStream_t st) {
+static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float eps, hipStream_t st) {
     constexpr int VEC = Elem<T>::VEC;
-    const int64_t rows = batch * seq;
-    const T* xp = static_cast<const T*>(x);
-    const T* scp = static_cast<const T*>(scale);
-    const T* shp = static_cast<const T*>(shift);
-    T* yp = static_cast<T*>(y);
-    RowPlan plan = plan_row(n, VEC);
-    const bool vec_ok = aligned16(x) && aligned16(y) && aligned16(scale) && aligned16(shift) && mod_stride % VEC == 0;
-    if (plan.G != 0 && vec_ok) {
+    const RowPlan plan = plan_row(n, VEC);
+    LnModSet<T> set;
+    set.n = n;
+    set.eps = eps;
+    int used = 0;
+    bool vec_ok = true;
+    for (int i = 0; i < count; ++i) {
+        if (a[i].batch * a[i].seq == 0) continue;
+        set.t[used++] = {static_cast<const T*>(a[i].x), static_cast<const T*>(a[i].scale), static_cast<const T*>(a[i].shift), static_cast<T*>(a[i].y),
+                         a[i].batch * a[i].seq, a[i].seq, a[i].mod_batch_stride};
+        vec_ok = vec_ok && aligned16(a[i].x) && aligned16(a[i].y) && aligned16(a[i].scale) && aligned16(a[i].shift) && a[i].mod_batch_stride % VEC == 0;
+    }
+    if (used == 0) return FLUX_OK;
+    if (plan.G == 0 || !vec_ok) {
+        for (int i = 0; i < used; ++i)
+            hipLaunchKernelGGL((ln_mod_fwd_block<T>), dim3((unsigned)set.t[i].rows), dim3(kBlock), 0, st, set.t[i].x, set.t[i].scale, set.t[i].shift,
+                               set.t[i].y, set.t[i].rows, set.t[i].seq, n, set.t[i].mod_stride, eps);
+        return check_launch("flux_layer_norm_modulation");
+    }
+    if (used == 1) set.t[1] = set.t[0];
 #define CALL(G_, I_)                                                                                        \
     do {                                                                                                    \
-        const dim3 grid_((unsigned)((rows + kBlock / G_ - 1) / (kBlock / G_)));                              \
+        constexpr int RPB_ = kBlock / G_;                                                                    \
         /* wave-per-row plans whose blocks stay inside one batch element stage the modulation vectors in LDS */ \
-        const bool lds_ = G_ == 64 && (batch == 1 || seq % (kBlock / G_) == 0);                             \
+        bool lds_ = G_ == 64;                                                                               \
+        unsigned grid_ = 0;                                                                                 \
+        for (int i = 0; i < used; ++i) {                                                                    \
+            lds_ = lds_ && (set.t[i].rows == set.t[i].seq || set.t[i].seq % RPB_ == 0);                      \
+            grid_ += (unsigned)((set.t[i].rows + RPB_ - 1) / RPB_);                                          \
+            if (i == 0) set.blocks0 = grid_;                                                                \
+        }                                                                                                   \
         if (n == G_ * I_ * VEC && lds_)                                                                     \
-            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, true, G_ == 64>), grid_, dim3(kBlock), 0, st, xp, scp, shp, yp, rows, seq, n, mod_stride, eps);  \
+            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, true, G_ == 64>), dim3(grid_), dim3(kBlock), 0, st, set);  \
         else if (n == G_ * I_ * VEC)                                                                        \
-            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, true, false>), grid_, dim3(kBlock), 0, st, xp, scp, shp, yp, rows, seq, n, mod_stride, eps);  \
+            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, true, false>), dim3(grid_), dim3(kBlock), 0, st, set);     \
         else if (lds_)                                                                                      \
-            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, false, G_ == 64>), grid_, dim3(kBlock), 0, st, xp, scp, shp, yp, rows, seq, n, mod_stride, eps); \
+            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, false, G_ == 64>), dim3(grid_), dim3(kBlock), 0, st, set); \
         else                                                                                                \
-            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, false, false>), grid_, dim3(kBlock), 0, st, xp, scp, shp, yp, rows, seq, n, mod_stride, eps); \
+            hipLaunchKernelGGL((ln_mod_fwd_regs<T, G_, I_, false, false>), dim3(grid_), dim3(kBlock), 0, st, set);    \
     } while (0)
-        FLUX_DISPATCH_GI(plan, CALL);
+    FLUX_DISPATCH_GI(plan, CALL);
 #undef CALL
-    } else {
-        hipLaunchKernelGGL((ln_mod_fwd_block<T>), dim3((unsigned)rows), dim3(kBlock), 0, st, xp, scp, shp, yp, rows, seq, n,
-                           mod_stride, eps);
-    }
     return check_launch("flux_layer_norm_modulation");
 }
 
@@ -583,16 +620,32 @@ extern "C" int flux_rms_norm_bwd(const void* dy, const void* x, const void* scal
     return fail(FLUX_E_DTYPE, "flux_rms_norm_bwd: unsupported dtype pair (%d,%d)", x_dtype, scale_dtype);
 }
 
+static int ln_mod_checked(const flux_layer_norm_args* a, int count, int32_t n, int32_t dtype, float eps, void* stream) {
+    int64_t rows = 0;
+    for (int i = 0; i < count; ++i) {
+        if (!a[i].x || !a[i].scale || !a[i].shift || !a[i].y) return fail(FLUX_E_NULL, "flux_layer_norm_modulation: null pointer");
+        if (a[i].batch < 0 || a[i].seq < 0 || n <= 0) return fail(FLUX_E_SHAPE, "flux_layer_norm_modulation: bad shape [%lld,%lld,%d]", (long long)a[i].batch, (long long)a[i].seq, n);
+        rows += a[i].batch * a[i].seq;
+    }
+    if (n > FLUX_MAX_ROW) return fail(FLUX_E_TOO_WIDE, "flux_layer_norm_modulation: n = %d exceeds the maximum row length %d", n, FLUX_MAX_ROW);
+    if (rows == 0) return FLUX_OK;
+    if (rows > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_layer_norm_modulation: too many rows");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (dtype == FLUX_BF16) return ln_mod_launch<bf16_t>(a, count, n, eps, st);
+    if (dtype == FLUX_F32) return ln_mod_launch<float>(a, count, n, eps, st);
+    return fail(FLUX_E_DTYPE, "flux_layer_norm_modulation: unsupported dtype %d", dtype);
+}
+
 extern "C" int flux_layer_norm_modulation(const void* x, const void* scale, const void* shift, void* y, int64_t batch,
                                           int64_t seq, int32_t n, int64_t mod_batch_stride, int32_t dtype, float eps,
                                           void* stream) {
-    if (!x || !scale || !shift || !y) return fail(FLUX_E_NULL, "flux_layer_norm_modulation: null pointer");
-    if (batch < 0 || seq < 0 || n <= 0) return fail(FLUX_E_SHAPE, "flux_layer_norm_modulation: bad shape [%lld,%lld,%d]", (long long)batch, (long long)seq, n);
-    if (n > FLUX_MAX_ROW) return fail(FLUX_E_TOO_WIDE, "flux_layer_norm_modulation: n = %d exceeds the maximum row length %d", n, FLUX_MAX_ROW);
-    if (batch * seq == 0) return FLUX_OK;
-    if (batch * seq > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_layer_norm_modulation: too many rows");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (dtype == FLUX_BF16) return ln_mod_launch<bf16_t>(x, scale, shift, y, batch, seq, n, mod_batch_stride, eps, st);
-    if (dtype == FLUX_F32) return ln_mod_launch<float>(x, scale, shift, y, batch, seq, n, mod_batch_stride, eps, st);
-    return fail(FLUX_E_DTYPE, "flux_layer_norm_modulation: unsupported dtype %d", dtype);
+    const flux_layer_norm_args a = {x, scale, shift, y, batch, seq, mod_batch_stride};
+    return ln_mod_checked(&a, 1, n, dtype, eps, stream);
+}
+
+extern "C" int flux_layer_norm_modulation_pair(const flux_layer_norm_args* first, const flux_layer_norm_args* second, int32_t n,
+                                               int32_t dtype, float eps, void* stream) {
+    if (!first || !second) return fail(FLUX_E_NULL, "flux_layer_norm_modulation_pair: null args");
+    const flux_layer_norm_args a[2] = {*first, *second};
+    return ln_mod_checked(a, 2, n, dtype, eps, stream);
 }

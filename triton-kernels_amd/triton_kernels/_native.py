@@ -66,6 +66,17 @@ class LinearArgs(Structure):
     ]
 
 
+class LinearPairArgs(Structure):
+    _fields_ = [("product", LinearArgs * 2), ("a_rows", c_int64 * 2), ("a_batch_stride", c_int64 * 2)]
+
+
+class LayerNormArgs(Structure):
+    _fields_ = [
+        ("x", c_void_p), ("scale", c_void_p), ("shift", c_void_p), ("y", c_void_p),
+        ("batch", c_int64), ("seq", c_int64), ("mod_batch_stride", c_int64),
+    ]
+
+
 class AttnArgs(Structure):
     _fields_ = [
         ("q", Src4), ("k", Src4), ("v", Src4),
@@ -86,10 +97,13 @@ SIGNATURES = {
                                     c_int32, c_int32, c_void_p]),
     "flux_layer_norm_modulation": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32,
                                              c_int64, c_int32, c_float, c_void_p]),
+    "flux_layer_norm_modulation_pair": (c_int32, [POINTER(LayerNormArgs), POINTER(LayerNormArgs), c_int32, c_int32, c_float, c_void_p]),
     "flux_qkv_prep": (c_int32, [POINTER(QkvPrepArgs), c_void_p]),
     "flux_linear_bf16": (c_int32, [POINTER(LinearArgs), c_void_p]),
     "flux_linear_workspace_bytes": (c_int64, [POINTER(LinearArgs)]),
     "flux_linear_bf16_ws": (c_int32, [POINTER(LinearArgs), c_void_p, c_int64, c_void_p]),
+    "flux_linear_pair_workspace_bytes": (c_int64, [POINTER(LinearPairArgs)]),
+    "flux_linear_bf16_pair": (c_int32, [POINTER(LinearPairArgs), c_void_p, c_int64, c_void_p]),
     "flux_attention_fwd_bf16": (c_int32, [POINTER(AttnArgs), c_void_p]),
     "flux_silu": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
     "flux_gelu_tanh": (c_int32, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int32, c_void_p]),
@@ -207,6 +221,6 @@ def src4(t: torch.Tensor | None) -> Src4:
 
 __all__ = [
     "lib", "lib_path", "check", "last_error", "dtype_code", "require_gpu", "stream_ptr", "on_device", "ptr", "src4",
-    "Src4", "QkvPrepArgs", "LinearArgs", "AttnArgs", "SIGNATURES", "byref",
+    "Src4", "QkvPrepArgs", "LinearArgs", "LinearPairArgs", "LayerNormArgs", "AttnArgs", "SIGNATURES", "byref",
     "FLUX_BF16", "FLUX_F32", "ACT_NONE", "ACT_GELU_TANH", "ACT_SILU", "LINEAR_SHARED_GPU", "MAX_ROW",
 ]

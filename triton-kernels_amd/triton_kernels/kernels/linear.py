@@ -55,20 +55,67 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
             that leaves CUs free in its last round instead of one that fills the GPU exactly (same
             result, only the schedule differs)
     """
+    a = nv.LinearArgs()
+    out, _keep = _fill_args(a, x, w, b, activation=activation, act_begin=act_begin, out=out, out2=out2, split=split, resid=resid,
+                            gate=gate, qk=qk, in_activation=in_activation, shared_gpu=shared_gpu)
+    dev = out.device
+    with nv.on_device(dev):
+        need = nv.lib().flux_linear_workspace_bytes(nv.byref(a))
+        if need:   # K cut over several workgroups: partial sums in memory of this launch's stream
+            ws = torch.empty((need,), dtype=torch.uint8, device=dev)
+            rc = nv.lib().flux_linear_bf16_ws(nv.byref(a), ws.data_ptr(), need, nv.stream_ptr(dev))
+        else:
+            rc = nv.lib().flux_linear_bf16(nv.byref(a), nv.stream_ptr(dev))
+    nv.check(rc, "flux_linear_bf16")
+    return out
+
+
+def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
+    """Two linear_into calls (each the keyword arguments of one, `x`, `w` and `b` among them) in one library
+    call: products of the same N, K and form of epilogue share a launch. An x of [B, L, K] may be a slice of
+    a longer sequence, whose batch elements are not evenly strided rows."""
+    args = nv.LinearPairArgs()
+    outs, keep = [], []
+    for i, call in enumerate((first, second)):
+        x = call["x"]
+        if x.dim() == 3 and x.shape[0] > 1 and x.stride(0) != x.shape[1] * x.stride(1):
+            B, L, K = x.shape
+            if B * L > 8 and x.stride(2) == 1 and x.stride(1) >= K and x.stride(0) % 8 == 0 and x.stride(0) >= L * x.stride(1) \
+                    and x.stride(1) % 8 == 0 and K % 8 == 0 and x.data_ptr() % 16 == 0 and call["w"].data_ptr() % 16 == 0 \
+                    and call["w"].is_contiguous() and B * x.stride(0) * 2 < 2**31:
+                args.a_rows[i], args.a_batch_stride[i] = L, x.stride(0)
+        out, kept = _fill_args(args.product[i], batches=bool(args.a_rows[i]), **call)
+        outs.append(out)
+        keep.append(kept)
+    dev = outs[0].device
+    nv.require_gpu(*outs)
+    with nv.on_device(dev):
+        need = nv.lib().flux_linear_pair_workspace_bytes(nv.byref(args))
+        ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None
+        rc = nv.lib().flux_linear_bf16_pair(nv.byref(args), nv.ptr(ws), need, nv.stream_ptr(dev))
+    nv.check(rc, "flux_linear_bf16_pair")
+    return outs[0], outs[1]
+
+
+def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "", act_begin: int = 0,
+               out: Tensor | None = None, out2: Tensor | None = None, split: int | None = None, resid: Tensor | None = None,
+               gate: Tensor | None = None, qk: dict | None = None, in_activation: str = "", shared_gpu: bool = False,
+               batches: bool = False):
+    """Checks one call and writes it into `a`; returns the output and what has to live until the launch.
+    batches: x is [B, L, K] with evenly strided rows inside a batch element only."""
     assert x.shape[-1] == w.shape[-1], "Incompatible dimensions"
     assert x.dtype == w.dtype, "Incompatible dtypes"
     _PLANS[x.dtype]  # KeyError for anything but bfloat16, as in the reference
     act = _ACTIVATIONS[activation]
     dev = nv.require_gpu(x, w, b, out, out2, resid, gate)
     N, K = w.shape
-    x2 = _rows_2d(x, K)
-    M = x2.shape[0]
+    x2 = x[0] if batches else _rows_2d(x, K)
+    M = x.numel() // K if batches else x2.shape[0]
     if w.stride(1) != 1 or (N > 1 and w.stride(0) < K):
         w = w.contiguous()
     if b is not None:
         assert b.shape[-1] == N
         b = b.to(x.dtype).contiguous()
-    a = nv.LinearArgs()
     a.A, a.W, a.bias = x2.data_ptr(), w.data_ptr(), nv.ptr(b)
     a.M, a.N, a.K = M, N, K
     a.lda = x2.stride(0) if M > 1 else K
@@ -84,6 +131,7 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
     else:
         assert out.shape[1] >= N
         a.Y2, a.split_n = None, N
+    keep = [x2, w, b]
     if gate is not None:
         assert resid is not None
         r2 = resid.reshape(-1, N)
@@ -95,13 +143,13 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
             g2 = g2.contiguous()
         nb = g2.shape[0]
         assert M % nb == 0
+        keep += [r2, g2]
         a.resid, a.ldresid = r2.data_ptr(), r2.stride(0)
         a.gate, a.gate_batch_stride, a.rows_per_batch = g2.data_ptr(), (g2.stride(0) if nb > 1 else N), M // nb
     a.act, a.act_begin = act, act_begin
     a.flags = nv.LINEAR_SHARED_GPU if shared_gpu else 0
     a.in_act = {"": nv.ACT_NONE, "SiLU": nv.ACT_SILU}[in_activation]
     assert a.in_act == nv.ACT_NONE or M <= 8, "the input activation is fused for at most 8 rows"
-    keep = None
     if qk is not None:
         f = nv.LinearQKFusion()
         q_out, k_out, pe = qk["q_out"], qk["k_out"], qk["pe"]
@@ -117,21 +165,12 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
         f.heads, f.seq_len, f.out_len, f.pos0 = heads, seq_len, out_len, int(qk.get("pos0", 0))
         f.eps = float(qk.get("eps", 1e-6))
         a.qk = ctypes.pointer(f)
-        keep = (f, qs, ks, pe2)
+        keep += [f, qs, ks, pe2]
     if launch_hook is not None:
         parts = [activation and f"{activation}>={act_begin}", split is not None and f"split@{split}", gate is not None and "gated-residual",
                  qk is not None and "qk-norm-rope", in_activation and f"in:{in_activation}"]
         launch_hook(linear_launch_metadata(M, N, K, x.element_size(), "+".join(p for p in parts if p)))
-    with nv.on_device(dev):
-        need = nv.lib().flux_linear_workspace_bytes(nv.byref(a))
-        if need:   # K cut over several workgroups: partial sums in memory of this launch's stream
-            ws = torch.empty((need,), dtype=torch.uint8, device=dev)
-            rc = nv.lib().flux_linear_bf16_ws(nv.byref(a), ws.data_ptr(), need, nv.stream_ptr(dev))
-        else:
-            rc = nv.lib().flux_linear_bf16(nv.byref(a), nv.stream_ptr(dev))
-    nv.check(rc, "flux_linear_bf16")
-    del keep
-    return out
+    return out, keep
 
 
 def qk_fusable(x: Tensor, w: Tensor, seq_len: int, head_dim: int) -> bool:

@@ -90,9 +90,32 @@ rms_norm = _rms_norm.apply
 def layer_norm_modulation(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps=1e-5) -> torch.Tensor:
     """(1 + weight) * layer_norm(x) + bias, where weight is the adaLN *scale* and bias the *shift*,
     each [B, 1, N] (or [B, N]); chunks of a wider modulation tensor are read in place."""
+    a, y, _keep = _layer_norm_args(x, weight, bias)
+    dev = y.device
+    with nv.on_device(dev):
+        rc = nv.lib().flux_layer_norm_modulation(
+            a.x, a.scale, a.shift, a.y, a.batch, a.seq, y.shape[-1], a.mod_batch_stride, nv.dtype_code(y), float(eps), nv.stream_ptr(dev))
+    nv.check(rc, "flux_layer_norm_modulation")
+    return y
+
+
+def layer_norm_modulation_pair(first: tuple, second: tuple, eps=1e-5) -> tuple[torch.Tensor, torch.Tensor]:
+    """layer_norm_modulation of two (x, weight, bias) triples of the same width and type in one launch."""
+    a0, y0, _keep0 = _layer_norm_args(*first)
+    a1, y1, _keep1 = _layer_norm_args(*second)
+    assert y0.shape[-1] == y1.shape[-1] and y0.dtype == y1.dtype and y0.device == y1.device
+    dev = y0.device
+    with nv.on_device(dev):
+        rc = nv.lib().flux_layer_norm_modulation_pair(nv.byref(a0), nv.byref(a1), y0.shape[-1], nv.dtype_code(y0), float(eps), nv.stream_ptr(dev))
+    nv.check(rc, "flux_layer_norm_modulation_pair")
+    return y0, y1
+
+
+def _layer_norm_args(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor):
+    """The call's arguments, its output and the tensors that have to live until it is launched."""
     assert x.shape[0] == weight.shape[0] == bias.shape[0]
     assert x.shape[-1] == weight.shape[-1] == bias.shape[-1]
-    dev = nv.require_gpu(x, weight, bias)
+    nv.require_gpu(x, weight, bias)
     batch, n = x.shape[0], x.shape[-1]
     calculate_settings(n)
     x = x.contiguous()
@@ -110,9 +133,5 @@ def layer_norm_modulation(x: torch.Tensor, weight: torch.Tensor, bias: torch.Ten
         mod_stride = weight.stride(0)
     y = torch.empty_like(x)
     rows = x.numel() // n
-    with nv.on_device(dev):
-        rc = nv.lib().flux_layer_norm_modulation(
-            x.data_ptr(), weight.data_ptr(), bias.data_ptr(), y.data_ptr(),
-            batch, rows // batch if batch else 0, n, mod_stride, nv.dtype_code(x), float(eps), nv.stream_ptr(dev))
-    nv.check(rc, "flux_layer_norm_modulation")
-    return y
+    a = nv.LayerNormArgs(x.data_ptr(), weight.data_ptr(), bias.data_ptr(), y.data_ptr(), batch, rows // batch if batch else 0, mod_stride)
+    return a, y, (x, weight, bias)

@@ -22,11 +22,12 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 from torch import Tensor
+from torch.nn.modules.module import _has_any_global_hook
 
 from triton_kernels import _native as nv
 from triton_kernels.kernels.attention import attention_into, scaled_dot_product_attention
-from triton_kernels.kernels.linear import linear, linear_into, qk_fusable
-from triton_kernels.kernels.normalization import layer_norm_modulation
+from triton_kernels.kernels.linear import linear, linear_into, linear_pair_into, qk_fusable
+from triton_kernels.kernels.normalization import layer_norm_modulation, layer_norm_modulation_pair
 from triton_kernels.kernels.positional_embedding import apply_rope, qkv_prep
 from triton_kernels.modules.normalization import QKNorm
 
@@ -132,12 +133,17 @@ class Modulation(nn.Module):
         self.lin = Linear(dim, self.multiplier * dim, bias=True)
 
     def forward(self, vec: Tensor) -> tuple[ModulationOut, ModulationOut | None]:
-        rows = vec.numel() // vec.shape[-1]
-        if self.fused_silu and vec.is_cuda and vec.dtype == torch.bfloat16 and rows <= 8:
+        if self.takes_fused_silu(vec):
             # one launch: the row-vector kernel applies SiLU to vec as it reads it
             out = linear_into(vec, self.lin.weight, self.lin.bias, in_activation="SiLU").reshape(*vec.shape[:-1], -1)
         else:
             out = self.lin(_silu(vec))
+        return self.chunks(out)
+
+    def takes_fused_silu(self, vec: Tensor) -> bool:
+        return self.fused_silu and vec.is_cuda and vec.dtype == torch.bfloat16 and vec.numel() // vec.shape[-1] <= 8
+
+    def chunks(self, out: Tensor) -> tuple[ModulationOut, ModulationOut | None]:
         chunks = out[:, None, :].chunk(self.multiplier, dim=-1)
         first = ModulationOut(*chunks[:3])
         return first, (ModulationOut(*chunks[3:]) if self.is_double else None)
@@ -150,6 +156,11 @@ def MLP(hidden_size: int, mlp_hidden_dim: int, bias: bool = True):
         nn.Identity(),
         Linear(mlp_hidden_dim, hidden_size, bias=bias),
     )
+
+
+def _plain(module: nn.Module, cls: type) -> bool:
+    """Whether calling `module` does what `cls` does and nothing else, so that its weights may be used directly."""
+    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks or _has_any_global_hook())
 
 
 def _fusable(*tensors: Tensor) -> bool:
@@ -257,32 +268,16 @@ class DoubleStreamBlock(nn.Module):
         self.txt_attn = SelfAttention(dim=hidden_size, num_heads=num_heads, qkv_bias=qkv_bias)
         self.txt_mlp = MLP(hidden_size, mlp_hidden_dim)
 
-    # The txt stream is a ninth of the img stream's work: its small GEMMs (96 tiles of 128 x 128)
-    # leave most CUs idle when they run alone, so the fused path runs the txt chain on a second HIP
-    # stream of default priority, next to the img chain, and joins the two around the joint attention.
+    # Kept for callers that set it. The text and the image products of a fused block share their launches,
+    # so there is no second stream to switch on or off.
     two_streams = True
-
-    def _side_stream(self, dev: torch.device) -> "torch.cuda.Stream":
-        """This block's second stream on `dev`. Each instance keeps its own (per device), so two blocks
-        driven from different host threads or streams never order their txt chains behind each
-        other; setdefault makes the lazy creation safe when one instance is called from two threads."""
-        streams = self.__dict__.setdefault("_side_streams", {})
-        st = streams.get(dev.index)
-        if st is None:
-            st = streams.setdefault(dev.index, torch.cuda.Stream(device=dev))
-        return st
-
-    def __getstate__(self):
-        state = self.__dict__.copy()
-        state.pop("_side_streams", None)   # streams are neither copied nor pickled with the block
-        return state
 
     def forward(self, img: Tensor, txt: Tensor, vec: Tensor, pe: Tensor) -> tuple[Tensor, Tensor]:
         H = self.num_heads
         Lt = txt.shape[1]
         fused = self.fused and _fusable(img, txt, self.img_attn.qkv.weight, self.img_attn.norm.query_norm.scale)
-        if fused and self.two_streams and not torch.is_grad_enabled():
-            return self._forward_two_streams(img, txt, vec, pe)
+        if fused:
+            return self._forward_fused(img, txt, vec, pe)
 
         img_mod1, img_mod2 = self.img_mod(vec)
         txt_mod1, txt_mod2 = self.txt_mod(vec)
@@ -290,89 +285,63 @@ class DoubleStreamBlock(nn.Module):
         txt_qkv = self.txt_attn.qkv(layer_norm_modulation(txt, txt_mod1.scale, txt_mod1.shift))
         img_q, img_k, img_v = _heads(img_qkv, H)
         txt_q, txt_k, txt_v = _heads(txt_qkv, H)
-
-        if fused:
-            B, Li, hid = img.shape
-            q, k, v = qkv_prep(img_q, img_k, img_v, txt_q, txt_k, txt_v, pe=pe,
-                               q_scale_img=self.img_attn.norm.query_norm.scale, k_scale_img=self.img_attn.norm.key_norm.scale,
-                               q_scale_txt=self.txt_attn.norm.query_norm.scale, k_scale_txt=self.txt_attn.norm.key_norm.scale)
-            attn = torch.empty((B, Lt + Li, hid), dtype=img.dtype, device=img.device)
-            attention_into(q, k, v, attn.view(B, Lt + Li, H, hid // H).permute(0, 2, 1, 3))
-        else:
-            img_q, img_k = self.img_attn.norm(img_q, img_k, img_v)
-            txt_q, txt_k = self.txt_attn.norm(txt_q, txt_k, txt_v)
-            q, k, v = qkv_prep(img_q, img_k, img_v, txt_q, txt_k, txt_v)   # torch.cat(dim=2) of the three pairs
-            attn = attention(q, k, v, pe=pe)
-        txt_attn, img_attn = attn[:, :Lt], attn[:, Lt:]
-
-        img = self._stream_tail(img, img_attn, img_mod1, img_mod2, self.img_attn.proj, self.img_mlp, fused)
-        txt = self._stream_tail(txt, txt_attn, txt_mod1, txt_mod2, self.txt_attn.proj, self.txt_mlp, fused)
+        img_q, img_k = self.img_attn.norm(img_q, img_k, img_v)
+        txt_q, txt_k = self.txt_attn.norm(txt_q, txt_k, txt_v)
+        q, k, v = qkv_prep(img_q, img_k, img_v, txt_q, txt_k, txt_v)   # torch.cat(dim=2) of the three pairs
+        attn = attention(q, k, v, pe=pe)
+        img = self._stream_tail(img, attn[:, Lt:], img_mod1, img_mod2, self.img_attn.proj, self.img_mlp)
+        txt = self._stream_tail(txt, attn[:, :Lt], txt_mod1, txt_mod2, self.txt_attn.proj, self.txt_mlp)
         return img, txt
 
-    def _forward_two_streams(self, img: Tensor, txt: Tensor, vec: Tensor, pe: Tensor) -> tuple[Tensor, Tensor]:
-        """Same arithmetic as the fused path of forward(), txt chain on a side stream. Everything the
-        main stream reads later is allocated on the main stream (the caching allocator ties a block
-        to the stream it was allocated on); temporaries of the side chain live and die on the side
-        stream."""
+    def _forward_fused(self, img: Tensor, txt: Tensor, vec: Tensor, pe: Tensor) -> tuple[Tensor, Tensor]:
+        """The text rows are a small part of the work (a ninth at 4096 + 512 tokens, a fifth at 1024 + 256):
+        by themselves their products leave most CUs idle or walk K one slab after the other, and every launch
+        of theirs costs the host as much as one of the image's. So every step takes both in one launch: the
+        weights of the same shape, two row ranges. Block passes with the text chain on a second stream ->
+        with shared launches: 1133 -> 1121 us at 4096 + 512 tokens, 567 -> 371 us at 1024 + 256 (19 launches
+        and five stream joins kept the host busy for longer than the GPU; now ten launches)."""
         H = self.num_heads
         B, Li, hid = img.shape
         Lt = txt.shape[1]
-        dev = img.device
-        main = torch.cuda.current_stream(dev)
-        side = self._side_stream(dev)
-        txt_qkv = torch.empty((B * Lt, 3 * hid), dtype=txt.dtype, device=dev)
-        txt_out = torch.empty((B, Lt, hid), dtype=txt.dtype, device=dev)
-        attn = torch.empty((B, Lt + Li, hid), dtype=img.dtype, device=dev)
-
-        side.wait_stream(main)            # inputs are ready on the main stream
-        with torch.cuda.stream(side):
-            txt_mod1, txt_mod2 = self.txt_mod(vec)
-            qkv_lin = self.txt_attn.qkv
-            linear_into(layer_norm_modulation(txt, txt_mod1.scale, txt_mod1.shift), qkv_lin.weight, qkv_lin.bias, out=txt_qkv,
-                        shared_gpu=True)
-        img_mod1, img_mod2 = self.img_mod(vec)
-        img_qkv = self.img_attn.qkv(layer_norm_modulation(img, img_mod1.scale, img_mod1.shift))
-        main.wait_stream(side)            # txt_qkv is complete
-
-        img_q, img_k, img_v = _heads(img_qkv, H)
+        img, txt = img.contiguous(), txt.contiguous()
+        img_mod1, img_mod2, txt_mod1, txt_mod2 = self._modulations(vec)
+        img_qkv_lin, txt_qkv_lin = self.img_attn.qkv, self.txt_attn.qkv
+        img_m, txt_m = layer_norm_modulation_pair((img, img_mod1.scale, img_mod1.shift), (txt, txt_mod1.scale, txt_mod1.shift))
+        if _plain(img_qkv_lin, Linear) and _plain(txt_qkv_lin, Linear):
+            img_qkv, txt_qkv = linear_pair_into(dict(x=img_m, w=img_qkv_lin.weight, b=img_qkv_lin.bias),
+                                                dict(x=txt_m, w=txt_qkv_lin.weight, b=txt_qkv_lin.bias))
+        else:
+            img_qkv, txt_qkv = img_qkv_lin(img_m), txt_qkv_lin(txt_m)
+        img_q, img_k, img_v = _heads(img_qkv.view(B, Li, 3 * hid), H)
         txt_q, txt_k, txt_v = _heads(txt_qkv.view(B, Lt, 3 * hid), H)
         q, k, v = qkv_prep(img_q, img_k, img_v, txt_q, txt_k, txt_v, pe=pe,
                            q_scale_img=self.img_attn.norm.query_norm.scale, k_scale_img=self.img_attn.norm.key_norm.scale,
                            q_scale_txt=self.txt_attn.norm.query_norm.scale, k_scale_txt=self.txt_attn.norm.key_norm.scale)
+        attn = torch.empty((B, Lt + Li, hid), dtype=img.dtype, device=img.device)
         attention_into(q, k, v, attn.view(B, Lt + Li, H, hid // H).permute(0, 2, 1, 3))
-        txt_attn, img_attn = attn[:, :Lt], attn[:, Lt:]
 
-        side.wait_stream(main)            # attention output is complete
-        with torch.cuda.stream(side):
-            self._stream_tail(txt, txt_attn, txt_mod1, txt_mod2, self.txt_attn.proj, self.txt_mlp, True, out=txt_out, side_chain=True)
-        img = self._stream_tail(img, img_attn, img_mod1, img_mod2, self.img_attn.proj, self.img_mlp, True, beside_txt=True)
-        main.wait_stream(side)
-        # tensors made on the side stream that the caller's stream may still be reading when they die
-        for t in (txt_mod1.shift, txt_mod1.scale, txt_mod1.gate, txt_mod2.shift, txt_mod2.scale, txt_mod2.gate):
-            t.record_stream(main)
-        return img, txt_out
+        def gated(x, lin, resid, gate):
+            return dict(x=x, w=lin.weight, b=lin.bias, resid=resid, gate=gate)
+
+        img_1, txt_1 = linear_pair_into(gated(attn[:, Lt:], self.img_attn.proj, img, img_mod1.gate),
+                                        gated(attn[:, :Lt], self.txt_attn.proj, txt, txt_mod1.gate))
+        img_1, txt_1 = img_1.view(B, Li, hid), txt_1.view(B, Lt, hid)
+        img_m, txt_m = layer_norm_modulation_pair((img_1, img_mod2.scale, img_mod2.shift), (txt_1, txt_mod2.scale, txt_mod2.shift))
+        img_h, txt_h = linear_pair_into(dict(x=img_m, w=self.img_mlp[0].weight, b=self.img_mlp[0].bias, activation="GELU"),
+                                        dict(x=txt_m, w=self.txt_mlp[0].weight, b=self.txt_mlp[0].bias, activation="GELU"))
+        img_2, txt_2 = linear_pair_into(gated(img_h, self.img_mlp[2], img_1, img_mod2.gate),
+                                        gated(txt_h, self.txt_mlp[2], txt_1, txt_mod2.gate))
+        return img_2.view(B, Li, hid), txt_2.view(B, Lt, hid)
+
+    def _modulations(self, vec: Tensor):
+        mods = (self.img_mod, self.txt_mod)
+        if not (all(_plain(m, Modulation) and m.takes_fused_silu(vec) for m in mods) and mods[0].multiplier == mods[1].multiplier):
+            return (*self.img_mod(vec), *self.txt_mod(vec))
+        outs = linear_pair_into(*(dict(x=vec, w=m.lin.weight, b=m.lin.bias, in_activation="SiLU") for m in mods))
+        pairs = [m.chunks(o.reshape(*vec.shape[:-1], -1)) for m, o in zip(mods, outs)]
+        return (*pairs[0], *pairs[1])
 
     @staticmethod
-    def _stream_tail(x: Tensor, attn: Tensor, mod1: ModulationOut, mod2: ModulationOut, proj: Linear, mlp: nn.Sequential,
-                     fused: bool, out: Tensor | None = None, beside_txt: bool = False, side_chain: bool = False) -> Tensor:
-        if not fused:
-            x = _gated_residual(x, mod1.gate, proj(attn))
-            return _gated_residual(x, mod2.gate, mlp(layer_norm_modulation(x, mod2.scale, mod2.shift)))
-        B, L, hid = x.shape
-        M = B * L
-        x = x.contiguous()
-        x1 = torch.empty_like(x)
-        # attn is a slice of the [B, Lt+Li, hid] buffer: rows of one batch element are evenly strided,
-        # batches are not, so flatten per call only when there is a single batch element.
-        a2 = attn.reshape(M, hid) if B > 1 else attn[0]
-        # beside_txt: the txt chain's projection runs on the other stream at the same time and lives on the
-        # CUs this launch leaves free (192 tiles at 4096 rows); a tile shape that fills all 256 CUs would
-        # push it behind. By the time of the last projection the txt chain has finished: measured at
-        # 4096 + 512 tokens, 1.18 ms like this, 1.23 ms with the flag on every launch or on none.
-        # side_chain: this is the txt chain on the side stream; its small launches keep few, larger workgroups
-        # instead of spreading over every CU the img chain is using (1.25 against 1.30 ms).
-        linear_into(a2, proj.weight, proj.bias, out=x1.view(M, hid), resid=x.view(M, hid), gate=mod1.gate, shared_gpu=beside_txt or side_chain)
-        h = linear(layer_norm_modulation(x1, mod2.scale, mod2.shift), mlp[0].weight, mlp[0].bias, activation="GELU", shared_gpu=side_chain)
-        x2 = torch.empty_like(x) if out is None else out
-        linear_into(h, mlp[2].weight, mlp[2].bias, out=x2.view(M, hid), resid=x1.view(M, hid), gate=mod2.gate, shared_gpu=side_chain)
-        return x2
+    def _stream_tail(x: Tensor, attn: Tensor, mod1: ModulationOut, mod2: ModulationOut, proj: Linear, mlp: nn.Sequential) -> Tensor:
+        x = _gated_residual(x, mod1.gate, proj(attn))
+        return _gated_residual(x, mod2.gate, mlp(layer_norm_modulation(x, mod2.scale, mod2.shift)))

@@ -67,6 +67,14 @@ int flux_rms_norm_bwd(const void* dy, const void* x, const void* scale, const fl
                       void* dx, float* dscale, int64_t rows, int32_t n,
                       int32_t x_dtype, int32_t scale_dtype, void* stream);
 
+/* The same with a workspace of flux_rms_norm_bwd_workspace_bytes bytes of device memory: dscale[n] is
+ * written, not added to, in dscale_dtype, its sums formed in fp32 in a fixed order and rounded once.
+ * Neither dscale nor the workspace needs to be cleared. rows == 0 writes zeros. */
+int64_t flux_rms_norm_bwd_workspace_bytes(int64_t rows, int32_t n, int32_t x_dtype);
+int flux_rms_norm_bwd_ws(const void* dy, const void* x, const void* scale, const float* rstd,
+                         void* dx, void* dscale, int32_t dscale_dtype, void* ws, int64_t ws_bytes,
+                         int64_t rows, int32_t n, int32_t x_dtype, int32_t scale_dtype, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * LayerNorm (no affine) + adaLN modulation.   y = (1 + scale[b]) * LN(x[b,l,:]) + shift[b]
  * Replaces layer_norm_modulation / _layer_norm_modulation_fwd (kernels/normalization.py:47-77,

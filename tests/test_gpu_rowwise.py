@@ -11,6 +11,7 @@ import torch
 
 import triton_kernels as tk
 from oracle import flux_oracle as oracle
+from triton_kernels import _native as nv
 from triton_kernels import testing as cfg
 from util import DEV, randn, seeded
 
@@ -81,6 +82,41 @@ def test_rms_norm_bf16_backward(shape, scale_dtype):
     torch.testing.assert_close(dw_ref.double(), dw64, atol=1e-3 * math.sqrt(xf.numel() / shape[-1]), rtol=1e-3)  # the oracle agrees with the closed form
     tol = (2.0 ** -8 if scale_dtype == torch.bfloat16 else 1e-5) * dw64.abs() + 2e-4 * math.sqrt(xf.numel() / shape[-1])
     assert ((w.grad.double() - dw64).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,n,offset", [(1, 128, 0), (63, 128, 0), (16384, 128, 0), (16385, 128, 0), (70001, 8, 0),   # one to 256 parts, whole and ragged
+                                           (1025, 1000, 0), (33, 2056, 0), (5, 99, 0), (64, 128, 1)])  # several vectors, block per row, unaligned
+def test_rms_norm_backward_dscale_parts(rows, n, offset, dtype):
+    """dscale summed from per-block parts (workspace full of NaN, written in the scale's type) and, through
+    the entry without a workspace, by atomics. Both against fp64: |error| <= 32 * 2^-24 * sum |terms| for the
+    fp32 sums (roundings add like a random walk over a chain of a few hundred terms), plus 2^-8 of the result where it is rounded to bf16."""
+    g = seeded(rows + n + offset)
+    x, dy = (torch.cat((torch.zeros(offset), randn(g, rows * n))).to(dtype).to(DEV)[offset:].view(rows, n) for _ in range(2))
+    w = (torch.rand(n, generator=g) + 0.5).to(dtype).to(DEV)
+    rstd = torch.rsqrt(x.float().pow(2).mean(-1) + 1e-6)
+    terms = dy.double() * x.double() * rstd.double()[:, None]
+    want, bound = terms.sum(0), 32 * 2.0 ** -24 * terms.abs().sum(0)
+    if dtype == torch.bfloat16:
+        bound = bound + 2.0 ** -8 * want.abs()
+    lib, code, st = nv.lib(), nv.dtype_code(x), nv.stream_ptr(x.device)
+    size = lib.flux_rms_norm_bwd_workspace_bytes(rows, n, code)
+    ws = torch.full((size // 4,), float("nan"), device=DEV)
+    results = []
+    for _ in range(2):
+        dx, ds = torch.empty_like(x), torch.full((n,), float("nan"), dtype=dtype, device=DEV)
+        nv.check(lib.flux_rms_norm_bwd_ws(dy.data_ptr(), x.data_ptr(), w.data_ptr(), rstd.data_ptr(), dx.data_ptr(), ds.data_ptr(), code,
+                                          ws.data_ptr(), size, rows, n, code, code, st), "flux_rms_norm_bwd_ws")
+        results.append((dx, ds))
+    assert ((results[0][1].double() - want).abs() <= bound).all()
+    dx2, ds2 = torch.empty_like(x), torch.zeros(n, device=DEV)
+    nv.check(lib.flux_rms_norm_bwd(dy.data_ptr(), x.data_ptr(), w.data_ptr(), rstd.data_ptr(), dx2.data_ptr(), ds2.data_ptr(),
+                                   rows, n, code, code, st), "flux_rms_norm_bwd")
+    assert torch.equal(dx2, results[0][0]) and ((ds2.double() - want).abs() <= bound).all()
+    if n % 8 == 0 and n <= 1024 and offset == 0:   # no atomics: the same bits each time
+        assert torch.equal(results[0][1], results[1][1])
+    assert lib.flux_rms_norm_bwd_ws(dy.data_ptr(), x.data_ptr(), w.data_ptr(), rstd.data_ptr(), dx2.data_ptr(), ds2.data_ptr(), code,
+                                    ws.data_ptr(), size - 1, rows, n, code, code, st) == nv.E_SHAPE
 
 
 def test_rms_norm_config1_cpu_oracle_and_strided_view():

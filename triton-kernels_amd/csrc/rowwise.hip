@@ -180,15 +180,21 @@ __global__ __launch_bounds__(kBlock) void rms_norm_fwd_block(
 // ------------------------------------------------------------------------------------------------
 // RMSNorm backward: dx = rstd*(dy*w) - rstd^3/n * sum(dy*w*x) * x ;  dscale += sum_rows dy*x*rstd.
 // One group of G lanes per row (register-resident); each block reduces its rows' dscale partials in
-// registers while its groups walk the block's rows, folds them in LDS and finishes with one atomic
-// per column per block. All blocks finish together and their atomics land on the few cache lines of
-// dscale, where they are served one at a time: short rows (one vector per lane) therefore run as
-// 256 blocks of 1024 threads rather than 1024 blocks of 256.
+// registers while its groups walk the block's rows, folds them in LDS and writes them as one row of
+// `part` [blocks, n], which rms_norm_dscale_reduce adds up in a fixed order. Without a workspace
+// (part = null) it finishes with one atomic per column per block into a dscale that the caller cleared.
+// Bound by HBM: x and dy in, dx out. With the workspace [98304, 128] bf16 takes 22.4 us for both launches
+// (75 MB, 3.4 TB/s) and [6144, 128] 7.0 us; clearing dscale, atomics and converting it took 27.2 and
+// 14.1 us. Short rows (one vector per lane) run as 256 blocks of 1024 threads: 512 and 1024 blocks of 1024, 512
+// or 256 threads take 22.8 to 25.1 us at the first shape and 7.1 to 7.4 us at the second, because the
+// reduction reads a row of partials per block.
+constexpr int kBwdThreads1 = 1024, kBwdBlocks1 = 256;
+
 // ------------------------------------------------------------------------------------------------
 template <typename T, typename TS, int G, int ITER, int BLK>
 __global__ __launch_bounds__(BLK) void rms_norm_bwd_regs(
     const T* __restrict__ dy, const T* __restrict__ x, const TS* __restrict__ scale, const float* __restrict__ rstd_in,
-    T* __restrict__ dx, float* __restrict__ dscale, int64_t rows, int n, int rows_per_group) {
+    T* __restrict__ dx, float* __restrict__ dscale, float* __restrict__ part, int64_t rows, int n, int rows_per_group) {
     constexpr int VEC = Elem<T>::VEC;
     constexpr int GROUPS = BLK / G;
     const int lane = threadIdx.x % G;
@@ -249,7 +255,7 @@ __global__ __launch_bounds__(BLK) void rms_norm_bwd_regs(
             }
         }
     }
-    // Fold the block's GROUPS partial rows in LDS, then one atomic per column per block.
+    // Fold the block's GROUPS partial rows in LDS.
     extern __shared__ float dw_lds[];  // [GROUPS][G*ITER*VEC]
     constexpr int COLS = G * ITER * VEC;
 #pragma unroll
@@ -263,8 +269,40 @@ __global__ __launch_bounds__(BLK) void rms_norm_bwd_regs(
         float t = 0.0f;
 #pragma unroll
         for (int g = 0; g < GROUPS; ++g) t += dw_lds[g * COLS + c];
-        atomicAdd(dscale + c, t);
+        if (part) part[static_cast<int64_t>(blockIdx.x) * n + c] = t;
+        else atomicAdd(dscale + c, t);
     }
+}
+
+// dscale[c] = the sum of part[0 .. parts)[c], rounded once to dscale's type. A workgroup takes 32 columns
+// with 32 threads each; a thread adds every 32nd part, the 32 sums are folded in LDS in order, so the
+// result does not depend on timing. At 256 parts of 128 columns (128 KB, out of the L2s) all eight loads of
+// a thread are in flight at once.
+constexpr int kDscaleCols = 32, kDscaleStrips = 32;
+template <typename TD>
+__global__ __launch_bounds__(kDscaleCols * kDscaleStrips) void rms_norm_dscale_reduce(
+    const float* __restrict__ part, TD* __restrict__ dscale, int parts, int n) {
+    __shared__ float sums[kDscaleStrips][kDscaleCols];
+    const int col = threadIdx.x % kDscaleCols, strip = threadIdx.x / kDscaleCols;
+    const int c = blockIdx.x * kDscaleCols + col;
+    float t = 0.0f;
+    if (c < n) {
+#pragma unroll 8
+        for (int i = strip; i < parts; i += kDscaleStrips) t += part[static_cast<int64_t>(i) * n + c];
+    }
+    sums[strip][col] = t;
+    __syncthreads();
+    if (strip == 0 && c < n) {
+        float total = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kDscaleStrips; ++i) total += sums[i][col];
+        dscale[c] = Elem<TD>::store(total);
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void zero_floats(float* __restrict__ p, int n) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) p[i] = 0.0f;
 }
 
 // Block-per-row backward for rows that do not fit the register path.
@@ -505,36 +543,64 @@ static int rms_fwd_launch(const void* x, const void* scale, void* y, float* rstd
     return check_launch("flux_rms_norm");
 }
 
+// How the register-resident backward splits `rows` rows; blocks == 0 where the row takes the block kernel.
+struct BwdPlan {
+    RowPlan row;
+    int threads;         // per workgroup
+    int rows_per_group;  // rows that a group of row.G lanes walks
+    unsigned blocks;
+};
+static BwdPlan plan_bwd(int64_t rows, int n, int vec) {
+    BwdPlan p = {plan_row(n, vec), 0, 0, 0};
+    if (p.row.G == 0 || p.row.ITER > 4) return p;
+    p.threads = p.row.ITER == 1 ? kBwdThreads1 : kBlock;
+    const int64_t want = p.row.ITER == 1 ? kBwdBlocks1 : 1024, groups = p.threads / p.row.G;
+    const int64_t rpg = (rows + want * groups - 1) / (want * groups);
+    p.rows_per_group = static_cast<int>(rpg < 1 ? 1 : rpg);
+    p.blocks = static_cast<unsigned>((rows + p.rows_per_group * groups - 1) / (p.rows_per_group * groups));
+    return p;
+}
+
+template <typename TD>
+static void dscale_reduce(const float* part, void* dscale, int parts, int n, hipStream_t st) {
+    hipLaunchKernelGGL((rms_norm_dscale_reduce<TD>), dim3((n + kDscaleCols - 1) / kDscaleCols), dim3(kDscaleCols * kDscaleStrips), 0, st,
+                       part, static_cast<TD*>(dscale), parts, n);
+}
+
+// With a workspace `ws` (plan_bwd's blocks * n floats, at least n) dscale is written, in dscale_dtype; without
+// one it is fp32 and is added to.
 template <typename T, typename TS>
-static int rms_bwd_launch(const void* dy, const void* x, const void* scale, const float* rstd, void* dx, float* dscale,
-                          int64_t rows, int n, hipStream_t st) {
+static int rms_bwd_launch(const void* dy, const void* x, const void* scale, const float* rstd, void* dx, void* dscale, int dscale_dtype,
+                          float* ws, int64_t rows, int n, hipStream_t st) {
     constexpr int VEC = Elem<T>::VEC;
     const T* dyp = static_cast<const T*>(dy);
     const T* xp = static_cast<const T*>(x);
     const TS* sp = static_cast<const TS*>(scale);
     T* dxp = static_cast<T*>(dx);
-    RowPlan plan = plan_row(n, VEC);
+    const BwdPlan bp = plan_bwd(rows, n, VEC);
+    const RowPlan plan = bp.row;
     const bool vec_ok = aligned16(dy) && aligned16(x) && aligned16(dx) && (sizeof(TS) * VEC != 16 || aligned16(scale));
-    if (plan.G != 0 && plan.ITER <= 4 && vec_ok) {
+    int parts = 0;
+    if (rows > 0 && bp.blocks != 0 && vec_ok) {
 #define CALL(G_, I_)                                                                                         \
     do {                                                                                                     \
         constexpr int IT = (I_ > 4 ? 4 : I_);                                                                \
-        constexpr int BLK = IT == 1 ? 1024 : kBlock;                                                         \
-        constexpr int GROUPS = BLK / G_;                                                                     \
-        const int64_t want_blocks = IT == 1 ? 256 : 1024;  /* few blocks: few atomics on dscale */           \
-        int64_t rpg = (rows + want_blocks * GROUPS - 1) / (want_blocks * GROUPS);                            \
-        if (rpg < 1) rpg = 1;                                                                                \
-        const unsigned grid = (unsigned)((rows + rpg * GROUPS - 1) / (rpg * GROUPS));                        \
+        constexpr int BLK = IT == 1 ? kBwdThreads1 : kBlock;                                                 \
         const size_t lds_bytes = sizeof(float) * BLK * IT * VEC;                                             \
-        hipLaunchKernelGGL((rms_norm_bwd_regs<T, TS, G_, IT, BLK>), dim3(grid), dim3(BLK), lds_bytes, st, dyp, xp, sp, \
-                           rstd, dxp, dscale, rows, n, (int)rpg);                                            \
+        hipLaunchKernelGGL((rms_norm_bwd_regs<T, TS, G_, IT, BLK>), dim3(bp.blocks), dim3(BLK), lds_bytes, st, dyp, xp, sp, \
+                           rstd, dxp, static_cast<float*>(dscale), ws, rows, n, bp.rows_per_group);          \
     } while (0)
         FLUX_DISPATCH_GI(plan, CALL);
 #undef CALL
-    } else {
+        parts = static_cast<int>(bp.blocks);
+    } else if (rows > 0) {
+        if (ws) hipLaunchKernelGGL(zero_floats, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, ws, n);
         hipLaunchKernelGGL((rms_norm_bwd_block<T, TS>), dim3((unsigned)rows), dim3(kBlock), 0, st, dyp, xp, sp, rstd, dxp,
-                           dscale, rows, n);
+                           ws ? ws : static_cast<float*>(dscale), rows, n);
+        parts = 1;
     }
+    if (ws && dscale_dtype == FLUX_BF16) dscale_reduce<bf16_t>(ws, dscale, parts, n, st);
+    else if (ws) dscale_reduce<float>(ws, dscale, parts, n, st);
     return check_launch("flux_rms_norm_bwd");
 }
 
@@ -605,19 +671,40 @@ extern "C" int flux_rms_norm(const void* x, const void* scale, void* y, float* r
     return fail(FLUX_E_DTYPE, "flux_rms_norm: unsupported dtype pair (%d,%d)", x_dtype, scale_dtype);
 }
 
-extern "C" int flux_rms_norm_bwd(const void* dy, const void* x, const void* scale, const float* rstd, void* dx,
-                                 float* dscale, int64_t rows, int32_t n, int32_t x_dtype, int32_t scale_dtype,
-                                 void* stream) {
+static int rms_bwd_checked(const void* dy, const void* x, const void* scale, const float* rstd, void* dx, void* dscale, int dscale_dtype,
+                           float* ws, int64_t rows, int32_t n, int32_t x_dtype, int32_t scale_dtype, void* stream) {
     if (!dy || !x || !scale || !rstd || !dx || !dscale) return fail(FLUX_E_NULL, "flux_rms_norm_bwd: null pointer");
     if (rows < 0 || n <= 0) return fail(FLUX_E_SHAPE, "flux_rms_norm_bwd: bad shape [%lld,%d]", (long long)rows, n);
     if (n > FLUX_MAX_ROW) return fail(FLUX_E_TOO_WIDE, "flux_rms_norm_bwd: n = %d exceeds the maximum row length %d", n, FLUX_MAX_ROW);
-    if (rows == 0) return FLUX_OK;
+    if (rows == 0 && !ws) return FLUX_OK;
     if (rows > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_rms_norm_bwd: too many rows");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_BF16) return rms_bwd_launch<bf16_t, bf16_t>(dy, x, scale, rstd, dx, dscale, rows, n, st);
-    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_F32) return rms_bwd_launch<bf16_t, float>(dy, x, scale, rstd, dx, dscale, rows, n, st);
-    if (x_dtype == FLUX_F32 && scale_dtype == FLUX_F32) return rms_bwd_launch<float, float>(dy, x, scale, rstd, dx, dscale, rows, n, st);
+    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_BF16) return rms_bwd_launch<bf16_t, bf16_t>(dy, x, scale, rstd, dx, dscale, dscale_dtype, ws, rows, n, st);
+    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_F32) return rms_bwd_launch<bf16_t, float>(dy, x, scale, rstd, dx, dscale, dscale_dtype, ws, rows, n, st);
+    if (x_dtype == FLUX_F32 && scale_dtype == FLUX_F32) return rms_bwd_launch<float, float>(dy, x, scale, rstd, dx, dscale, dscale_dtype, ws, rows, n, st);
     return fail(FLUX_E_DTYPE, "flux_rms_norm_bwd: unsupported dtype pair (%d,%d)", x_dtype, scale_dtype);
+}
+
+extern "C" int flux_rms_norm_bwd(const void* dy, const void* x, const void* scale, const float* rstd, void* dx,
+                                 float* dscale, int64_t rows, int32_t n, int32_t x_dtype, int32_t scale_dtype,
+                                 void* stream) {
+    return rms_bwd_checked(dy, x, scale, rstd, dx, dscale, FLUX_F32, nullptr, rows, n, x_dtype, scale_dtype, stream);
+}
+
+extern "C" int64_t flux_rms_norm_bwd_workspace_bytes(int64_t rows, int32_t n, int32_t x_dtype) {
+    if (rows < 0 || rows > 0x7fffffffLL || n <= 0 || n > FLUX_MAX_ROW) return 0;
+    const int64_t blocks = plan_bwd(rows, n, x_dtype == FLUX_BF16 ? Elem<bf16_t>::VEC : Elem<float>::VEC).blocks;
+    return static_cast<int64_t>(sizeof(float)) * n * (blocks > 1 ? blocks : 1);
+}
+
+extern "C" int flux_rms_norm_bwd_ws(const void* dy, const void* x, const void* scale, const float* rstd, void* dx,
+                                    void* dscale, int32_t dscale_dtype, void* ws, int64_t ws_bytes, int64_t rows, int32_t n,
+                                    int32_t x_dtype, int32_t scale_dtype, void* stream) {
+    if (!ws) return fail(FLUX_E_NULL, "flux_rms_norm_bwd_ws: null workspace");
+    if (dscale_dtype != FLUX_BF16 && dscale_dtype != FLUX_F32) return fail(FLUX_E_DTYPE, "flux_rms_norm_bwd_ws: unsupported dscale dtype %d", dscale_dtype);
+    if (reinterpret_cast<uintptr_t>(ws) % sizeof(float) != 0) return fail(FLUX_E_ALIGN, "flux_rms_norm_bwd_ws: the workspace must be 4-byte aligned");
+    if (ws_bytes < flux_rms_norm_bwd_workspace_bytes(rows, n, x_dtype)) return fail(FLUX_E_SHAPE, "flux_rms_norm_bwd_ws: workspace of %lld bytes is too small", (long long)ws_bytes);
+    return rms_bwd_checked(dy, x, scale, rstd, dx, dscale, dscale_dtype, static_cast<float*>(ws), rows, n, x_dtype, scale_dtype, stream);
 }
 
 static int ln_mod_checked(const flux_layer_norm_args* a, int count, int32_t n, int32_t dtype, float eps, void* stream) {

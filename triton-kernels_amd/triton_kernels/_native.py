@@ -95,6 +95,9 @@ SIGNATURES = {
                                 c_int64, c_int64, c_int64, c_int32, c_int32, c_float, c_void_p]),
     "flux_rms_norm_bwd": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
                                     c_int32, c_int32, c_void_p]),
+    "flux_rms_norm_bwd_workspace_bytes": (c_int64, [c_int64, c_int32, c_int32]),
+    "flux_rms_norm_bwd_ws": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_int64,
+                                       c_int64, c_int32, c_int32, c_int32, c_void_p]),
     "flux_layer_norm_modulation": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32,
                                              c_int64, c_int32, c_float, c_void_p]),
     "flux_layer_norm_modulation_pair": (c_int32, [POINTER(LayerNormArgs), POINTER(LayerNormArgs), c_int32, c_int32, c_float, c_void_p]),

@@ -75,11 +75,14 @@ class _rms_norm(torch.autograd.Function):
         if sc.dtype != x2.dtype and not (x2.dtype == torch.bfloat16 and sc.dtype == torch.float32):
             sc = sc.to(x2.dtype)
         dx = torch.empty_like(x2)
-        dscale = torch.zeros((n,), dtype=torch.float32, device=dev)
+        # the kernel's types; the gradient of a scale of another type is converted from fp32 below
+        dscale = torch.empty((n,), dtype=scale.dtype if scale.dtype == torch.bfloat16 else torch.float32, device=dev)
+        xcode = nv.dtype_code(x2)
+        ws = torch.empty((nv.lib().flux_rms_norm_bwd_workspace_bytes(rows, n, xcode),), dtype=torch.uint8, device=dev)
         with nv.on_device(dev):
-            rc = nv.lib().flux_rms_norm_bwd(
-                dy2.data_ptr(), x2.data_ptr(), sc.data_ptr(), rstd.data_ptr(), dx.data_ptr(), dscale.data_ptr(),
-                rows, n, nv.dtype_code(x2), nv.dtype_code(sc), nv.stream_ptr(dev))
+            rc = nv.lib().flux_rms_norm_bwd_ws(
+                dy2.data_ptr(), x2.data_ptr(), sc.data_ptr(), rstd.data_ptr(), dx.data_ptr(), dscale.data_ptr(), nv.dtype_code(dscale),
+                ws.data_ptr(), ws.numel(), rows, n, xcode, nv.dtype_code(sc), nv.stream_ptr(dev))
         nv.check(rc, "flux_rms_norm_bwd")
         return dx.reshape(dy.shape), dscale.to(scale.dtype).reshape(scale.shape), None
 

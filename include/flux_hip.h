@@ -60,6 +60,14 @@ int flux_rms_norm(const void* x, const void* scale, void* y, float* rstd,
                   int64_t s0, int64_t s1, int64_t s2,
                   int32_t x_dtype, int32_t scale_dtype, float eps, void* stream);
 
+/* The same on two tensors of the same width and types in one launch (q and k of a q/k norm). */
+typedef struct flux_rms_norm_args {
+    const void* x; const void* scale; void* y; float* rstd;
+    int64_t d0, d1, d2, s0, s1, s2;
+} flux_rms_norm_args;
+int flux_rms_norm_pair(const flux_rms_norm_args* first, const flux_rms_norm_args* second, int32_t n,
+                       int32_t x_dtype, int32_t scale_dtype, float eps, void* stream);
+
 /* RMSNorm backward. Replaces _rms_norm.backward / _rms_norm_bwd (kernels/normalization.py:110-139,
  * 171-190). x, dy, dx contiguous [rows, n]; rstd from the forward; dscale[n] is fp32 and is
  * accumulated with atomics, so the caller zero-fills it first. */

@@ -119,6 +119,44 @@ def test_rms_norm_backward_dscale_parts(rows, n, offset, dtype):
                                     ws.data_ptr(), size - 1, rows, n, code, code, st) == nv.E_SHAPE
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens,width,heads", [((256, 256), 128, 24), ((1, 77), 128, 3), ((33, 5), 1536, 1), ((7, 9), 100, 2), ((19, 3), 4104, 1)])
+def test_qk_norm_pair_equals_two_calls(tokens, width, heads, dtype):
+    """QKNorm without gradients norms q and k in one launch: the same bits as two calls, on views of a
+    projection and on views that are not 16-byte addressable, with frozen and unfrozen scales; hooks still see
+    both norms."""
+    g = seeded(sum(tokens) + width)
+    norm = tk.QKNorm(width).to(DEV, dtype).eval()
+    with torch.no_grad():
+        for p in norm.parameters():
+            p.copy_(torch.rand(width, generator=g) + 0.5)
+    def views(extra):
+        return [randn(g, 2, t, 3 * heads * width + extra, dtype=dtype).to(DEV)[..., extra:].unflatten(-1, (3, heads, width)).permute(2, 0, 3, 1, 4)[i]
+                for i, t in enumerate(tokens)]
+    for q, k in (views(0), views(1)):
+        want = [tk.rms_norm(x.contiguous(), p.detach()) for x, p in ((q, norm.query_norm.scale), (k, norm.key_norm.scale))]
+        for frozen in (False, True):
+            norm.requires_grad_(not frozen)
+            with torch.no_grad():
+                got = norm(q, k, q)
+            for a, b in zip(got, want):
+                if frozen and (width % 8 or q.storage_offset()):
+                    # read in place, by elements: another order of the fp32 sums. In bf16 the normalised value and the
+                    # product may each round the other way: two units of at most 2^-7.
+                    torch.testing.assert_close(a, b, atol=1e-6, rtol=2.0 ** -6 if dtype == torch.bfloat16 else 1e-6)
+                else:
+                    assert torch.equal(a, b)
+    seen = []
+    norm.query_norm.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    with torch.no_grad():
+        norm(q, k, q)
+    assert seen == [q.shape]
+    norm.requires_grad_(True)
+    gq, gk = norm(q, k, q)          # differentiated: the two calls
+    (gq.float().sum() + gk.float().sum()).backward()
+    assert norm.query_norm.scale.grad.isfinite().all() and norm.key_norm.scale.grad.isfinite().all()
+
+
 def test_rms_norm_config1_cpu_oracle_and_strided_view():
     x, w = cfg.config1("cpu", scale=0.25)
     want = oracle.rms_norm_ref(x, w)                       # CPU oracle, same bits

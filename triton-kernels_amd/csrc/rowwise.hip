@@ -55,14 +55,38 @@ __device__ __forceinline__ void load_vecf(const TS* p, float (&out)[VEC]) {
 // R rows per thread (a block covers R * kBlock / G rows, row j of a thread being kBlock / G rows behind row
 // j - 1). One row per thread is what is launched: two rows of one vector each, which put twice the loads
 // in flight per wave and halve the number of workgroups, measured 14.7 us against 13.8 us at the Flux shape.
+//
+// One or two tensors of the same width and types per launch (t[1]'s blocks follow the blocks0 of t[0]): q and
+// k of a q/k norm. At [1, 24, 256, 128] the kernel is 3 us of work behind a launch, and the second launch
+// costs the host more than both kernels take.
+template <typename T, typename TS>
+struct RmsFwd {
+    const T* x; const TS* scale; T* y; float* rstd;
+    int64_t rows, d1, d2, s0, s1, s2;
+};
+template <typename T, typename TS>
+struct RmsFwdSet {
+    RmsFwd<T, TS> t[2];
+    unsigned blocks0;
+    int n;
+    float eps;
+};
 template <typename T, typename TS, int G, int ITER, int R>
-__global__ __launch_bounds__(kBlock) void rms_norm_fwd_regs(
-    const T* __restrict__ x, const TS* __restrict__ scale, T* __restrict__ y, float* __restrict__ rstd_out,
-    int64_t rows, int64_t d1, int64_t d2, int n, int64_t s0, int64_t s1, int64_t s2, float eps) {
+__global__ __launch_bounds__(kBlock) void rms_norm_fwd_regs(RmsFwdSet<T, TS> set) {
+    const bool second = blockIdx.x >= set.blocks0;
+    const RmsFwd<T, TS>& t = set.t[second];
+    const unsigned block = blockIdx.x - (second ? set.blocks0 : 0u);
+    const T* __restrict__ const x = t.x;
+    const TS* __restrict__ const scale = t.scale;
+    T* __restrict__ const y = t.y;
+    float* __restrict__ const rstd_out = t.rstd;
+    const int64_t rows = t.rows, d1 = t.d1, d2 = t.d2, s0 = t.s0, s1 = t.s1, s2 = t.s2;
+    const int n = set.n;
+    const float eps = set.eps;
     constexpr int VEC = Elem<T>::VEC;
     constexpr int ROWS_PER_PASS = kBlock / G;
     const int lane = threadIdx.x % G;
-    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * (ROWS_PER_PASS * R) + threadIdx.x / G;
+    const int64_t row0 = static_cast<int64_t>(block) * (ROWS_PER_PASS * R) + threadIdx.x / G;
 
     // Offset of a row in the strided [d0, d1, d2] view. The host merges dimensions whose strides
     // allow it, so an evenly strided tensor arrives as d1 = 1 and needs no division; other views
@@ -510,35 +534,56 @@ static RowPlan plan_row(int n, int vec) {
     } while (0)
 
 template <typename T, typename TS>
-static int rms_fwd_launch(const void* x, const void* scale, void* y, float* rstd, int64_t d0, int64_t d1, int64_t d2,
-                          int n, int64_t s0, int64_t s1, int64_t s2, float eps, hipStream_t st) {
+static int rms_fwd_launch(const flux_rms_norm_args* a, int count, int n, float eps, hipStream_t st) {
     constexpr int VEC = Elem<T>::VEC;
-    const int64_t rows = d0 * d1 * d2;
-    const T* xp = static_cast<const T*>(x);
-    const TS* sp = static_cast<const TS*>(scale);
-    T* yp = static_cast<T*>(y);
-    RowPlan plan = plan_row(n, VEC);
-    const bool vec_ok = aligned16(x) && aligned16(y) && s0 % VEC == 0 && s1 % VEC == 0 && s2 % VEC == 0 &&
-                        (sizeof(TS) * VEC != 16 || aligned16(scale));
-    // merge dimensions that are evenly strided: [d0, d1, d2] -> [1, 1, rows] for a contiguous tensor
-    if (d0 == 1 || s0 == d1 * s1) { d1 *= d0; d0 = 1; }
-    if (d0 == 1 && (d1 == 1 || s1 == d2 * s2)) { d2 *= d1; d1 = 1; }
-    if (plan.G != 0 && vec_ok) {
+    const RowPlan plan = plan_row(n, VEC);
+    RmsFwdSet<T, TS> set;
+    set.n = n;
+    set.eps = eps;
+    int used = 0;
+    bool vec_ok[2];
+    for (int i = 0; i < count; ++i) {
+        int64_t d0 = a[i].d0, d1 = a[i].d1, d2 = a[i].d2, s0 = a[i].s0, s1 = a[i].s1, s2 = a[i].s2;
+        const int64_t rows = d0 * d1 * d2;
+        if (rows == 0) continue;
+        vec_ok[used] = aligned16(a[i].x) && aligned16(a[i].y) && s0 % VEC == 0 && s1 % VEC == 0 && s2 % VEC == 0 &&
+                       (sizeof(TS) * VEC != 16 || aligned16(a[i].scale));
+        // merge dimensions that are evenly strided: [d0, d1, d2] -> [1, 1, rows] for a contiguous tensor
+        if (d0 == 1 || s0 == d1 * s1) { d1 *= d0; d0 = 1; }
+        if (d0 == 1 && (d1 == 1 || s1 == d2 * s2)) { d2 *= d1; d1 = 1; }
+        set.t[used++] = {static_cast<const T*>(a[i].x), static_cast<const TS*>(a[i].scale), static_cast<T*>(a[i].y), a[i].rstd, rows, d1, d2, s0, s1, s2};
+    }
+    if (used == 0) return FLUX_OK;
+    if (plan.G != 0 && vec_ok[0] && vec_ok[used - 1]) {
 #define CALL(G_, I_)                                                                                          \
     do {                                                                                                      \
         constexpr int R_ = 1;   /* two short rows per thread measured 6 % slower at the Flux shape */            \
         constexpr int RPB_ = (kBlock / G_) * R_;                                                              \
-        hipLaunchKernelGGL((rms_norm_fwd_regs<T, TS, G_, I_, R_>), dim3((unsigned)((rows + RPB_ - 1) / RPB_)), \
-                           dim3(kBlock), 0, st, xp, sp, yp, rstd, rows, d1, d2, n, s0, s1, s2, eps);           \
+        unsigned grid_ = 0;                                                                                   \
+        for (int i = 0; i < used; ++i) {                                                                      \
+            grid_ += (unsigned)((set.t[i].rows + RPB_ - 1) / RPB_);                                            \
+            if (i == 0) set.blocks0 = grid_;                                                                  \
+        }                                                                                                     \
+        hipLaunchKernelGGL((rms_norm_fwd_regs<T, TS, G_, I_, R_>), dim3(grid_), dim3(kBlock), 0, st, set);     \
     } while (0)
+        if (used == 1) set.t[1] = set.t[0];
         FLUX_DISPATCH_GI(plan, CALL);
 #undef CALL
-    } else if (n % VEC == 0 && vec_ok) {
-        hipLaunchKernelGGL((rms_norm_fwd_block<T, TS, VEC>), dim3((unsigned)rows), dim3(kBlock), 0, st, xp, sp, yp, rstd,
-                           rows, d1, d2, n, s0, s1, s2, eps);
-    } else {
-        hipLaunchKernelGGL((rms_norm_fwd_block<T, TS, 1>), dim3((unsigned)rows), dim3(kBlock), 0, st, xp, sp, yp, rstd,
-                           rows, d1, d2, n, s0, s1, s2, eps);
+        return check_launch("flux_rms_norm");
+    }
+    for (int i = 0; i < used; ++i) {
+        const RmsFwd<T, TS>& t = set.t[i];
+        if (plan.G != 0 && vec_ok[i]) {   // the other one of a pair is not 16-byte addressable
+            flux_rms_norm_args one = a[a[0].d0 * a[0].d1 * a[0].d2 == 0 ? 1 : i];
+            const int rc = rms_fwd_launch<T, TS>(&one, 1, n, eps, st);
+            if (rc != FLUX_OK) return rc;
+        } else if (n % VEC == 0 && vec_ok[i]) {
+            hipLaunchKernelGGL((rms_norm_fwd_block<T, TS, VEC>), dim3((unsigned)t.rows), dim3(kBlock), 0, st, t.x, t.scale, t.y, t.rstd,
+                               t.rows, t.d1, t.d2, n, t.s0, t.s1, t.s2, eps);
+        } else {
+            hipLaunchKernelGGL((rms_norm_fwd_block<T, TS, 1>), dim3((unsigned)t.rows), dim3(kBlock), 0, st, t.x, t.scale, t.y, t.rstd,
+                               t.rows, t.d1, t.d2, n, t.s0, t.s1, t.s2, eps);
+        }
     }
     return check_launch("flux_rms_norm");
 }
@@ -656,19 +701,36 @@ static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float 
 
 using namespace flux;
 
+static int rms_fwd_checked(const flux_rms_norm_args* a, int count, int32_t n, int32_t x_dtype, int32_t scale_dtype, float eps, void* stream) {
+    int64_t rows = 0;
+    for (int i = 0; i < count; ++i) {
+        if (!a[i].x || !a[i].scale || !a[i].y) return fail(FLUX_E_NULL, "flux_rms_norm: null pointer");
+        if (a[i].d0 < 0 || a[i].d1 < 0 || a[i].d2 < 0 || n <= 0)
+            return fail(FLUX_E_SHAPE, "flux_rms_norm: bad shape [%lld,%lld,%lld,%d]", (long long)a[i].d0, (long long)a[i].d1, (long long)a[i].d2, n);
+        rows += a[i].d0 * a[i].d1 * a[i].d2;
+    }
+    if (n > FLUX_MAX_ROW) return fail(FLUX_E_TOO_WIDE, "flux_rms_norm: n = %d exceeds the maximum row length %d", n, FLUX_MAX_ROW);
+    if (rows == 0) return FLUX_OK;
+    if (rows > 0x7fffffffLL * 4) return fail(FLUX_E_SHAPE, "flux_rms_norm: too many rows");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_BF16) return rms_fwd_launch<bf16_t, bf16_t>(a, count, n, eps, st);
+    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_F32) return rms_fwd_launch<bf16_t, float>(a, count, n, eps, st);
+    if (x_dtype == FLUX_F32 && scale_dtype == FLUX_F32) return rms_fwd_launch<float, float>(a, count, n, eps, st);
+    return fail(FLUX_E_DTYPE, "flux_rms_norm: unsupported dtype pair (%d,%d)", x_dtype, scale_dtype);
+}
+
 extern "C" int flux_rms_norm(const void* x, const void* scale, void* y, float* rstd, int64_t d0, int64_t d1, int64_t d2,
                              int32_t n, int64_t s0, int64_t s1, int64_t s2, int32_t x_dtype, int32_t scale_dtype,
                              float eps, void* stream) {
-    if (!x || !scale || !y) return fail(FLUX_E_NULL, "flux_rms_norm: null pointer");
-    if (d0 < 0 || d1 < 0 || d2 < 0 || n <= 0) return fail(FLUX_E_SHAPE, "flux_rms_norm: bad shape [%lld,%lld,%lld,%d]", (long long)d0, (long long)d1, (long long)d2, n);
-    if (n > FLUX_MAX_ROW) return fail(FLUX_E_TOO_WIDE, "flux_rms_norm: n = %d exceeds the maximum row length %d", n, FLUX_MAX_ROW);
-    if (d0 * d1 * d2 == 0) return FLUX_OK;
-    if (d0 * d1 * d2 > 0x7fffffffLL * 4) return fail(FLUX_E_SHAPE, "flux_rms_norm: too many rows");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_BF16) return rms_fwd_launch<bf16_t, bf16_t>(x, scale, y, rstd, d0, d1, d2, n, s0, s1, s2, eps, st);
-    if (x_dtype == FLUX_BF16 && scale_dtype == FLUX_F32) return rms_fwd_launch<bf16_t, float>(x, scale, y, rstd, d0, d1, d2, n, s0, s1, s2, eps, st);
-    if (x_dtype == FLUX_F32 && scale_dtype == FLUX_F32) return rms_fwd_launch<float, float>(x, scale, y, rstd, d0, d1, d2, n, s0, s1, s2, eps, st);
-    return fail(FLUX_E_DTYPE, "flux_rms_norm: unsupported dtype pair (%d,%d)", x_dtype, scale_dtype);
+    const flux_rms_norm_args a = {x, scale, y, rstd, d0, d1, d2, s0, s1, s2};
+    return rms_fwd_checked(&a, 1, n, x_dtype, scale_dtype, eps, stream);
+}
+
+extern "C" int flux_rms_norm_pair(const flux_rms_norm_args* first, const flux_rms_norm_args* second, int32_t n,
+                                  int32_t x_dtype, int32_t scale_dtype, float eps, void* stream) {
+    if (!first || !second) return fail(FLUX_E_NULL, "flux_rms_norm_pair: null args");
+    const flux_rms_norm_args a[2] = {*first, *second};
+    return rms_fwd_checked(a, 2, n, x_dtype, scale_dtype, eps, stream);
 }
 
 static int rms_bwd_checked(const void* dy, const void* x, const void* scale, const float* rstd, void* dx, void* dscale, int dscale_dtype,

@@ -70,6 +70,13 @@ class LinearPairArgs(Structure):
     _fields_ = [("product", LinearArgs * 2), ("a_rows", c_int64 * 2), ("a_batch_stride", c_int64 * 2)]
 
 
+class RmsNormArgs(Structure):
+    _fields_ = [
+        ("x", c_void_p), ("scale", c_void_p), ("y", c_void_p), ("rstd", c_void_p),
+        ("d0", c_int64), ("d1", c_int64), ("d2", c_int64), ("s0", c_int64), ("s1", c_int64), ("s2", c_int64),
+    ]
+
+
 class LayerNormArgs(Structure):
     _fields_ = [
         ("x", c_void_p), ("scale", c_void_p), ("shift", c_void_p), ("y", c_void_p),
@@ -93,6 +100,7 @@ SIGNATURES = {
     "flux_last_error": (c_char_p, []),
     "flux_rms_norm": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int32,
                                 c_int64, c_int64, c_int64, c_int32, c_int32, c_float, c_void_p]),
+    "flux_rms_norm_pair": (c_int32, [POINTER(RmsNormArgs), POINTER(RmsNormArgs), c_int32, c_int32, c_int32, c_float, c_void_p]),
     "flux_rms_norm_bwd": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
                                     c_int32, c_int32, c_void_p]),
     "flux_rms_norm_bwd_workspace_bytes": (c_int64, [c_int64, c_int32, c_int32]),
@@ -224,6 +232,6 @@ def src4(t: torch.Tensor | None) -> Src4:
 
 __all__ = [
     "lib", "lib_path", "check", "last_error", "dtype_code", "require_gpu", "stream_ptr", "on_device", "ptr", "src4",
-    "Src4", "QkvPrepArgs", "LinearArgs", "LinearPairArgs", "LayerNormArgs", "AttnArgs", "SIGNATURES", "byref",
+    "Src4", "QkvPrepArgs", "LinearArgs", "LinearPairArgs", "RmsNormArgs", "LayerNormArgs", "AttnArgs", "SIGNATURES", "byref",
     "FLUX_BF16", "FLUX_F32", "ACT_NONE", "ACT_GELU_TANH", "ACT_SILU", "LINEAR_SHARED_GPU", "MAX_ROW",
 ]

@@ -22,14 +22,13 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 from torch import Tensor
-from torch.nn.modules.module import _has_any_global_hook
 
 from triton_kernels import _native as nv
 from triton_kernels.kernels.attention import attention_into, scaled_dot_product_attention
 from triton_kernels.kernels.linear import linear, linear_into, linear_pair_into, qk_fusable
 from triton_kernels.kernels.normalization import layer_norm_modulation, layer_norm_modulation_pair
 from triton_kernels.kernels.positional_embedding import apply_rope, qkv_prep
-from triton_kernels.modules.normalization import QKNorm
+from triton_kernels.modules.normalization import QKNorm, plain
 
 
 def _heads(qkv: Tensor, num_heads: int) -> tuple[Tensor, Tensor, Tensor]:
@@ -156,11 +155,6 @@ def MLP(hidden_size: int, mlp_hidden_dim: int, bias: bool = True):
         nn.Identity(),
         Linear(mlp_hidden_dim, hidden_size, bias=bias),
     )
-
-
-def _plain(module: nn.Module, cls: type) -> bool:
-    """Whether calling `module` does what `cls` does and nothing else, so that its weights may be used directly."""
-    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks or _has_any_global_hook())
 
 
 def _fusable(*tensors: Tensor) -> bool:
@@ -307,7 +301,7 @@ class DoubleStreamBlock(nn.Module):
         img_mod1, img_mod2, txt_mod1, txt_mod2 = self._modulations(vec)
         img_qkv_lin, txt_qkv_lin = self.img_attn.qkv, self.txt_attn.qkv
         img_m, txt_m = layer_norm_modulation_pair((img, img_mod1.scale, img_mod1.shift), (txt, txt_mod1.scale, txt_mod1.shift))
-        if _plain(img_qkv_lin, Linear) and _plain(txt_qkv_lin, Linear):
+        if plain(img_qkv_lin, Linear) and plain(txt_qkv_lin, Linear):
             img_qkv, txt_qkv = linear_pair_into(dict(x=img_m, w=img_qkv_lin.weight, b=img_qkv_lin.bias),
                                                 dict(x=txt_m, w=txt_qkv_lin.weight, b=txt_qkv_lin.bias))
         else:
@@ -335,7 +329,7 @@ class DoubleStreamBlock(nn.Module):
 
     def _modulations(self, vec: Tensor):
         mods = (self.img_mod, self.txt_mod)
-        if not (all(_plain(m, Modulation) and m.takes_fused_silu(vec) for m in mods) and mods[0].multiplier == mods[1].multiplier):
+        if not (all(plain(m, Modulation) and m.takes_fused_silu(vec) for m in mods) and mods[0].multiplier == mods[1].multiplier):
             return (*self.img_mod(vec), *self.txt_mod(vec))
         outs = linear_pair_into(*(dict(x=vec, w=m.lin.weight, b=m.lin.bias, in_activation="SiLU") for m in mods))
         pairs = [m.chunks(o.reshape(*vec.shape[:-1], -1)) for m, o in zip(mods, outs)]

@@ -254,6 +254,12 @@ typedef struct flux_attn_args {
 } flux_attn_args;
 
 int flux_attention_fwd_bf16(const flux_attn_args* args, void* stream);
+/* The same with a workspace of device memory (16-byte aligned, the launch's own until it has run), which
+ * lets few rows use the whole GPU: the keys are cut over workgroups, whose fp32 partial results are added
+ * in a fixed order. flux_attention_workspace_bytes says how much that takes, 0 where it would not help; with
+ * less the call runs as without. */
+int64_t flux_attention_workspace_bytes(int64_t B, int64_t H, int64_t L, int32_t D);
+int flux_attention_fwd_bf16_ws(const flux_attn_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Small element-wise kernels (the reference's inductor-derived `ops`, plus nn.GELU on a view).

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import triton_kernels as tk
+from triton_kernels import _native as nv
 from oracle import flux_oracle as oracle
 from triton_kernels import testing as cfg
 from util import DEV, randn, seeded
@@ -125,8 +126,9 @@ _WIDE = [(4, 24, 512),    # 64-row-per-wave kernel, one launch of 256-row tiles
          (4, 24, 1000),   # the same with a ragged last tile
          (1, 24, 4336),   # two launches (256- and 192-row tiles), ragged
          (3, 24, 1536),   # two launches, odd batch * even heads
-         (8, 24, 31),     # one partial tile per head
+         (8, 24, 31),     # one partial tile per head, 128-row workgroups
          (6, 24, 97),
+         (12, 24, 31),    # one partial tile per head, 256-row tiles
          (1, 8, 4100),    # few heads, long ragged sequence
          (2, 43, 770),    # both tile sizes in one launch, ragged, 4 tiles of 256 rows per head
          (1, 170, 520),   # the same just under two rounds of tiles
@@ -229,3 +231,74 @@ def test_attention_lse_at_the_flux_shape():
     s = torch.einsum("bhqd,bhkd->bhqk", q[:, :, rows].float(), k.float()) * (math.log2(math.e) / math.sqrt(q.shape[-1]))
     total = torch.exp2(s - lse[:, :, rows, None]).sum(-1)
     torch.testing.assert_close(total, torch.ones_like(total), atol=5e-3, rtol=0)
+
+
+# 128-row workgroups whose keys are cut in parts: equal and shorter last parts, a last tile of one key, ragged rows
+_SPLIT = [(1, 2, 2048), (1, 2, 4096), (2, 1, 2049), (1, 2, 1793), (1, 4, 2500), (1, 1, 3000)]
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("B,H,L", _SPLIT)
+def test_attention_keys_in_parts(B, H, L, D):
+    """On views of a packed projection, with lse; the same call without a workspace (one part) agrees to the
+    rounding of the output and of P (2^-8 relative each)."""
+    lib = nv.lib()
+    need = lib.flux_attention_workspace_bytes(B, H, L, D)
+    assert need > 0
+    g = seeded(L + D)
+    qkv = randn(g, B, L, 3 * H * D, dtype=torch.bfloat16).to(DEV)
+    q, k, v = oracle.split_heads_ref(qkv, H)
+    buf = torch.zeros(B, L, H * D + 64, dtype=torch.bfloat16, device=DEV)
+    out = buf[..., :H * D].view(B, L, H, D).permute(0, 2, 1, 3)
+    lse, lse1 = (torch.empty(B, H, L, dtype=torch.float32, device=DEV) for _ in range(2))
+    tk.attention_into(q, k, v, out, lse=lse)
+    torch.testing.assert_close(out.float(), oracle.attention_ref_fp32(q, k, v), atol=1e-2, rtol=0)
+    torch.testing.assert_close(lse, oracle.attention_lse_ref(q, k), atol=5e-3, rtol=5e-4)
+    assert (buf[..., H * D:] == 0).all()
+    one = torch.empty(B, H, L, D, dtype=torch.bfloat16, device=DEV)
+    a = nv.AttnArgs()
+    a.q, a.k, a.v = nv.src4(q), nv.src4(k), nv.src4(v)
+    a.o, a.o_sb, a.o_sh, a.o_sl = one.data_ptr(), *one.stride()[:3]
+    a.lse, a.B, a.H, a.L, a.D, a.sm_scale = lse1.data_ptr(), B, H, L, D, 1 / math.sqrt(D)
+    assert lib.flux_attention_fwd_bf16(nv.byref(a), nv.stream_ptr(one.device)) == 0
+    torch.testing.assert_close(out.float(), one.float(), atol=4e-3, rtol=2.0 ** -7)
+    # a row's sum is that of its probabilities rounded to bf16, at most 2^-9 relative per term on either side, and
+    # the two round them against different maxima: |lse - lse1| <= 2 * 2^-9 * log2(e)
+    torch.testing.assert_close(lse, lse1, atol=2.0 ** -8 * math.log2(math.e), rtol=0)
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_attention_keys_in_parts_infinite_and_nan_scores(D):
+    """Keys that score -inf in one whole part drop out; NaN in a part reaches exactly the rows it belongs to."""
+    L = 2048
+    g = seeded(D)
+    q = randn(g, 1, 2, L, D, dtype=torch.bfloat16).abs().to(DEV)
+    k, v = (randn(g, 1, 2, L, D, dtype=torch.bfloat16).to(DEV) for _ in range(2))
+    assert nv.lib().flux_attention_workspace_bytes(1, 2, L, D) > 0
+    k[:, :, 1024:] = 0
+    k[:, :, 1024:, 0] = -math.inf          # q > 0 there: the second half of the keys scores -inf
+    q[..., 0] = q[..., 0].clamp_min(0.1)
+    q[..., 1:] = q[..., 1:].clamp_min(1e-3)
+    o = tk.scaled_dot_product_attention(q, k, v)
+    torch.testing.assert_close(o.float(), oracle.attention_ref_fp32(q, k[:, :, :1024], v[:, :, :1024]), atol=1e-2, rtol=0)
+    k[:, 1, 700] = math.nan
+    o = tk.scaled_dot_product_attention(q, k, v)
+    assert torch.isnan(o[:, 1]).all() and torch.isfinite(o[:, 0]).all()
+
+
+def test_attention_keys_in_parts_replayed_from_a_graph():
+    g = seeded(3)
+    q, k, v = (randn(g, 1, 2, 1100, 128, dtype=torch.bfloat16).to(DEV) for _ in range(3))
+    o = torch.empty_like(q)
+    tk.attention_into(q, k, v, o)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tk.attention_into(q, k, v, o)
+    for i in range(3):
+        q.copy_(randn(g, 1, 2, 1100, 128, dtype=torch.bfloat16))
+        eager = tk.scaled_dot_product_attention(q, k, v)
+        o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, eager), i

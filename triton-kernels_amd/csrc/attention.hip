@@ -29,7 +29,7 @@
 // refilled is the one read a whole iteration earlier.
 #include "common.h"
 #include "attention_params.h"
-#include <stdlib.h>
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -116,8 +116,11 @@ constexpr bool attn_units_in_time(int qb_count, int ns, int db_count, int nslot,
     return true;
 }
 
-template <int D, int QB, int BN>  // BN = keys per tile (32 or 64)
-__global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(AttnParams p) {
+// SPLIT: the keys are cut in `splits` parts of part_keys (the last may be shorter, none is empty) and a
+// workgroup takes one part of them; it stores O^T unnormalised, the reference maximum and the sum of
+// its rows as fp32 to ws, and attn_combine_kernel adds the parts.
+template <int D, int QB, int BN, bool SPLIT>  // BN = keys per tile (32 or 64)
+__global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(AttnParams p, float* ws, int splits, int part_keys) {
     constexpr int KB = BN / 32;         // 32-key blocks of S^T per tile
     constexpr int PS = BN / 16;         // 16-key steps of P^T per tile
     constexpr int KSTEPS = D / 16;      // contraction steps of S^T = K Q^T
@@ -144,16 +147,20 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
     const int per_xcd = gridDim.x / 8;
     const int vt = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (vt >= p.total_tiles) return;
-    const int bh = vt / p.n_qtiles, qt = vt % p.n_qtiles;
+    const int qt = vt % p.n_qtiles;
+    const int part = SPLIT ? vt / p.n_qtiles % splits : 0;   // workgroups that share K and V stay on one XCD
+    const int bh = SPLIT ? vt / p.n_qtiles / splits : vt / p.n_qtiles;
     const int b = bh / p.H, h = bh % p.H;
+    const int key_begin = SPLIT ? part * part_keys : 0;
+    const int keys = SPLIT ? min(p.L - key_begin, part_keys) : p.L;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int frow = lane & 31, fhalf = lane >> 5;
     const int q0 = qt * (128 * QB) + wave * (32 * QB);
 
-    const bf16_t* kbase = p.k + b * p.k_sb + h * p.k_sh;
-    const bf16_t* vbase = p.v + b * p.v_sb + h * p.v_sh;
+    const bf16_t* kbase = p.k + b * p.k_sb + h * p.k_sh + key_begin * p.k_sl;
+    const bf16_t* vbase = p.v + b * p.v_sb + h * p.v_sh + key_begin * p.v_sl;
 
     // LDS row swizzles (64 banks of 4 bytes; a b128 read is served 16 lanes per clock):
     //   K rows are read whole-chunk by 16 lanes on 16 consecutive rows  -> chunk ^ kswz(row)
@@ -190,11 +197,11 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
         k_voff[i] = static_cast<uint32_t>((r * p.k_sl + (l_pos ^ kswz(r)) * 8) * 2);
         v_voff[i] = static_cast<uint32_t>((r * p.v_sl + (l_pos ^ vswz(r)) * 8) * 2);
     }
-    // Buffer resource of a 64-key tile starting at key0; keys at or past L are outside it and read
-    // as zeros (a tile wholly past L has an empty resource: its base is never dereferenced).
+    // Buffer resource of a 64-key tile starting at key0; keys at or past the end are outside it and read
+    // as zeros (a tile wholly past the end has an empty resource: its base is never dereferenced).
     const int k_row2 = static_cast<int>(p.k_sl * 2), v_row2 = static_cast<int>(p.v_sl * 2);
     auto tile_rsrc = [&](const bf16_t* base, int row2, int key0) -> u32x4 {
-        const int rows = min(p.L - key0, BN);
+        const int rows = min(keys - key0, BN);
         const int bytes = rows > 0 ? (rows - 1) * row2 + D * 2 : 0;
         const uint64_t addr = reinterpret_cast<uint64_t>(base) + static_cast<uint64_t>(static_cast<int64_t>(key0) * row2);
         u32x4 r;
@@ -236,7 +243,7 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
     }
     constexpr float c = 1.0f;  // the scale is already in Q
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const int ntiles = (p.L + BN - 1) / BN;
+    const int ntiles = (keys + BN - 1) / BN;
 
     bf16x8 kf[KRN];  // K fragment ring, indexed by fragment number % KRN
     bf16x8 vf[VRN];  // V^T fragment ring
@@ -304,7 +311,7 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
         const int key0 = t * BN;
 #pragma unroll
         for (int db = 0; db < DB; ++db) v_cur_addr[db] = v_addr[db] + vcur;
-        if (key0 + BN > p.L) {  // ragged tail: keys past L get -inf
+        if (key0 + BN > keys) {  // ragged tail: keys past the end get -inf
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
@@ -312,7 +319,7 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int key = key0 + kb * 32 + 8 * (r >> 2) + 4 * fhalf + (r & 3);
-                        if (key >= p.L) s_cur[qb][kb][r] = -INFINITY;
+                        if (key >= keys) s_cur[qb][kb][r] = -INFINITY;
                     }
         }
         const u32x4 rk = tile_rsrc(kbase, k_row2, key0 + 3 * BN);
@@ -376,7 +383,8 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
                         for (int r = 0; r < 16; ++r) acc[qb][db][r] *= alpha;
                     m_run[qb] = m_new;
                 }
-                mc[qb] = m_new * c;
+                // a part whose scores are all -inf so far adds nothing, whatever the other parts hold
+                mc[qb] = SPLIT && m_new == -INFINITY ? 0.0f : m_new * c;
                 sum[qb] = 0.0f;
             }
             // ... and the exponentials, two accumulator values per unit, in the order the MFMAs of
@@ -430,7 +438,19 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
         const float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 32, 64);
         const float inv = 1.0f / l_tot;
         const int row = q0 + qb * 32 + frow;
-        if (row < p.L) {
+        if constexpr (SPLIT) {
+            // in the order the lanes hold it (1 KB per store, rows past L included): block = 32 rows of a (batch, head)
+            const int64_t blocks = static_cast<int64_t>(p.total_tiles / splits) * (4 * QB);
+            const int64_t at = part * blocks + (static_cast<int64_t>(bh) * p.n_qtiles + qt) * (4 * QB) + wave * QB + qb;
+            u32x4* wblk = reinterpret_cast<u32x4*>(ws + at * (32 * D)) + lane;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    wblk[(db * 4 + g) * 64] = u32x4{__float_as_uint(acc[qb][db][g * 4 + 0]), __float_as_uint(acc[qb][db][g * 4 + 1]),
+                                                    __float_as_uint(acc[qb][db][g * 4 + 2]), __float_as_uint(acc[qb][db][g * 4 + 3])};
+            if (fhalf == 0) *reinterpret_cast<f32x2*>(ws + splits * blocks * (32 * D) + (at * 32 + frow) * 2) = f32x2{m_run[qb] * c, l_tot};
+        } else if (row < p.L) {
             bf16_t* orow = p.o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(row) * p.o_sl;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
@@ -447,6 +467,49 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
     }
 }
 
+// O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s over the parts of a row, in the order of the keys. A wave
+// takes 32 rows x 32 columns, in the layout the kernel above leaves them in.
+// A part of all -inf scores has m_s = -inf, l_s = 0, O_s = 0 and weight 0; NaNs stay in l_s and O_s.
+template <int D>
+__global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p, const float* ws, int splits, int blocks) {
+    constexpr int DB = D / 32, BPG = 4 / DB;   // blocks of 32 rows per workgroup
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, frow = lane & 31, fhalf = lane >> 5;
+    const int64_t blk = static_cast<int64_t>(blockIdx.x) * BPG + wave / DB;
+    const int db = wave % DB;
+    if (blk >= blocks) return;
+    const int per_bh = p.n_qtiles * 4;
+    const int bh = static_cast<int>(blk / per_bh), row = static_cast<int>(blk % per_bh) * 32 + frow;
+    const f32x2* ml = reinterpret_cast<const f32x2*>(ws + static_cast<int64_t>(splits) * blocks * (32 * D)) + blk * 32 + frow;
+    const Vec16<float>* part = reinterpret_cast<const Vec16<float>*>(ws) + (blk * (8 * D) + db * 256 + lane);
+    float m = -INFINITY, l = 0.0f, acc[16];
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) m = fmaxf(m, ml[static_cast<int64_t>(s) * blocks * 32].x);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+#pragma unroll 2
+    for (int s = 0; s < splits; ++s) {
+        const f32x2 t = ml[static_cast<int64_t>(s) * blocks * 32];
+        const float w = t.x == m ? 1.0f : __builtin_amdgcn_exp2f(t.x - m);
+        l += t.y * w;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const Vec16<float> a = part[static_cast<int64_t>(s) * blocks * (8 * D) + g * 64];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[g * 4 + e] = __builtin_fmaf(a.v[e], w, acc[g * 4 + e]);
+        }
+    }
+    if (row >= p.L) return;
+    const float inv = 1.0f / l;
+    bf16_t* orow = p.o + (bh / p.H) * p.o_sb + (bh % p.H) * p.o_sh + row * p.o_sl + db * 32 + fhalf * 4;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        u32x2 y;
+        y.x = pack2_bf16(acc[g * 4 + 0] * inv, acc[g * 4 + 1] * inv);
+        y.y = pack2_bf16(acc[g * 4 + 2] * inv, acc[g * 4 + 3] * inv);
+        *reinterpret_cast<u32x2*>(orow + g * 8) = y;
+    }
+    if (p.lse != nullptr && db == 0 && fhalf == 0) p.lse[static_cast<int64_t>(bh) * p.L + row] = m + __builtin_amdgcn_logf(l);
+}
 
 #endif  // FLUX_ATTN_W64_D64_UNIT
 
@@ -1144,18 +1207,56 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel_pair(AttnParams p4
     else attn_w64_tile<D, 3, 4>(p3, lds, static_cast<int>(blockIdx.x) - n4, static_cast<int>(gridDim.x) - n4);
 }
 
+constexpr int kAttnCUs = 256;
+
 #ifndef FLUX_ATTN_W64_D64_UNIT
-template <int D, int QB, int BN>
-static void attn_launch_pipe(AttnParams& p, int64_t BH, hipStream_t st) {
-    p.n_qtiles = (p.L + 128 * QB - 1) / (128 * QB);
-    p.total_tiles = static_cast<int>(p.n_qtiles * BH);
+// Parts that the keys are cut in where 128-row workgroups leave half the GPU idle or more, and the keys of a
+// part. A workgroup alone on its CU takes 1.03 us per 64 keys (head dim 128; 0.68 at 64), whatever the
+// rest of the GPU does; a part costs the traffic of its fp32 results, 0.033 us (0.016) per workgroup, and the
+// second launch about 2 us, both fitted to 46 problems of 2 to 24 heads. More than 256 workgroups would
+// share CUs, which gains nothing (LDS-bound). us before -> after at head dim 128, [1, 2, L]: L 1024
+// 22.5 -> 14.1, 2048 38.7 -> 20.2, 4096 70.6 -> 33.3; [1, 4, 4096] 72.5 -> 51.3; [1, 8, 1500] 31.0 -> 27.3 is
+// not taken: below 6 us the host's part in the second launch can cost what the GPU gains.
+static int attn_splits(int64_t BH, int64_t L, int D, int& part_keys) {
+    const int64_t groups = BH * ((L + 127) / 128), key_tiles = (L + 63) / 64;
+    const double tile_us = D == 128 ? 1.03 : 0.68, fixed_us = D == 128 ? 1.8 : 2.4, group_us = D == 128 ? 0.033 : 0.016;
+    double best = 6.0;
+    int parts = 1;
+    part_keys = static_cast<int>(L);
+    for (int64_t s = 2; s <= 8 && s * groups <= kAttnCUs && s <= key_tiles; ++s) {
+        const int64_t part_tiles = (key_tiles + s - 1) / s;
+        const double gain = tile_us * static_cast<double>(key_tiles - part_tiles) - (fixed_us + 0.3 * s + group_us * static_cast<double>(groups * s));
+        if (gain <= best) continue;
+        best = gain;
+        part_keys = static_cast<int>(part_tiles * 64);
+        parts = static_cast<int>((key_tiles + part_tiles - 1) / part_tiles);   // every part has keys
+    }
+    return parts;
+}
+
+// fp32 O, reference maximum and sum of every row of every part; rows in whole workgroups
+static int64_t attn_split_bytes(int64_t BH, int64_t L, int D, int splits) {
+    return splits > 1 ? splits * BH * ((L + 127) / 128 * 128) * (D + 2) * 4 : 0;
+}
+
+template <int D>
+static void attn_launch_pipe(AttnParams& p, int64_t BH, float* ws, int64_t ws_bytes, hipStream_t st) {
+    p.n_qtiles = (p.L + 127) / 128;
+    int part_keys;
+    const int splits = attn_splits(BH, p.L, D, part_keys);
+    const bool split = splits > 1 && ws != nullptr && ws_bytes >= attn_split_bytes(BH, p.L, D, splits);
+    p.total_tiles = static_cast<int>(p.n_qtiles * BH * (split ? splits : 1));
     const int grid = ((p.total_tiles + 7) / 8) * 8;
-    hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, QB, BN>), dim3(grid), dim3(256), 0, st, p);
+    if (!split) {
+        hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, false>), dim3(grid), dim3(256), 0, st, p, nullptr, 1, p.L);
+        return;
+    }
+    hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, true>), dim3(grid), dim3(256), 0, st, p, ws, splits, part_keys);
+    const int blocks = static_cast<int>(p.n_qtiles * BH) * 4, per_group = 128 / D;
+    hipLaunchKernelGGL(attn_combine_kernel<D>, dim3((blocks + per_group - 1) / per_group), dim3(256), 0, st, p, ws, splits, blocks);
 }
 
 #endif
-
-constexpr int64_t kW64MinTiles = 128;
 
 // One workgroup per CU, so a launch of more than one round's worth of equal tiles costs whole
 // rounds: 432 tiles of 256 rows on 256 CUs take as long as 512 would. The rows of every (batch, head)
@@ -1164,8 +1265,6 @@ constexpr int64_t kW64MinTiles = 128;
 // that the last workgroup finishes earliest (attn_launch_w64). 110 592 rows of the Flux shape become
 // 252 + 240 workgroups, 1.8 tile times instead of 2. The two parts are the two block ranges of one
 // launch (attn_fwd_w64_kernel_pair).
-constexpr int kAttnCUs = 256;
-
 // Fills in the tile mapping of one part and returns its grid (a multiple of eight, 0 = no tiles).
 static int attn_w64_part(AttnParams& p, int64_t BH, int cnt_even, int cnt_odd, int first_even, int first_odd) {
     p.cnt_even = cnt_even; p.cnt_odd = cnt_odd; p.first_even = first_even; p.first_odd = first_odd;
@@ -1265,11 +1364,17 @@ void attn_launch_w64_d64(AttnParams& p, int64_t BH, hipStream_t st) { attn_launc
 #ifndef FLUX_ATTN_W64_D64_UNIT
 using namespace flux;
 
+// Whether 128-row workgroups (32 rows per wave) are few enough for one per CU; then they end sooner than half
+// as many 256-row ones (64 rows per wave), which are faster per row only. us on the 32-row and the 64-row kernel,
+// head dim 128: [1, 24, 1280] (240 workgroups) 29 and 35, [1, 8, 4096] (256) 77 and 88, [1, 24, 1500] (288)
+// 47 and 40; head dim 64: 19 and 24, 50 and 60, 32 and 28.
+static bool attn_short(int64_t BH, int64_t L) { return BH * ((L + 127) / 128) <= kAttnCUs; }
+
 static bool view_ok(const void* ptr, int64_t sb, int64_t sh, int64_t sl) {
     return ptr != nullptr && aligned16(ptr) && sb % 8 == 0 && sh % 8 == 0 && sl % 8 == 0;
 }
 
-extern "C" int flux_attention_fwd_bf16(const flux_attn_args* a, void* stream) {
+static int attention_launch(const flux_attn_args* a, void* workspace, int64_t workspace_bytes, hipStream_t st) {
     if (!a) return fail(FLUX_E_NULL, "flux_attention_fwd_bf16: null args");
     if (a->B < 0 || a->H <= 0 || a->L < 0) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: bad shape B=%lld H=%lld L=%lld", (long long)a->B, (long long)a->H, (long long)a->L);
     if (a->D != 16 && a->D != 32 && a->D != 64 && a->D != 128 && a->D != 256)
@@ -1292,17 +1397,30 @@ extern "C" int flux_attention_fwd_bf16(const flux_attn_args* a, void* stream) {
     p.H = (int)a->H; p.L = (int)a->L;
     p.scale_log2 = a->sm_scale * 1.4426950408889634f;
     const int64_t BH = a->B * a->H;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    // Head dim 128: 64 rows per wave (256 per workgroup, one workgroup per CU) once there are enough
-    // such tiles to occupy the chip; smaller problems get 128-row workgroups, two per CU.
-    const int64_t tiles256 = BH * ((a->L + 255) / 256);
     if (a->D != 64 && a->D != 128) {
         if (BH * ((a->L + 63) / 64) > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: problem too large");
         attn_launch_plain(p, BH, a->D, st);
-    } else if (a->D == 128 && tiles256 >= kW64MinTiles) attn_launch_w64<128>(p, BH, st);
-    else if (a->D == 128) attn_launch_pipe<128, 1, 64>(p, BH, st);
-    else if (tiles256 >= kW64MinTiles) attn_launch_w64_d64(p, BH, st);
-    else attn_launch_pipe<64, 1, 64>(p, BH, st);
+    } else if (a->D == 128 && !attn_short(BH, a->L)) attn_launch_w64<128>(p, BH, st);
+    else if (a->D == 128) attn_launch_pipe<128>(p, BH, static_cast<float*>(workspace), workspace_bytes, st);
+    else if (!attn_short(BH, a->L)) attn_launch_w64_d64(p, BH, st);
+    else attn_launch_pipe<64>(p, BH, static_cast<float*>(workspace), workspace_bytes, st);
     return check_launch("flux_attention_fwd_bf16");
+}
+
+extern "C" int flux_attention_fwd_bf16(const flux_attn_args* a, void* stream) {
+    return attention_launch(a, nullptr, 0, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t flux_attention_workspace_bytes(int64_t B, int64_t H, int64_t L, int32_t D) {
+    if (B <= 0 || H <= 0 || L <= 0 || (D != 64 && D != 128) || L > 0x7fffffff / 64 || B > 0x7fffffff / 64 / H) return 0;
+    if (!attn_short(B * H, L)) return 0;
+    int part_keys;
+    return attn_split_bytes(B * H, L, D, attn_splits(B * H, L, D, part_keys));
+}
+
+extern "C" int flux_attention_fwd_bf16_ws(const flux_attn_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace))))
+        return fail(FLUX_E_NULL, "flux_attention_fwd_bf16_ws: workspace must be 16-byte aligned memory");
+    return attention_launch(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 #endif  // FLUX_ATTN_W64_D64_UNIT

@@ -37,7 +37,12 @@ def attention_into(q: Tensor, k: Tensor, v: Tensor, out: Tensor, sm_scale: float
     a.lse = nv.ptr(lse)
     a.B, a.H, a.L, a.D, a.sm_scale = B, H, L, D, float(sm_scale)
     with nv.on_device(dev):
-        rc = nv.lib().flux_attention_fwd_bf16(nv.byref(a), nv.stream_ptr(dev))
+        need = nv.lib().flux_attention_workspace_bytes(B, H, L, D)
+        if need:   # keys cut over several workgroups: partial sums in memory of this launch's stream
+            ws = torch.empty((need,), dtype=torch.uint8, device=dev)
+            rc = nv.lib().flux_attention_fwd_bf16_ws(nv.byref(a), ws.data_ptr(), need, nv.stream_ptr(dev))
+        else:
+            rc = nv.lib().flux_attention_fwd_bf16(nv.byref(a), nv.stream_ptr(dev))
     nv.check(rc, "flux_attention_fwd_bf16")
     return out
 

@@ -229,6 +229,16 @@ typedef struct flux_linear_pair_args {
 int64_t flux_linear_pair_workspace_bytes(const flux_linear_pair_args* args);
 int flux_linear_bf16_pair(const flux_linear_pair_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* What a call would launch, without launching it (nothing here touches the GPU): the kernel family, the output
+ * tile of a workgroup, the parts K is cut in with a workspace of workspace_bytes, and how many of the two
+ * products the launch takes (second may be null; where the two do not share one, first is described). Returns
+ * what the call itself would return for its arguments. */
+enum { FLUX_LINEAR_NOTHING = 0, FLUX_LINEAR_SCALAR = 1, FLUX_LINEAR_ROWS = 2, FLUX_LINEAR_SQUARE = 3, FLUX_LINEAR_RECT = 4, FLUX_LINEAR_EIGHT_WAVES = 5 };
+typedef struct flux_linear_plan {
+    int32_t family, tile_m, tile_n, splits, products;
+} flux_linear_plan;
+int flux_linear_plan_of(const flux_linear_args* first, const flux_linear_args* second, int64_t workspace_bytes, flux_linear_plan* plan);
+
 /* ---------------------------------------------------------------------------------------------
  * Non-causal attention forward: O = softmax(Q K^T * sm_scale) V, bf16 in/out, fp32 online softmax.
  * Replaces scaled_dot_product_attention / _attn_fwd (kernels/attention.py:173-221, 70-170).

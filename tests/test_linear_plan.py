@@ -1,0 +1,69 @@
+"""Which kernel a linear call takes, asked of the library on the host (flux_linear_plan_of): nothing here
+launches or needs a GPU."""
+import ctypes
+import random
+
+import pytest
+
+from triton_kernels import _native as nv
+
+NOTHING, SCALAR, ROWS, SQUARE, RECT, EIGHT_WAVES = range(6)
+PTR = 1 << 20   # stands for an aligned device address; the query reads the arguments only
+NO_LIMIT = 2 ** 62
+
+
+def linear_args(M, N, K, **fields):
+    a = nv.LinearArgs()
+    a.A = a.W = a.Y = PTR
+    a.M, a.N, a.K, a.lda, a.ldw, a.ldy, a.split_n = M, N, K, K, K, N, N
+    for name, value in fields.items():
+        setattr(a, name, value)
+    return a
+
+
+def qk_args(B, L, heads, mlp, K=None, **fields):
+    """linear1 of a single-stream block: q, k and v heads of 128 and the mlp columns behind them."""
+    f = nv.LinearQKFusion()
+    f.q_out = f.k_out = f.q_scale = f.k_scale = f.pe = PTR
+    f.heads, f.seq_len, f.out_len = heads, L, L
+    qkv = 3 * heads * 128
+    split = dict(Y2=PTR, ldy=qkv, ldy2=qkv + mlp, split_n=qkv, act=nv.ACT_GELU_TANH, act_begin=qkv) if mlp else dict(ldy=qkv, act_begin=qkv)
+    a = linear_args(B * L, qkv + mlp, K or heads * 128, **{**split, **fields})
+    a.qk = ctypes.pointer(f)
+    return a
+
+
+def plan_of(first, second=None, workspace=NO_LIMIT):
+    p = nv.LinearPlan()
+    rc = nv.lib().flux_linear_plan_of(nv.byref(first), nv.byref(second) if second is not None else None, workspace, nv.byref(p))
+    assert rc == 0, nv.last_error()
+    return p
+
+
+def test_plan_names_the_route():
+    assert plan_of(linear_args(0, 8, 8)).family == NOTHING
+    assert plan_of(linear_args(4, 8, 8)).family == ROWS
+    assert plan_of(linear_args(4, 8, 7)).family == SCALAR
+    assert plan_of(linear_args(9, 8, 8)).family in (SQUARE, RECT, EIGHT_WAVES)
+    assert plan_of(linear_args(64, 96, 128), linear_args(32, 96, 128)).products == 2
+    assert plan_of(linear_args(64, 96, 128), linear_args(32, 104, 128)).products == 1
+    bad = nv.LinearPlan()
+    assert nv.lib().flux_linear_plan_of(nv.byref(linear_args(9, 8, 8, lda=4)), None, 0, nv.byref(bad)) == -2
+
+
+@pytest.mark.parametrize("far", ["", "ldy", "ldy2", "both"])
+def test_qk_columns_take_a_tile_whose_waves_hold_whole_heads(far):
+    """The q/k epilogue exists where a wave owns 128 columns: tiles of 256 columns. Any admitted fused call
+    must get one, also where a row stride is too long for 32-bit offsets inside a tile (3.73 million
+    elements of 2 bytes times 288 rows)."""
+    rng = random.Random(len(far))
+    for _ in range(300):
+        B, L, heads = rng.randint(1, 3), rng.randint(256, 4700), rng.choice([1, 2, 8, 24])
+        mlp = 256 * rng.choice([0, 1, 2 * heads]) + (128 * heads) % 256   # columns in multiples of 256
+        fields = {}
+        if far in ("ldy", "both"):
+            fields["ldy"] = 3_800_000 // 8 * 8
+        if far in ("ldy2", "both") and mlp:
+            fields["ldy2"] = 4_000_000
+        p = plan_of(qk_args(B, L, heads, mlp, **fields))
+        assert p.tile_n == 256 and p.family in (SQUARE, RECT, EIGHT_WAVES), (B, L, heads, mlp, p.family, p.tile_m, p.tile_n)

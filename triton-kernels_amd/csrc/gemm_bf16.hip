@@ -948,7 +948,7 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
         return (p.split_n >= p.N || p.split_n % w == 0) && (p.act == FLUX_ACT_NONE || p.act_begin >= p.N || p.act_begin % w == 0);
     };
     if (!form) {   // 256-wide tiles once they fill most of the chip, else 128-wide ones, two workgroups per CU
-        const bool big = square_tiles >= 160;
+        const bool big = p.qk_cols > 0 || square_tiles >= 160;   // (whole heads per wave: 256-wide tiles only)
         return {kSquare, big ? 8 : 4, big ? 8 : 4, 1, 0.0};
     }
     TilePlan best = {kSquare, 8, 8, 1, 1e30};
@@ -1110,6 +1110,13 @@ static int set_a_batches(GemmParams& p, int64_t rows, int64_t stride, LinearRout
     return FLUX_OK;
 }
 
+static bool share_launch(const GemmSet& g, const LinearRoute (&route)[2]) {
+    const GemmParams &p = g.p[0], &q = g.p[1];
+    const bool same = route[0] == route[1] && p.N == q.N && p.K == q.K && p.act == q.act && p.act_begin == q.act_begin && p.split_n == q.split_n &&
+                      p.in_silu == q.in_silu && (p.gate != nullptr) == (q.gate != nullptr) && p.qk_cols == q.qk_cols;
+    return same && (route[0] == kTiles || (route[0] == kRows && p.M == q.M));
+}
+
 // One launch for both products where they have the same N, K and form of epilogue, so that the tile grid is
 // that of their rows together; else one after the other through the same workspace (the stream orders them).
 // 1024 + 256 rows of the double-stream block, one launch against two on two streams: 3072 x 9216 weights 59 us
@@ -1123,17 +1130,11 @@ static int linear_pair_launch(const flux_linear_pair_args* a, void* workspace, i
         if (rc == FLUX_OK) rc = set_a_batches(g.p[i], a->a_rows[i], a->a_batch_stride[i], route[i], "flux_linear_bf16_pair");
         if (rc != FLUX_OK) return rc;
     }
-    const GemmParams &p = g.p[0], &q = g.p[1];
-    const bool same = route[0] == route[1] && p.N == q.N && p.K == q.K && p.act == q.act && p.act_begin == q.act_begin && p.split_n == q.split_n &&
-                      p.in_silu == q.in_silu && (p.gate != nullptr) == (q.gate != nullptr) && p.qk_cols == q.qk_cols;
     const bool shared_gpu = ((a->product[0].flags | a->product[1].flags) & FLUX_LINEAR_SHARED_GPU) != 0;
     if (need != nullptr) *need = 0;
-    if (same && route[0] == kTiles) {
+    if (share_launch(g, route)) {
         g.n = 2;
-        return launch_tiles(g, shared_gpu, workspace, workspace_bytes, need, st);
-    }
-    if (same && route[0] == kRows && p.M == q.M) {
-        g.n = 2;
+        if (route[0] == kTiles) return launch_tiles(g, shared_gpu, workspace, workspace_bytes, need, st);
         return need != nullptr ? FLUX_OK : launch_rows(g, st);
     }
     for (int i = 0; i < 2; ++i) {
@@ -1175,4 +1176,25 @@ extern "C" int64_t flux_linear_pair_workspace_bytes(const flux_linear_pair_args*
 extern "C" int flux_linear_bf16_pair(const flux_linear_pair_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
     if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace)))) return fail(FLUX_E_NULL, "flux_linear_bf16_pair: workspace must be 16-byte aligned memory");
     return linear_pair_launch(a, workspace, workspace_bytes, nullptr, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int flux_linear_plan_of(const flux_linear_args* first, const flux_linear_args* second, int64_t workspace_bytes, flux_linear_plan* plan) {
+    if (!plan) return fail(FLUX_E_NULL, "flux_linear_plan_of: null plan");
+    *plan = {FLUX_LINEAR_NOTHING, 0, 0, 1, 1};
+    GemmSet g;
+    LinearRoute route[2];
+    int rc = read_linear_args(first, g.p[0], route[0]);
+    if (rc == FLUX_OK && second) rc = read_linear_args(second, g.p[1], route[1]);
+    if (rc != FLUX_OK) return rc;
+    plan->products = g.n = second && share_launch(g, route) ? 2 : 1;
+    if (route[0] == kScalar) plan->family = FLUX_LINEAR_SCALAR;
+    if (route[0] == kRows) plan->family = FLUX_LINEAR_ROWS;
+    if (route[0] != kTiles) return FLUX_OK;
+    const bool shared_gpu = ((first->flags | (g.n > 1 ? second->flags : 0)) & FLUX_LINEAR_SHARED_GPU) != 0;
+    const TilePlan t = plan_tiles(g, shared_gpu, workspace_bytes);
+    plan->family = t.family == kSquare ? FLUX_LINEAR_SQUARE : t.family == kRect ? FLUX_LINEAR_RECT : FLUX_LINEAR_EIGHT_WAVES;
+    plan->tile_m = 32 * t.fm;
+    plan->tile_n = 32 * t.fn;
+    plan->splits = t.splits;
+    return FLUX_OK;
 }

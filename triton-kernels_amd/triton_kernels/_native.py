@@ -70,6 +70,10 @@ class LinearPairArgs(Structure):
     _fields_ = [("product", LinearArgs * 2), ("a_rows", c_int64 * 2), ("a_batch_stride", c_int64 * 2)]
 
 
+class LinearPlan(Structure):
+    _fields_ = [("family", c_int32), ("tile_m", c_int32), ("tile_n", c_int32), ("splits", c_int32), ("products", c_int32)]
+
+
 class RmsNormArgs(Structure):
     _fields_ = [
         ("x", c_void_p), ("scale", c_void_p), ("y", c_void_p), ("rstd", c_void_p),
@@ -115,6 +119,7 @@ SIGNATURES = {
     "flux_linear_bf16_ws": (c_int32, [POINTER(LinearArgs), c_void_p, c_int64, c_void_p]),
     "flux_linear_pair_workspace_bytes": (c_int64, [POINTER(LinearPairArgs)]),
     "flux_linear_bf16_pair": (c_int32, [POINTER(LinearPairArgs), c_void_p, c_int64, c_void_p]),
+    "flux_linear_plan_of": (c_int32, [POINTER(LinearArgs), POINTER(LinearArgs), c_int64, POINTER(LinearPlan)]),
     "flux_attention_fwd_bf16": (c_int32, [POINTER(AttnArgs), c_void_p]),
     "flux_attention_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int32]),
     "flux_attention_fwd_bf16_ws": (c_int32, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p]),
@@ -234,6 +239,6 @@ def src4(t: torch.Tensor | None) -> Src4:
 
 __all__ = [
     "lib", "lib_path", "check", "last_error", "dtype_code", "require_gpu", "stream_ptr", "on_device", "ptr", "src4",
-    "Src4", "QkvPrepArgs", "LinearArgs", "LinearPairArgs", "RmsNormArgs", "LayerNormArgs", "AttnArgs", "SIGNATURES", "byref",
+    "Src4", "QkvPrepArgs", "LinearArgs", "LinearPairArgs", "LinearPlan", "RmsNormArgs", "LayerNormArgs", "AttnArgs", "SIGNATURES", "byref",
     "FLUX_BF16", "FLUX_F32", "ACT_NONE", "ACT_GELU_TANH", "ACT_SILU", "LINEAR_SHARED_GPU", "MAX_ROW",
 ]

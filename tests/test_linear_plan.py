@@ -67,3 +67,15 @@ def test_qk_columns_take_a_tile_whose_waves_hold_whole_heads(far):
             fields["ldy2"] = 4_000_000
         p = plan_of(qk_args(B, L, heads, mlp, **fields))
         assert p.tile_n == 256 and p.family in (SQUARE, RECT, EIGHT_WAVES), (B, L, heads, mlp, p.family, p.tile_m, p.tile_n)
+
+
+@pytest.mark.parametrize("stride", ["ldy", "ldy2", "ldresid"])
+@pytest.mark.parametrize("M", [40, 320, 700, 2700])
+def test_rows_too_far_apart_for_32_bit_offsets_take_the_checked_epilogue(M, stride):
+    """The rectangular and eight-wave tiles address the rows of a tile by 32-bit byte offsets; the square
+    tiles have an epilogue that does not."""
+    fields = dict(gate=PTR, resid=PTR, rows_per_batch=M, ldresid=3072)
+    if stride == "ldy2":
+        fields.update(Y2=PTR, split_n=1536, ldy2=1536)
+    assert plan_of(linear_args(M, 3072, 3072, **fields)).family != SQUARE
+    assert plan_of(linear_args(M, 3072, 3072, **{**fields, stride: 160_000_000})).family == SQUARE

@@ -265,7 +265,8 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
     const bool fast = p.vec_io && m0 + BM <= p.M && n0 + BN <= p.N && (gelu_all || gelu_none) &&
                       (p.gate == nullptr || m0 / p.rows_per_batch == (m0 + BM - 1) / p.rows_per_batch) &&
                       (wave_n0 + WCOLS <= p.split_n || wave_n0 >= p.split_n) && (p.bias == nullptr || p.bias_vec) &&
-                      static_cast<int64_t>(BM) * p.ldy * 2 < 0x7fffffffLL && static_cast<int64_t>(BM) * p.ldy2 * 2 < 0x7fffffffLL;
+                      static_cast<int64_t>(BM) * p.ldy * 2 < 0x7fffffffLL && static_cast<int64_t>(BM) * p.ldy2 * 2 < 0x7fffffffLL &&
+                      static_cast<int64_t>(BM) * p.ldresid * 2 < 0x7fffffffLL;
     if (fast) {
         if (p.gate != nullptr) {
             if (gelu_all) gemm_epilogue_fast<MI, NJ, true, true>(p, acc, lds, m0, n0, wave, lane);
@@ -940,7 +941,7 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
         const GemmParams& q = g.p[i];
         form = form && q.vec_io && q.N % 8 == 0 && (q.bias == nullptr || q.bias_vec) && !(q.gate != nullptr && q.act != FLUX_ACT_NONE) &&
                q.lda * 2 * 288 < 0x7fffffffLL && q.ldw * 2 * 256 < 0x7fffffffLL && q.ldy * 2 * 288 < 0x7fffffffLL &&
-               q.ldy2 * 2 * 288 < 0x7fffffffLL;   // 32-bit byte offsets inside a tile's rows
+               q.ldy2 * 2 * 288 < 0x7fffffffLL && q.ldresid * 2 * 288 < 0x7fffffffLL;   // 32-bit byte offsets inside a tile's rows
         square_tiles += static_cast<int64_t>((q.M + 255) / 256) * ((q.N + 255) / 256);
     }
     auto columns_ok = [&](int fn) {

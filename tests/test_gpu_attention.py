@@ -233,6 +233,25 @@ def test_attention_lse_at_the_flux_shape():
     torch.testing.assert_close(total, torch.ones_like(total), atol=5e-3, rtol=0)
 
 
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("B,H,L", [(1, 8, 4096), (1, 8, 4000), (2, 24, 520), (128, 1, 100), (1, 24, 1536)])
+def test_attention_lse_sums_unrounded_probabilities(B, H, L, D):
+    """From 128 tiles of 256 rows on a row's sum is that of its fp32 exponentials, on the 128-row and on the
+    256-row workgroups. Every score is exactly -5/64 in the base-2 domain but one, which is 0: the bf16 value of
+    2^(-5/64) is 2.0e-3 (relative) off, the sum of L fp32 terms at most L/2 * 2^-24."""
+    q, k = (torch.zeros(B, H, L, D, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    q[..., 0] = 1
+    k[:, :, 1:, 0] = -5 / 64
+    v = torch.ones_like(q)
+    o = torch.empty_like(q)
+    lse = torch.empty(B, H, L, dtype=torch.float32, device=DEV)
+    tk.attention_into(q, k, v, o, sm_scale=math.log(2.0), lse=lse)
+    want = math.log2(1 + (L - 1) * 2.0 ** (-5 / 64))
+    assert (lse - want).abs().max().item() <= L / 2 * 2.0 ** -24 * math.log2(math.e) + 2.0 ** -20, (lse - want).abs().max().item()
+    # numerator from bf16 probabilities, denominator from fp32 ones: off by that rounding, then rounded to bf16 itself
+    assert (o.float() - 1).abs().max().item() <= 2.0 ** -7
+
+
 # 128-row workgroups whose keys are cut in parts: equal and shorter last parts, a last tile of one key, ragged rows
 _SPLIT = [(1, 2, 2048), (1, 2, 4096), (2, 1, 2049), (1, 2, 1793), (1, 4, 2500), (1, 1, 3000)]
 

@@ -119,7 +119,9 @@ constexpr bool attn_units_in_time(int qb_count, int ns, int db_count, int nslot,
 // SPLIT: the keys are cut in `splits` parts of part_keys (the last may be shorter, none is empty) and a
 // workgroup takes one part of them; it stores O^T unnormalised, the reference maximum and the sum of
 // its rows as fp32 to ws, and attn_combine_kernel adds the parts.
-template <int D, int QB, int BN, bool SPLIT>  // BN = keys per tile (32 or 64)
+// FSUM: a row's sum is that of its fp32 exponentials, as in the 64-row kernel; else that of the probabilities
+// rounded to bf16, one instruction for two of them, which round like the numerator they divide.
+template <int D, int QB, int BN, bool SPLIT, bool FSUM>  // BN = keys per tile (32 or 64)
 __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(AttnParams p, float* ws, int splits, int part_keys) {
     constexpr int KB = BN / 32;         // 32-key blocks of S^T per tile
     constexpr int PS = BN / 16;         // 16-key steps of P^T per tile
@@ -401,8 +403,9 @@ __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(A
                 const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(a0, c, -mc[qb]));
                 const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(a1, c, -mc[qb]));
                 pw[qb][u] = pack2_bf16(p0, p1);
+                if (FSUM) sum[qb] += p0 + p1;
                 // row sum from the rounded values, two per instruction: sum += p0*1 + p1*1
-                sum[qb] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pw[qb][u]), __builtin_bit_cast(bf16x2, 0x3f803f80u), sum[qb], false);
+                else sum[qb] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pw[qb][u]), __builtin_bit_cast(bf16x2, 0x3f803f80u), sum[qb], false);
                 if (u % 4 == 3) {  // a 16-key step of P^T is complete
                     const u32x4 v4 = {pw[qb][u - 3], pw[qb][u - 2], pw[qb][u - 1], pw[qb][u]};
                     pf[qb][u / 4] = __builtin_bit_cast(bf16x8, v4);
@@ -1239,6 +1242,12 @@ static int64_t attn_split_bytes(int64_t BH, int64_t L, int D, int splits) {
     return splits > 1 ? splits * BH * ((L + 127) / 128 * 128) * (D + 2) * 4 : 0;
 }
 
+// From this many tiles of 256 rows on a call sums its fp32 exponentials whichever kernel it takes (FSUM). us on the
+// 64-row kernel, on this one with rounded and with fp32 sums, head dim 128 (64): [1, 8, 4096] 88.9 (61.0), 83 (50.6),
+// 85.7 (52.1); [2, 24, 640] 23.7 (16.7), 18.8 (13.8), 19.0 (13.3); [1, 16, 2000] 50.6 (35.1), 42.7 (28.2), 43.4 (28.9).
+// Relative error of O against float64, same order, [1, 8, 4096]: 2.87e-3 (2.89e-3), 2.81e-3 (2.83e-3) for both sums.
+constexpr int64_t kFsumTiles = 128;
+
 template <int D>
 static void attn_launch_pipe(AttnParams& p, int64_t BH, float* ws, int64_t ws_bytes, hipStream_t st) {
     p.n_qtiles = (p.L + 127) / 128;
@@ -1248,10 +1257,11 @@ static void attn_launch_pipe(AttnParams& p, int64_t BH, float* ws, int64_t ws_by
     p.total_tiles = static_cast<int>(p.n_qtiles * BH * (split ? splits : 1));
     const int grid = ((p.total_tiles + 7) / 8) * 8;
     if (!split) {
-        hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, false>), dim3(grid), dim3(256), 0, st, p, nullptr, 1, p.L);
+        if (BH * ((p.L + 255) / 256) >= kFsumTiles) hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, false, true>), dim3(grid), dim3(256), 0, st, p, nullptr, 1, p.L);
+        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, false, false>), dim3(grid), dim3(256), 0, st, p, nullptr, 1, p.L);
         return;
     }
-    hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, true>), dim3(grid), dim3(256), 0, st, p, ws, splits, part_keys);
+    hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, true, false>), dim3(grid), dim3(256), 0, st, p, ws, splits, part_keys);
     const int blocks = static_cast<int>(p.n_qtiles * BH) * 4, per_group = 128 / D;
     hipLaunchKernelGGL(attn_combine_kernel<D>, dim3((blocks + per_group - 1) / per_group), dim3(256), 0, st, p, ws, splits, blocks);
 }
@@ -1366,8 +1376,8 @@ using namespace flux;
 
 // Whether 128-row workgroups (32 rows per wave) are few enough for one per CU; then they end sooner than half
 // as many 256-row ones (64 rows per wave), which are faster per row only. us on the 32-row and the 64-row kernel,
-// head dim 128: [1, 24, 1280] (240 workgroups) 29 and 35, [1, 8, 4096] (256) 77 and 88, [1, 24, 1500] (288)
-// 47 and 40; head dim 64: 19 and 24, 50 and 60, 32 and 28.
+// head dim 128: [1, 24, 1280] (240 workgroups) 29 and 35, [1, 8, 4096] (256) 86 and 89, [1, 24, 1500] (288)
+// 47 and 40; head dim 64: 19 and 24, 52 and 61, 32 and 28.
 static bool attn_short(int64_t BH, int64_t L) { return BH * ((L + 127) / 128) <= kAttnCUs; }
 
 static bool view_ok(const void* ptr, int64_t sb, int64_t sh, int64_t sl) {

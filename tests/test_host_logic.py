@@ -150,3 +150,19 @@ def test_bench_reads_traffic_from_the_committed_summary_and_refuses_more_gpus():
     assert algorithmic < traffic < 8 * algorithmic
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0 and "one GPU" in (r.stderr + r.stdout)
+
+
+def test_attention_asks_for_a_workspace_wherever_the_library_wants_one():
+    """The Python rule that spares a call the question must not answer no where the library cuts the keys."""
+    from triton_kernels import _native as nv
+    from triton_kernels.kernels.attention import _may_cut_keys
+    asked = 0
+    for L in [*range(1, 1500, 7), *range(640, 1025), *range(1500, 20000, 61)]:
+        for H in (1, 2, 3, 5, 8, 12, 16, 20, 21, 24, 43, 64, 128, 129, 256):
+            for D in (64, 128):
+                if not _may_cut_keys(H, L):
+                    assert nv.lib().flux_attention_workspace_bytes(1, H, L, D) == 0, (H, L, D)
+                else:
+                    asked += nv.lib().flux_attention_workspace_bytes(1, H, L, D) > 0
+    assert asked > 100                                                       # and it does say yes
+    assert not _may_cut_keys(96, 1024) and not _may_cut_keys(24, 1280)      # 24 heads: never

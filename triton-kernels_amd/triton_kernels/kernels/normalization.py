@@ -21,27 +21,28 @@ def _as_4d_view(x: torch.Tensor):
         x = x.contiguous()
         if x.dim() > 4:
             x = x.reshape(-1, x.shape[-1])
-    lead = list(x.shape[:-1])
-    strides = list(x.stride()[:-1])
-    while len(lead) < 3:
-        lead.insert(0, 1)
-        strides.insert(0, 0)
+    lead, strides = tuple(x.shape)[:-1], x.stride()[:-1]
+    short = 3 - len(lead)
+    if short:
+        lead, strides = (1,) * short + lead, (0,) * short + strides
     return x, lead, strides
 
 
 def _rms_norm_args(x: torch.Tensor, scale: torch.Tensor, want_rstd: bool = False):
-    """The call's arguments, its outputs and the tensors that have to live until it is launched."""
-    assert x.shape[-1] == scale.shape[-1]
+    """The call's arguments in the order of nv.RmsNormArgs, its outputs and the tensors that have to live until
+    it is launched."""
+    shape, dtype = x.shape, x.dtype
+    assert shape[-1] == scale.shape[-1]
     dev = nv.require_gpu(x, scale)
-    calculate_settings(x.shape[-1])  # raises for rows wider than 65536, like the reference
+    if shape[-1] > nv.MAX_ROW:
+        calculate_settings(shape[-1])  # raises, like the reference
     scale = scale.contiguous()
-    if scale.dtype != x.dtype and not (x.dtype == torch.bfloat16 and scale.dtype == torch.float32):
-        scale = scale.to(x.dtype)
+    if scale.dtype != dtype and not (dtype == torch.bfloat16 and scale.dtype == torch.float32):
+        scale = scale.to(dtype)
     xv, lead, strides = _as_4d_view(x)
-    y = torch.empty(x.shape, dtype=x.dtype, device=dev)
+    y = torch.empty(shape, dtype=dtype, device=dev)
     rstd = torch.empty((lead[0] * lead[1] * lead[2],), dtype=torch.float32, device=dev) if want_rstd else None
-    a = nv.RmsNormArgs(xv.data_ptr(), scale.data_ptr(), y.data_ptr(), nv.ptr(rstd), *lead, *strides)
-    return a, y, rstd, (xv, scale)
+    return (xv.data_ptr(), scale.data_ptr(), y.data_ptr(), rstd.data_ptr() if want_rstd else None, *lead, *strides), y, rstd, (xv, scale)
 
 
 def rms_norm_forward(x: torch.Tensor, scale: torch.Tensor, eps: float = 1e-6, want_rstd: bool = False):
@@ -49,7 +50,7 @@ def rms_norm_forward(x: torch.Tensor, scale: torch.Tensor, eps: float = 1e-6, wa
     dev = y.device
     with nv.on_device(dev):
         rc = nv.lib().flux_rms_norm(
-            a.x, a.scale, a.y, a.rstd, a.d0, a.d1, a.d2, y.shape[-1], a.s0, a.s1, a.s2,
+            *a[:7], y.shape[-1], *a[7:],
             nv.dtype_code(y), nv.dtype_code(scale), float(eps), nv.stream_ptr(dev))
     nv.check(rc, "flux_rms_norm")
     return y, rstd, xv
@@ -118,7 +119,7 @@ class _rms_norm_pair(torch.autograd.Function):
         dev = y0.device
         with nv.on_device(dev):
             rc = nv.lib().flux_rms_norm_pair(
-                nv.byref(a0), nv.byref(a1), y0.shape[-1], nv.dtype_code(y0), nv.dtype_code(s0), float(eps), nv.stream_ptr(dev))
+                nv.byref(nv.RmsNormArgs(*a0)), nv.byref(nv.RmsNormArgs(*a1)), y0.shape[-1], nv.dtype_code(y0), nv.dtype_code(s0), float(eps), nv.stream_ptr(dev))
         nv.check(rc, "flux_rms_norm_pair")
         return y0, y1
 
@@ -140,7 +141,7 @@ def layer_norm_modulation(x: torch.Tensor, weight: torch.Tensor, bias: torch.Ten
     dev = y.device
     with nv.on_device(dev):
         rc = nv.lib().flux_layer_norm_modulation(
-            a.x, a.scale, a.shift, a.y, a.batch, a.seq, y.shape[-1], a.mod_batch_stride, nv.dtype_code(y), float(eps), nv.stream_ptr(dev))
+            *a[:6], y.shape[-1], a[6], nv.dtype_code(y), float(eps), nv.stream_ptr(dev))
     nv.check(rc, "flux_layer_norm_modulation")
     return y
 
@@ -152,18 +153,22 @@ def layer_norm_modulation_pair(first: tuple, second: tuple, eps=1e-5) -> tuple[t
     assert y0.shape[-1] == y1.shape[-1] and y0.dtype == y1.dtype and y0.device == y1.device
     dev = y0.device
     with nv.on_device(dev):
-        rc = nv.lib().flux_layer_norm_modulation_pair(nv.byref(a0), nv.byref(a1), y0.shape[-1], nv.dtype_code(y0), float(eps), nv.stream_ptr(dev))
+        rc = nv.lib().flux_layer_norm_modulation_pair(
+            nv.byref(nv.LayerNormArgs(*a0)), nv.byref(nv.LayerNormArgs(*a1)), y0.shape[-1], nv.dtype_code(y0), float(eps), nv.stream_ptr(dev))
     nv.check(rc, "flux_layer_norm_modulation_pair")
     return y0, y1
 
 
 def _layer_norm_args(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor):
-    """The call's arguments, its output and the tensors that have to live until it is launched."""
-    assert x.shape[0] == weight.shape[0] == bias.shape[0]
-    assert x.shape[-1] == weight.shape[-1] == bias.shape[-1]
+    """The call's arguments in the order of nv.LayerNormArgs, its output and the tensors that have to live until
+    it is launched."""
+    shape, weight_shape, bias_shape = x.shape, weight.shape, bias.shape
+    batch, n = shape[0], shape[-1]
+    assert batch == weight_shape[0] == bias_shape[0]
+    assert n == weight_shape[-1] == bias_shape[-1]
     nv.require_gpu(x, weight, bias)
-    batch, n = x.shape[0], x.shape[-1]
-    calculate_settings(n)
+    if n > nv.MAX_ROW:
+        calculate_settings(n)
     x = x.contiguous()
     if weight.dtype != x.dtype:
         weight = weight.to(x.dtype)
@@ -179,5 +184,4 @@ def _layer_norm_args(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor):
         mod_stride = weight.stride(0)
     y = torch.empty_like(x)
     rows = x.numel() // n
-    a = nv.LayerNormArgs(x.data_ptr(), weight.data_ptr(), bias.data_ptr(), y.data_ptr(), batch, rows // batch if batch else 0, mod_stride)
-    return a, y, (x, weight, bias)
+    return (x.data_ptr(), weight.data_ptr(), bias.data_ptr(), y.data_ptr(), batch, rows // batch if batch else 0, mod_stride), y, (x, weight, bias)

@@ -158,3 +158,24 @@ def test_gemm_generated_code_does_not_spill(tmp_path):
         pytest.skip("library not built in this tree")
     assert chk.check(path, "gemm_nt_ring_kernel") == []
     assert chk.check(path, "gemm_nt_rect_kernel") == []
+
+
+def test_gemm_kernels_load_their_parameters_once(tmp_path):
+    """A kernel that serves one of two products must not load its parameters again at every use: the checker
+    counts scalar loads, and the assembly the build keeps passes it."""
+    import importlib.util
+    import pytest
+    here = os.path.dirname(os.path.abspath(__file__))
+    spec = importlib.util.spec_from_file_location("check_no_scratch", os.path.join(here, "..", "triton-kernels_amd", "csrc", "check_no_scratch.py"))
+    chk = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(chk)
+    f = tmp_path / "g.s"
+    f.write_text("_ZN4flux19gemm_nt_rect_kernelE:\n" + "\ts_load_dword s0, s[0:1], 0x0\n" * 5 + "\ts_endpgm\n.Lfunc_end0:\n\ts_load_dword s0, s[0:1], 0x0\n")
+    assert chk.check(str(f), "gemm_nt_rect_kernel", 5) == [] and len(chk.check(str(f), "gemm_nt_rect_kernel", 4)) == 1
+    unit = os.path.join(here, "..", "build", "csrc", "%s-hip-amdgcn-amd-amdhsa-gfx950.s")
+    if not os.path.exists(unit % "gemm_bf16"):
+        pytest.skip("library not built in this tree")
+    for name in ("gemm_nt_ring_kernelILi2E", "gemm_nt_ring_kernelILi4ELb0ELb0E", "gemm_nt_ring_kernelILi4ELb1ELb0E", "gemm_nt_rect_kernel", "gemv_small_m_kernel"):
+        assert chk.check(unit % "gemm_bf16", name, 64) == [], name
+    for name in ("gemm_nt_pair_kernel", "gemm_reduce_kernel"):
+        assert chk.check(unit % "gemm_pair", name, 64) == [], name

@@ -494,13 +494,16 @@ __device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, 
 }
 
 
-template <int MI, bool KTAIL>
+// TWO: the launch may hold two products. The 256-wide tile has a form without, which reads its parameters as plain
+// kernel arguments: a copy of them (see product_of_tile) does not fit its scalar registers, and with two products
+// it takes them by reference.
+template <int MI, bool KTAIL, bool TWO>
 __global__ __launch_bounds__(kGemmThreads) void gemm_nt_ring_kernel(GemmLaunch L) {
     constexpr int BM = 64 * MI, BK = 64, NU = 5, UNIT = BM * BK * 2;
     __shared__ __attribute__((aligned(1024))) char lds[NU * UNIT];
     int tm, tn;
     if (L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BM, tm, tn) : !tile_of_block(L, tm, tn)) return;
-    const GemmParams& p = product_of_tile(L, tm);
+    std::conditional_t<MI == 4, const GemmParams&, const GemmParams> p = L.p[TWO ? product_of_tile(L, tm) : 0];
     const int m0 = tm * BM, n0 = tn * BM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -686,7 +689,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_rect_kernel(GemmLaunch L
     __shared__ __attribute__((aligned(1024))) char lds[(3 * BM + 2 * BN) * BK * 2];
     int tm, tn;
     if (FN == 8 && L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
-    const GemmParams& p = product_of_tile(L, tm);
+    const GemmParams p = L.p[product_of_tile(L, tm)];
     const int m0 = tm * BM, n0 = tn * BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -716,7 +719,7 @@ constexpr int gemv_depth(int rows) { return rows <= 2 ? 6 : 3; }
 // EXACT: K = 512 * U, so every lane has exactly U vectors per row and the K loop runs once, without tests.
 template <int MM, bool SILU_LDS, bool EXACT>
 __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
-    const GemmParams& p = g.p[blockIdx.y];
+    const GemmParams p = g.p[blockIdx.y];
     constexpr int CPW = kGemvCols, U = gemv_depth(MM);  // CPW * U 16-byte loads of W in flight per lane: a whole row of 3072
     extern __shared__ __attribute__((aligned(16))) char act_lds[];
     const int lane = threadIdx.x & 63;
@@ -857,11 +860,11 @@ __global__ __launch_bounds__(256) void gemm_nt_scalar_kernel(GemmParams p) {
     *dst = f2bf(t);
 }
 
-template <int MI>
+template <int MI, bool TWO>
 static void launch_tiled(const GemmSet& g, hipStream_t st) {
     const GemmLaunch L = make_launch(g, 64 * MI, 64 * MI);
-    if (g.p[0].K % 64 == 0) hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, false>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
-    else hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, true>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+    if (g.p[0].K % 64 == 0) hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, false, TWO>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+    else hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, true, TWO>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
 }
 
 template <int FM, int FN>
@@ -1073,7 +1076,11 @@ static int launch_tiles(const GemmSet& g, bool shared_gpu, void* workspace, int6
         return FLUX_OK;
     }
     switch (plan.family) {
-        case kSquare: if (plan.fm == 8) launch_tiled<4>(g, st); else launch_tiled<2>(g, st); break;
+        case kSquare:
+            if (plan.fm != 8) launch_tiled<2, true>(g, st);
+            else if (g.n > 1) launch_tiled<4, true>(g, st);
+            else launch_tiled<4, false>(g, st);
+            break;
         case kRect:
             if (plan.fm == 9) launch_rect<9, 6>(g, st);
             else if (plan.fm == 8) launch_rect<8, 6>(g, st);

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
     } else {
         if (FN == 8 && L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
     }
-    const GemmParams& p = product_of_tile(L, tm);
+    const GemmParams p = L.p[product_of_tile(L, tm)];
     const int m0 = tm * BM, n0 = tn * BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_reduce_kernel(GemmLaunch L)
     const int t = blockIdx.x / FM, row = blockIdx.x - t * FM;
     int tm, tn;
     tile_at(L, t, tm, tn);
-    const GemmParams& p = product_of_tile(L, tm);
+    const GemmParams p = L.p[product_of_tile(L, tm)];
     const int m0 = tm * BM, n0 = tn * BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -236,6 +236,8 @@ int flux_linear_bf16_pair(const flux_linear_pair_args* args, void* workspace, in
 enum { FLUX_LINEAR_NOTHING = 0, FLUX_LINEAR_SCALAR = 1, FLUX_LINEAR_ROWS = 2, FLUX_LINEAR_SQUARE = 3, FLUX_LINEAR_RECT = 4, FLUX_LINEAR_EIGHT_WAVES = 5 };
 typedef struct flux_linear_plan {
     int32_t family, tile_m, tile_n, splits, products;
+    int32_t head_rows;   /* > 0: only this many rows take that tile, the others follow on eight-wave tiles */
+    int32_t checked;     /* 1: the tile's epilogue can decide per column and address rows in 64 bits (square tiles always) */
 } flux_linear_plan;
 int flux_linear_plan_of(const flux_linear_args* first, const flux_linear_args* second, int64_t workspace_bytes, flux_linear_plan* plan);
 

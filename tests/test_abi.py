@@ -175,7 +175,7 @@ def test_gemm_kernels_load_their_parameters_once(tmp_path):
     unit = os.path.join(here, "..", "build", "csrc", "%s-hip-amdgcn-amd-amdhsa-gfx950.s")
     if not os.path.exists(unit % "gemm_bf16"):
         pytest.skip("library not built in this tree")
-    for name in ("gemm_nt_ring_kernelILi2E", "gemm_nt_ring_kernelILi4ELb0ELb0E", "gemm_nt_ring_kernelILi4ELb1ELb0E", "gemm_nt_rect_kernel", "gemv_small_m_kernel"):
+    for name in ("gemm_nt_ring_kernelILi4ELb0ELb0E", "gemm_nt_ring_kernelILi4ELb1ELb0E", "gemm_nt_rect_kernel", "gemv_small_m_kernel"):
         assert chk.check(unit % "gemm_bf16", name, 64) == [], name
     for name in ("gemm_nt_pair_kernel", "gemm_reduce_kernel"):
         assert chk.check(unit % "gemm_pair", name, 64) == [], name

@@ -348,6 +348,42 @@ def test_linear_tile_edges(B, L, N, K, splits):
     assert ((y0.float() - ref32).abs() <= half_ulp_bound(ref32)).all()
 
 
+@pytest.mark.parametrize("B,L,N,K,split,act_begin", [
+    (1, 9, 3, 64, None, 0), (1, 65, 97, 128, 50, 33),        # less than a tile; a segment of 8 columns on both sides of the split
+    (2, 100, 1001, 72, 1000, 1000), (3, 43, 201, 4096, None, 7),   # K tail; K over several workgroups, batch elements inside a tile
+    (1, 320, 3073, 640, 8, 3000), (1, 700, 6001, 64, 3080, 3080),  # several sizes of eight-wave tiles
+    (3, 1000, 1001, 192, 500, 0), (1, 2300, 6001, 192, None, 0), (4, 1000, 3073, 3072, 500, 0),
+    (6, 250, 12289, 3072, 12000, 12288), (6, 256, 12289, 3072, None, 0),   # 256-wide tiles, the last rows on 128-wide ones
+])
+def test_linear_outside_the_branch_free_form(B, L, N, K, split, act_begin):
+    """Columns of any number, outputs that are not 16-byte addressable, a split and the first GELU column
+    anywhere, GELU in front of the gate: against the fp32 product, half a bf16 ulp per rounding plus the spread of an
+    fp32 sum in another order."""
+    g = seeded(B + L + N + K)
+    M, S = B * L, N if split is None else split
+    a = randn(g, M, K, dtype=torch.bfloat16).to(DEV)
+    w = randn(g, N, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV)
+    b = randn(g, N, dtype=torch.bfloat16, std=0.5).to(DEV)
+    plain32, gelu32 = oracle.linear_ref_fp32(a, w, b), oracle.linear_ref_fp32(a, w, b, "GELU")
+    ref32 = torch.cat([plain32[:, :act_begin], gelu32[:, act_begin:]], dim=1)
+    for pad in (0, 1):     # outputs with rows at any element
+        y = torch.full((M, S + pad), float("nan"), dtype=torch.bfloat16, device=DEV)
+        y2 = torch.full((M, N - S + 3), float("nan"), dtype=torch.bfloat16, device=DEV)
+        tk.linear_into(a, w, b, activation="GELU", act_begin=act_begin, out=y[:, pad:], **({} if split is None else dict(out2=y2[:, 3:], split=split)))
+        got = torch.cat([y[:, pad:], y2[:, 3:]], dim=1).float()
+        assert ((got - ref32).abs() <= half_ulp_bound(ref32)).all()
+        assert y[:, :pad].isnan().all() and y2[:, :3].isnan().all()    # nothing beside the outputs is written
+    if split is None:
+        x = randn(g, B, L, N, dtype=torch.bfloat16).to(DEV)
+        gate = randn(g, B, 1, N, dtype=torch.bfloat16).to(DEV)
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        tk.linear_into(a, w, b, activation="GELU", act_begin=act_begin, out=out, resid=x.view(M, N), gate=gate)
+        gy = (gate.float() * ref32.view(B, L, N)).view(M, N)
+        want32 = x.view(M, N).float() + gy
+        bound = half_ulp_bound(ref32) * gate.float().abs().expand(B, L, N).reshape(M, N) + 2.0 ** -8 * 1.01 * (gy.abs() + want32.abs()) + 1e-6
+        assert ((out.float() - want32).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("B,L0,L1,N,K", [
     (1, 65, 9, 96, 128),          # one tile row each, the smallest tiles
     (3, 43, 21, 3072, 4096),      # K over several workgroups, batch elements inside a tile

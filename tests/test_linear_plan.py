@@ -72,10 +72,37 @@ def test_qk_columns_take_a_tile_whose_waves_hold_whole_heads(far):
 @pytest.mark.parametrize("stride", ["ldy", "ldy2", "ldresid"])
 @pytest.mark.parametrize("M", [40, 320, 700, 2700])
 def test_rows_too_far_apart_for_32_bit_offsets_take_the_checked_epilogue(M, stride):
-    """The rectangular and eight-wave tiles address the rows of a tile by 32-bit byte offsets; the square
-    tiles have an epilogue that does not."""
+    """The branch-free epilogue of the rectangular and eight-wave tiles addresses the rows of a tile by 32-bit
+    byte offsets; the checked one does not."""
     fields = dict(gate=PTR, resid=PTR, rows_per_batch=M, ldresid=3072)
     if stride == "ldy2":
         fields.update(Y2=PTR, split_n=1536, ldy2=1536)
-    assert plan_of(linear_args(M, 3072, 3072, **fields)).family != SQUARE
-    assert plan_of(linear_args(M, 3072, 3072, **{**fields, stride: 160_000_000})).family == SQUARE
+    assert not plan_of(linear_args(M, 3072, 3072, **fields)).checked
+    assert plan_of(linear_args(M, 3072, 3072, **{**fields, stride: 160_000_000})).checked
+
+
+@pytest.mark.parametrize("M", [9, 64, 128, 300, 512, 1024])
+@pytest.mark.parametrize("N,fields", [
+    (100, {}), (1001, {}), (3073, {}),                                                    # columns no multiple of 8
+    (3072, dict(Y2=PTR, split_n=1000, ldy=1000, ldy2=2072)),                              # a split no tile has at a wave's edge
+    (3072, dict(act=nv.ACT_GELU_TANH, act_begin=1000)), (3072, dict(Y=PTR + 2)),
+    (3072, dict(act=nv.ACT_GELU_TANH, gate=PTR, resid=PTR, rows_per_batch=1 << 20, ldresid=3072)),
+])
+def test_calls_outside_the_branch_free_form_still_get_small_tiles(M, N, fields):
+    """256-wide tiles leave almost the whole GPU idle at these sizes, and 128-wide ones walk K with too few
+    loads in flight: 64 x 3072 x 3072 with 1000 columns in the first output takes 12 us on eight-wave tiles and 63 us
+    on the 256-wide one, 300 x 1001 x 3072 13 us and 30 us on 128-wide ones."""
+    p = plan_of(linear_args(M, N, 3072, **fields))
+    assert p.family == EIGHT_WAVES and p.checked, (p.family, p.tile_m, p.tile_n)
+    pair = plan_of(linear_args(M, N, 3072, **fields), linear_args(M // 3 + 9, N, 3072, **fields))
+    assert pair.products == 2 and pair.family == EIGHT_WAVES and pair.checked
+
+
+def test_a_nearly_empty_last_round_is_cut_off():
+    """1500 x 12289 outputs are 294 tiles of 256 x 256, a second round of 38 of them: five tile rows are one round,
+    and the 220 rows behind them go to 128-wide tiles. Only where one batch element's rows stay together."""
+    p = plan_of(linear_args(1500, 12289, 3072))
+    assert (p.family, p.tile_m, p.head_rows) == (SQUARE, 256, 1280)
+    gated = dict(gate=PTR, resid=PTR, ldresid=12289)
+    assert plan_of(linear_args(1500, 12289, 3072, rows_per_batch=256, **gated)).head_rows == 1280
+    assert plan_of(linear_args(1500, 12289, 3072, rows_per_batch=1500, **gated)).head_rows == 0

@@ -24,113 +24,6 @@
 
 namespace flux {
 
-template <int MI, int NJ>
-__device__ __forceinline__ void gemm_epilogue_checked(const GemmParams& p, f32x4 (&acc)[2 * MI][2 * NJ], char* lds, int m0, int n0,
-                                                   int wave, int lane) {
-    constexpr int WROWS = 32 * MI, WCOLS = 32 * NJ;
-    constexpr int C_PITCH = WCOLS * 2, C_CH = WCOLS / 8;  // bytes per row, 16-byte chunks per row
-    constexpr int RPI = 64 / C_CH;                         // rows one wave-wide 16-byte access covers
-    constexpr int NQ = 2 * NJ;                             // column quads of a lane: one per 16-column fragment
-    const int wm = wave >> 1, wn = wave & 1;
-    const int frow = lane & 15, fq = lane >> 4;            // accumulator: row frow of a 16-row fragment, columns fq*4..+3
-    char* cw = lds + wave * (WROWS * C_PITCH);
-    const int wave_n0 = n0 + wn * WCOLS;
-    const int wave_m0 = m0 + wm * WROWS;
-
-    // bias for the lane's NQ column quads
-    float bv[NQ][4];
-    const bool bias_fast = p.bias != nullptr && p.bias_vec;
-    if (bias_fast) {
-        const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.bias), 0, p.N * 2, kRsrcFlags);
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const u32x2 raw = __builtin_amdgcn_raw_buffer_load_b64(rb, (wave_n0 + q * 16 + fq * 4) * 2, 0, 0);
-            bv[q][0] = __uint_as_float(raw.x << 16);
-            bv[q][1] = __uint_as_float(raw.x & 0xffff0000u);
-            bv[q][2] = __uint_as_float(raw.y << 16);
-            bv[q][3] = __uint_as_float(raw.y & 0xffff0000u);
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int n = wave_n0 + q * 16 + fq * 4 + e;
-                bv[q][e] = (p.bias != nullptr && n < p.N) ? bf2f(p.bias[n]) : 0.0f;
-            }
-    }
-
-    // LDS write address of column quad q in this lane's row, without the 16-row fragment offset
-    int waddr[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) waddr[q] = frow * C_PITCH + (((q * 2 + (fq >> 1)) ^ (frow & (C_CH - 1))) * 16) + (fq & 1) * 8;
-    // read side: lane -> (row within the pass = lane / C_CH, chunk = lane % C_CH)
-    const int rrow = lane / C_CH, rch = lane % C_CH;
-
-    const bool gelu_all = p.act == FLUX_ACT_GELU_TANH && wave_n0 >= p.act_begin;
-    const bool gelu_some = p.act == FLUX_ACT_GELU_TANH && !gelu_all && wave_n0 + WCOLS > p.act_begin;
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        // ---- accumulators of block row i (two 16-row fragments) -> bf16 -> LDS
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = acc[2 * i + t][q][e] + bv[q][e];
-                if (gelu_all) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = tanh_gelu_fast(v[e]);
-                } else if (gelu_some) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (wave_n0 + q * 16 + fq * 4 + e >= p.act_begin) v[e] = tanh_gelu_fast(v[e]);
-                }
-                *reinterpret_cast<u32x2*>(cw + (i * 32 + t * 16) * C_PITCH + waddr[q]) = pack4_bf16(v[0], v[1], v[2], v[3]);
-            }
-        __builtin_amdgcn_wave_barrier();  // LDS operations of one wave complete in order
-
-        // ---- the 32 rows leave as 16-byte segments
-#pragma unroll
-        for (int it = 0; it < 32 / RPI; ++it) {
-            const int row = i * 32 + it * RPI + rrow;
-            const int m = wave_m0 + row, n = wave_n0 + rch * 8;
-            Vec16<bf16_t> y = *reinterpret_cast<const Vec16<bf16_t>*>(cw + row * C_PITCH + ((rch ^ (row & (C_CH - 1))) * 16));
-            if (m >= p.M || n >= p.N) continue;
-            const bool full = p.vec_io && n + 8 <= p.N;
-            if (p.gate != nullptr) {
-                const bf16_t* gp = p.gate + static_cast<int64_t>(m / p.rows_per_batch) * p.gate_stride + n;
-                const bf16_t* rp = p.resid + static_cast<int64_t>(m) * p.ldresid + n;
-                if (full) {
-                    Vec16<bf16_t> gt = ld16(gp), rs = ld16(rp);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) y.v[e] = f2bf(bf2f(rs.v[e]) + bf2f(f2bf(bf2f(gt.v[e]) * bf2f(y.v[e]))));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (n + e < p.N) y.v[e] = f2bf(bf2f(rp[e]) + bf2f(f2bf(bf2f(gp[e]) * bf2f(y.v[e]))));
-                }
-            }
-            if (full && (n + 8 <= p.split_n || n >= p.split_n)) {
-                bf16_t* dst = n < p.split_n ? p.Y + static_cast<int64_t>(m) * p.ldy + n
-                                            : p.Y2 + static_cast<int64_t>(m) * p.ldy2 + (n - p.split_n + p.y2_col0);
-                st16(dst, y);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int ne = n + e;
-                    if (ne < p.N) {
-                        bf16_t* dst = ne < p.split_n ? p.Y + static_cast<int64_t>(m) * p.ldy + ne
-                                                     : p.Y2 + static_cast<int64_t>(m) * p.ldy2 + (ne - p.split_n + p.y2_col0);
-                        *dst = y.v[e];
-                    }
-                }
-            }
-        }
-    }
-}
-
 // Branch-free epilogue for interior tiles whose outputs (and residual operands) are 16-byte
 // addressable and whose columns all go to one destination. GELU is all-or-nothing for the wave.
 // Everything lane-dependent is computed once; per store only a wave-uniform row offset changes, so
@@ -276,7 +169,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
             else gemm_epilogue_fast<MI, NJ, false, false>(p, acc, lds, m0, n0, wave, lane);
         }
     } else {
-        gemm_epilogue_checked<MI, NJ>(p, acc, lds, m0, n0, wave, lane);
+        gemm_epilogue_checked<2 * MI, 2 * NJ, 2 * MI>(p, acc, lds, m0, n0, 0, wave, lane);
     }
 }
 
@@ -494,16 +387,15 @@ __device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, 
 }
 
 
-// TWO: the launch may hold two products. The 256-wide tile has a form without, which reads its parameters as plain
-// kernel arguments: a copy of them (see product_of_tile) does not fit its scalar registers, and with two products
-// it takes them by reference.
+// TWO: the launch may hold two products, whose parameters are taken by reference (a copy, see product_of_tile, does
+// not fit the scalar registers of the 256-wide tile); the form for one reads them as plain kernel arguments.
 template <int MI, bool KTAIL, bool TWO>
 __global__ __launch_bounds__(kGemmThreads) void gemm_nt_ring_kernel(GemmLaunch L) {
     constexpr int BM = 64 * MI, BK = 64, NU = 5, UNIT = BM * BK * 2;
     __shared__ __attribute__((aligned(1024))) char lds[NU * UNIT];
     int tm, tn;
     if (L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BM, tm, tn) : !tile_of_block(L, tm, tn)) return;
-    std::conditional_t<MI == 4, const GemmParams&, const GemmParams> p = L.p[TWO ? product_of_tile(L, tm) : 0];
+    const GemmParams& p = L.p[TWO ? product_of_tile(L, tm) : 0];
     const int m0 = tm * BM, n0 = tn * BM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -695,7 +587,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_rect_kernel(GemmLaunch L
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     f32x4 acc[FM][FN];
     gemm_rect_slabs<FM, FN, KTAIL>(p, lds, m0, n0, (p.K + BK - 1) / BK, acc);
-    gemm_finish_rect<FM, FN, FM>(p, acc, lds, m0, n0, 0, wave, lane);
+    gemm_finish_rect<FM, FN, FM, false>(p, acc, lds, m0, n0, 0, wave, lane);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -860,11 +752,16 @@ __global__ __launch_bounds__(256) void gemm_nt_scalar_kernel(GemmParams p) {
     *dst = f2bf(t);
 }
 
-template <int MI, bool TWO>
-static void launch_tiled(const GemmSet& g, hipStream_t st) {
-    const GemmLaunch L = make_launch(g, 64 * MI, 64 * MI);
-    if (g.p[0].K % 64 == 0) hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, false, TWO>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
-    else hipLaunchKernelGGL((gemm_nt_ring_kernel<MI, true, TWO>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+template <bool KTAIL>
+static void launch_ring(const GemmSet& g, hipStream_t st) {
+    const GemmLaunch L = make_launch(g, 256, 256);
+    if (g.n == 1) hipLaunchKernelGGL((gemm_nt_ring_kernel<4, KTAIL, false>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+    else hipLaunchKernelGGL((gemm_nt_ring_kernel<4, KTAIL, true>), dim3(grid_of(L)), dim3(kGemmThreads), 0, st, L);
+}
+
+static void launch_square(const GemmSet& g, hipStream_t st) {
+    if (g.p[0].K % 64 == 0) launch_ring<false>(g, st);
+    else launch_ring<true>(g, st);
 }
 
 template <int FM, int FN>
@@ -901,6 +798,8 @@ struct TilePlan {
     TileFamily family;
     int fm, fn, splits;
     double us;
+    bool checked = false;   // eight-wave tiles with the epilogue that decides per column
+    int head_rows = 0;      // > 0: this many rows on these tiles, the rest on eight-wave ones behind them
 };
 struct TileShape {
     TileFamily family;
@@ -934,39 +833,81 @@ static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
     return kLaunch + std::max(us, 2e-3 * g.n * g.p[0].N * g.p[0].K / kWeightGBs) + (splits > 1 ? kReduce + 2e-3 * split_bytes(g, t, splits) / kSplitGBs : 0.0);
 }
 
+// The best eight-wave tile for a product whose K is not cut.
+static TilePlan plan_eight_waves(const GemmSet& g) {
+    TilePlan best = {kPair, 0, 0, 1, 1e30, true};
+    for (const TileShape& t : kTileShapes) {
+        if (t.family != kPair || t.fn == 8) continue;
+        const double us = tile_cost_us(g, t, 1);
+        if (us < best.us) best = {kPair, t.fm, t.fn, 1, us, true};
+    }
+    return best;
+}
+
+// The first `rows` rows of a product, or those behind them.
+static GemmSet rows_before(const GemmSet& g, int rows) {
+    GemmSet head = g;
+    head.p[0].M = rows;
+    return head;
+}
+static GemmSet rows_behind(const GemmSet& g, int rows) {
+    GemmSet tail = g;
+    GemmParams& t = tail.p[0];
+    const int64_t row0 = rows;
+    t.M -= rows;
+    t.A += row0 * t.lda;
+    t.Y += row0 * t.ldy;
+    if (t.Y2 != nullptr) t.Y2 += row0 * t.ldy2;
+    if (t.gate != nullptr) {
+        t.resid += row0 * t.ldresid;
+        t.gate += row0 / t.rows_per_batch * t.gate_stride;
+    }
+    return tail;
+}
+
 static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_bytes) {
-    // The rectangular and eight-wave tiles have one epilogue: 16-byte outputs, a wave's columns on one side of
-    // split_n and act_begin, no GELU in front of a gate. Anything else takes the square tiles' checked one.
+    // The branch-free epilogue of the rectangular and eight-wave tiles: 16-byte outputs, a wave's columns on one
+    // side of split_n and act_begin, no GELU in front of a gate. The square and the eight-wave tiles have one for
+    // anything else as well. (Without it on the eight-wave tiles, calls outside the form ran on square ones: 64 x 3072
+    // x 3072 with 1000 columns in the first output 13 -> 63 us, 300 x 1001 x 3072 14 -> 30 us.)
     const GemmParams& p = g.p[0];
     bool form = true;
-    int64_t square_tiles = 0;
     for (int i = 0; i < g.n; ++i) {
         const GemmParams& q = g.p[i];
         form = form && q.vec_io && q.N % 8 == 0 && (q.bias == nullptr || q.bias_vec) && !(q.gate != nullptr && q.act != FLUX_ACT_NONE) &&
                q.lda * 2 * 288 < 0x7fffffffLL && q.ldw * 2 * 256 < 0x7fffffffLL && q.ldy * 2 * 288 < 0x7fffffffLL &&
                q.ldy2 * 2 * 288 < 0x7fffffffLL && q.ldresid * 2 * 288 < 0x7fffffffLL;   // 32-bit byte offsets inside a tile's rows
-        square_tiles += static_cast<int64_t>((q.M + 255) / 256) * ((q.N + 255) / 256);
     }
     auto columns_ok = [&](int fn) {
         const int w = 16 * fn;
-        return (p.split_n >= p.N || p.split_n % w == 0) && (p.act == FLUX_ACT_NONE || p.act_begin >= p.N || p.act_begin % w == 0);
+        return form && (p.split_n >= p.N || p.split_n % w == 0) && (p.act == FLUX_ACT_NONE || p.act_begin >= p.N || p.act_begin % w == 0);
     };
-    if (!form) {   // 256-wide tiles once they fill most of the chip, else 128-wide ones, two workgroups per CU
-        const bool big = p.qk_cols > 0 || square_tiles >= 160;   // (whole heads per wave: 256-wide tiles only)
-        return {kSquare, big ? 8 : 4, big ? 8 : 4, 1, 0.0};
-    }
+    if (!form && p.qk_cols > 0) return {kSquare, 8, 8, 1, 0.0};   // (whole heads per wave: 256-wide tiles only)
     TilePlan best = {kSquare, 8, 8, 1, 1e30};
     // First the best shape for the plain product: whether a tile sums K in one run (four-wave tiles) or in two
     // interleaved halves (eight-wave tiles) is decided by M, N and K alone, so that a product rounds the same
     // way whatever its epilogue is.
     for (const TileShape& t : kTileShapes) {
         if (t.fn == 8 && t.family != kSquare) continue;       // only there for whole heads per wave
-        if (t.family != kSquare && !columns_ok(t.fn)) continue;
+        if (t.family == kRect && !columns_ok(t.fn)) continue;
         const int most = t.family == kPair && p.K % 64 == 0 && p.qk_cols == 0 ? 10 : 1;
         for (int s = 1; s <= most; ++s) {
             if (s > 1 && (tile_count(g, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(g, t, s) > workspace_bytes)) break;
             const double us = tile_cost_us(g, t, s);
-            if (us < best.us) best = {t.family, t.fm, t.fn, s, us};
+            if (us < best.us) best = {t.family, t.fm, t.fn, s, us, t.family == kPair && !columns_ok(t.fn)};
+        }
+    }
+    // Where rectangles may be missing (192 columns are whole waves of every tile): whole rounds of 256-wide tiles
+    // with the rows left over on eight-wave ones behind them, instead of a last round that is mostly empty.
+    // Only along the edge of a batch element, whose gate vector a part starts with.
+    const int64_t tiles = tile_count(g, kTileShapes[0]), tiles_n = (p.N + 255) / 256;
+    if (!columns_ok(12) && p.qk_cols == 0 && g.n == 1 && p.a_skip == 0 && tiles > kGemmCUs) {
+        const int64_t most = tiles / kGemmCUs * kGemmCUs / tiles_n;   // tile rows in whole rounds
+        for (int64_t c = most; c > 0 && c > most - 4; --c) {
+            const int rows = static_cast<int>(c * 256);
+            if (rows >= p.M || (p.gate != nullptr && rows % p.rows_per_batch != 0)) continue;
+            const double us = tile_cost_us(rows_before(g, rows), kTileShapes[0], 1) + plan_eight_waves(rows_behind(g, rows)).us;
+            if (us < best.us) best = {kSquare, 8, 8, 1, us, false, rows};
         }
     }
     // Beside another stream's work: square tiles leave that work the CUs of their last round.
@@ -1015,6 +956,7 @@ static int read_linear_args(const flux_linear_args* a, GemmParams& p, LinearRout
     p.y2_col0 = split ? (int)a->y2_col0 : 0;
     p.rows_per_batch = a->gate ? (int)a->rows_per_batch : 1;
     p.in_silu = a->in_act == FLUX_ACT_SILU;
+    p.checked = 0;
     p.act = a->act; p.act_begin = (int)(a->act_begin < 0 ? 0 : (a->act_begin > a->N ? a->N : a->act_begin));
     p.bias_vec = a->bias != nullptr && (reinterpret_cast<uintptr_t>(a->bias) & 3u) == 0 && a->N % 4 == 0;
     p.vec_io = aligned16(a->Y) && a->ldy % 8 == 0 &&
@@ -1069,18 +1011,23 @@ static int launch_rows(const GemmSet& g, hipStream_t st) {
 }
 
 // With `need` nothing is launched: it receives the workspace the launch would like to have.
-static int launch_tiles(const GemmSet& g, bool shared_gpu, void* workspace, int64_t workspace_bytes, int64_t* need, hipStream_t st) {
+static int launch_tiles(GemmSet& g, bool shared_gpu, void* workspace, int64_t workspace_bytes, int64_t* need, hipStream_t st) {
     const TilePlan plan = plan_tiles(g, shared_gpu, need != nullptr ? INT64_MAX : workspace_bytes);
     if (need != nullptr) {
         if (plan.splits > 1) *need = split_bytes(g, {plan.family, plan.fm, plan.fn, 0.0}, plan.splits);
         return FLUX_OK;
     }
+    if (plan.head_rows > 0) {
+        GemmSet tail = rows_behind(g, plan.head_rows);
+        const TilePlan behind = plan_eight_waves(tail);
+        tail.p[0].checked = 1;
+        launch_square(rows_before(g, plan.head_rows), st);
+        launch_pair_tiles(behind.fm, behind.fn, tail, 1, nullptr, st);
+        return check_launch("flux_linear_bf16");
+    }
+    for (int i = 0; i < g.n; ++i) g.p[i].checked = plan.checked;
     switch (plan.family) {
-        case kSquare:
-            if (plan.fm != 8) launch_tiled<2, true>(g, st);
-            else if (g.n > 1) launch_tiled<4, true>(g, st);
-            else launch_tiled<4, false>(g, st);
-            break;
+        case kSquare: launch_square(g, st); break;
         case kRect:
             if (plan.fm == 9) launch_rect<9, 6>(g, st);
             else if (plan.fm == 8) launch_rect<8, 6>(g, st);
@@ -1188,7 +1135,7 @@ extern "C" int flux_linear_bf16_pair(const flux_linear_pair_args* a, void* works
 
 extern "C" int flux_linear_plan_of(const flux_linear_args* first, const flux_linear_args* second, int64_t workspace_bytes, flux_linear_plan* plan) {
     if (!plan) return fail(FLUX_E_NULL, "flux_linear_plan_of: null plan");
-    *plan = {FLUX_LINEAR_NOTHING, 0, 0, 1, 1};
+    *plan = {FLUX_LINEAR_NOTHING, 0, 0, 1, 1, 0, 0};
     GemmSet g;
     LinearRoute route[2];
     int rc = read_linear_args(first, g.p[0], route[0]);
@@ -1204,5 +1151,7 @@ extern "C" int flux_linear_plan_of(const flux_linear_args* first, const flux_lin
     plan->tile_m = 32 * t.fm;
     plan->tile_n = 32 * t.fn;
     plan->splits = t.splits;
+    plan->head_rows = t.head_rows;
+    plan->checked = t.checked || t.family == kSquare;
     return FLUX_OK;
 }

@@ -25,6 +25,7 @@ struct GemmParams {
     int in_silu;  // 1: A passes through x * sigmoid(x), rounded to bf16, on the way in (row-vector and scalar kernels)
     int bias_vec;  // 1: bias may be read with 8-byte buffer loads (4-byte aligned base)
     int vec_io;  // 1: every output/residual row segment of 8 columns may be accessed as 16 bytes
+    int checked; // 1: an eight-wave tile takes the epilogue that decides per column
     // fused QK RMSNorm + RoPE for columns [0, qk_cols): q heads first, then k heads, 128 columns each
     bf16_t* q_out; bf16_t* k_out;
     const bf16_t* q_scale; const bf16_t* k_scale;
@@ -440,10 +441,108 @@ __device__ __forceinline__ void gemm_epilogue_rect(const GemmParams& p, f32x4 (&
     }
 }
 
+// Epilogue for what the branch-free forms cannot express: columns of any number and alignment, split_n and
+// act_begin anywhere, GELU in front of a gate, rows any distance apart. The steps are those of
+// gemm_epilogue_rect, decided per segment of 8 columns or per column. ROWS of the wave's FM fragment rows from `row0` on.
 template <int FM, int FN, int ROWS>
+__device__ __forceinline__ void gemm_epilogue_checked(const GemmParams& p, f32x4 (&acc)[ROWS][FN], char* lds, int m0, int n0, int row0, int wave, int lane) {
+    constexpr int WCOLS = 16 * FN, C_CH = WCOLS / 8, C_PITCH = WCOLS * 2 + 16;
+    constexpr int SEGS = 16 * C_CH;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int frow = lane & 15, fq = lane >> 4;            // accumulator: row frow of a 16-row fragment, columns fq*4..+3
+    char* cw = lds + wave * (2 * 16 * C_PITCH);
+    const int wave_n0 = n0 + wn * WCOLS;
+    const int wave_m0 = m0 + wm * (16 * FM) + row0 * 16;
+
+    float bv[FN][4];
+    if (p.bias != nullptr && p.bias_vec) {
+        const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.bias), 0, p.N * 2, kRsrcFlags);
+#pragma unroll
+        for (int q = 0; q < FN; ++q) {
+            const u32x2 raw = __builtin_amdgcn_raw_buffer_load_b64(rb, (wave_n0 + q * 16 + fq * 4) * 2, 0, 0);
+            bv[q][0] = __uint_as_float(raw.x << 16);
+            bv[q][1] = __uint_as_float(raw.x & 0xffff0000u);
+            bv[q][2] = __uint_as_float(raw.y << 16);
+            bv[q][3] = __uint_as_float(raw.y & 0xffff0000u);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < FN; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = wave_n0 + q * 16 + fq * 4 + e;
+                bv[q][e] = (p.bias != nullptr && n < p.N) ? bf2f(p.bias[n]) : 0.0f;
+            }
+    }
+    const bool gelu_all = p.act == FLUX_ACT_GELU_TANH && wave_n0 >= p.act_begin;
+    const bool gelu_some = p.act == FLUX_ACT_GELU_TANH && !gelu_all && wave_n0 + WCOLS > p.act_begin;
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        char* const blk = cw + (i & 1) * (16 * C_PITCH);
+#pragma unroll
+        for (int q = 0; q < FN; ++q) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = acc[i][q][e] + bv[q][e];
+            if (gelu_all) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = tanh_gelu_fast(v[e]);
+            } else if (gelu_some) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (wave_n0 + q * 16 + fq * 4 + e >= p.act_begin) v[e] = tanh_gelu_fast(v[e]);
+            }
+            *reinterpret_cast<u32x2*>(blk + frow * C_PITCH + fq * 8 + q * 32) = pack4_bf16(v[0], v[1], v[2], v[3]);
+        }
+        __builtin_amdgcn_wave_barrier();  // LDS operations of one wave complete in order
+#pragma unroll
+        for (int a = 0; a < (SEGS + 63) / 64; ++a) {
+            const int seg = a * 64 + lane, row = seg / C_CH, ch = seg % C_CH;
+            if (SEGS % 64 != 0 && seg >= SEGS) continue;
+            const int m = wave_m0 + i * 16 + row, n = wave_n0 + ch * 8;
+            Vec16<bf16_t> y = *reinterpret_cast<const Vec16<bf16_t>*>(blk + row * C_PITCH + ch * 16);
+            if (m >= p.M || n >= p.N) continue;
+            const bool full = p.vec_io && n + 8 <= p.N;
+            if (p.gate != nullptr) {
+                const bf16_t* gp = p.gate + static_cast<int64_t>(m / p.rows_per_batch) * p.gate_stride + n;
+                const bf16_t* rp = p.resid + static_cast<int64_t>(m) * p.ldresid + n;
+                if (full) {
+                    Vec16<bf16_t> gt = ld16(gp), rs = ld16(rp);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) y.v[e] = f2bf(bf2f(rs.v[e]) + bf2f(f2bf(bf2f(gt.v[e]) * bf2f(y.v[e]))));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (n + e < p.N) y.v[e] = f2bf(bf2f(rp[e]) + bf2f(f2bf(bf2f(gp[e]) * bf2f(y.v[e]))));
+                }
+            }
+            if (full && (n + 8 <= p.split_n || n >= p.split_n)) {
+                bf16_t* dst = n < p.split_n ? p.Y + static_cast<int64_t>(m) * p.ldy + n
+                                            : p.Y2 + static_cast<int64_t>(m) * p.ldy2 + (n - p.split_n + p.y2_col0);
+                st16(dst, y);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int ne = n + e;
+                    if (ne < p.N) {
+                        bf16_t* dst = ne < p.split_n ? p.Y + static_cast<int64_t>(m) * p.ldy + ne
+                                                     : p.Y2 + static_cast<int64_t>(m) * p.ldy2 + (ne - p.split_n + p.y2_col0);
+                        *dst = y.v[e];
+                    }
+                }
+            }
+        }
+    }
+}
+
+// CHECKED: the tile has the checked epilogue too, for calls that carry p.checked.
+template <int FM, int FN, int ROWS, bool CHECKED>
 __device__ __forceinline__ void gemm_finish_rect(const GemmParams& p, f32x4 (&acc)[ROWS][FN], char* lds, int m0, int n0, int row0, int wave, int lane) {
     constexpr int BM = 32 * FM, WCOLS = 16 * FN;
     const int wave_n0 = n0 + (wave & 1) * WCOLS;
+    if constexpr (CHECKED) {
+        if (p.checked) return gemm_epilogue_checked<FM, FN, ROWS>(p, acc, lds, m0, n0, row0, wave, lane);
+    }
     const bool gelu = p.act == FLUX_ACT_GELU_TANH && wave_n0 >= p.act_begin;
     const bool edge = m0 + BM > p.M || n0 + 32 * FN > p.N || (p.gate != nullptr && m0 / p.rows_per_batch != (m0 + BM - 1) / p.rows_per_batch);
     if constexpr (FN == 8 && ROWS > 1) {

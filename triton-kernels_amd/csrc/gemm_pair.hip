@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
                 for (int j = 0; j < FN; ++j) dst[((OWN0 + i) * FN + j) * 64] = own[i][j];
         } else {
             __syncthreads();                   // the exchange has been read: its LDS is the epilogue's now
-            gemm_finish_rect<FM, FN, OWN>(p, own, lds + G * (ST * (BM + BN) * BK), m0, n0, OWN0, w4, lane);
+            gemm_finish_rect<FM, FN, OWN, FN != 8>(p, own, lds + G * (ST * (BM + BN) * BK), m0, n0, OWN0, w4, lane);
         }
     };
     f32x4 acc[FM][FN];
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_reduce_kernel(GemmLaunch L)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[0][j] += src[j * 64];
     }
-    gemm_finish_rect<FM, FN, 1>(p, acc, lds, m0, n0, row, wave, lane);
+    gemm_finish_rect<FM, FN, 1, FN != 8>(p, acc, lds, m0, n0, row, wave, lane);
 }
 
 template <int FM, int FN, int ST>

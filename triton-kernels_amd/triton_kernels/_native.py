@@ -71,7 +71,7 @@ class LinearPairArgs(Structure):
 
 
 class LinearPlan(Structure):
-    _fields_ = [("family", c_int32), ("tile_m", c_int32), ("tile_n", c_int32), ("splits", c_int32), ("products", c_int32)]
+    _fields_ = [("family", c_int32), ("tile_m", c_int32), ("tile_n", c_int32), ("splits", c_int32), ("products", c_int32), ("head_rows", c_int32), ("checked", c_int32)]
 
 
 class RmsNormArgs(Structure):

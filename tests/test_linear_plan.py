@@ -106,3 +106,15 @@ def test_a_nearly_empty_last_round_is_cut_off():
     gated = dict(gate=PTR, resid=PTR, ldresid=12289)
     assert plan_of(linear_args(1500, 12289, 3072, rows_per_batch=256, **gated)).head_rows == 1280
     assert plan_of(linear_args(1500, 12289, 3072, rows_per_batch=1500, **gated)).head_rows == 0
+
+
+@pytest.mark.parametrize("rows,family,tile_m", [
+    (260, EIGHT_WAVES, 128), (384, EIGHT_WAVES, 128), (513, RECT, 224), (640, RECT, 224), (960, RECT, 224), (1153, RECT, 224), (1344, RECT, 224),
+    (1600, RECT, 224), (1760, RECT, 224), (1920, RECT, 224), (2049, SQUARE, 256), (2112, SQUARE, 256), (2560, RECT, 224), (3329, RECT, 224),
+    (4096, SQUARE, 256), (4608, SQUARE, 256)])
+def test_qk_projection_takes_the_tile_that_is_fastest_for_it(rows, family, tile_m):
+    """The tile measured fastest for the single block's fused projection at each row count. Eight-wave tiles are the
+    best for the plain product up to 2100 rows, but their only shape with whole heads per wave is slow: 1920 rows 257
+    us against 215 on 224 x 256 tiles, 2049 rows 290 against 237 on 256 x 256."""
+    p = plan_of(qk_args(1, rows, 24, 12288))
+    assert (p.family, p.tile_m, p.tile_n) == (family, tile_m, 256)

@@ -884,12 +884,13 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     };
     if (!form && p.qk_cols > 0) return {kSquare, 8, 8, 1, 0.0};   // (whole heads per wave: 256-wide tiles only)
     TilePlan best = {kSquare, 8, 8, 1, 1e30};
-    // First the best shape for the plain product: whether a tile sums K in one run (four-wave tiles) or in two
-    // interleaved halves (eight-wave tiles) is decided by M, N and K alone, so that a product rounds the same
-    // way whatever its epilogue is.
+    // Calls with the q/k epilogue take the cheapest shape whose waves hold whole heads (128 columns), whatever the plain
+    // product of that size takes. Fused projection of the single block (21504 x 3072, weights from HBM), us on 256 x
+    // 256, 224 x 256 and eight-wave 128 x 256 tiles: 320 rows 79 75 58, 640 88 79 108, 1153 159 142 173, 1920 243 215
+    // 256, 2049 237 263 290, 3329 409 367 424, 4608 492 517 560. (The eight-wave tile sums K in another order.)
     for (const TileShape& t : kTileShapes) {
-        if (t.fn == 8 && t.family != kSquare) continue;       // only there for whole heads per wave
-        if (t.family == kRect && !columns_ok(t.fn)) continue;
+        if (p.qk_cols > 0 ? t.fn != 8 : t.fn == 8 && t.family != kSquare) continue;   // (the others of that width are there for q/k only)
+        if ((t.family == kRect || (t.family == kPair && t.fn == 8)) && !columns_ok(t.fn)) continue;
         const int most = t.family == kPair && p.K % 64 == 0 && p.qk_cols == 0 ? 10 : 1;
         for (int s = 1; s <= most; ++s) {
             if (s > 1 && (tile_count(g, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(g, t, s) > workspace_bytes)) break;
@@ -912,15 +913,6 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     }
     // Beside another stream's work: square tiles leave that work the CUs of their last round.
     if (shared_gpu && best.family == kRect) best = {kSquare, 8, 8, 1, best.us};
-    if (p.qk_cols > 0 && best.family != kSquare) {            // a wave's 128 columns are one head
-        const bool pair = best.family == kPair;
-        best = {kSquare, 8, 8, 1, 1e30};
-        for (const TileShape& t : kTileShapes) {
-            if (t.fn != 8 || (t.family == kPair) != pair || (t.family != kSquare && !columns_ok(8))) continue;
-            const double us = tile_cost_us(g, t, 1);
-            if (us < best.us) best = {t.family, t.fm, t.fn, 1, us};
-        }
-    }
     return best;
 }
 

@@ -118,3 +118,13 @@ def test_qk_projection_takes_the_tile_that_is_fastest_for_it(rows, family, tile_
     us against 215 on 224 x 256 tiles, 2049 rows 290 against 237 on 256 x 256."""
     p = plan_of(qk_args(1, rows, 24, 12288))
     assert (p.family, p.tile_m, p.tile_n) == (family, tile_m, 256)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (9, 12288, 3072, (64, 64)), (64, 12288, 3072, (64, 64)), (48, 21504, 3072, (64, 96)), (81, 21504, 3072, (96, 96)), (28, 18432, 3072, (64, 96)),
+    (335, 9216, 3072, (160, 128))])
+def test_tiles_of_like_price(M, N, K, tile):
+    """Few rows of wide products wait for the weights whatever the tile: those took the first shape of the table that
+    was fast enough (64 x 12288 x 3072 25 us, 48 x 21504 39) and take the one that does least beside (20 and 27)."""
+    p = plan_of(linear_args(M, N, K))
+    assert (p.family, p.tile_m, p.tile_n, p.splits) == (EIGHT_WAVES, *tile, 1)

@@ -233,7 +233,7 @@ static void launch_pair(const GemmSet& g, int splits, float* partial, hipStream_
 void launch_pair_tiles(int fm, int fn, const GemmSet& g, int splits, float* partial, hipStream_t st) {
 #define FLUX_PAIR(FM, FN, ST) if (fm == FM && fn == FN) return launch_pair<FM, FN, ST>(g, splits, partial, st)
     FLUX_PAIR(5, 6, 3); FLUX_PAIR(6, 6, 3); FLUX_PAIR(4, 6, 3); FLUX_PAIR(8, 4, 3); FLUX_PAIR(7, 4, 3); FLUX_PAIR(6, 4, 4);
-    FLUX_PAIR(5, 4, 4); FLUX_PAIR(4, 4, 4); FLUX_PAIR(5, 3, 4); FLUX_PAIR(4, 3, 4); FLUX_PAIR(3, 3, 4); FLUX_PAIR(2, 3, 4);
+    FLUX_PAIR(5, 4, 4); FLUX_PAIR(5, 3, 4); FLUX_PAIR(4, 3, 4); FLUX_PAIR(3, 3, 4); FLUX_PAIR(2, 3, 4);
     FLUX_PAIR(2, 2, 6); FLUX_PAIR(4, 8, 3);
 #undef FLUX_PAIR
 }

@@ -312,7 +312,7 @@ def test_linear_head_and_tail_launches(gated):
 
 @pytest.mark.parametrize("B,L,N,K,splits", [
     (1, 9, 64, 64, 1), (1, 65, 96, 128, 1),          # one slab, two slabs; a row past the smallest tile
-    (3, 43, 200, 4096, 2), (1, 320, 384, 3072, 2),   # few tiles, long K: K over several workgroups (batch elements inside a tile)
+    (3, 43, 200, 8192, 2), (1, 320, 384, 6144, 2),   # few tiles, long K: K over several workgroups (batch elements inside a tile)
     (7, 19, 1000, 520, 1),                           # K tail, columns past the last tile, seven batch elements in two tiles
     (1, 333, 9216, 192, 1), (2, 640, 3072, 640, 1),  # eight-wave tiles, ragged and exact
     (1, 2700, 3072, 192, 1), (3, 1445, 3072, 128, 1), (1, 2049, 9224, 72, 1),   # four-wave rectangles with rows and columns to spare
@@ -350,7 +350,7 @@ def test_linear_tile_edges(B, L, N, K, splits):
 
 @pytest.mark.parametrize("B,L,N,K,split,act_begin", [
     (1, 9, 3, 64, None, 0), (1, 65, 97, 128, 50, 33),        # less than a tile; a segment of 8 columns on both sides of the split
-    (2, 100, 1001, 72, 1000, 1000), (3, 43, 201, 4096, None, 7),   # K tail; K over several workgroups, batch elements inside a tile
+    (2, 100, 1001, 72, 1000, 1000), (3, 43, 201, 8192, None, 7),   # K tail; K over several workgroups, batch elements inside a tile
     (1, 320, 3073, 640, 8, 3000), (1, 700, 6001, 64, 3080, 3080),  # several sizes of eight-wave tiles
     (3, 1000, 1001, 192, 500, 0), (1, 2300, 6001, 192, None, 0), (4, 1000, 3073, 3072, 500, 0),
     (6, 250, 12289, 3072, 12000, 12288), (6, 256, 12289, 3072, None, 0),   # 256-wide tiles, the last rows on 128-wide ones
@@ -386,7 +386,7 @@ def test_linear_outside_the_branch_free_form(B, L, N, K, split, act_begin):
 
 @pytest.mark.parametrize("B,L0,L1,N,K", [
     (1, 65, 9, 96, 128),          # one tile row each, the smallest tiles
-    (3, 43, 21, 3072, 4096),      # K over several workgroups, batch elements inside a tile
+    (2, 100, 33, 1000, 8192),     # K over several workgroups, batch elements inside a tile
     (2, 300, 77, 200, 520),       # K tail, columns past the last tile
     (2, 1445, 256, 3072, 192),    # four-wave rectangles, ragged rows in both products
     (1, 4096, 512, 1024, 64),     # square tiles or exact rectangles

@@ -6,6 +6,7 @@ import random
 import pytest
 
 from triton_kernels import _native as nv
+from triton_kernels.kernels.linear import _may_cut_k
 
 NOTHING, SCALAR, ROWS, SQUARE, RECT, EIGHT_WAVES = range(6)
 PTR = 1 << 20   # stands for an aligned device address; the query reads the arguments only
@@ -128,3 +129,26 @@ def test_tiles_of_like_price(M, N, K, tile):
     was fast enough (64 x 12288 x 3072 25 us, 48 x 21504 39) and take the one that does least beside (20 and 27)."""
     p = plan_of(linear_args(M, N, K))
     assert (p.family, p.tile_m, p.tile_n, p.splits) == (EIGHT_WAVES, *tile, 1)
+
+
+def test_no_workspace_is_needed_where_the_question_is_not_asked():
+    rng, cut = random.Random(5), 0
+    for _ in range(6000):
+        M, N = (round(2 ** rng.uniform(*r)) for r in ((0, 14), (3, 15)))
+        K = rng.choice([64, 1024, 2048, 3072, 3136, 4096, 4608, 6144, 9216, 12288, 15360])
+        a = linear_args(M, N, K)
+        need = nv.lib().flux_linear_workspace_bytes(nv.byref(a))
+        assert need == 0 or _may_cut_k(M, N, K), (M, N, K, need)
+        cut += need > 0
+        other = round(2 ** rng.uniform(0, 12))
+        pair = nv.LinearPairArgs()
+        pair.product[0], pair.product[1] = a, linear_args(other, N, K)
+        need = nv.lib().flux_linear_pair_workspace_bytes(nv.byref(pair))
+        assert need == 0 or _may_cut_k(M + other, N, K), (M, other, N, K, need)
+    assert cut > 100
+
+
+def test_k_is_cut_only_for_a_gain_above_what_it_costs_the_host():
+    assert plan_of(linear_args(64, 3072, 3072)).splits == 1      # 2 us of the GPU for 6 us of the host
+    assert plan_of(linear_args(320, 3072, 15360)).splits > 1     # 30 us
+    assert plan_of(linear_args(320, 3072, 15360), workspace=0).splits == 1

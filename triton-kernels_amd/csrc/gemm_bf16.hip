@@ -814,17 +814,20 @@ static const TileShape kTileShapes[] = {
 };
 
 static int64_t tile_count(const GemmSet& g, const TileShape& t) {
+    const uint32_t bm = 32 * t.fm, bn = 32 * t.fn;   // (32-bit divisions: the search below does some forty per call)
     int64_t rows = 0;
-    for (int i = 0; i < g.n; ++i) rows += (g.p[i].M + 32 * t.fm - 1) / (32 * t.fm);
-    return rows * ((g.p[0].N + 32 * t.fn - 1) / (32 * t.fn));
+    for (int i = 0; i < g.n; ++i) rows += (static_cast<uint32_t>(g.p[i].M) + bm - 1) / bm;
+    return rows * ((static_cast<uint32_t>(g.p[0].N) + bn - 1) / bn);
 }
 static int64_t split_bytes(const GemmSet& g, const TileShape& t, int splits) {
     return tile_count(g, t) * splits * (32 * t.fm) * (32 * t.fn) * 4;
 }
 
+static const double kLaunch = 4.6, kTileLarge = 4.3, kTilePair = 2.7, kReduce = 1.7, kSplitGBs = 5970.0, kWeightGBs = 4500.0;
+static const double kIdleShare = 0.31;   // a workgroup runs up to this much faster the emptier the GPU is
+static const double kSplitHostUs = 6.0;  // K in parts costs the host this much
+
 static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
-    const double kLaunch = 4.6, kTileLarge = 4.3, kTilePair = 2.7, kReduce = 1.7, kSplitGBs = 5970.0, kWeightGBs = 4500.0;
-    const double kIdleShare = 0.31;   // a workgroup runs up to this much faster the emptier the GPU is
     const int64_t tiles = tile_count(g, t) * splits;
     const int64_t rounds = (tiles + kGemmCUs - 1) / kGemmCUs;
     const double fill = static_cast<double>(tiles) / (rounds * kGemmCUs);
@@ -834,6 +837,11 @@ static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
     // (12288 columns of 3072 at 64 rows: 64 x 64 tiles 19 us, 96 x 96 23, 192 x 128 30).
     const double weights_us = 2e-3 * g.n * g.p[0].N * g.p[0].K / kWeightGBs;
     return kLaunch + std::max(us, weights_us) + 0.05 * std::min(us, weights_us) + (splits > 1 ? kReduce + 2e-3 * split_bytes(g, t, splits) / kSplitGBs : 0.0);
+}
+
+// No more than tile_cost_us in `splits` or more parts: the work spread evenly over the CUs, and the traffic of the parts.
+static double split_floor_us(const GemmSet& g, const TileShape& t, int splits) {
+    return kLaunch + kReduce + kTilePair + tile_count(g, t) * (g.p[0].K / 64) * t.slab_us / kGemmCUs + 2e-3 * split_bytes(g, t, splits) / kSplitGBs;
 }
 
 // The best eight-wave tile for a product whose K is not cut.
@@ -894,12 +902,24 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     for (const TileShape& t : kTileShapes) {
         if (p.qk_cols > 0 ? t.fn != 8 : t.fn == 8 && t.family != kSquare) continue;   // (the others of that width are there for q/k only)
         if ((t.family == kRect || (t.family == kPair && t.fn == 8)) && !columns_ok(t.fn)) continue;
-        const int most = t.family == kPair && p.K % 64 == 0 && p.qk_cols == 0 ? 10 : 1;
-        for (int s = 1; s <= most; ++s) {
-            if (s > 1 && (tile_count(g, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(g, t, s) > workspace_bytes)) break;
-            const double us = tile_cost_us(g, t, s);
-            if (us < best.us) best = {t.family, t.fm, t.fn, s, us, t.family == kPair && !columns_ok(t.fn)};
+        const double us = tile_cost_us(g, t, 1);
+        if (us < best.us) best = {t.family, t.fm, t.fn, 1, us, t.family == kPair && !columns_ok(t.fn)};
+    }
+    // K in parts, where that gains more than the host pays for it: a workspace to allocate and a second launch, 6 us
+    // per call (64 x 3072 x 3072 takes 11 us of the GPU in two parts and 13 in one, but the host 20 and 14).
+    if (workspace_bytes > 0 && p.K % 64 == 0 && p.K / 64 >= 8 && p.qk_cols == 0) {
+        const double bar = best.us - kSplitHostUs;
+        TilePlan split = {kPair, 0, 0, 1, bar};
+        for (const TileShape& t : kTileShapes) {
+            if (t.family != kPair || t.fn == 8) continue;
+            for (int s = 2; s <= 10; ++s) {
+                if (tile_count(g, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(g, t, s) > workspace_bytes) break;
+                if (split_floor_us(g, t, s) > split.us) break;
+                const double us = tile_cost_us(g, t, s);
+                if (us < split.us) split = {kPair, t.fm, t.fn, s, us, !columns_ok(t.fn)};
+            }
         }
+        if (split.splits > 1) best = split;
     }
     // Where rectangles may be missing (192 columns are whole waves of every tile): whole rounds of 256-wide tiles
     // with the rows left over on eight-wave ones behind them, instead of a last round that is mostly empty.

@@ -36,6 +36,13 @@ def _rows_2d(x: Tensor, K: int) -> Tensor:
     return x2
 
 
+def _may_cut_k(rows: int, N: int, K: int) -> bool:
+    """False where flux_linear_workspace_bytes is known to be 0, so that the call is spared the question (0.5 us of
+    14 us of host time, 1 to 3 us where the library has tiles to choose from): K is cut where that gains more than 6
+    us, which takes more than 3072 of it, and only up to 256 tiles of 192 x 192."""
+    return K > 3072 and rows > 8 and rows * N <= 1 << 24
+
+
 def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "", act_begin: int = 0,
                 out: Tensor | None = None, out2: Tensor | None = None, split: int | None = None,
                 resid: Tensor | None = None, gate: Tensor | None = None, qk: dict | None = None,
@@ -56,11 +63,9 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
             result, only the schedule differs)
     """
     a = nv.LinearArgs()
-    out, _keep = _fill_args(a, x, w, b, activation=activation, act_begin=act_begin, out=out, out2=out2, split=split, resid=resid,
-                            gate=gate, qk=qk, in_activation=in_activation, shared_gpu=shared_gpu)
-    dev = out.device
+    out, dev, M, N, K, _keep = _fill_args(a, x, w, b, activation, act_begin, out, out2, split, resid, gate, qk, in_activation, shared_gpu)
     with nv.on_device(dev):
-        need = nv.lib().flux_linear_workspace_bytes(nv.byref(a))
+        need = nv.lib().flux_linear_workspace_bytes(nv.byref(a)) if K > 3072 and _may_cut_k(M, N, K) else 0
         if need:   # K cut over several workgroups: partial sums in memory of this launch's stream
             ws = torch.empty((need,), dtype=torch.uint8, device=dev)
             rc = nv.lib().flux_linear_bf16_ws(nv.byref(a), ws.data_ptr(), need, nv.stream_ptr(dev))
@@ -75,7 +80,7 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
     call: products of the same N, K and form of epilogue share a launch. An x of [B, L, K] may be a slice of
     a longer sequence, whose batch elements are not evenly strided rows."""
     args = nv.LinearPairArgs()
-    outs, keep = [], []
+    outs, keep, sizes = [], [], []
     for i, call in enumerate((first, second)):
         x = call["x"]
         if x.dim() == 3 and x.shape[0] > 1 and x.stride(0) != x.shape[1] * x.stride(1):
@@ -84,24 +89,25 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
                     and x.stride(1) % 8 == 0 and K % 8 == 0 and x.data_ptr() % 16 == 0 and call["w"].data_ptr() % 16 == 0 \
                     and call["w"].is_contiguous() and B * x.stride(0) * 2 < 2**31:
                 args.a_rows[i], args.a_batch_stride[i] = L, x.stride(0)
-        out, kept = _fill_args(args.product[i], batches=bool(args.a_rows[i]), **call)
+        out, dev, M, N, K, kept = _fill_args(args.product[i], batches=bool(args.a_rows[i]), **call)
         outs.append(out)
         keep.append(kept)
-    dev = outs[0].device
+        sizes.append((M, N, K))
     nv.require_gpu(*outs)
     with nv.on_device(dev):
-        need = nv.lib().flux_linear_pair_workspace_bytes(nv.byref(args))
+        (M0, N0, K0), (M1, N1, K1) = sizes
+        need = nv.lib().flux_linear_pair_workspace_bytes(nv.byref(args)) if _may_cut_k(M0 + M1, min(N0, N1), max(K0, K1)) else 0
         ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None
         rc = nv.lib().flux_linear_bf16_pair(nv.byref(args), nv.ptr(ws), need, nv.stream_ptr(dev))
     nv.check(rc, "flux_linear_bf16_pair")
     return outs[0], outs[1]
 
 
-def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "", act_begin: int = 0,
+def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, activation: str = "", act_begin: int = 0,
                out: Tensor | None = None, out2: Tensor | None = None, split: int | None = None, resid: Tensor | None = None,
                gate: Tensor | None = None, qk: dict | None = None, in_activation: str = "", shared_gpu: bool = False,
                batches: bool = False):
-    """Checks one call and writes it into `a`; returns the output and what has to live until the launch.
+    """Checks one call and writes it into `a`; returns the output, its device, M, N, K and what has to live until the launch.
     batches: x is [B, L, K] with evenly strided rows inside a batch element only."""
     assert x.shape[-1] == w.shape[-1], "Incompatible dimensions"
     assert x.dtype == w.dtype, "Incompatible dtypes"
@@ -122,7 +128,8 @@ def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, *, ac
     a.ldw = w.stride(0) if N > 1 else K
     if out is None:
         out = torch.empty((M, N if split is None else split), device=dev, dtype=x.dtype)
-    assert out.dim() == 2 and out.shape[0] == M and out.stride(1) == 1 and out.dtype == x.dtype
+    else:
+        assert out.dim() == 2 and out.shape[0] == M and out.stride(1) == 1 and out.dtype == x.dtype
     a.Y, a.ldy = out.data_ptr(), out.stride(0)
     if split is not None and split < N:
         assert out2 is not None and out2.dim() == 2 and out2.shape[0] == M and out2.stride(1) == 1
@@ -170,7 +177,7 @@ def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, *, ac
         parts = [activation and f"{activation}>={act_begin}", split is not None and f"split@{split}", gate is not None and "gated-residual",
                  qk is not None and "qk-norm-rope", in_activation and f"in:{in_activation}"]
         launch_hook(linear_launch_metadata(M, N, K, x.element_size(), "+".join(p for p in parts if p)))
-    return out, keep
+    return out, dev, M, N, K, keep
 
 
 def qk_fusable(x: Tensor, w: Tensor, seq_len: int, head_dim: int) -> bool:

@@ -50,6 +50,21 @@ def test_rms_norm_bf16_shapes(shape):
     torch.testing.assert_close(y2, oracle.rms_norm_ref(x, w.float()).to(torch.bfloat16), atol=1e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("dtype,width", [(torch.bfloat16, 4104), (torch.bfloat16, 6144), (torch.float32, 2052), (torch.float32, 3072)])
+@pytest.mark.parametrize("rows", [2, 2559, 2560])
+def test_rms_norm_long_rows(rows, dtype, width):
+    """Rows of nine to twelve vectors per lane: a block per row up to 2559 rows, a wave per row from there on. A row is
+    the same sum in another order: fp32 to 1e-5, bf16 to the ulp on either side of a rounding boundary (2^-7)."""
+    g = seeded(rows + width)
+    x = randn(g, rows, width, dtype=dtype).to(DEV)
+    w = (torch.rand(width, generator=g) + 0.5).to(dtype).to(DEV)
+    y = tk.rms_norm(x, w)
+    want = oracle.rms_norm_ref(x, w)
+    torch.testing.assert_close(y, want, **(dict(atol=1e-5, rtol=0) if dtype == torch.float32 else dict(atol=1e-2, rtol=1e-2)))
+    one = torch.cat([tk.rms_norm(x[:1], w), tk.rms_norm(x[-1:], w)])   # always the block kernel
+    torch.testing.assert_close(y[[0, -1]], one, atol=1e-6, rtol=1e-5 if dtype == torch.float32 else 2.0 ** -7)
+
+
 @pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", [(1, 24, 4608, 128),   # the Flux q/k shape: one vector per lane
                                    (3, 700, 512),         # two vectors per lane

@@ -6,6 +6,7 @@
 // (more than 64*ITER_MAX vectors) or not 16-byte addressable take a block-per-row kernel that
 // re-reads the row from cache.
 #include "common.h"
+#include <algorithm>
 
 namespace flux {
 
@@ -533,10 +534,19 @@ static RowPlan plan_row(int n, int vec) {
         else { CALL(64, 12); }                                         \
     } while (0)
 
+// RMS norm reads a row twice in the block-per-row kernel, the second time from a cache, and needs many rows before a
+// wave per row with twelve vectors per lane is the faster: us on the block kernel and in registers at 4608 bf16, 256 rows
+// 3.8 and 5.8, 2048 rows 8.9 and 10.1, 3072 rows 13.5 and 12.8, 4096 rows 17.5 and 14.4; at 3072 fp32 3.8 and 4.8,
+// 10.7 and 10.4, 17.6 and 13.7, 22.7 and 16.9.
+constexpr int64_t kRmsLongRows = 2560;
+
 template <typename T, typename TS>
 static int rms_fwd_launch(const flux_rms_norm_args* a, int count, int n, float eps, hipStream_t st) {
     constexpr int VEC = Elem<T>::VEC;
-    const RowPlan plan = plan_row(n, VEC);
+    RowPlan plan = plan_row(n, VEC);
+    int64_t most_rows = 0;
+    for (int i = 0; i < count; ++i) most_rows = std::max(most_rows, a[i].d0 * a[i].d1 * a[i].d2);
+    if (plan.ITER == 12 && most_rows < kRmsLongRows) plan = {0, 0};
     RmsFwdSet<T, TS> set;
     set.n = n;
     set.eps = eps;

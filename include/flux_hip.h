@@ -76,8 +76,10 @@ int flux_rms_norm_bwd(const void* dy, const void* x, const void* scale, const fl
                       int32_t x_dtype, int32_t scale_dtype, void* stream);
 
 /* The same with a workspace of flux_rms_norm_bwd_workspace_bytes bytes of device memory: dscale[n] is
- * written, not added to, in dscale_dtype, its sums formed in fp32 in a fixed order and rounded once.
- * Neither dscale nor the workspace needs to be cleared. rows == 0 writes zeros. */
+ * written, not added to, in dscale_dtype, from sums formed in fp32 and rounded once. The order of the sums is
+ * fixed for 16-byte addressable rows of up to 256 vectors of 16 bytes (2048 bf16, 1024 fp32 values); longer and
+ * unaligned rows are added with atomics. Neither dscale nor the workspace needs to be cleared. rows == 0 writes
+ * zeros (all pointers must be non-null all the same). */
 int64_t flux_rms_norm_bwd_workspace_bytes(int64_t rows, int32_t n, int32_t x_dtype);
 int flux_rms_norm_bwd_ws(const void* dy, const void* x, const void* scale, const float* rstd,
                          void* dx, void* dscale, int32_t dscale_dtype, void* ws, int64_t ws_bytes,

@@ -648,10 +648,11 @@ static int rms_bwd_launch(const void* dy, const void* x, const void* scale, cons
         FLUX_DISPATCH_GI(plan, CALL);
 #undef CALL
         parts = static_cast<int>(bp.blocks);
-    } else if (rows > 0) {
-        if (ws) hipLaunchKernelGGL(zero_floats, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, ws, n);
-        hipLaunchKernelGGL((rms_norm_bwd_block<T, TS>), dim3((unsigned)rows), dim3(kBlock), 0, st, dyp, xp, sp, rstd, dxp,
-                           ws ? ws : static_cast<float*>(dscale), rows, n);
+    } else if (rows > 0) {   // sums by atomics: straight into an fp32 dscale
+        float* const sums = ws && dscale_dtype == FLUX_BF16 ? ws : static_cast<float*>(dscale);
+        if (ws) hipLaunchKernelGGL(zero_floats, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, sums, n);
+        hipLaunchKernelGGL((rms_norm_bwd_block<T, TS>), dim3((unsigned)rows), dim3(kBlock), 0, st, dyp, xp, sp, rstd, dxp, sums, rows, n);
+        if (sums == dscale) return check_launch("flux_rms_norm_bwd");
         parts = 1;
     }
     if (ws && dscale_dtype == FLUX_BF16) dscale_reduce<bf16_t>(ws, dscale, parts, n, st);

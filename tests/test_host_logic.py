@@ -166,3 +166,44 @@ def test_attention_asks_for_a_workspace_wherever_the_library_wants_one():
                     asked += nv.lib().flux_attention_workspace_bytes(1, H, L, D) > 0
     assert asked > 100                                                       # and it does say yes
     assert not _may_cut_keys(96, 1024) and not _may_cut_keys(24, 1280)      # 24 heads: never
+
+
+def test_launch_hook_is_called_once_right_before_every_launch(monkeypatch):
+    """linear_pair_into launches two products at once or one after the other; a hook that opens a range per
+    call must see one call per launch. The library is asked for its plan and not launched."""
+    import contextlib
+    import importlib
+    from triton_kernels import _native as nv
+    lin = importlib.import_module("triton_kernels.kernels.linear")
+    real, events = nv.lib(), []
+
+    class Lib:
+        flux_linear_plan_of = real.flux_linear_plan_of
+        flux_linear_workspace_bytes = flux_linear_pair_workspace_bytes = staticmethod(lambda *a: 0)
+        flux_linear_bf16 = staticmethod(lambda *a: events.append("launch") or 0)
+
+        @staticmethod
+        def flux_linear_bf16_pair(args, *rest):
+            pair = args._obj
+            events.append(("pair", pair.product[0].M, pair.product[1].M, pair.a_rows[0], pair.a_batch_stride[0]))
+            return 0
+
+    monkeypatch.setattr(nv, "lib", lambda: Lib)
+    monkeypatch.setattr(nv, "require_gpu", lambda *t: t[0].device)
+    monkeypatch.setattr(nv, "on_device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(nv, "stream_ptr", lambda d: 0)
+    monkeypatch.setattr(lin, "launch_hook", events.append)
+    K, N = 64, 96
+    seq = torch.zeros(2, 100, K, dtype=torch.bfloat16)
+    w = torch.zeros(N, K, dtype=torch.bfloat16)
+    lin.linear_pair_into(dict(x=seq[:, 10:], w=w, b=None), dict(x=seq[:, :10], w=w, b=None))
+    assert [type(e) for e in events] == [dict, tuple] and events[1][1:] == (180, 20, 90, 100 * K)
+    assert events[0] == {"name": "flux_linear_bf16 [M=180+20, N=96, K=64]", "flops16": 2.0 * 200 * N * K, "bytes": 2 * (200 * K + 2 * N * K + 200 * N)}
+    del events[:]
+    lin.linear_pair_into(dict(x=seq[:, 10:], w=w, b=None), dict(x=seq[:, :10], w=w[:8], b=None))   # not of the same N: two launches
+    assert [type(e) for e in events] == [dict, tuple, dict, tuple]
+    assert "M=180," in events[0]["name"] and events[1][1:] == (180, 0, 90, 100 * K)
+    assert "M=20," in events[2]["name"] and events[3][1:] == (20, 0, 10, 100 * K)
+    del events[:]
+    lin.linear(seq, w, None)
+    assert [type(e) for e in events] == [dict, str]

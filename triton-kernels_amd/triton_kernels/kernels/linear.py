@@ -18,13 +18,18 @@ _PLANS = {torch.bfloat16: {"tile": (256, 256, 64), "waves": 4, "mfma": "16x16x32
 # thread, right before the launch. Profilers and benchmarks set it (e.g. to open a named range); None
 # costs nothing. The dictionary is what the reference attaches to its launches for its profiler
 # (kernels/linear.py:9-19): "name" with the problem size, "flops16" = 2 M N K and "bytes" = the three
-# matrices once.
+# matrices once; a launch of two products names both row counts ("M=4096+512") and counts both.
 launch_hook = None
 
 
 def linear_launch_metadata(M: int, N: int, K: int, elem_bytes: int = 2, epilogue: str = "") -> dict:
     name = f"flux_linear_bf16 [M={M}, N={N}, K={K}]" + (f" {epilogue}" if epilogue else "")
     return {"name": name, f"flops{elem_bytes * 8}": 2.0 * M * N * K, "bytes": elem_bytes * (M * K + N * K + M * N)}
+
+
+def _pair_launch_metadata(first: dict, second: dict, sizes: list) -> dict:
+    both = {key: first[key] + second[key] for key in first if key != "name"}
+    return {"name": first["name"].replace(f"[M={sizes[0][0]},", f"[M={sizes[0][0]}+{sizes[1][0]},"), **both}
 
 
 def _rows_2d(x: Tensor, K: int) -> Tensor:
@@ -80,7 +85,7 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
     call: products of the same N, K and form of epilogue share a launch. An x of [B, L, K] may be a slice of
     a longer sequence, whose batch elements are not evenly strided rows."""
     args = nv.LinearPairArgs()
-    outs, keep, sizes = [], [], []
+    outs, keep, sizes, notes = [], [], [], []
     for i, call in enumerate((first, second)):
         x = call["x"]
         if x.dim() == 3 and x.shape[0] > 1 and x.stride(0) != x.shape[1] * x.stride(1):
@@ -89,26 +94,45 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
                     and x.stride(1) % 8 == 0 and K % 8 == 0 and x.data_ptr() % 16 == 0 and call["w"].data_ptr() % 16 == 0 \
                     and call["w"].is_contiguous() and B * x.stride(0) * 2 < 2**31:
                 args.a_rows[i], args.a_batch_stride[i] = L, x.stride(0)
-        out, dev, M, N, K, kept = _fill_args(args.product[i], batches=bool(args.a_rows[i]), **call)
+        out, dev, M, N, K, kept = _fill_args(args.product[i], batches=bool(args.a_rows[i]), notes=notes, **call)
         outs.append(out)
         keep.append(kept)
         sizes.append((M, N, K))
     nv.require_gpu(*outs)
     with nv.on_device(dev):
-        (M0, N0, K0), (M1, N1, K1) = sizes
-        need = nv.lib().flux_linear_pair_workspace_bytes(nv.byref(args)) if _may_cut_k(M0 + M1, min(N0, N1), max(K0, K1)) else 0
-        ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None
-        rc = nv.lib().flux_linear_bf16_pair(nv.byref(args), nv.ptr(ws), need, nv.stream_ptr(dev))
-    nv.check(rc, "flux_linear_bf16_pair")
+        if launch_hook is None:
+            _launch_pair(args, sizes, dev)
+            return outs[0], outs[1]
+        plan = nv.LinearPlan()
+        nv.check(nv.lib().flux_linear_plan_of(nv.byref(args.product[0]), nv.byref(args.product[1]), 0, nv.byref(plan)), "flux_linear_plan_of")
+        if plan.products == 2:
+            launch_hook(_pair_launch_metadata(*notes, sizes))
+            _launch_pair(args, sizes, dev)
+            return outs[0], outs[1]
+        for i in range(2):   # a launch each: each alone, beside a product without rows
+            one = nv.LinearPairArgs()
+            one.product[0], one.product[1] = args.product[i], args.product[i]
+            one.product[1].M = 0
+            one.a_rows[0], one.a_batch_stride[0] = args.a_rows[i], args.a_batch_stride[i]
+            launch_hook(notes[i])
+            _launch_pair(one, sizes[i:i + 1], dev)
     return outs[0], outs[1]
+
+
+def _launch_pair(args: "nv.LinearPairArgs", sizes: list, dev: torch.device) -> None:
+    rows, N, K = sum(s[0] for s in sizes), min(s[1] for s in sizes), max(s[2] for s in sizes)
+    need = nv.lib().flux_linear_pair_workspace_bytes(nv.byref(args)) if _may_cut_k(rows, N, K) else 0
+    ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None
+    nv.check(nv.lib().flux_linear_bf16_pair(nv.byref(args), nv.ptr(ws), need, nv.stream_ptr(dev)), "flux_linear_bf16_pair")
 
 
 def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, activation: str = "", act_begin: int = 0,
                out: Tensor | None = None, out2: Tensor | None = None, split: int | None = None, resid: Tensor | None = None,
                gate: Tensor | None = None, qk: dict | None = None, in_activation: str = "", shared_gpu: bool = False,
-               batches: bool = False):
+               batches: bool = False, notes: list | None = None):
     """Checks one call and writes it into `a`; returns the output, its device, M, N, K and what has to live until the launch.
-    batches: x is [B, L, K] with evenly strided rows inside a batch element only."""
+    batches: x is [B, L, K] with evenly strided rows inside a batch element only. notes: receives the launch
+    hook's metadata instead of the hook, for a caller that launches two products at once."""
     assert x.shape[-1] == w.shape[-1], "Incompatible dimensions"
     assert x.dtype == w.dtype, "Incompatible dtypes"
     _PLANS[x.dtype]  # KeyError for anything but bfloat16, as in the reference
@@ -176,7 +200,7 @@ def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, activ
     if launch_hook is not None:
         parts = [activation and f"{activation}>={act_begin}", split is not None and f"split@{split}", gate is not None and "gated-residual",
                  qk is not None and "qk-norm-rope", in_activation and f"in:{in_activation}"]
-        launch_hook(linear_launch_metadata(M, N, K, x.element_size(), "+".join(p for p in parts if p)))
+        (launch_hook if notes is None else notes.append)(linear_launch_metadata(M, N, K, x.element_size(), "+".join(p for p in parts if p)))
     return out, dev, M, N, K, keep
 
 

@@ -191,11 +191,11 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
 //
 // Ring offsets are wave-uniform scalars that advance by two units per slab.
 // ------------------------------------------------------------------------------------------------
-// Multiplies K slabs [kb, ke) of the tile at (m0, n0) into acc (cleared first). On return every
+// Multiplies the first ke K slabs of the tile at (m0, n0) into acc (cleared first). On return every
 // buffer load of the wave has landed and all waves have passed a barrier, so the ring may be
 // reused (the epilogue parks its bf16 blocks there).
 template <int MI, bool KTAIL>
-__device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, int m0, int n0, int kb, int ke,
+__device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, int m0, int n0, int ke,
                                                 f32x4 (&acc)[2 * MI][2 * MI]) {
     constexpr int NJ = MI;
     constexpr int FM = 2 * MI, FN = 2 * NJ;      // 16-row fragments per wave and side
@@ -352,15 +352,15 @@ __device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, 
 
     // Prologue: slab 0, A(1) and the first loads of G(0); slab 0 must have landed, the rest flies on.
     {
-        const uint32_t k0 = slab_mask(kb), k1 = slab_mask(kb + 1);
+        const uint32_t k0 = slab_mask(0), k1 = slab_mask(1);
 #pragma unroll
-        for (int i = 0; i < PU; ++i) load_a(0, i, kb, k0);
+        for (int i = 0; i < PU; ++i) load_a(0, i, 0, k0);
 #pragma unroll
-        for (int i = 0; i < PU; ++i) load_w(UNIT, i, kb, k0);
+        for (int i = 0; i < PU; ++i) load_w(UNIT, i, 0, k0);
 #pragma unroll
-        for (int i = 0; i < PU; ++i) load_a(2 * UNIT, i, kb + 1, k1);
+        for (int i = 0; i < PU; ++i) load_a(2 * UNIT, i, 1, k1);
 #pragma unroll
-        for (int i = 0; i < EARLY; ++i) load_w(3 * UNIT, i, kb + 1, k1);
+        for (int i = 0; i < EARLY; ++i) load_w(3 * UNIT, i, 1, k1);
         wait_loads_and_barrier<PU + EARLY>();
 #pragma unroll
         for (int r = 0; r < READS; ++r) read_frag(0, 0, UNIT, 0, r);
@@ -370,8 +370,8 @@ __device__ __forceinline__ void gemm_tile_slabs(const GemmParams& p, char* lds, 
 
     {
         int ua = 0, uw = UNIT, ua1 = 2 * UNIT, uw1 = 3 * UNIT, ua2 = 4 * UNIT;
-        uint32_t m2 = slab_mask(kb + 2);
-        for (int kt = kb; kt < ke; ++kt) {
+        uint32_t m2 = slab_mask(2);
+        for (int kt = 0; kt < ke; ++kt) {
             uint32_t m3;
             slab(kt, ua, uw, ua1, uw1, ua2, m2, m3);
             // the ring advances by two units
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_ring_kernel(GemmLaunch L
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     f32x4 acc[2 * MI][2 * MI];
-    gemm_tile_slabs<MI, KTAIL>(p, lds, m0, n0, 0, (p.K + BK - 1) / BK, acc);
+    gemm_tile_slabs<MI, KTAIL>(p, lds, m0, n0, (p.K + BK - 1) / BK, acc);
     gemm_epilogue<MI, MI>(p, acc, lds, m0, n0, wave, lane);
 }
 

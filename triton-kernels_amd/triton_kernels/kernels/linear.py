@@ -65,7 +65,7 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
             qk_fusable() for the shapes this form takes
     shared_gpu : the launch runs beside another stream's work; the library then keeps a tile shape
             that leaves CUs free in its last round instead of one that fills the GPU exactly (same
-            result, only the schedule differs)
+            result, only the schedule differs); for callers that run streams side by side
     """
     a = nv.LinearArgs()
     out, dev, M, N, K, _keep = _fill_args(a, x, w, b, activation, act_begin, out, out2, split, resid, gate, qk, in_activation, shared_gpu)
@@ -206,9 +206,9 @@ def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, activ
 
 def qk_fusable(x: Tensor, w: Tensor, seq_len: int, head_dim: int) -> bool:
     """Whether linear_into(..., qk=...) takes this projection and is worth it: bf16, heads of 128,
-    columns in multiples of the 256-wide tile, sequences of at least one tile (a tile then holds rows
-    of at most two batch elements; ragged row counts and sequence lengths are fine), and enough
-    tiles that the library would pick the 256-wide ones anyway (the fused epilogue exists for them only)."""
+    columns in multiples of 256 (a wave's 128 columns are one head), sequences of at least 256 rows (a tile then holds
+    rows of at most two batch elements; ragged row counts and sequence lengths are fine), and at least 160 outputs
+    of 256 x 256, below which the preparation kernel behind a plain product is left alone."""
     M = x.numel() // x.shape[-1]
     N = w.shape[0]
     return (x.dtype == torch.bfloat16 and head_dim == 128 and seq_len >= 256 and M % seq_len == 0

@@ -358,7 +358,7 @@ def test_linear_tile_edges(B, L, N, K, splits):
 # Every tile that a product can get, by a product of few operations that gets it: with rows and columns to spare, with
 # and without a K tail, and with K in parts.
 EVERY_TILE = [
-    (EIGHT_WAVES, 64, 64, (9, 72, 64), (11, 72, 72), (9, 72, 6144)),
+    (EIGHT_WAVES, 64, 64, (9, 72, 64), (11, 72, 72), (9, 72, 8192)),
     (EIGHT_WAVES, 64, 96, (132, 5968, 64), (131, 6256, 72), (1397, 72, 6144)),
     (EIGHT_WAVES, 96, 96, (65, 8624, 64), (93, 8472, 80), (74, 1488, 6144)),
     (EIGHT_WAVES, 128, 96, (108, 12648, 64), (229, 8904, 72), (201, 1376, 12288)),

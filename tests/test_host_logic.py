@@ -168,6 +168,14 @@ def test_attention_asks_for_a_workspace_wherever_the_library_wants_one():
     assert not _may_cut_keys(96, 1024) and not _may_cut_keys(24, 1280)      # 24 heads: never
 
 
+def test_attention_keys_stay_whole_where_the_host_would_take_longer():
+    """A call in parts takes the host 22 us: [1, 2, 1420, 64] is done in 20.7 us without."""
+    from triton_kernels import _native as nv
+    need = nv.lib().flux_attention_workspace_bytes
+    assert need(1, 2, 1420, 64) == 0 and need(1, 2, 1024, 128) == 0
+    assert need(1, 2, 1793, 64) > 0 and need(1, 2, 1100, 128) > 0
+
+
 def test_launch_hook_is_called_once_right_before_every_launch(monkeypatch):
     """linear_pair_into launches two products at once or one after the other; a hook that opens a range per
     call must see one call per launch. The library is asked for its plan and not launched."""

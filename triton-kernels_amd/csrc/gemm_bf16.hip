@@ -825,7 +825,8 @@ static int64_t split_bytes(const GemmSet& g, const TileShape& t, int splits) {
 
 static const double kLaunch = 4.6, kTileLarge = 4.3, kTilePair = 2.7, kReduce = 1.7, kSplitGBs = 5970.0, kWeightGBs = 4500.0;
 static const double kIdleShare = 0.31;   // a workgroup runs up to this much faster the emptier the GPU is
-static const double kSplitHostUs = 6.0;  // K in parts costs the host this much
+static const double kSplitHostUs = 6.0;  // K in parts costs the host this much more, ...
+static const double kSplitCallUs = 20.0; // ... in all about this much
 
 static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
     const int64_t tiles = tile_count(g, t) * splits;
@@ -906,8 +907,9 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
         if (us < best.us) best = {t.family, t.fm, t.fn, 1, us, t.family == kPair && !columns_ok(t.fn)};
     }
     // K in parts, where that gains more than the host pays for it: a workspace to allocate and a second launch, 6 us
-    // per call (64 x 3072 x 3072 takes 11 us of the GPU in two parts and 13 in one, but the host 20 and 14).
-    if (workspace_bytes > 0 && p.K % 64 == 0 && p.K / 64 >= 8 && p.qk_cols == 0) {
+    // per call (64 x 3072 x 3072 takes 11 us of the GPU in two parts and 13 in one, but the host 20 and 14), and where
+    // the product in one piece takes the GPU longer than the call in parts takes the host.
+    if (workspace_bytes > 0 && best.us > kSplitCallUs && p.K % 64 == 0 && p.K / 64 >= 8 && p.qk_cols == 0) {
         const double bar = best.us - kSplitHostUs;
         TilePlan split = {kPair, 0, 0, 1, bar};
         for (const TileShape& t : kTileShapes) {

@@ -18,9 +18,9 @@ def _bhld_view(t: Tensor) -> Tensor:
 
 def _may_cut_keys(BH: int, L: int) -> bool:
     """False where flux_attention_workspace_bytes is known to be 0, so that the call is spared the question (0.4 of
-    16 us of host time): keys are cut in two or more parts up to 256 workgroups of 128 rows in all, and eleven tiles
-    of 64 keys are too few to pay for the second launch."""
-    return L > 704 and BH * ((L + 127) // 128) <= 128
+    16 us of host time): keys are cut in two or more parts up to 256 workgroups of 128 rows in all, and sixteen
+    tiles of 64 keys are too few to pay for the second launch."""
+    return L > 1024 and BH * ((L + 127) // 128) <= 128
 
 
 def attention_into(q: Tensor, k: Tensor, v: Tensor, out: Tensor, sm_scale: float | None = None,

@@ -478,3 +478,25 @@ def test_linear_pair_of_row_vectors(rows):
              for _ in range(2)]
     for y, call in zip(linear_pair_into(*calls), calls):
         assert torch.equal(y, tk.linear_into(**call))
+
+
+@pytest.mark.parametrize("M,K", [(1, 8), (1, 2048), (1, 4096), (1, 4104), (1, 24576), (2, 3080), (3, 3072), (3, 3416), (4, 3072),
+                                 (4, 3080), (5, 3072), (6, 4096), (7, 3072), (8, 3072), (8, 3080)])
+@pytest.mark.parametrize("N", [1, 129])
+def test_linear_row_vector_activation_shares(M, K, N):
+    """The activation rows of a row-vector product reach the workgroup in shares of 2048 values, some of them requested in
+    front of the weights: K at the edges of the shares, one past them, and past the memory they are staged in. Against
+    the float64 product of the separate operator's activations: half a bf16 ulp, and the fp32 sum's own error of at
+    most K 2^-24 of the sum of its terms' sizes."""
+    from triton_kernels.modules.blocks import _silu
+    g = seeded(M * K + N)
+    x = randn(g, M, K, dtype=torch.bfloat16, std=2.0).to(DEV)
+    w = randn(g, N, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV)
+    b = randn(g, N, dtype=torch.bfloat16).to(DEV)
+    got = tk.linear_into(x, w, b, in_activation="SiLU")
+    torch.testing.assert_close(_silu(x), oracle.silu_ref(x), atol=1e-6, rtol=2.0 ** -7)
+    a = _silu(x).double()
+    ref = a @ w.double().T + b.double()
+    sizes = a.abs() @ w.double().abs().T + b.double().abs()
+    assert ((got.double() - ref).abs() <= ref.abs() * (2.0 ** -8 * 1.01) + sizes * (K * 2.0 ** -24)).all()
+    assert torch.equal(tk.linear_into(x, w, None, in_activation="SiLU"), tk.linear_into(x, w, torch.zeros_like(b), in_activation="SiLU"))

@@ -65,6 +65,11 @@ template <typename T> struct alignas(16) Vec16 {
 template <typename T> __device__ __forceinline__ Vec16<T> ld16(const T* p) {
     return *reinterpret_cast<const Vec16<T>*>(p);
 }
+// The same for data that nothing reads again soon (weights of a product that passes over them once).
+template <typename T> __device__ __forceinline__ Vec16<T> ld16_once(const T* p) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(Vec16<T>, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
+}
 template <typename T> __device__ __forceinline__ void st16(T* p, const Vec16<T>& v) {
     *reinterpret_cast<Vec16<T>*>(p) = v;
 }

@@ -593,32 +593,57 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_rect_kernel(GemmLaunch L
 // ------------------------------------------------------------------------------------------------
 // Skinny problems (M <= 8, e.g. the Modulation projection of one conditioning vector per batch
 // element): HBM-bound on W. A wave streams the W rows of two output columns with 16-byte loads,
-// six in flight per lane, while the few activation rows come from cache; the dot products are
+// twelve in flight per lane, while the few activation rows come from cache; the dot products are
 // folded with a wave butterfly. The kernel is instantiated per row count, so it has no row tests.
+// Everything a wave needs beside W is requested in front of it: with the activation rows behind the W loads, and the
+// bias behind the sums, each was a wait of its own while all waves of the launch stood at the same place. W is read
+// once, so its loads carry the non-temporal hint (a bare read of 113 MB: 18.4 -> 17.4 us). us, weights from HBM,
+// before -> now: 1 x 9216 x 3072 with SiLU 14.0 -> 11.2 (the bare read 9.5), two such products of 18432 columns in one launch
+// 38.7 -> 33.8 (6.7 TB/s), 3 rows 17.8 -> 15.8, 8 rows 33.2 -> 31.2, 1 x 3072 x 12288 20.7 -> 19.1.
 // ------------------------------------------------------------------------------------------------
 constexpr int kGemvCols = 2;  // output columns per wave
 constexpr int kGemvSiluLds = 48 * 1024;  // bytes of LDS for the (activated) input rows (bf16)
-// 16-byte vectors of a W row a lane requests at once: a whole row of 3072 for one or two activation rows,
-// half of that when more rows' products need the registers
-constexpr int gemv_depth(int rows) { return rows <= 2 ? 6 : 3; }
+// 16-byte vectors of a W row a lane requests at once: a whole row of 3072 for up to four activation rows, half of
+// that when more rows' products need the registers (8 rows: 33 us, 49 with whole rows)
+constexpr int gemv_depth(int rows) { return rows <= 4 ? 6 : 3; }
 
 // SILU_LDS: the few activation rows are staged in LDS once per workgroup, with the input activation
 // x * sigmoid(x) applied on the way (rounded to bf16, as the separate operator would leave it). Every
 // wave needs all K values of every row: read from memory inside the K loop they queue behind the W
 // loads of the wave (the memory counter is in-order), and the activation, two transcendentals per
-// value, would be repeated by each of the N / 2 waves. Rows that do not fit the LDS budget are read
+// value, would be repeated by each of the N / 2 waves. For the same reason the workgroup's share of them is
+// requested in front of the first W loads, not behind. Rows that do not fit the LDS budget are read
 // from memory as they are needed.
 // EXACT: K = 512 * U, so every lane has exactly U vectors per row and the K loop runs once, without tests.
 template <int MM, bool SILU_LDS, bool EXACT>
 __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
     const GemmParams p = g.p[blockIdx.y];
-    constexpr int CPW = kGemvCols, U = gemv_depth(MM);  // CPW * U 16-byte loads of W in flight per lane: a whole row of 3072
+    constexpr int CPW = kGemvCols, U = gemv_depth(MM);  // CPW * U 16-byte loads of W in flight per lane
+    constexpr int PRE = MM <= 4 ? MM + (MM + 1) / 2 : 2;  // activation vectors requested in front: a thread's share at K = 3072
     extern __shared__ __attribute__((aligned(16))) char act_lds[];
     const int lane = threadIdx.x & 63;
     const int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * CPW;
     const bf16_t* wrow[CPW];
 #pragma unroll
     for (int c = 0; c < CPW; ++c) wrow[c] = p.W + static_cast<int64_t>(n0 + c < p.N ? n0 + c : (n0 < p.N ? n0 : p.N - 1)) * p.ldw;
+    const int act_n = MM * p.K;
+    auto act_at = [&](int i) {   // K is a multiple of 8: a vector stays inside one row
+        const int m = MM == 1 ? 0 : i / p.K, k = i - m * p.K;
+        return p.A + static_cast<int64_t>(m) * p.lda + k;
+    };
+    // (the bias goes in front too: behind the sums it was a round trip to memory with nothing beside it)
+    bf16_t bias_raw[CPW];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) bias_raw[c] = p.bias ? p.bias[min(n0 + c, p.N - 1)] : static_cast<bf16_t>(0);
+    Vec16<bf16_t> pre[PRE];
+    if (SILU_LDS) {
+#pragma unroll
+        for (int j = 0; j < PRE; ++j) {
+            const int i = static_cast<int>(threadIdx.x) * 8 + j * 2048;
+            pre[j] = ld16(act_at(i < act_n ? i : 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     // the first group of W loads goes out before the activation is worked on
     Vec16<bf16_t> w[U][CPW];
     auto request_w = [&](int k0) {
@@ -627,15 +652,14 @@ __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
             const int k = k0 + u * 512;
             // past the end: a harmless re-read, skipped below
 #pragma unroll
-            for (int c = 0; c < CPW; ++c) w[u][c] = ld16(wrow[c] + (EXACT || k < p.K ? k : k0));
+            for (int c = 0; c < CPW; ++c) w[u][c] = ld16_once(wrow[c] + (EXACT || k < p.K ? k : k0));
         }
     };
     if (EXACT || lane * 8 < p.K) request_w(lane * 8);
     if (SILU_LDS) {
+        __builtin_amdgcn_sched_barrier(0);
         bf16_t* dst = reinterpret_cast<bf16_t*>(act_lds);
-        for (int i = threadIdx.x * 8; i < MM * p.K; i += 256 * 8) {   // K is a multiple of 8: a vector stays inside one row
-            const int m = i / p.K, k = i - m * p.K;
-            const Vec16<bf16_t> a = ld16(p.A + static_cast<int64_t>(m) * p.lda + k);
+        auto stage = [&](int i, const Vec16<bf16_t>& a) {
             Vec16<bf16_t> o = a;
             if (p.in_silu) {
 #pragma unroll
@@ -645,7 +669,13 @@ __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
                 }
             }
             *reinterpret_cast<Vec16<bf16_t>*>(dst + i) = o;
+        };
+#pragma unroll
+        for (int j = 0; j < PRE; ++j) {
+            const int i = static_cast<int>(threadIdx.x) * 8 + j * 2048;
+            if (i < act_n) stage(i, pre[j]);
         }
+        for (int i = threadIdx.x * 8 + PRE * 2048; i < act_n; i += 2048) stage(i, ld16(act_at(i)));
         __syncthreads();
     }
     if (n0 >= p.N) return;  // whole wave leaves together (after the barrier)
@@ -692,7 +722,7 @@ __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
         for (int c = 0; c < CPW; ++c) {
             const int n = n0 + c;
             if (n >= p.N) break;
-            const float b = p.bias ? bf2f(p.bias[n]) : 0.0f;
+            const float b = bf2f(bias_raw[c]);
 #pragma unroll
             for (int m = 0; m < MM; ++m) {
                 float t = acc[c][m] + b;

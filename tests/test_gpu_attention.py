@@ -168,6 +168,21 @@ def test_attention_wide_tile_strided_views(D):
 
 
 @pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("row", [1 << 24, (1 << 24) - 8])
+def test_attention_far_apart_query_rows(row, D):
+    """Rows of q at the distance from which 64 of them no longer lie within 31-bit byte offsets, and just below it: the
+    64-row kernel fetches q through such offsets, a call beyond them takes the 32-row kernel."""
+    H, L = 130, 130                                              # 260 workgroups of 128 rows
+    g = seeded(D)
+    flat = torch.empty((L - 1) * row + H * D, dtype=torch.bfloat16, device=DEV)
+    q = flat.as_strided((1, H, L, D), (0, D, row, 1))
+    q.copy_(randn(g, 1, H, L, D, dtype=torch.bfloat16))
+    k, v = (randn(g, 1, H, L, D, dtype=torch.bfloat16).to(DEV) for _ in range(2))
+    o = tk.scaled_dot_product_attention(q, k, v)
+    torch.testing.assert_close(o.float(), oracle.attention_ref_fp32(q.contiguous(), k, v), atol=1e-2, rtol=0)
+
+
+@pytest.mark.parametrize("D", [128, 64])
 @pytest.mark.parametrize("H", [24, 4])   # 24 heads: 64-row-per-wave kernel; 4 heads: 128-row workgroups
 @pytest.mark.parametrize("kind", ["hot", "ramp"])
 def test_attention_large_scores_move_the_reference_maximum(H, kind, D):

@@ -81,6 +81,13 @@ __device__ __forceinline__ void lds_load16_raw_at(u32x4 rsrc, uint32_t lds_base,
                  : "s"(lds_base), "v"(voff), "s"(rsrc), "n"(OFF)
                  : "memory", "scc", "m0");
 }
+// Brings the cache lines that the lanes point at into the L2: one dword each, to 256 bytes of LDS that nothing reads.
+__device__ __forceinline__ void touch_raw(u32x4 rsrc, uint32_t lds_addr, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(rsrc)
+                 : "memory", "m0");
+}
 __device__ __forceinline__ uint32_t lds_addr_of(const char* p) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
 }
@@ -760,8 +767,23 @@ constexpr int attn_load_slot(int j, int ns, int bs, int sp, bool second) {
 // 32 keys) and the same softmax work, so there the VALU sets the pace: every slot carries an
 // exponential. Rows of K and V are 128 bytes, a wave-wide load covers eight of them, and the swizzles
 // are those of 128-byte rows (below).
-template <int D, int QB, int NW>
-__device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, const int block, const int nblocks) {
+// Tile of a block of one of the two parts of a launch: (batch, head) and first row; false where there is none.
+__device__ __forceinline__ bool attn_w64_find(const AttnParams& p, int rows, int block, int nblocks, int& bh, int& row0) {
+    const int per_xcd = nblocks / 8;
+    const int vt = (block % 8) * per_xcd + block / 8;
+    if (vt >= p.total_tiles) return false;
+    const int per_pair = p.cnt_even + p.cnt_odd;
+    const int pair = vt / per_pair, rem = vt % per_pair;
+    const bool odd = rem >= p.cnt_even;
+    bh = 2 * pair + odd;
+    row0 = (odd ? p.first_odd : p.first_even) + (odd ? rem - p.cnt_even : rem) * rows;
+    return true;
+}
+
+// `next` finds the tile that this CU, or another of its XCD, will probably take next: its first loads are brought into
+// the L2 from here (see the end of the common loop).
+template <int D, int QB, int NW, typename Next>
+__device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, const int block, const int nblocks, Next&& next) {
     static_assert(NW == 4 && (QB == 3 || QB == 4) && (D == 64 || D == 128), "configurations that have been laid out and measured");
     constexpr int ROWS = 16 * QB * NW;         // query rows per workgroup
     constexpr int KS = D / 32, DBN = D / 16, ROWB = D * 2, TB = 64 * ROWB, HALF = 32 * ROWB;
@@ -780,19 +802,14 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     static_assert(attn_load_slot(LPW - 1, NS, BS, NS / 8, false) != -2, "load slots");
     constexpr float kRebase = 1.0995116e12f;  // 2^40
     // lds: 8 * TB bytes, K ring of 4 tiles, V ring of 4 tiles
-    const int per_xcd = nblocks / 8;
-    const int vt = (block % 8) * per_xcd + block / 8;
-    if (vt >= p.total_tiles) return;
-    const int per_pair = p.cnt_even + p.cnt_odd;
-    const int pair = vt / per_pair, rem = vt % per_pair;
-    const bool odd = rem >= p.cnt_even;
-    const int bh = 2 * pair + odd, qt = odd ? rem - p.cnt_even : rem;
+    int bh, row0;
+    if (!attn_w64_find(p, ROWS, block, nblocks, bh, row0)) return;
     const int b = bh / p.H, h = bh % p.H;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int q0 = (odd ? p.first_odd : p.first_even) + qt * ROWS + wave * (16 * QB);
+    const int q0 = row0 + wave * (16 * QB);
     const float c = p.scale_log2;
 
     const bf16_t* kbase = p.k + b * p.k_sb + h * p.k_sh;
@@ -838,6 +855,39 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
         for (int i = 0; i < PP; ++i) lds_load16_raw(rs, lds_base + V0 + buf * TB + i * (NW * 1024), v_voff[i]);
     };
 
+    // Q: a wave fetches its own 16*QB rows into one of the four ring buffers that stay empty until the loop is
+    // about to start (K 2 and 3, V 1 and 2), whole rows per load and swizzled like K, and reads its fragments from
+    // there. (Fragments loaded straight into registers are pieces of 64 bytes of 16 rows, 64 cycles of the CU's
+    // address path each, and 64 registers.) Sixteen rows at a time have a descriptor of their own, rows past the end
+    // read as zeros. K(0) goes first, V(0) and K(1) last: the first scores do not wait for those.
+    load_k(0, 0);
+    char* const q_lds = lds + (2 + wave + (wave >> 1)) * TB;
+    {
+        constexpr int LPB = 16 / RPL;   // loads per 16 rows
+        const uint32_t q_at = lds_addr_of(q_lds);
+        const int q_row2 = static_cast<int>(p.q_sl * 2);
+        uint32_t q_voff[LPB];
+#pragma unroll
+        for (int i = 0; i < LPB; ++i) {
+            const int r = i * RPL + l_row;
+            q_voff[i] = static_cast<uint32_t>(r * q_row2 + (l_pos ^ k_swz(r)) * 16);
+        }
+        uint64_t at = reinterpret_cast<uint64_t>(p.q + b * p.q_sb + h * p.q_sh) + static_cast<uint64_t>(static_cast<int64_t>(q0) * q_row2);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            const int rows = min(p.L - q0 - qb * 16, 16);
+            u32x4 r;
+            r.x = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
+            r.y = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32) & 0xffffu);
+            r.z = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(rows > 0 ? (rows - 1) * q_row2 + D * 2 : 0));
+            r.w = kAttnRsrcFlags;
+#pragma unroll
+            for (int i = 0; i < LPB; ++i) lds_load16_raw(r, q_at + (qb * LPB + i) * 1024, q_voff[i]);
+            at += static_cast<uint64_t>(16) * static_cast<uint64_t>(static_cast<int64_t>(q_row2));
+        }
+    }
+    load_v(0, 0);
+    load_k(1, 1);
     // The first pass through the loop multiplies P = 0 with whatever the last V buffer holds:
     // make that finite.
     {
@@ -845,32 +895,24 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
 #pragma unroll
         for (int i = 0; i < PP; ++i) *reinterpret_cast<u32x4*>(lds + V0 + 3 * TB + i * (NW * 1024) + tid * 16) = z;
     }
-    load_k(0, 0);
-    load_v(0, 0);
-    load_k(1, 1);
 
     // Q fragments ("B" operand of S^T): lane holds row q0 + qb*16 + r16, d = ks*32 + g*8 .. +8,
     // scaled by sm_scale*log2(e) and rounded to bf16.
     attn_claim_agprs<(D == 128 ? 48 * QB : 96)>();
+    static_for<0, kAccQ>([&](auto i_c) { acc_write<decltype(i_c)::value>(0u); });  // O^T = 0, while the loads are on their way
     {
-        u32x4 qraw[QB][KS];  // all loads in flight before the first conversion
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PP) : "memory");   // K(0) and Q have landed
+        u32x4 qraw[QB][KS];
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-            const int row = q0 + qb * 16 + r16;
-            const bool ok = row < p.L;
-            const bf16_t* rp = p.q + b * p.q_sb + h * p.q_sh + static_cast<int64_t>(ok ? row : 0) * p.q_sl;
+        for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                qraw[qb][ks] = *reinterpret_cast<const u32x4*>(rp + ks * 32 + g * 8);
-                if (!ok) qraw[qb][ks] = u32x4{0u, 0u, 0u, 0u};
-            }
-        }
+            for (int ks = 0; ks < KS; ++ks)
+                qraw[qb][ks] = *reinterpret_cast<const u32x4*>(q_lds + (qb * 16 + r16) * ROWB + (((ks * 4 + g) ^ k_swz(r16)) * 16));
         static_for<0, QB * KS * 4>([&](auto i_c) {
             constexpr int i = decltype(i_c)::value, qb = i / kQRegs, ks = (i / 4) % KS, e = i % 4;
             const uint32_t t = qraw[qb][ks][e];
             acc_write<kAccQ + i>(pack2_bf16(__uint_as_float(t << 16) * c, __uint_as_float(t & 0xffff0000u) * c));
         });
-        static_for<0, kAccQ>([&](auto i_c) { acc_write<decltype(i_c)::value>(0u); });  // O^T = 0
     }
 
     // fragment addresses, lane part (the ring offset of the sub-tile is added once per iteration,
@@ -926,7 +968,7 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     };
 
     // ---- prologue: S^T(0) from the first half of K(0), then the rows' first reference maxima
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     static_for<0, 2 * KS>([&](auto n_c) {
         constexpr int n = decltype(n_c)::value, kb = n / KS, ks = n % KS;
         const bf16x8 f = *reinterpret_cast<const bf16x8*>(lds + k_addr[ks] + kb * 16 * ROWB);
@@ -1159,6 +1201,35 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
         body(std::integral_constant<int, 2>{}, std::false_type{}, T + 2);
         body(std::integral_constant<int, 3>{}, std::false_type{}, T + 3);
     }
+    // A workgroup that starts behind this one waits for its first 112 KB to come from HBM with the matrix pipe idle
+    // (3.8 us from its start to its first MFMA at head dim 128), so the rows of Q and of the first K and V tile of the
+    // tile 256 blocks on are touched here, a few microseconds ahead. us, with the fetch of Q above, before -> now:
+    // [4, 24, 1024, 128] 58.2 -> 57.2, [4, 24, 800, 128] 45.8 -> 45.2, [2, 24, 2048, 128] 97.8 -> 96.8, [4, 24, 2000, 64]
+    // 112.0 -> 110.6; launches of one round and of many long ones stay as they were.
+    {
+        int nbh, nrow0;
+        if (next(nbh, nrow0)) {
+            const int nb = nbh / p.H, nh = nbh % p.H;
+            const bool is_v = wave >= 2;
+            constexpr int LPR = D / 64, RPT = 64 / LPR;   // 128-byte lines per row; rows a touch covers
+            const int t_row = lane / LPR, t_col = (lane % LPR) * 128;
+            auto touch = [&](const bf16_t* base, int64_t sl, int row_first, int rows) {
+                const int left = min(p.L - row_first, rows);
+                const uint64_t at = reinterpret_cast<uint64_t>(base + row_first * sl);
+                u32x4 r;
+                r.x = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
+                r.y = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32) & 0xffffu);
+                r.z = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(left > 0 ? (left - 1) * static_cast<int>(sl * 2) + D * 2 : 0));
+                r.w = kAttnRsrcFlags;
+                touch_raw(r, lds_addr_of(lds) + 8 * TB, static_cast<uint32_t>(t_row * static_cast<int>(sl * 2) + t_col));
+            };
+            const bf16_t* const nq = p.q + nb * p.q_sb + nh * p.q_sh;
+#pragma unroll
+            for (int i = 0; i < 64 / RPT; ++i) touch(nq, p.q_sl, nrow0 + wave * 64 + i * RPT, RPT);
+            if (is_v) touch(p.v + nb * p.v_sb + nh * p.v_sh, p.v_sl, (wave & 1) * 32, 32);
+            else touch(p.k + nb * p.k_sb + nh * p.k_sh, p.k_sl, (wave & 1) * 32, 32);
+        }
+    }
     for (;; T += 4) {
         if (!body(std::integral_constant<int, 0>{}, std::true_type{}, T)) break;
         if (!body(std::integral_constant<int, 1>{}, std::true_type{}, T + 1)) break;
@@ -1175,6 +1246,11 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     // reads both spread over all banks, and a 16-byte chunk stays contiguous.
     asm volatile("s_barrier" ::: "memory");
     char* const stage = lds + wave * (16 * QB * ROWB);
+    int o_row = lane / CH;   // (opaque: row numbers shared with the fetch of Q would live in registers through the loop)
+    asm volatile("" : "+v"(o_row));
+    const int o_chunk = lane % CH;
+    bf16_t* o_at = p.o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(q0 + o_row) * p.o_sl + o_chunk * 8;
+    const int64_t o_step = RPL * p.o_sl;
     static_for<0, QB>([&](auto qb_c) {
         constexpr int qb = decltype(qb_c)::value, QBC = qb;
         float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 16, 64);
@@ -1193,16 +1269,12 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
             p.lse[static_cast<int64_t>(bh) * p.L + row] = -seed[qb][0] + __builtin_amdgcn_logf(l_tot);
     });
     __builtin_amdgcn_wave_barrier();  // LDS operations of one wave complete in order
-    {
-        bf16_t* const obase = p.o + b * p.o_sb + h * p.o_sh;
-        const int chunk = lane % CH;
 #pragma unroll
-        for (int it = 0; it < 16 * QB / RPL; ++it) {
-            const int rl = it * RPL + lane / CH;
-            const u32x4 y = *reinterpret_cast<const u32x4*>(stage + rl * ROWB + ((chunk ^ (rl % CH)) * 16));
-            const int row = q0 + rl;
-            if (row < p.L) *reinterpret_cast<u32x4*>(obase + static_cast<int64_t>(row) * p.o_sl + chunk * 8) = y;
-        }
+    for (int it = 0; it < 16 * QB / RPL; ++it) {
+        const int rl = it * RPL + o_row;
+        const u32x4 y = *reinterpret_cast<const u32x4*>(stage + rl * ROWB + ((o_chunk ^ (rl % CH)) * 16));
+        if (q0 + rl < p.L) *reinterpret_cast<u32x4*>(o_at) = y;
+        o_at += o_step;
     }
 }
 
@@ -1213,14 +1285,21 @@ constexpr int w64_lds_bytes(int d) { return 8 * 64 * 2 * d; }  // K ring and V r
 // p3. Workgroups are handed out in order, so the 192-row tiles start on each CU as it finishes its
 // 256-row tile, with no launch boundary in between. n4 and the remainder are multiples of eight, so
 // a block's XCD is the same counted from either start. A launch of 256-row tiles only has n4 = grid.
+constexpr int kAttnCUs = 256;
+
 template <int D>
 __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel_pair(AttnParams p4, AttnParams p3, int n4) {
-    __shared__ __attribute__((aligned(1024))) char lds[w64_lds_bytes(D)];
-    if (static_cast<int>(blockIdx.x) < n4) attn_w64_tile<D, 4, 4>(p4, lds, blockIdx.x, n4);
-    else attn_w64_tile<D, 3, 4>(p3, lds, static_cast<int>(blockIdx.x) - n4, static_cast<int>(gridDim.x) - n4);
+    __shared__ __attribute__((aligned(1024))) char lds[w64_lds_bytes(D) + 256];
+    const int grid = static_cast<int>(gridDim.x), block = static_cast<int>(blockIdx.x);
+    auto next = [&](int& bh, int& row0) {
+        const int nb = block + kAttnCUs;   // the same XCD
+        if (nb < n4) return attn_w64_find(p4, 256, nb, n4, bh, row0);
+        return nb < grid && attn_w64_find(p3, 192, nb - n4, grid - n4, bh, row0);
+    };
+    if (block < n4) attn_w64_tile<D, 4, 4>(p4, lds, block, n4, next);
+    else attn_w64_tile<D, 3, 4>(p3, lds, block - n4, grid - n4, next);
 }
 
-constexpr int kAttnCUs = 256;
 
 #ifndef FLUX_ATTN_W64_D64_UNIT
 // Parts that the keys are cut in where 128-row workgroups leave half the GPU idle or more, and the keys of a
@@ -1392,6 +1471,8 @@ using namespace flux;
 // head dim 128: [1, 24, 1280] (240 workgroups) 29 and 35, [1, 8, 4096] (256) 86 and 89, [1, 24, 1500] (288)
 // 47 and 40; head dim 64: 19 and 24, 52 and 61, 32 and 28.
 static bool attn_short(int64_t BH, int64_t L) { return BH * ((L + 127) / 128) <= kAttnCUs; }
+// The 64-row kernel reaches the rows of q with 32-bit offsets inside 64 rows; the 32-row one has no such limit.
+static bool attn_q_near(const flux_attn_args* a) { return a->q.sl * 2 * 64 < 0x7fffffffLL; }
 
 static bool view_ok(const void* ptr, int64_t sb, int64_t sh, int64_t sl) {
     return ptr != nullptr && aligned16(ptr) && sb % 8 == 0 && sh % 8 == 0 && sl % 8 == 0;
@@ -1423,9 +1504,9 @@ static int attention_launch(const flux_attn_args* a, void* workspace, int64_t wo
     if (a->D != 64 && a->D != 128) {
         if (BH * ((a->L + 63) / 64) > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: problem too large");
         attn_launch_plain(p, BH, a->D, st);
-    } else if (a->D == 128 && !attn_short(BH, a->L)) attn_launch_w64<128>(p, BH, st);
+    } else if (a->D == 128 && !attn_short(BH, a->L) && attn_q_near(a)) attn_launch_w64<128>(p, BH, st);
     else if (a->D == 128) attn_launch_pipe<128>(p, BH, static_cast<float*>(workspace), workspace_bytes, st);
-    else if (!attn_short(BH, a->L)) attn_launch_w64_d64(p, BH, st);
+    else if (!attn_short(BH, a->L) && attn_q_near(a)) attn_launch_w64_d64(p, BH, st);
     else attn_launch_pipe<64>(p, BH, static_cast<float*>(workspace), workspace_bytes, st);
     return check_launch("flux_attention_fwd_bf16");
 }

@@ -1,0 +1,243 @@
+"""The operators' calls in native code (csrc/torch_ops.cpp) against the Python launchers of the same operators, over the forms
+they accept, and the calls that they leave to the launchers."""
+import threading
+
+import pytest
+import torch
+import torch.autograd.forward_ad as fwad
+
+import triton_kernels as tk
+from triton_kernels import _native as nv
+from triton_kernels.kernels import attention as attention_mod
+from triton_kernels.kernels import linear as linear_mod
+from triton_kernels.kernels import normalization as norm_mod
+from triton_kernels.kernels import positional_embedding as rope_mod
+from util import DEV, randn, seeded
+
+gpu = pytest.mark.gpu
+BF, F32 = torch.bfloat16, torch.float32
+
+
+class _Refuses:
+    """Native calls that take nothing: every operator goes through its Python launcher."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def launcher(monkeypatch, fn, *args, **kw):
+    with monkeypatch.context() as m:
+        m.setattr(nv, "ops", lambda: _Refuses())
+        return fn(*args, **kw)
+
+
+def test_tensors_without_a_gpu_are_left_to_the_launchers():
+    ops, x = nv.ops(), torch.ones(2, 2, 4, 8)
+    assert ops.rms_norm(x, torch.ones(8), 1e-6) is None
+    assert ops.rms_norm_pair(x, torch.ones(8), x, torch.ones(8), 1e-6) is None
+    assert ops.layer_norm_modulation(x, x, x, 1e-5) is None
+    assert ops.apply_rope(x, x, x) is None
+    assert ops.linear(x.bfloat16(), torch.ones(8, 8, dtype=BF), None, 0) is None
+    assert ops.attention(x.bfloat16(), x.bfloat16(), x.bfloat16(), None) is None
+    for bad in (None, 3, "x", [x]):
+        assert ops.rms_norm(bad, torch.ones(8), 1e-6) is None
+    with pytest.raises(RuntimeError, match="GPU"):
+        tk.rms_norm(x, torch.ones(8))
+
+
+def _views(g, dtype):
+    """Rows of one to 300 values in every order and stride that a norm reads in place, and those it copies or refuses."""
+    base = randn(g, 3, 4, 5, 128, dtype=dtype).to(DEV)
+    wide = randn(g, 2, 6, 3 * 256, dtype=dtype).to(DEV)
+    return [base, base[0, 0, 0], base[1], base.permute(2, 0, 1, 3), base.transpose(1, 2)[::2], wide[..., 256:512], wide.view(2, 6, 3, 2, 128).permute(2, 0, 3, 1, 4)[1],
+            base[..., :100], base[..., 1:129:1][..., :50], base[:, :, :1].expand(3, 4, 7, 128), base.flatten()[:7 * 300].view(7, 300), base.flatten()[3:3 + 5 * 33].view(5, 33),
+            base[..., ::2], base.view(3, 2, 2, 5, 128), base[:0], base.flatten()[:9].view(9, 1)]
+
+
+@gpu
+@pytest.mark.parametrize("dtype,scale_dtype", [(BF, BF), (BF, F32), (F32, F32), (F32, BF)])
+def test_rms_norm_forms(monkeypatch, dtype, scale_dtype):
+    g = seeded(1)
+    for x in _views(g, dtype):
+        for scale in (randn(g, x.shape[-1], dtype=scale_dtype).to(DEV), randn(g, 1, x.shape[-1], dtype=scale_dtype).to(DEV)):
+            if x.numel():
+                got = tk.rms_norm(x, scale)
+                want = launcher(monkeypatch, tk.rms_norm, x, scale)
+                assert torch.equal(got, want) and got.stride() == want.stride() and got.dtype == want.dtype
+            xs = [x.detach().clone(memory_format=torch.preserve_format).requires_grad_(True) for _ in range(2)]
+            ss = [scale.detach().clone().requires_grad_(True) for _ in range(2)]
+            dy = randn(g, *x.shape, dtype=dtype).to(DEV)
+            if not x.numel():
+                continue
+            ys = tk.rms_norm(xs[0], ss[0]), launcher(monkeypatch, tk.rms_norm, xs[1], ss[1])
+            for y in ys:
+                y.backward(dy)
+            assert torch.equal(ys[0], ys[1]) and torch.equal(xs[0].grad, xs[1].grad) and xs[0].grad.stride() == xs[1].grad.stride()
+            # (rows that are no 16-byte vectors add the scale's gradient with atomics, in any order)
+            torch.testing.assert_close(ss[0].grad, ss[1].grad, atol=1e-5 if scale_dtype == F32 else 2e-2, rtol=1e-5 if scale_dtype == F32 else 2.0 ** -7)
+            assert ss[0].grad.dtype == scale_dtype and ss[0].grad.shape == scale.shape
+
+
+@gpu
+def test_rms_norm_pair_and_layer_norm_forms(monkeypatch):
+    g = seeded(2)
+    for dtype in (BF, F32):
+        views = [v for v in _views(g, dtype) if v.numel()]
+        with torch.no_grad():
+            for x0 in views:
+                for x1 in views:
+                    if x0.shape[-1] == x1.shape[-1]:
+                        s = [randn(g, x0.shape[-1], dtype=dtype).to(DEV) for _ in range(2)]
+                        got, want = norm_mod.rms_norm_pair(x0, s[0], x1, s[1]), launcher(monkeypatch, norm_mod.rms_norm_pair, x0, s[0], x1, s[1])
+                        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        for x in views:
+            if x.dim() < 2:
+                continue
+            B, N = x.shape[0], x.shape[-1]
+            mod = randn(g, B, 1, 3 * N, dtype=dtype).to(DEV)
+            for w, b in (mod.chunk(3, -1)[:2], (mod[..., :N].contiguous(), mod[..., N:2 * N]), (mod[:, 0, :N], mod[:, 0, N:2 * N]), (mod[..., ::3], mod[..., 1::3]),
+                         (mod[:1, :, :N].expand(B, 1, N), mod[:1, :, N:2 * N].expand(B, 1, N)), (mod[..., :N].float(), mod[..., N:2 * N].float())):
+                assert torch.equal(tk.layer_norm_modulation(x, w, b), launcher(monkeypatch, tk.layer_norm_modulation, x, w, b))
+
+
+@gpu
+def test_rope_linear_attention_forms(monkeypatch):
+    g = seeded(3)
+    for dtype in (BF, F32):
+        for D in (128, 64, 16):
+            qkv = randn(g, 2, 9, 3 * 4 * D, dtype=dtype).to(DEV).view(2, 9, 3, 4, D).permute(2, 0, 3, 1, 4)
+            pes = [randn(g, *lead, 9, D // 2, 2, 2).to(DEV) for lead in ((1, 1), (), (2, 1), (1, 4), (1,))]
+            for q, k in ((qkv[0], qkv[1]), (qkv[0].contiguous(), qkv[1].contiguous()), (qkv[0].transpose(2, 3).contiguous().transpose(2, 3), qkv[1])):
+                for pe in pes + [pes[0].double(), pes[0].transpose(-1, -2)]:
+                    got, want = tk.apply_rope(q, k, pe), launcher(monkeypatch, tk.apply_rope, q, k, pe)
+                    assert all(torch.equal(a, b) and a.stride() == b.stride() for a, b in zip(got, want))
+    for M, N, K in ((1, 64, 64), (8, 40, 72), (9, 40, 72), (300, 136, 3080), (64, 33, 50), (256, 256, 3136)):
+        x, w, b = randn(g, M, K, dtype=BF).to(DEV), randn(g, N, K, dtype=BF, std=K ** -0.5).to(DEV), randn(g, N, dtype=BF).to(DEV)
+        half = randn(g, M, 2 * K, dtype=BF).to(DEV)[:, :K]
+        for xx in (x, x.view(1, M, K), x.t().contiguous().t(), half, x[0]):
+            for ww in (w, randn(g, K, N, dtype=BF).to(DEV).t()):
+                for bb in (b, None, b.float(), b.view(1, N)):
+                    for act in ("", "GELU"):
+                        got, want = tk.linear(xx, ww, bb, activation=act), launcher(monkeypatch, tk.linear, xx, ww, bb, activation=act)
+                        assert torch.equal(got, want) and got.shape == want.shape and got.stride() == want.stride()
+    for B, H, L, D in ((1, 2, 1, 64), (2, 3, 77, 128), (1, 2, 1500, 64), (1, 2, 40, 32), (4, 24, 300, 128)):
+        qkv = randn(g, B, L, 3, H, D, dtype=BF).to(DEV).permute(2, 0, 3, 1, 4)
+        for q, k, v in (qkv.unbind(0), [t.contiguous() for t in qkv], (qkv[0], qkv[1].transpose(2, 3).contiguous().transpose(2, 3), qkv[2])):
+            for scale in (None, 0.3, 0.0, torch.tensor(0.2)):
+                got, want = tk.scaled_dot_product_attention(q, k, v, scale), launcher(monkeypatch, tk.scaled_dot_product_attention, q, k, v, scale)
+                assert torch.equal(got, want) and got.stride() == want.stride()
+
+
+@gpu
+def test_refusals_stay_what_they_were(monkeypatch):
+    x, w = torch.ones(4, 64, device=DEV, dtype=BF), torch.ones(32, 64, device=DEV, dtype=BF)
+    h = x.view(1, 1, 4, 64)
+    calls = [(tk.rms_norm, x, torch.ones(32, device=DEV, dtype=BF)), (tk.rms_norm, torch.ones(1, 70000, device=DEV), torch.ones(70000, device=DEV)),
+             (tk.rms_norm, x.half(), w[0].half()), (tk.rms_norm, x, w[0].cpu()), (tk.linear, x, w[:, :32], None), (tk.linear, x.float(), w, None), (tk.linear, x.float(), w.float(), None),
+             (tk.linear, x, w, None, "RELU"), (tk.linear, x, w, torch.ones(7, device=DEV, dtype=BF)), (tk.scaled_dot_product_attention, h, h, h.float()),
+             (tk.scaled_dot_product_attention, h, h, h, float("nan")), (tk.scaled_dot_product_attention, h[..., :24], h[..., :24], h[..., :24]),
+             (tk.scaled_dot_product_attention, h, h, h[:, :, :2]), (tk.apply_rope, h, h, torch.ones(1, 1, 5, 32, 2, 2, device=DEV)), (tk.apply_rope, h, h.float(), h), (tk.apply_rope, h[..., :24], h[..., :24], torch.ones(1, 1, 4, 12, 2, 2, device=DEV)),
+             (tk.layer_norm_modulation, h, h[:, :, 0], h[:, :, :1, :32]), (tk.layer_norm_modulation, x, x[:2], x)]
+    for fn, *args in calls:
+        errors = []
+        for call in (lambda: fn(*args), lambda: launcher(monkeypatch, fn, *args)):
+            with pytest.raises(Exception) as e:
+                call()
+            errors.append(e)
+        assert errors[0].type is errors[1].type and str(errors[0].value) == str(errors[1].value)
+
+
+@gpu
+def test_transforms_tracing_and_forward_mode_see_the_launchers():
+    ops, g = nv.ops(), seeded(4)
+    x, s = randn(g, 3, 64).to(DEV), randn(g, 64).to(DEV)
+    assert ops.rms_norm(x, s, 1e-6) is not None
+    for transform in (torch.func.vmap, lambda f: torch.func.grad(lambda t: f(t).sum())):
+        with pytest.raises(RuntimeError):
+            transform(lambda t: tk.rms_norm(t, s))(x)
+    with fwad.dual_level():
+        assert ops.rms_norm(x, s, 1e-6) is None
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            tk.rms_norm(fwad.make_dual(x, torch.ones_like(x)), s)
+        with torch.no_grad(), pytest.raises((RuntimeError, NotImplementedError)):
+            norm_mod.rms_norm_pair(fwad.make_dual(x, torch.ones_like(x)), s, x, s)
+    seen = []
+
+    def traced(t):
+        seen.append(ops.rms_norm(t, s, 1e-6))
+        return t + 1
+
+    torch.jit.trace(traced, x, check_trace=False)
+    assert seen == [None]
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert ops.rms_norm(x.as_subclass(Sub), s, 1e-6) is None
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert ops.rms_norm(x, s, 1e-6) is None
+    with torch.inference_mode():
+        assert torch.equal(tk.rms_norm(x, s), norm_mod.rms_norm_forward(x, s)[0])
+
+
+@gpu
+def test_rms_norm_graph_behaves_like_the_function():
+    g = seeded(5)
+    x, s = randn(g, 8, 128, dtype=BF).to(DEV).requires_grad_(True), randn(g, 128, dtype=BF).to(DEV).requires_grad_(True)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.to(DEV)):
+        y = tk.rms_norm(x, s)
+    assert packed == [(8, 128), (128,), (8,)]
+    plain = tk.rms_norm(x, s)
+    dy = torch.ones_like(y)
+    for a, b in zip(torch.autograd.grad(y, (x, s), dy), torch.autograd.grad(plain, (x, s), dy, retain_graph=True)):
+        assert torch.equal(a, b)
+    assert torch.autograd.grad(plain, x, dy, retain_graph=True)[0].shape == x.shape
+    assert torch.equal(torch.autograd.grad(plain, s, torch.ones(1, 1, device=DEV, dtype=BF).expand(8, 128), retain_graph=True)[0], torch.autograd.grad(plain, s, dy, retain_graph=True)[0])
+    dx = torch.autograd.grad(plain, x, dy, create_graph=True)[0]
+    assert not dx.requires_grad
+    torch.autograd.grad(plain, x, dy)
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(plain, x, dy)
+    y = tk.rms_norm(x, s)
+    with torch.no_grad():
+        s.add_(1)
+    with pytest.raises(RuntimeError, match="inplace"):
+        torch.autograd.grad(y, x, dy)
+
+
+@gpu
+def test_streams_and_threads():
+    """Every thread trains on a stream of its own: launches, allocations and the backward follow the stream."""
+    g = seeded(6)
+    x0, s0 = randn(g, 4096, 128).to(DEV), randn(g, 128).to(DEV)
+    want_y = norm_mod.rms_norm_forward(x0, s0)[0]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work():
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                x = torch.zeros_like(x0)
+                torch.cuda._sleep(200000)
+                x.add_(x0).requires_grad_(True)            # late on this stream: a launch on another one would read zeros
+                y = tk.rms_norm(x, s0)
+                (dx,) = torch.autograd.grad(y, x, y.detach())
+                ok = torch.equal(y, want_y) & torch.isfinite(dx).all()
+                if not bool(ok):
+                    bad.append(1)
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad

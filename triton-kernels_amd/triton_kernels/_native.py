@@ -158,6 +158,22 @@ def lib():
     return _lib
 
 
+_ops = None
+
+
+def ops():
+    """The operators' common calls in native code (csrc/torch_ops.cpp): each answers None for a call that it leaves to the
+    Python launcher."""
+    global _ops
+    if _ops is None:
+        try:
+            from triton_kernels import _torch_ops
+        except ImportError as e:
+            raise RuntimeError("_torch_ops.so is not built: run `make -C triton-kernels_amd/csrc`") from e
+        _ops = _torch_ops
+    return _ops
+
+
 def last_error() -> str:
     msg = lib().flux_last_error()
     return msg.decode() if msg else ""

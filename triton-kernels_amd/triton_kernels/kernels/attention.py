@@ -6,6 +6,7 @@ import math
 
 import torch
 from torch import Tensor
+from torch.compiler import is_compiling
 
 from triton_kernels import _native as nv
 
@@ -55,5 +56,8 @@ def attention_into(q: Tensor, k: Tensor, v: Tensor, out: Tensor, sm_scale: float
 
 
 def scaled_dot_product_attention(q: Tensor, k: Tensor, v: Tensor, sm_scale: float = None) -> Tensor:
+    o = None if is_compiling() else nv.ops().attention(q, k, v, sm_scale)
+    if o is not None:
+        return o
     o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     return attention_into(q, k, v, o, sm_scale)

@@ -6,6 +6,7 @@ import ctypes
 
 import torch
 from torch import Tensor
+from torch.compiler import is_compiling
 
 from triton_kernels import _native as nv
 
@@ -216,6 +217,11 @@ def qk_fusable(x: Tensor, w: Tensor, seq_len: int, head_dim: int) -> bool:
 
 
 def linear(x: Tensor, w: Tensor, b: Tensor | None, activation: str = "", shared_gpu: bool = False) -> Tensor:
+    act = _ACTIVATIONS.get(activation)
+    if act is not None and launch_hook is None and not shared_gpu and not is_compiling():
+        y = nv.ops().linear(x, w, b, act)
+        if y is not None:
+            return y
     N = w.shape[0]
     y = linear_into(x, w, b, activation=activation, shared_gpu=shared_gpu)
     return y.reshape(*x.shape[:-1], N)

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor
+from torch.compiler import is_compiling
 
 from triton_kernels import _native as nv
 
@@ -104,6 +105,9 @@ def qkv_prep(q_img: Tensor | None, k_img: Tensor | None, v_img: Tensor | None,
 
 
 def apply_rope(xq: Tensor, xk: Tensor, freqs_cis: Tensor) -> tuple[Tensor, Tensor]:
+    both = None if is_compiling() else nv.ops().apply_rope(xq, xk, freqs_cis)
+    if both is not None:
+        return both
     assert xq.dim() == 4 and xq.shape == xk.shape and xq.dtype == xk.dtype
     q, k, _ = qkv_prep(xq, xk, None, pe=freqs_cis)
     return q, k

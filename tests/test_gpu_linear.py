@@ -500,3 +500,33 @@ def test_linear_row_vector_activation_shares(M, K, N):
     sizes = a.abs() @ w.double().abs().T + b.double().abs()
     assert ((got.double() - ref).abs() <= ref.abs() * (2.0 ** -8 * 1.01) + sizes * (K * 2.0 ** -24)).all()
     assert torch.equal(tk.linear_into(x, w, None, in_activation="SiLU"), tk.linear_into(x, w, torch.zeros_like(b), in_activation="SiLU"))
+
+
+@pytest.mark.parametrize("tile_m,tile_n,M,N,K", [(256, 224, 916, 12384, 1024), (256, 224, 1178, 9944, 1032), (224, 256, 880, 12320, 1024), (224, 256, 872, 12376, 1032),
+                                                 (224, 288, 1586, 8200, 1024), (224, 288, 1580, 8312, 1032)])
+def test_linear_wide_rectangles(tile_m, tile_n, M, N, K):
+    """Rectangles of 50000 and more outputs with rows and columns to spare, with and without a K tail, against the fp32
+    product (half a bf16 ulp plus the spread of an fp32 sum in another order): plain, two outputs with GELU in the second
+    from a wave's edge on, a gated residual whose batch elements end inside a tile, and two products in one launch."""
+    assert (lambda p: (p.family, p.tile_m, p.tile_n))(plan_of(linear_args(M, N, K))) == (RECT, tile_m, tile_n)
+    g = seeded(M + N + K)
+    a = randn(g, M, K, dtype=torch.bfloat16).to(DEV)
+    w = randn(g, N, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV)
+    b = randn(g, N, dtype=torch.bfloat16, std=0.5).to(DEV)
+    y = tk.linear(a, w, b)
+    ref32 = oracle.linear_ref_fp32(a, w, b)
+    assert ((y.float() - ref32).abs() <= half_ulp_bound(ref32)).all()
+    cut = tile_n // 2 * 3
+    out = [torch.full((M, n), float("nan"), dtype=torch.bfloat16, device=DEV) for n in (cut, N - cut)]
+    tk.linear_into(a, w, b, activation="GELU", act_begin=cut, out=out[0], out2=out[1], split=cut)
+    assert torch.equal(out[0], y[:, :cut])
+    gelu32 = torch.nn.functional.gelu(ref32[:, cut:], approximate="tanh")
+    assert ((out[1].float() - gelu32).abs() <= half_ulp_bound(gelu32) + 2.0 ** -10).all()   # (tanh by exp2 and rcp: 1e-3 at most)
+    x, gate = randn(g, 2, M // 2, N, dtype=torch.bfloat16).to(DEV), randn(g, 2, 1, N, dtype=torch.bfloat16).to(DEV)
+    both = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    tk.linear_into(a, w, b, out=both, resid=x.view(M, N), gate=gate)
+    assert torch.equal(both.view(2, M // 2, N), oracle.gated_residual_ref(x, gate, y.view(2, M // 2, N)))
+    rows = M // 3
+    pair = linear_pair_into(dict(x=a[:rows], w=w, b=b), dict(x=a[rows:], w=w, b=b))
+    # (its rows of tiles are others, and with them the tile: the same product at half an ulp)
+    assert ((torch.cat(pair).float() - ref32).abs() <= half_ulp_bound(ref32)).all()

@@ -816,6 +816,11 @@ using namespace flux;
 //   512 x 3072 x 12288   98 -> 50 us (69)       2048 x 3072 x 3072   50 -> 40 us (40)
 //   768 x 3072 x 12288   138 -> 62 us (95)      2700 x 3072 x 15360  342 -> 216 us (297)
 // (before: 128-wide tiles, or 64-wide ones up to 128 tiles of 128; tiles with rows to spare excluded).
+// The rectangles of 256 x 224, 224 x 256 and 224 x 288 came later, for rounds that the others leave half empty (us before
+// -> now, weights from HBM; two numbers of rows share a launch):
+//   4096 + 512 x 9216 x 3072   215 -> 202     1305 + 357 x 9216 x 3072   98 -> 77      1500 x 9216 x 3072    80 -> 66
+//   4096 + 512 x 12288 x 3072  294 -> 278     1336 + 207 x 9216 x 3072   83 -> 71      5000 x 3072 x 3072    80 -> 71
+//   4096 + 512 x 3072 x 12288  261 -> 250     876 + 138 x 12288 x 3072   85 -> 74      4702 x 3072 x 15360  317 -> 299
 // A product of at least a few thousand rows fills the CUs with large tiles: one workgroup of four waves per
 // CU, 256 x 256 or whichever rectangle's rounds come out shortest. Below that the eight-wave tiles, down
 // to 64 x 64; what the fit shows to bound those is the load path of a CU (a slab costs in proportion to
@@ -837,7 +842,7 @@ struct TileShape {
     double slab_us;
 };
 static const TileShape kTileShapes[] = {
-    {kSquare, 8, 8, 1.475}, {kRect, 9, 6, 1.200}, {kRect, 8, 6, 1.136}, {kRect, 7, 6, 1.042}, {kRect, 7, 8, 1.300},
+    {kSquare, 8, 8, 1.475}, {kRect, 9, 6, 1.200}, {kRect, 8, 6, 1.136}, {kRect, 7, 6, 1.042}, {kRect, 8, 7, 1.290}, {kRect, 7, 8, 1.300}, {kRect, 7, 9, 1.450},
     {kPair, 6, 6, 0.869}, {kPair, 5, 6, 0.756}, {kPair, 4, 6, 0.647}, {kPair, 8, 4, 0.838}, {kPair, 7, 4, 0.760},
     {kPair, 6, 4, 0.626}, {kPair, 5, 4, 0.568}, {kPair, 5, 3, 0.502}, {kPair, 4, 3, 0.458},
     {kPair, 3, 3, 0.325}, {kPair, 2, 3, 0.287}, {kPair, 2, 2, 0.183}, {kPair, 4, 8, 0.900},
@@ -931,7 +936,10 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     // 256, 224 x 256 and eight-wave 128 x 256 tiles: 320 rows 79 75 58, 640 88 79 108, 1153 159 142 173, 1920 243 215
     // 256, 2049 237 263 290, 3329 409 367 424, 4608 492 517 560. (The eight-wave tile sums K in another order.)
     for (const TileShape& t : kTileShapes) {
-        if (p.qk_cols > 0 ? t.fn != 8 : t.fn == 8 && t.family != kSquare) continue;   // (the others of that width are there for q/k only)
+        if (p.qk_cols > 0 ? t.fn != 8 : t.fn == 8 && t.family == kPair) continue;   // (eight waves of that width are there for q/k only)
+        // Rectangles of 50000 outputs and more: measured from K = 1024 on. Their epilogues, which a slab's price does not
+        // hold, are as long as the square tile's.
+        if (t.family == kRect && t.fn > 6 && p.qk_cols == 0 && p.K < 1024) continue;
         if ((t.family == kRect || (t.family == kPair && t.fn == 8)) && !columns_ok(t.fn)) continue;
         const double us = tile_cost_us(g, t, 1);
         if (us < best.us) best = {t.family, t.fm, t.fn, 1, us, t.family == kPair && !columns_ok(t.fn)};
@@ -1077,7 +1085,9 @@ static int launch_tiles(GemmSet& g, bool shared_gpu, void* workspace, int64_t wo
         case kSquare: launch_square(g, st); break;
         case kRect:
             if (plan.fm == 9) launch_rect<9, 6>(g, st);
+            else if (plan.fm == 8 && plan.fn == 7) launch_rect<8, 7>(g, st);
             else if (plan.fm == 8) launch_rect<8, 6>(g, st);
+            else if (plan.fn == 9) launch_rect<7, 9>(g, st);
             else if (plan.fn == 6) launch_rect<7, 6>(g, st);
             else launch_rect<7, 8>(g, st);
             break;

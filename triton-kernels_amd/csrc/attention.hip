@@ -81,6 +81,10 @@ __device__ __forceinline__ void lds_load16_raw_at(u32x4 rsrc, uint32_t lds_base,
                  : "s"(lds_base), "v"(voff), "s"(rsrc), "n"(OFF)
                  : "memory", "scc", "m0");
 }
+// The same from an address per lane.
+__device__ __forceinline__ void lds_load16_global(const void* src, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_addr), "v"(src) : "memory", "m0");
+}
 // Brings the cache lines that the lanes point at into the L2: one dword each, to 256 bytes of LDS that nothing reads.
 __device__ __forceinline__ void touch_raw(u32x4 rsrc, uint32_t lds_addr, uint32_t voff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
@@ -176,26 +180,6 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
     auto kswz = [](int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); };
     auto vswz = [](int row) { return D == 128 ? ((row & 3) * 4) : (((row >> 1) & 1) * 4); };
 
-    // Q fragments ("B" operand): lane holds row q0 + qb*32 + frow, d = (kk*2 + fhalf)*8 .. +8
-    bf16x8 qf[QB][KSTEPS];
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-        const int row = q0 + qb * 32 + frow;
-        const bool ok = row < p.L;
-        const bf16_t* rp = p.q + b * p.q_sb + h * p.q_sh + static_cast<int64_t>(ok ? row : 0) * p.q_sl;
-#pragma unroll
-        for (int kk = 0; kk < KSTEPS; ++kk) {
-            u32x4 t = *reinterpret_cast<const u32x4*>(rp + (kk * 2 + fhalf) * 8);
-            if (!ok) t = u32x4{0u, 0u, 0u, 0u};
-            // sm_scale*log2(e) goes into Q once (rounded to bf16), so scores leave the MFMA in the
-            // base-2 domain whatever the sign of the scale, and masked keys stay -inf for scale 0
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                t[e] = pack2_bf16(__uint_as_float(t[e] << 16) * p.scale_log2, __uint_as_float(t[e] & 0xffff0000u) * p.scale_log2);
-            qf[qb][kk] = __builtin_bit_cast(bf16x8, t);
-        }
-    }
-
     // loader: thread -> LDS slot (row = pass*4*RPW + wave*RPW + lane/CH, position lane%CH)
     const int l_row = lane / CH, l_pos = lane % CH;
     uint32_t k_voff[PASSES], v_voff[PASSES];
@@ -270,17 +254,46 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
         vf[m % VRN] = __builtin_bit_cast(bf16x8, both);
     };
 
-    // ---- prologue: K(0), V(0), K(1); S^T(0) without overlap; then K(2), V(1) on their way
+    // ---- prologue: Q, K(0), V(0), K(1); S^T(0) without overlap; then K(2), V(1) on their way
+    // Q: a wave fetches its own rows into the V buffers that are empty until then, whole rows per load and swizzled like
+    // K, and reads its fragments from there. (Fragments loaded straight into registers are pieces of 32 bytes of 32 rows,
+    // 64 cycles of the CU's address path each.) Rows past the end repeat the last one; they are not stored. K(0) goes
+    // first, V(0) and K(1) last: the first scores do not wait for those. us, with the output through LDS below, before ->
+    // now: [1, 24, 320, 128] 11.4 -> 10.3, [1, 24, 640, 128] 17.1 -> 15.9, [1, 24, 1280, 128] 30.9 -> 29.8, [1, 2, 1000, 128] 23.0 -> 21.6,
+    // [1, 24, 320, 64] 8.2 -> 7.8, [1, 24, 1280, 64] 19.3 -> 19.1; keys in parts [1, 2, 4096, 128] 33.6 -> 33.9, [1, 2, 2048, 64] 15.5 -> 15.3.
+    static_assert(128 * QB * ROWB <= 2 * T_BYTES, "Q must fit the idle V buffers");
+    bf16x8 qf[QB][KSTEPS];   // "B" operand: lane holds row q0 + qb*32 + frow, d = (kk*2 + fhalf)*8 .. +8
     {
         const u32x4 rk0 = tile_rsrc(kbase, k_row2, 0), rv0 = tile_rsrc(vbase, v_row2, 0);
         const u32x4 rk1 = tile_rsrc(kbase, k_row2, BN);
+        const bf16_t* const qbase = p.q + b * p.q_sb + h * p.q_sh;
+        char* const q_lds = lds + V0 + T_BYTES + wave * (32 * QB * ROWB);
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) lds_load16_raw(rk0, lds_base + i * 4096, k_voff[i]);
+#pragma unroll
+        for (int i = 0; i < 32 * QB / RPW; ++i) {
+            const int r = i * RPW + l_row;
+            lds_load16_global(qbase + static_cast<int64_t>(min(q0 + r, p.L - 1)) * p.q_sl + (l_pos ^ kswz(r)) * 8, lds_addr_of(q_lds) + i * 1024);
+        }
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
-            lds_load16_raw(rk0, lds_base + i * 4096, k_voff[i]);
             lds_load16_raw(rv0, lds_base + V0 + i * 4096, v_voff[i]);
             lds_load16_raw(rk1, lds_base + T_BYTES + i * 4096, k_voff[i]);
         }
-        attn_wait_and_barrier<0>();
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PASSES) : "memory");   // K(0) and Q have landed; V(0) and K(1) fly on
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+            for (int kk = 0; kk < KSTEPS; ++kk) {
+                u32x4 t = *reinterpret_cast<const u32x4*>(q_lds + (qb * 32 + frow) * ROWB + (((kk * 2 + fhalf) ^ kswz(frow)) * 16));
+                // sm_scale*log2(e) goes into Q once (rounded to bf16), so scores leave the MFMA in the
+                // base-2 domain whatever the sign of the scale, and masked keys stay -inf for scale 0
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    t[e] = pack2_bf16(__uint_as_float(t[e] << 16) * p.scale_log2, __uint_as_float(t[e] & 0xffff0000u) * p.scale_log2);
+                qf[qb][kk] = __builtin_bit_cast(bf16x8, t);
+            }
+        attn_wait_and_barrier<2 * PASSES>();
     }
     f32x16 sa[QB][KB], sb[QB][KB];  // S^T of the tile in its softmax / of the tile being multiplied
 #pragma unroll
@@ -442,6 +455,8 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
     wait_all_vmem();  // loads of tiles past the end are empty but still count
 
     // ---- finish: fold the two half-waves' partial sums, normalise, store
+    if constexpr (!SPLIT) asm volatile("s_barrier" ::: "memory");   // the buffers are everyone's until here
+    char* const stage = lds + wave * (32 * QB * ROWB);
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         const float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 32, 64);
@@ -459,8 +474,9 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
                     wblk[(db * 4 + g) * 64] = u32x4{__float_as_uint(acc[qb][db][g * 4 + 0]), __float_as_uint(acc[qb][db][g * 4 + 1]),
                                                     __float_as_uint(acc[qb][db][g * 4 + 2]), __float_as_uint(acc[qb][db][g * 4 + 3])};
             if (fhalf == 0) *reinterpret_cast<f32x2*>(ws + splits * blocks * (32 * D) + (at * 32 + frow) * 2) = f32x2{m_run[qb] * c, l_tot};
-        } else if (row < p.L) {
-            bf16_t* orow = p.o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(row) * p.o_sl;
+        } else {
+            // 8-byte slot s of row r sits at slot s ^ 2(r mod chunks per row), as in the 64-row kernel
+            char* const srow = stage + (qb * 32 + frow) * ROWB;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -468,10 +484,27 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
                     u32x2 w;
                     w.x = pack2_bf16(acc[qb][db][g * 4 + 0] * inv, acc[qb][db][g * 4 + 1] * inv);
                     w.y = pack2_bf16(acc[qb][db][g * 4 + 2] * inv, acc[qb][db][g * 4 + 3] * inv);
-                    *reinterpret_cast<u32x2*>(orow + db * 32 + g * 8 + fhalf * 4) = w;
+                    *reinterpret_cast<u32x2*>(srow + (((db * 8 + g * 2 + fhalf) ^ ((frow % CH) * 2)) * 8)) = w;
                 }
-            if (p.lse != nullptr && fhalf == 0)
+            if (row < p.L && p.lse != nullptr && fhalf == 0)
                 p.lse[static_cast<int64_t>(bh) * p.L + row] = m_run[qb] * c + __builtin_amdgcn_logf(l_tot);
+        }
+    }
+    if constexpr (!SPLIT) {
+        // A lane holds runs of four columns of one row, which would leave as 8-byte pieces of 32 rows; through LDS they leave
+        // as 16-byte pieces of whole rows.
+        __builtin_amdgcn_wave_barrier();   // LDS operations of one wave complete in order
+        int o_row = lane / CH;   // (opaque: row numbers shared with the fetch of Q would live in registers through the loop)
+        asm volatile("" : "+v"(o_row));
+        const int chunk = lane % CH;
+        bf16_t* o_at = p.o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(q0 + o_row) * p.o_sl + chunk * 8;
+        const int64_t o_step = RPW * p.o_sl;
+#pragma unroll
+        for (int it = 0; it < 32 * QB / RPW; ++it) {
+            const int rl = it * RPW + o_row;
+            const u32x4 y = *reinterpret_cast<const u32x4*>(stage + rl * ROWB + ((chunk ^ (rl % CH)) * 16));
+            if (q0 + rl < p.L) *reinterpret_cast<u32x4*>(o_at) = y;
+            o_at += o_step;
         }
     }
 }

@@ -359,3 +359,18 @@ def test_qkv_prep_norm_rope_matches_unfused_sequence():
     torch.testing.assert_close(q, rq, atol=1e-2, rtol=1e-2)
     torch.testing.assert_close(k, rk, atol=1e-2, rtol=1e-2)
     assert torch.equal(v, torch.cat((tv, iv), 2))
+
+
+@pytest.mark.parametrize("rows", [(256 << 20) // (3 * 4 * 3072), (256 << 20) // (3 * 4 * 3072) + 1])
+@pytest.mark.parametrize("width", [3072, 3068])
+def test_layer_norm_modulation_inputs_read_once(rows, width):
+    """fp32 inputs of more than a third of the cache are read past it: the same bits as a part of them that is read
+    through it, at the size where that begins (3072 values a row) and one row below it."""
+    g = torch.Generator(device=DEV).manual_seed(rows + width)
+    x = torch.randn(1, rows, width, generator=g, device=DEV)
+    scale, shift = (torch.randn(1, 1, width, generator=g, device=DEV) for _ in range(2))
+    y = tk.layer_norm_modulation(x, scale, shift)
+    for first, last in ((0, 1000), (rows - 1000, rows)):
+        part = x[:, first:last].contiguous()
+        assert torch.equal(y[:, first:last], tk.layer_norm_modulation(part, scale, shift))
+        torch.testing.assert_close(y[:, first:last], oracle.layer_norm_modulation_ref(part, scale, shift), atol=1e-5, rtol=1e-5)

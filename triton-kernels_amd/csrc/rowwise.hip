@@ -371,6 +371,7 @@ struct LnModSet {
     unsigned blocks0;
     int n;
     float eps;
+    bool once;   // x is read past the caches (see ln_mod_launch)
 };
 
 // Straight-line: rows past the end and columns past n are clamped for the loads (x, scale and shift
@@ -407,12 +408,19 @@ __global__ __launch_bounds__(kBlock) void ln_mod_fwd_regs(LnModSet<T> set) {
 
     Vec16<T> xv[ITER], av[ITER], dv[ITER];
     bool in[ITER];
+    const bool once = sizeof(T) == 4 && set.once;
+#pragma unroll
+    for (int it = 0; it < ITER; ++it) in[it] = FULL || (it * G + lane) * VEC < n;
+    if (once) {
+#pragma unroll
+        for (int it = 0; it < ITER; ++it) xv[it] = ld16_once(xr + (in[it] ? (it * G + lane) * VEC : 0));
+    } else {
+#pragma unroll
+        for (int it = 0; it < ITER; ++it) xv[it] = ld16(xr + (in[it] ? (it * G + lane) * VEC : 0));
+    }
 #pragma unroll
     for (int it = 0; it < ITER; ++it) {
-        const int c = (it * G + lane) * VEC;
-        in[it] = FULL || c < n;
-        const int cl = in[it] ? c : 0;
-        xv[it] = ld16(xr + cl);
+        const int cl = in[it] ? (it * G + lane) * VEC : 0;
         if (!MODLDS) {
             av[it] = ld16(sc + cl);
             dv[it] = ld16(sh + cl);
@@ -660,6 +668,15 @@ static int rms_bwd_launch(const void* dy, const void* x, const void* scale, cons
     return check_launch("flux_rms_norm_bwd");
 }
 
+// fp32 inputs of more than a third of the 256 MB cache in front of HBM are read with the non-temporal hint: what the
+// operation in front read, the input it wrote and this output do not fit there together, so much of the input comes from
+// HBM. us, ordinary -> non-temporal: inputs from HBM [4, 2048, 3072] (101 MB) 40.8 -> 34.1; between two additions, all
+// three: 201 MB 207 -> 193, 147 MB 151 -> 140, but 101 MB, just written, 96 -> 101. Smaller ones mostly come from that cache, where the
+// hint costs more than it gives (50 MB 15.5 -> 17.0), and bf16 gains a third of what fp32 does. (Stores with the hint make the
+// call faster still, 10.3 us for 13.9 at [1, 4608, 3072] bf16, and the reader of the output slower: the single-stream block
+// at 3 x 4336 tokens 2840 -> 2873.)
+constexpr int64_t kCacheBytes = 256 << 20;
+
 template <typename T>
 static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float eps, hipStream_t st) {
     constexpr int VEC = Elem<T>::VEC;
@@ -669,8 +686,10 @@ static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float 
     set.eps = eps;
     int used = 0;
     bool vec_ok = true;
+    int64_t bytes = 0;
     for (int i = 0; i < count; ++i) {
         if (a[i].batch * a[i].seq == 0) continue;
+        bytes += a[i].batch * a[i].seq * n * static_cast<int64_t>(sizeof(T));
         set.t[used++] = {static_cast<const T*>(a[i].x), static_cast<const T*>(a[i].scale), static_cast<const T*>(a[i].shift), static_cast<T*>(a[i].y),
                          a[i].batch * a[i].seq, a[i].seq, a[i].mod_batch_stride};
         vec_ok = vec_ok && aligned16(a[i].x) && aligned16(a[i].y) && aligned16(a[i].scale) && aligned16(a[i].shift) && a[i].mod_batch_stride % VEC == 0;
@@ -683,6 +702,7 @@ static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float 
         return check_launch("flux_layer_norm_modulation");
     }
     if (used == 1) set.t[1] = set.t[0];
+    set.once = 3 * bytes > kCacheBytes;
 #define CALL(G_, I_)                                                                                        \
     do {                                                                                                    \
         constexpr int RPB_ = kBlock / G_;                                                                    \

@@ -59,6 +59,14 @@ bool same_kind(const Tensor& a, const Tensor& b) { return a.scalar_type() == b.s
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
+// Lets other Python threads run while outputs are allocated and kernels launched (a launch waits where the queue is full).
+struct WithoutInterpreter {
+    PyThreadState* const state = PyEval_SaveThread();
+    WithoutInterpreter() = default;
+    WithoutInterpreter(const WithoutInterpreter&) = delete;
+    ~WithoutInterpreter() { PyEval_RestoreThread(state); }
+};
+
 Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const Tensor& beside) {
     return at::empty(sizes, at::TensorOptions().dtype(type).device(beside.device()));
 }
@@ -143,10 +151,19 @@ PyObject* py_rms_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!x || !scale || !quiet() || !norm_args_ok(*x, *scale)) Py_RETURN_NONE;
     const double eps = PyFloat_AsDouble(args[2]);
     if (PyErr_Occurred()) return nullptr;
-    if (at::GradMode::is_enabled() && (x->requires_grad() || scale->requires_grad())) return THPVariable_Wrap(RmsNorm::apply(*x, *scale, eps));
-    if ((x->requires_grad() || scale->requires_grad()) && !vector_rows(*x)) Py_RETURN_NONE;   // (copied first)
-    const Tensor y = empty(x->sizes(), x->scalar_type(), *x);
-    launch_norm(*x, *scale, y, nullptr, eps);
+    const bool differentiable = x->requires_grad() || scale->requires_grad(), recorded = differentiable && at::GradMode::is_enabled();
+    if (differentiable && !recorded && !vector_rows(*x)) Py_RETURN_NONE;   // (copied first)
+    Tensor y;
+    {
+        const Tensor x_kept = *x, scale_kept = *scale;   // (the caller's objects are another thread's to drop from here on)
+        const WithoutInterpreter free;
+        if (recorded) {
+            y = RmsNorm::apply(x_kept, scale_kept, eps);
+        } else {
+            y = empty(x_kept.sizes(), x_kept.scalar_type(), x_kept);
+            launch_norm(x_kept, scale_kept, y, nullptr, eps);
+        }
+    }
     return THPVariable_Wrap(y);
     END_HANDLE_TH_ERRORS
 }
@@ -169,10 +186,16 @@ PyObject* py_rms_norm_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Py_RETURN_NONE;
     const double eps = PyFloat_AsDouble(args[4]);
     if (PyErr_Occurred()) return nullptr;
-    const c10::DeviceGuard guard(x0->device());
-    const Tensor y0 = empty(x0->sizes(), x0->scalar_type(), *x0), y1 = empty(x1->sizes(), x1->scalar_type(), *x1);
-    const flux_rms_norm_args a0 = norm_args(*x0, *s0, y0, nullptr), a1 = norm_args(*x1, *s1, y1, nullptr);
-    check(flux_rms_norm_pair(&a0, &a1, static_cast<int32_t>(x0->size(-1)), type_code(*x0), type_code(*s0), static_cast<float>(eps), stream_of(*x0)), "flux_rms_norm_pair");
+    Tensor y0, y1;
+    {
+        const Tensor xa = *x0, xb = *x1, sa = *s0, sb = *s1;
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(xa.device());
+        y0 = empty(xa.sizes(), xa.scalar_type(), xa);
+        y1 = empty(xb.sizes(), xb.scalar_type(), xb);
+        const flux_rms_norm_args a0 = norm_args(xa, sa, y0, nullptr), a1 = norm_args(xb, sb, y1, nullptr);
+        check(flux_rms_norm_pair(&a0, &a1, static_cast<int32_t>(xa.size(-1)), type_code(xa), type_code(sa), static_cast<float>(eps), stream_of(xa)), "flux_rms_norm_pair");
+    }
     return two(y0, y1);
     END_HANDLE_TH_ERRORS
 }
@@ -192,10 +215,16 @@ PyObject* py_layer_norm_modulation(PyObject*, PyObject* const* args, Py_ssize_t 
     if (n > kMaxRow || !modulates(*scale) || !modulates(*shift)) Py_RETURN_NONE;
     const double eps = PyFloat_AsDouble(args[3]);
     if (PyErr_Occurred()) return nullptr;
-    const c10::DeviceGuard guard(x->device());
-    const Tensor y = empty(x->sizes(), x->scalar_type(), *x);
-    const int rc = flux_layer_norm_modulation(x->data_ptr(), scale->data_ptr(), shift->data_ptr(), y.data_ptr(), batch, rows / batch, static_cast<int32_t>(n),
-                                              batch > 1 ? scale->stride(0) : n, type_code(*x), static_cast<float>(eps), stream_of(*x));
+    Tensor y;
+    int rc;
+    {
+        const Tensor xa = *x, sc = *scale, sh = *shift;
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(xa.device());
+        y = empty(xa.sizes(), xa.scalar_type(), xa);
+        rc = flux_layer_norm_modulation(xa.data_ptr(), sc.data_ptr(), sh.data_ptr(), y.data_ptr(), batch, rows / batch, static_cast<int32_t>(n),
+                                        batch > 1 ? sc.stride(0) : n, type_code(xa), static_cast<float>(eps), stream_of(xa));
+    }
     if (rc < 0) Py_RETURN_NONE;   // (a refusal: its kind of error is the launcher's)
     check(rc, "flux_layer_norm_modulation");
     return THPVariable_Wrap(y);
@@ -220,19 +249,26 @@ PyObject* py_apply_rope(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Py_RETURN_NONE;
     const int64_t tables = pe->numel() / (L * D * 2);
     if (tables != 1 && !(lead == 2 && pe->size(0) == B && pe->size(1) == 1)) Py_RETURN_NONE;
-    const c10::DeviceGuard guard(q->device());
-    const Tensor yq = empty(q->sizes(), q->scalar_type(), *q), yk = empty(q->sizes(), q->scalar_type(), *q);
-    flux_qkv_prep_args a = {};
-    a.q_img = source(*q);
-    a.k_img = source(*k);
-    a.q_out = yq.data_ptr();
-    a.k_out = yk.data_ptr();
-    a.pe = static_cast<const float*>(pe->data_ptr());
-    a.pe_batch_stride = tables == 1 ? 0 : L * D * 2;
-    a.B = B; a.H = H; a.Li = L; a.D = static_cast<int32_t>(D);
-    a.dtype = a.scale_dtype = type_code(*q);
-    a.eps = 1e-6f;
-    const int rc = flux_qkv_prep(&a, stream_of(*q));
+    Tensor yq, yk;
+    int rc;
+    {
+        const Tensor qa = *q, ka = *k, table = *pe;
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(qa.device());
+        yq = empty(qa.sizes(), qa.scalar_type(), qa);
+        yk = empty(qa.sizes(), qa.scalar_type(), qa);
+        flux_qkv_prep_args a = {};
+        a.q_img = source(qa);
+        a.k_img = source(ka);
+        a.q_out = yq.data_ptr();
+        a.k_out = yk.data_ptr();
+        a.pe = static_cast<const float*>(table.data_ptr());
+        a.pe_batch_stride = tables == 1 ? 0 : L * D * 2;
+        a.B = B; a.H = H; a.Li = L; a.D = static_cast<int32_t>(D);
+        a.dtype = a.scale_dtype = type_code(qa);
+        a.eps = 1e-6f;
+        rc = flux_qkv_prep(&a, stream_of(qa));
+    }
     if (rc < 0) Py_RETURN_NONE;
     check(rc, "flux_qkv_prep");
     return two(yq, yk);
@@ -253,21 +289,27 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (b && (!same_kind(*x, *b) || b->dim() != 1 || b->numel() != N || b->stride(0) != 1)) Py_RETURN_NONE;
     const long act = PyLong_AsLong(args[3]);
     if (PyErr_Occurred()) return nullptr;
-    const c10::DeviceGuard guard(x->device());
-    at::DimVector sizes(x->sizes().begin(), x->sizes().end());
-    sizes.back() = N;
-    const Tensor y = empty(sizes, at::kBFloat16, *x);
-    flux_linear_args a = {};
-    a.A = x->data_ptr(); a.W = w->data_ptr(); a.bias = b ? b->data_ptr() : nullptr;
-    a.Y = y.data_ptr();
-    a.M = M; a.N = N; a.K = K;
-    a.lda = a.ldw = K;
-    a.ldy = a.split_n = N;
-    a.act = static_cast<int32_t>(act);
-    // (K is cut over workgroups beyond 3072 of it only, and up to 256 tiles of 192 x 192)
-    const int64_t need = K > 3072 && M > 8 && M * N <= (int64_t{1} << 24) ? flux_linear_workspace_bytes(&a) : 0;
-    const Tensor ws = need ? empty({need}, at::kByte, *x) : Tensor();
-    const int rc = flux_linear_bf16_ws(&a, need ? ws.data_ptr() : nullptr, need, stream_of(*x));
+    Tensor y;
+    int rc;
+    {
+        const Tensor xa = *x, wa = *w, ba = b ? *b : Tensor();
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(xa.device());
+        at::DimVector sizes(xa.sizes().begin(), xa.sizes().end());
+        sizes.back() = N;
+        y = empty(sizes, at::kBFloat16, xa);
+        flux_linear_args a = {};
+        a.A = xa.data_ptr(); a.W = wa.data_ptr(); a.bias = ba.defined() ? ba.data_ptr() : nullptr;
+        a.Y = y.data_ptr();
+        a.M = M; a.N = N; a.K = K;
+        a.lda = a.ldw = K;
+        a.ldy = a.split_n = N;
+        a.act = static_cast<int32_t>(act);
+        // (K is cut over workgroups beyond 3072 of it only, and up to 256 tiles of 192 x 192)
+        const int64_t need = K > 3072 && M > 8 && M * N <= (int64_t{1} << 24) ? flux_linear_workspace_bytes(&a) : 0;
+        const Tensor ws = need ? empty({need}, at::kByte, xa) : Tensor();
+        rc = flux_linear_bf16_ws(&a, need ? ws.data_ptr() : nullptr, need, stream_of(xa));
+    }
     if (rc < 0) Py_RETURN_NONE;
     check(rc, "flux_linear_bf16");
     return THPVariable_Wrap(y);
@@ -288,17 +330,23 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (t->stride(3) != 1 || !vector_rows(*t)) Py_RETURN_NONE;
     const double scale = args[3] == Py_None ? 1.0 / std::sqrt(static_cast<double>(q->size(3))) : PyFloat_AsDouble(args[3]);
     if (PyErr_Occurred()) return nullptr;
-    const c10::DeviceGuard guard(q->device());
-    const Tensor o = empty(q->sizes(), at::kBFloat16, *q);
-    flux_attn_args a = {};
-    a.q = source(*q); a.k = source(*k); a.v = source(*v);
-    a.o = o.data_ptr();
-    a.o_sb = o.stride(0); a.o_sh = o.stride(1); a.o_sl = o.stride(2);
-    a.B = q->size(0); a.H = q->size(1); a.L = q->size(2); a.D = static_cast<int32_t>(q->size(3));
-    a.sm_scale = static_cast<float>(scale);
-    const int64_t need = flux_attention_workspace_bytes(a.B, a.H, a.L, a.D);   // keys cut over several workgroups
-    const Tensor ws = need ? empty({need}, at::kByte, *q) : Tensor();
-    const int rc = flux_attention_fwd_bf16_ws(&a, need ? ws.data_ptr() : nullptr, need, stream_of(*q));
+    Tensor o;
+    int rc;
+    {
+        const Tensor qa = *q, ka = *k, va = *v;
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(qa.device());
+        o = empty(qa.sizes(), at::kBFloat16, qa);
+        flux_attn_args a = {};
+        a.q = source(qa); a.k = source(ka); a.v = source(va);
+        a.o = o.data_ptr();
+        a.o_sb = o.stride(0); a.o_sh = o.stride(1); a.o_sl = o.stride(2);
+        a.B = qa.size(0); a.H = qa.size(1); a.L = qa.size(2); a.D = static_cast<int32_t>(qa.size(3));
+        a.sm_scale = static_cast<float>(scale);
+        const int64_t need = flux_attention_workspace_bytes(a.B, a.H, a.L, a.D);   // keys cut over several workgroups
+        const Tensor ws = need ? empty({need}, at::kByte, qa) : Tensor();
+        rc = flux_attention_fwd_bf16_ws(&a, need ? ws.data_ptr() : nullptr, need, stream_of(qa));
+    }
     if (rc < 0) Py_RETURN_NONE;
     check(rc, "flux_attention_fwd_bf16");
     return THPVariable_Wrap(o);

@@ -152,3 +152,17 @@ def test_k_is_cut_only_for_a_gain_above_what_it_costs_the_host():
     assert plan_of(linear_args(64, 3072, 3072)).splits == 1      # 2 us of the GPU for 6 us of the host
     assert plan_of(linear_args(320, 3072, 15360)).splits > 1     # 30 us
     assert plan_of(linear_args(320, 3072, 15360), workspace=0).splits == 1
+
+
+@pytest.mark.parametrize("ldw", [3_728_264, 3_728_272, 4_000_000, 4_194_296])
+def test_weight_rows_of_a_tile_stay_within_31_bit_offsets(ldw):
+    """A tile reaches its weight rows with byte offsets below 2^31, where the offset that stands for "out of range" begins:
+    288 rows of them up to 3728269 values apart, 256 up to 4194303."""
+    rng, widest = random.Random(ldw), 0
+    shapes = [(57344, 288, 1032), (1580, 8312, 1032)]
+    shapes += [(round(2 ** rng.uniform(8, 14)), 8 * round(2 ** rng.uniform(4, 11)), 8 * rng.randint(128, 600)) for _ in range(3000)]
+    for M, N, K in shapes:
+        p = plan_of(linear_args(M, N, K, ldw=ldw))
+        assert p.tile_n * ldw * 2 < 2 ** 31, (M, N, K, p.tile_m, p.tile_n)
+        widest = max(widest, p.tile_n)
+    assert widest == (288 if ldw == 3_728_264 else 256)

@@ -918,16 +918,19 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     // anything else as well. (Without it on the eight-wave tiles, calls outside the form ran on square ones: 64 x 3072
     // x 3072 with 1000 columns in the first output 13 -> 63 us, 300 x 1001 x 3072 14 -> 30 us.)
     const GemmParams& p = g.p[0];
-    bool form = true;
+    // near288: also 288 rows of W lie within 32-bit byte offsets, as 256 of them do on every call that gets here. Past
+    // that, offsets reach kOutOfRange and the K tail of those rows is no longer read as zeros.
+    bool form = true, near288 = true;
     for (int i = 0; i < g.n; ++i) {
         const GemmParams& q = g.p[i];
+        near288 = near288 && q.ldw * 2 * 288 < 0x7fffffffLL;
         form = form && q.vec_io && q.N % 8 == 0 && (q.bias == nullptr || q.bias_vec) && !(q.gate != nullptr && q.act != FLUX_ACT_NONE) &&
                q.lda * 2 * 288 < 0x7fffffffLL && q.ldw * 2 * 256 < 0x7fffffffLL && q.ldy * 2 * 288 < 0x7fffffffLL &&
                q.ldy2 * 2 * 288 < 0x7fffffffLL && q.ldresid * 2 * 288 < 0x7fffffffLL;   // 32-bit byte offsets inside a tile's rows
     }
     auto columns_ok = [&](int fn) {
         const int w = 16 * fn;
-        return form && (p.split_n >= p.N || p.split_n % w == 0) && (p.act == FLUX_ACT_NONE || p.act_begin >= p.N || p.act_begin % w == 0);
+        return form && (fn <= 8 || near288) && (p.split_n >= p.N || p.split_n % w == 0) && (p.act == FLUX_ACT_NONE || p.act_begin >= p.N || p.act_begin % w == 0);
     };
     if (!form && p.qk_cols > 0) return {kSquare, 8, 8, 1, 0.0};   // (whole heads per wave: 256-wide tiles only)
     TilePlan best = {kSquare, 8, 8, 1, 1e30};

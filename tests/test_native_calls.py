@@ -241,3 +241,23 @@ def test_streams_and_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+@gpu
+@pytest.mark.parametrize("grad", [False, True])
+def test_refusals_of_the_library_keep_their_kind(monkeypatch, grad):
+    """Tensors whose memory has been given back are refused by the library (null pointers): the norm's native calls raise
+    what the launchers raise."""
+    x, s = torch.ones(4, 64, device=DEV), torch.ones(64, device=DEV)
+    gone, s_gone = torch.ones(4, 64, device=DEV), torch.ones(64, device=DEV)
+    for t in (gone, s_gone):
+        t.untyped_storage().resize_(0)
+        t.requires_grad_(grad)
+    for fn, *args in ((tk.rms_norm, gone, s), (tk.rms_norm, x, s_gone), (norm_mod.rms_norm_pair, gone, s, x, s), (norm_mod.rms_norm_pair, x, s, x, s_gone)):
+        with torch.set_grad_enabled(grad):
+            errors = []
+            for call in (lambda: fn(*args), lambda: launcher(monkeypatch, fn, *args)):
+                with pytest.raises(Exception) as e:
+                    call()
+                errors.append(e)
+        assert errors[0].type is errors[1].type is ValueError and str(errors[0].value) == str(errors[1].value)

@@ -22,6 +22,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <cmath>
+#include <string>
 
 #include "../../include/flux_hip.h"
 
@@ -71,10 +72,16 @@ Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const Tensor& beside) {
     return at::empty(sizes, at::TensorOptions().dtype(type).device(beside.device()));
 }
 
+// Raises what the library answered, as the kind of error that the Python launchers make of it (_native.check).
 void check(int rc, const char* what) {
     if (rc == FLUX_OK) return;
-    const char* msg = flux_last_error();
-    TORCH_CHECK(false, msg && *msg ? msg : what, " (hipError ", rc, ")");
+    const char* const last = flux_last_error();
+    const std::string msg = last && *last ? last : what;
+    TORCH_CHECK_TYPE(rc != FLUX_E_DTYPE, msg);
+    TORCH_CHECK_VALUE(rc != FLUX_E_SHAPE && rc != FLUX_E_NULL && rc != FLUX_E_ALIGN, msg);
+    TORCH_CHECK_NOT_IMPLEMENTED(rc != FLUX_E_UNSUPPORTED, msg);
+    TORCH_CHECK(rc != FLUX_E_TOO_WIDE, msg);
+    TORCH_CHECK(false, msg, " (hipError ", rc, ")");
 }
 
 // Rows of 16-byte vectors from the first one on.

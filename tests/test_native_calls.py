@@ -261,3 +261,24 @@ def test_refusals_of_the_library_keep_their_kind(monkeypatch, grad):
                     call()
                 errors.append(e)
         assert errors[0].type is errors[1].type is ValueError and str(errors[0].value) == str(errors[1].value)
+
+
+@gpu
+def test_numbers_that_float_takes(monkeypatch):
+    """eps and the attention's scale may be anything that float() makes a number of, texts among them."""
+    g = seeded(7)
+    x, s = randn(g, 2, 4, 6, 64, dtype=BF).to(DEV), randn(g, 64, dtype=BF).to(DEV)
+    mod = randn(g, 2, 1, 64, dtype=BF).to(DEV)
+    with torch.no_grad():
+        for fn, args in ((tk.rms_norm, (x, s)), (norm_mod.rms_norm_pair, (x, s, x, s)), (tk.layer_norm_modulation, (x, mod, mod)), (tk.scaled_dot_product_attention, (x, x, x))):
+            for number in ("1e-3", b"0.25", torch.tensor(0.5), 1, True):
+                got, want = fn(*args, number), launcher(monkeypatch, fn, *args, number)
+                pairs = zip(got, want) if isinstance(got, tuple) else [(got, want)]
+                assert all(torch.equal(a, b) for a, b in pairs)
+            for bad in ("x", [], object()):
+                errors = []
+                for call in (lambda: fn(*args, bad), lambda: launcher(monkeypatch, fn, *args, bad)):
+                    with pytest.raises((TypeError, ValueError)) as e:
+                        call()
+                    errors.append(e)
+                assert errors[0].type is errors[1].type and str(errors[0].value) == str(errors[1].value)

@@ -58,6 +58,15 @@ int type_code(const Tensor& t) {
 }
 bool same_kind(const Tensor& a, const Tensor& b) { return a.scalar_type() == b.scalar_type() && a.device() == b.device(); }
 
+// The number that float() makes of a Python object; false where that is more than a number's own conversion (a text, or
+// nothing that float() takes), which is left to the launchers.
+bool number(PyObject* o, double& value) {
+    value = PyFloat_AsDouble(o);
+    if (value != -1.0 || !PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
+}
+
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 // Lets other Python threads run while outputs are allocated and kernels launched (a launch waits where the queue is full).
@@ -156,8 +165,8 @@ PyObject* py_rms_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     TORCH_CHECK(nargs == 3, "rms_norm takes 3 arguments");
     const Tensor *x = tensor_of(args[0]), *scale = tensor_of(args[1]);
     if (!x || !scale || !quiet() || !norm_args_ok(*x, *scale)) Py_RETURN_NONE;
-    const double eps = PyFloat_AsDouble(args[2]);
-    if (PyErr_Occurred()) return nullptr;
+    double eps;
+    if (!number(args[2], eps)) Py_RETURN_NONE;
     const bool differentiable = x->requires_grad() || scale->requires_grad(), recorded = differentiable && at::GradMode::is_enabled();
     if (differentiable && !recorded && !vector_rows(*x)) Py_RETURN_NONE;   // (copied first)
     Tensor y;
@@ -191,8 +200,8 @@ PyObject* py_rms_norm_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!x0 || !s0 || !x1 || !s1 || at::GradMode::is_enabled() || !quiet() || !norm_args_ok(*x0, *s0) || !norm_args_ok(*x1, *s1) ||
         !same_kind(*x0, *x1) || !same_kind(*s0, *s1) || x0->size(-1) != x1->size(-1) || !vector_rows(*x0) || !vector_rows(*x1))
         Py_RETURN_NONE;
-    const double eps = PyFloat_AsDouble(args[4]);
-    if (PyErr_Occurred()) return nullptr;
+    double eps;
+    if (!number(args[4], eps)) Py_RETURN_NONE;
     Tensor y0, y1;
     {
         const Tensor xa = *x0, xb = *x1, sa = *s0, sb = *s1;
@@ -220,8 +229,8 @@ PyObject* py_layer_norm_modulation(PyObject*, PyObject* const* args, Py_ssize_t 
         return m.dim() >= 2 && m.size(0) == batch && m.size(-1) == n && m.numel() == batch * n && m.stride(-1) == 1 && (batch == 1 || (m.stride(0) == scale->stride(0) && m.stride(0) >= n));
     };
     if (n > kMaxRow || !modulates(*scale) || !modulates(*shift)) Py_RETURN_NONE;
-    const double eps = PyFloat_AsDouble(args[3]);
-    if (PyErr_Occurred()) return nullptr;
+    double eps;
+    if (!number(args[3], eps)) Py_RETURN_NONE;
     Tensor y;
     int rc;
     {
@@ -335,8 +344,8 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Py_RETURN_NONE;
     for (const Tensor* t : {q, k, v})
         if (t->stride(3) != 1 || !vector_rows(*t)) Py_RETURN_NONE;
-    const double scale = args[3] == Py_None ? 1.0 / std::sqrt(static_cast<double>(q->size(3))) : PyFloat_AsDouble(args[3]);
-    if (PyErr_Occurred()) return nullptr;
+    double scale = 1.0 / std::sqrt(static_cast<double>(q->size(3)));
+    if (args[3] != Py_None && !number(args[3], scale)) Py_RETURN_NONE;
     Tensor o;
     int rc;
     {

@@ -282,3 +282,52 @@ def test_numbers_that_float_takes(monkeypatch):
                         call()
                     errors.append(e)
                 assert errors[0].type is errors[1].type and str(errors[0].value) == str(errors[1].value)
+
+
+@gpu
+@pytest.mark.parametrize("dtype,scale_dtype", [(BF, BF), (BF, F32), (F32, F32)])
+@pytest.mark.parametrize("kept", [torch.float32, torch.float64])
+@pytest.mark.parametrize("scale_too", [False, True])
+def test_saved_tensors_of_another_type(monkeypatch, dtype, scale_dtype, kept, scale_too):
+    """What a saved-tensor hook hands back may have another type than what was saved: the launcher's backward converts the
+    scale to what the kernels take beside x, and refuses an x they do not take; so does the native one."""
+    g = seeded(8)
+    x0, s0, dy = randn(g, 40, 96, dtype=dtype).to(DEV), randn(g, 96, dtype=scale_dtype).to(DEV), randn(g, 40, 96, dtype=dtype).to(DEV)
+    got = []
+    for call in (tk.rms_norm, lambda *a: launcher(monkeypatch, tk.rms_norm, *a)):
+        x, s = x0.clone().requires_grad_(True), s0.clone().requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.to(kept) if t.dim() == 2 or scale_too and t.numel() == 96 else t):
+            y = call(x, s)
+        if kept == torch.float64:
+            with pytest.raises(TypeError):
+                y.backward(dy)
+            continue
+        y.backward(dy)
+        got.append((x.grad, s.grad))
+    if got:
+        assert torch.equal(got[0][0], got[1][0]) and got[0][0].dtype == dtype and got[0][1].dtype == scale_dtype
+        torch.testing.assert_close(got[0][1], got[1][1], atol=2e-2, rtol=2.0 ** -7)
+
+
+@gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_saved_row_norms_of_another_type(monkeypatch, native):
+    """The kernel reads one fp32 value a row of what the forward kept; a hook that halves everything it keeps gets the
+    gradients of the halved input, and values that came back too few or on the CPU are refused."""
+    g = seeded(10)
+    x0, s0, dy = randn(g, 40, 96).to(DEV), randn(g, 96).to(DEV), randn(g, 40, 96).to(DEV)
+
+    def step(unpack):
+        x, s = x0.clone().requires_grad_(True), s0.clone().requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = tk.rms_norm(x, s) if native else launcher(monkeypatch, tk.rms_norm, x, s)
+        y.backward(dy)
+        return x.grad, s.grad
+
+    dx, ds = step(lambda t: t.bfloat16())
+    rx, rs = step(lambda t: t)
+    # (three roundings to bf16 of half an ulp, 2^-9 of the value, and the gradient's own)
+    assert (dx - rx).norm() <= 2.0 ** -6 * rx.norm() and (ds - rs).norm() <= 2.0 ** -6 * rs.norm() and dx.dtype == ds.dtype == F32
+    for bad in (lambda t: t[:20] if t.numel() == 40 else t, lambda t: t[:50] if t.numel() == 96 else t, lambda t: t.cpu() if t.dim() == 1 else t):
+        with pytest.raises(RuntimeError):
+            step(bad)

@@ -140,22 +140,29 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
     }
 
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
-        const auto saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &scale = saved[1], &rstd = saved[2];
+        const auto saved = ctx->get_saved_variables();   // (what saved-tensor hooks gave back, of any type)
+        const Tensor x = saved[0].contiguous(), r = saved[2].to(at::kFloat).contiguous();
+        Tensor s = saved[1].contiguous();
         const Tensor& dy = grads[0];
-        TORCH_CHECK(dy.is_cuda() && dy.device() == x.device(), "tensors on different devices: ", dy.device(), " and ", x.device());
+        for (const Tensor* t : std::initializer_list<const Tensor*>{&dy, &s, &r})
+            TORCH_CHECK(t->is_cuda() && t->device() == x.device(), "tensors on different devices: ", t->device(), " and ", x.device());
+        TORCH_CHECK(x.dim() == 2 && s.numel() == x.size(1) && r.numel() == x.size(0), "rms_norm: saved tensors came back with other sizes");
+        const int xc = type_code(x);
+        TORCH_CHECK_TYPE(xc >= 0, "unsupported dtype ", x.scalar_type(), ": the HIP kernels take bfloat16 or float32");
+        const at::ScalarType scale_type = s.scalar_type();
+        if (scale_type != x.scalar_type() && !(xc == FLUX_BF16 && scale_type == at::kFloat)) s = s.to(x.scalar_type());
         const int64_t rows = x.size(0), n = x.size(1);
         Tensor dy2 = dy.contiguous().reshape({rows, n});
         if (dy2.scalar_type() != x.scalar_type()) dy2 = dy2.to(x.scalar_type());
         const void* const dy_at = dy2.data_ptr();   // (a wrapper without memory ends here)
-        const Tensor x2 = x.contiguous(), s = scale.contiguous(), r = rstd.contiguous();   // (what a saved-tensor hook gave back)
         const c10::DeviceGuard guard(x.device());
-        const Tensor dx = empty(x2.sizes(), x2.scalar_type(), x2), dscale = empty(s.sizes(), s.scalar_type(), x2);
-        const int64_t ws_bytes = flux_rms_norm_bwd_workspace_bytes(rows, static_cast<int32_t>(n), type_code(x2));
-        const Tensor ws = empty({ws_bytes}, at::kByte, x2);
-        check(flux_rms_norm_bwd_ws(dy_at, x2.data_ptr(), s.data_ptr(), static_cast<const float*>(r.data_ptr()), dx.data_ptr(), dscale.data_ptr(), type_code(dscale),
-                                   ws.data_ptr(), ws_bytes, rows, static_cast<int32_t>(n), type_code(x2), type_code(s), stream_of(x2)), "flux_rms_norm_bwd");
-        return {dx.reshape(dy.sizes()), dscale, Tensor()};
+        // the kernel's types; the gradient of a scale of another type is converted from fp32
+        const Tensor dx = empty(x.sizes(), x.scalar_type(), x), dscale = empty(s.sizes(), scale_type == at::kBFloat16 ? at::kBFloat16 : at::kFloat, x);
+        const int64_t ws_bytes = flux_rms_norm_bwd_workspace_bytes(rows, static_cast<int32_t>(n), xc);
+        const Tensor ws = empty({ws_bytes}, at::kByte, x);
+        check(flux_rms_norm_bwd_ws(dy_at, x.data_ptr(), s.data_ptr(), static_cast<const float*>(r.data_ptr()), dx.data_ptr(), dscale.data_ptr(), type_code(dscale),
+                                   ws.data_ptr(), ws_bytes, rows, static_cast<int32_t>(n), xc, type_code(s), stream_of(x)), "flux_rms_norm_bwd");
+        return {dx.reshape(dy.sizes()), dscale.scalar_type() == scale_type ? dscale : dscale.to(scale_type), Tensor()};
     }
 };
 

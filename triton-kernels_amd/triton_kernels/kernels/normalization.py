@@ -83,13 +83,16 @@ class _rms_norm(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy: torch.Tensor):
-        x2, scale, rstd = ctx.saved_tensors
-        dev = nv.require_gpu(dy, x2)
+        x2, scale, rstd = ctx.saved_tensors   # (what saved-tensor hooks gave back, of any type)
+        dev = nv.require_gpu(dy, x2, scale, rstd)
         rows, n = x2.shape
+        if scale.numel() != n or rstd.numel() != rows:
+            raise RuntimeError("rms_norm: saved tensors came back with other sizes")
+        x2, rstd = x2.contiguous(), rstd.float().contiguous()
         dy2 = dy.contiguous().reshape(rows, n)
         if dy2.dtype != x2.dtype:
             dy2 = dy2.to(x2.dtype)
-        sc = scale
+        sc = scale.contiguous()
         if sc.dtype != x2.dtype and not (x2.dtype == torch.bfloat16 and sc.dtype == torch.float32):
             sc = sc.to(x2.dtype)
         dx = torch.empty_like(x2)

@@ -331,3 +331,13 @@ def test_saved_row_norms_of_another_type(monkeypatch, native):
     for bad in (lambda t: t[:20] if t.numel() == 40 else t, lambda t: t[:50] if t.numel() == 96 else t, lambda t: t.cpu() if t.dim() == 1 else t):
         with pytest.raises(RuntimeError):
             step(bad)
+
+
+@gpu
+def test_layer_norm_output_is_laid_out_like_its_input(monkeypatch):
+    """A dimension of one element may have any stride in a contiguous input; the output has the same."""
+    g = seeded(9)
+    x, mod = randn(g, 1, 5, 64).to(DEV)[:, :1], randn(g, 1, 1, 64).to(DEV)
+    assert x.is_contiguous() and x.stride(0) == 320
+    got, want = tk.layer_norm_modulation(x, mod, mod), launcher(monkeypatch, tk.layer_norm_modulation, x, mod, mod)
+    assert torch.equal(got, want) and got.stride() == want.stride()

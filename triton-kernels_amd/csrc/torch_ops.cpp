@@ -244,7 +244,7 @@ PyObject* py_layer_norm_modulation(PyObject*, PyObject* const* args, Py_ssize_t 
         const Tensor xa = *x, sc = *scale, sh = *shift;
         const WithoutInterpreter free;
         const c10::DeviceGuard guard(xa.device());
-        y = empty(xa.sizes(), xa.scalar_type(), xa);
+        y = at::empty_like(xa);
         rc = flux_layer_norm_modulation(xa.data_ptr(), sc.data_ptr(), sh.data_ptr(), y.data_ptr(), batch, rows / batch, static_cast<int32_t>(n),
                                         batch > 1 ? sc.stride(0) : n, type_code(xa), static_cast<float>(eps), stream_of(xa));
     }

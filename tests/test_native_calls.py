@@ -1,5 +1,6 @@
 """The operators' calls in native code (csrc/torch_ops.cpp) against the Python launchers of the same operators, over the forms
 they accept, and the calls that they leave to the launchers."""
+import sys
 import threading
 
 import pytest
@@ -52,6 +53,38 @@ def _views(g, dtype):
     return [base, base[0, 0, 0], base[1], base.permute(2, 0, 1, 3), base.transpose(1, 2)[::2], wide[..., 256:512], wide.view(2, 6, 3, 2, 128).permute(2, 0, 3, 1, 4)[1],
             base[..., :100], base[..., 1:129:1][..., :50], base[:, :, :1].expand(3, 4, 7, 128), base.flatten()[:7 * 300].view(7, 300), base.flatten()[3:3 + 5 * 33].view(5, 33),
             base[..., ::2], base.view(3, 2, 2, 5, 128), base[:0], base.flatten()[:9].view(9, 1)]
+
+
+def test_the_extension_says_why_it_does_not_load(monkeypatch, tmp_path):
+    """Not there, not loadable, built for another torch: three messages, and the library's own comes before them."""
+    import triton_kernels
+    monkeypatch.setattr(nv, "_ops", None)
+
+    class _Broken:
+        def find_spec(self, name, *args):
+            if name == "triton_kernels._torch_ops":
+                raise ImportError("undefined symbol: _ZN2at5emptyE")
+
+    with monkeypatch.context() as m:
+        m.setattr(nv, "_OPS_PATH", str(tmp_path / "_torch_ops.so"))
+        with pytest.raises(RuntimeError, match="_torch_ops.so is not built"):
+            nv.ops()
+    with monkeypatch.context() as m:
+        m.delitem(sys.modules, "triton_kernels._torch_ops", raising=False)
+        m.delattr(triton_kernels, "_torch_ops", raising=False)
+        m.setattr(sys, "meta_path", [_Broken(), *sys.meta_path])
+        with pytest.raises(RuntimeError, match="undefined symbol.*make -B"):
+            nv.ops()
+    with monkeypatch.context() as m:
+        m.setattr(nv, "_lib", None)
+        m.setattr(nv, "ABI_VERSION", nv.ABI_VERSION + 1)
+        with pytest.raises(RuntimeError, match="ABI version"):
+            nv.ops()
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "1.0.0+other")
+        with pytest.raises(RuntimeError, match=r"built for torch 2.*this is torch 1\.0\.0"):
+            nv.ops()
+    assert nv.ops().rms_norm(3, 3, 3) is None
 
 
 @gpu

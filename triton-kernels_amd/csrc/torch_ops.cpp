@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
@@ -385,6 +386,18 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_ops", nullptr, -1, methods,
 
 }  // namespace
 
+#define FLUX_TEXT_(x) #x
+#define FLUX_TEXT(x) FLUX_TEXT_(x)
+
 PyMODINIT_FUNC PyInit__torch_ops() {
-    return PyModule_Create(&module);
+    if (flux_abi_version() != FLUX_ABI_VERSION) {
+        PyErr_Format(PyExc_ImportError, "libfluxhip.so has ABI version %d, the extension was built for %d", flux_abi_version(), FLUX_ABI_VERSION);
+        return nullptr;
+    }
+    PyObject* const m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "built_for", "torch " TORCH_VERSION ", Python " FLUX_TEXT(PY_MAJOR_VERSION) "." FLUX_TEXT(PY_MINOR_VERSION)) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
 from ctypes import POINTER, Structure, byref, c_char_p, c_float, c_int32, c_int64, c_void_p
 
 import torch
@@ -20,6 +21,7 @@ ACT_NONE, ACT_GELU_TANH, ACT_SILU = 0, 1, 2
 LINEAR_SHARED_GPU = 1
 E_NULL, E_SHAPE, E_DTYPE, E_ALIGN, E_TOO_WIDE, E_UNSUPPORTED = -1, -2, -3, -4, -5, -6
 MAX_ROW = 65536
+ABI_VERSION = 4
 
 _DTYPE_CODE = {torch.bfloat16: FLUX_BF16, torch.float32: FLUX_F32}
 
@@ -152,24 +154,33 @@ def lib():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-        if handle.flux_abi_version() != 4:
+        if handle.flux_abi_version() != ABI_VERSION:
             raise RuntimeError("libfluxhip.so: ABI version mismatch")
         _lib = handle
     return _lib
 
 
+_OPS_PATH = os.path.join(os.path.dirname(_LIB_PATH), "_torch_ops.so")
 _ops = None
 
 
 def ops():
     """The operators' common calls in native code (csrc/torch_ops.cpp): each answers None for a call that it leaves to the
-    Python launcher."""
+    Python launcher. The library under it is loaded and checked first; the extension links torch's C++ interface, so it
+    serves the torch and the Python that it was built for."""
     global _ops
     if _ops is None:
+        lib()
+        if not os.path.exists(_OPS_PATH):
+            raise RuntimeError(f"{_OPS_PATH} is not built: run `make -C triton-kernels_amd/csrc`")
+        again = "build it again with `make -B -C triton-kernels_amd/csrc`"
         try:
             from triton_kernels import _torch_ops
         except ImportError as e:
-            raise RuntimeError("_torch_ops.so is not built: run `make -C triton-kernels_amd/csrc`") from e
+            raise RuntimeError(f"{_OPS_PATH} does not load ({e}): {again}") from e
+        here = "torch {}, Python {}.{}".format(torch.__version__.split("+")[0], *sys.version_info[:2])
+        if _torch_ops.built_for != here:
+            raise RuntimeError(f"{_OPS_PATH} is built for {_torch_ops.built_for}, this is {here}: {again}")
         _ops = _torch_ops
     return _ops
 

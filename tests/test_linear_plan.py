@@ -166,3 +166,18 @@ def test_weight_rows_of_a_tile_stay_within_31_bit_offsets(ldw):
         assert p.tile_n * ldw * 2 < 2 ** 31, (M, N, K, p.tile_m, p.tile_n)
         widest = max(widest, p.tile_n)
     assert widest == (288 if ldw == 3_728_264 else 256)
+
+
+def test_calls_beside_another_stream_keep_their_eight_wave_tiles():
+    """A call that shares the GPU takes square tiles where a rectangle of up to 192 columns would be the best. The wider ones
+    stand in for eight-wave tiles as well as for square ones (6100 x 9216 x 3072: 272 us on eight-wave tiles, 292 on square), so
+    they are no reason to leave those."""
+    assert (lambda p: (p.family, p.tile_m, p.tile_n))(plan_of(linear_args(6100, 9216, 3072))) == (RECT, 224, 288)
+    p = plan_of(linear_args(6100, 9216, 3072, flags=nv.LINEAR_SHARED_GPU))
+    assert p.family == EIGHT_WAVES
+    p = plan_of(linear_args(4608, 12288, 3072, flags=nv.LINEAR_SHARED_GPU))
+    assert (p.family, p.tile_m, p.tile_n) == (SQUARE, 256, 256)
+    rng = random.Random(3)
+    for _ in range(2000):
+        M, N, K = round(2 ** rng.uniform(8, 14)), 8 * round(2 ** rng.uniform(7, 11.5)), 64 * rng.randint(16, 240)
+        assert plan_of(linear_args(M, N, K, flags=nv.LINEAR_SHARED_GPU)).family != RECT

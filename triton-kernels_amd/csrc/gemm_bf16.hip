@@ -941,8 +941,9 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     for (const TileShape& t : kTileShapes) {
         if (p.qk_cols > 0 ? t.fn != 8 : t.fn == 8 && t.family == kPair) continue;   // (eight waves of that width are there for q/k only)
         // Rectangles of 50000 outputs and more: measured from K = 1024 on. Their epilogues, which a slab's price does not
-        // hold, are as long as the square tile's.
-        if (t.family == kRect && t.fn > 6 && p.qk_cols == 0 && p.K < 1024) continue;
+        // hold, are as long as the square tile's. Beside another stream no rectangle is taken in the end (below), and these,
+        // which replace eight-wave tiles too, would only hide those: 6100 x 9216 x 3072 272 us, 292 on square tiles.
+        if (t.family == kRect && t.fn > 6 && p.qk_cols == 0 && (p.K < 1024 || shared_gpu)) continue;
         if ((t.family == kRect || (t.family == kPair && t.fn == 8)) && !columns_ok(t.fn)) continue;
         const double us = tile_cost_us(g, t, 1);
         if (us < best.us) best = {t.family, t.fm, t.fn, 1, us, t.family == kPair && !columns_ok(t.fn)};

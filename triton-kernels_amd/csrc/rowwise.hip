@@ -668,14 +668,18 @@ static int rms_bwd_launch(const void* dy, const void* x, const void* scale, cons
     return check_launch("flux_rms_norm_bwd");
 }
 
-// fp32 inputs of more than a third of the 256 MB cache in front of HBM are read with the non-temporal hint: what the
-// operation in front read, the input it wrote and this output do not fit there together, so much of the input comes from
-// HBM. us, ordinary -> non-temporal: inputs from HBM [4, 2048, 3072] (101 MB) 40.8 -> 34.1; between two additions, all
-// three: 201 MB 207 -> 193, 147 MB 151 -> 140, but 101 MB, just written, 96 -> 101. Smaller ones mostly come from that cache, where the
-// hint costs more than it gives (50 MB 15.5 -> 17.0), and bf16 gains a third of what fp32 does. (Stores with the hint make the
-// call faster still, 10.3 us for 13.9 at [1, 4608, 3072] bf16, and the reader of the output slower: the single-stream block
-// at 3 x 4336 tokens 2840 -> 2873.)
-constexpr int64_t kCacheBytes = 256 << 20;
+// fp32 inputs of more than 136 MiB are read with the non-temporal hint: input and output together no longer fit in the
+// 256 MiB cache in front of HBM, so whatever came before the call and comes behind it, much of the input comes from
+// HBM. us, ordinary -> non-temporal, rows of 3072:
+//                                                        96 MiB           128 MiB          132 MiB          144 MiB          192 MiB
+//   input from HBM                                       35.4 -> 34.6     44.6 -> 43.9     46.8 -> 45.1     55.5 -> 49.4     73.7 -> 62.8
+//   the same input again                                 30.1 -> 34.8     40.6 -> 44.0     45.3 -> 45.2     54.1 -> 49.4     73.6 -> 62.9
+//   between additions in place, all three                87.5 -> 90.9    115.5 -> 118.0   124.0 -> 122.3   136.2 -> 132.7   199.2 -> 175.9
+//   between additions from and to other memory          103.1 -> 94.0    134.5 -> 124.9   142.1 -> 130.5   157.4 -> 141.2   208.3 -> 193.8
+// With the line at a third of the cache the last kind gained from 90 MiB on, but the second lost up to 15 % and the
+// third up to 4 % until 128 MiB. bf16 gains a third of what fp32 does. (Stores with the hint make the call faster still, 10.3 us
+// for 13.9 at [1, 4608, 3072] bf16, and the reader of the output slower: the single-stream block at 3 x 4336 tokens 2840 -> 2873.)
+constexpr int64_t kReadPastCache = 136 << 20;
 
 template <typename T>
 static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float eps, hipStream_t st) {
@@ -702,7 +706,7 @@ static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float 
         return check_launch("flux_layer_norm_modulation");
     }
     if (used == 1) set.t[1] = set.t[0];
-    set.once = 3 * bytes > kCacheBytes;
+    set.once = bytes > kReadPastCache;
 #define CALL(G_, I_)                                                                                        \
     do {                                                                                                    \
         constexpr int RPB_ = kBlock / G_;                                                                    \

@@ -502,6 +502,22 @@ def test_linear_row_vector_activation_shares(M, K, N):
     assert torch.equal(tk.linear_into(x, w, None, in_activation="SiLU"), tk.linear_into(x, w, torch.zeros_like(b), in_activation="SiLU"))
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("K", [1528, 1536, 1544, 3064, 3072, 3080, 6152])
+def test_linear_row_vector_weight_depths(M, K):
+    """K where a lane has three or six vectors of a weight row in flight, and one vector to either side: the same bound as
+    above, and the columns of a wider call have the same bits."""
+    g = seeded(M * K)
+    x = randn(g, M, K, dtype=torch.bfloat16, std=2.0).to(DEV)
+    w = randn(g, 75, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV)
+    b = randn(g, 75, dtype=torch.bfloat16).to(DEV)
+    got = tk.linear(x, w, b)
+    ref = x.double() @ w.double().T + b.double()
+    sizes = x.double().abs() @ w.double().abs().T + b.double().abs()
+    assert ((got.double() - ref).abs() <= ref.abs() * (2.0 ** -8 * 1.01) + sizes * (K * 2.0 ** -24)).all()
+    assert torch.equal(got[:, :9], tk.linear(x, w[:9], b[:9]))
+
+
 @pytest.mark.parametrize("tile_m,tile_n,M,N,K", [(256, 224, 916, 12384, 1024), (256, 224, 1178, 9944, 1032), (224, 256, 880, 12320, 1024), (224, 256, 872, 12376, 1032),
                                                  (224, 288, 1586, 8200, 1024), (224, 288, 1580, 8312, 1032)])
 def test_linear_wide_rectangles(tile_m, tile_n, M, N, K):

@@ -593,19 +593,16 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_rect_kernel(GemmLaunch L
 // ------------------------------------------------------------------------------------------------
 // Skinny problems (M <= 8, e.g. the Modulation projection of one conditioning vector per batch
 // element): HBM-bound on W. A wave streams the W rows of two output columns with 16-byte loads,
-// twelve in flight per lane, while the few activation rows come from cache; the dot products are
+// six or twelve in flight per lane, while the few activation rows come from cache; the dot products are
 // folded with a wave butterfly. The kernel is instantiated per row count, so it has no row tests.
 // Everything a wave needs beside W is requested in front of it: with the activation rows behind the W loads, and the
 // bias behind the sums, each was a wait of its own while all waves of the launch stood at the same place. W is read
 // once, so its loads carry the non-temporal hint (a bare read of 113 MB: 18.4 -> 17.4 us). us, weights from HBM,
 // before -> now: 1 x 9216 x 3072 with SiLU 14.0 -> 11.2 (the bare read 9.5), two such products of 18432 columns in one launch
-// 38.7 -> 33.8 (6.7 TB/s), 3 rows 17.8 -> 15.8, 8 rows 33.2 -> 31.2, 1 x 3072 x 12288 20.7 -> 19.1.
+// 38.7 -> 33.8 (6.7 TB/s), 3 rows 17.9 -> 15.8, 8 rows 33.6 -> 31.2, 1 x 3072 x 12288 22.3 -> 20.2.
 // ------------------------------------------------------------------------------------------------
 constexpr int kGemvCols = 2;  // output columns per wave
 constexpr int kGemvSiluLds = 48 * 1024;  // bytes of LDS for the (activated) input rows (bf16)
-// 16-byte vectors of a W row a lane requests at once: a whole row of 3072 for up to four activation rows, half of
-// that when more rows' products need the registers (8 rows: 33 us, 49 with whole rows)
-constexpr int gemv_depth(int rows) { return rows <= 4 ? 6 : 3; }
 
 // SILU_LDS: the few activation rows are staged in LDS once per workgroup, with the input activation
 // x * sigmoid(x) applied on the way (rounded to bf16, as the separate operator would leave it). Every
@@ -614,12 +611,15 @@ constexpr int gemv_depth(int rows) { return rows <= 4 ? 6 : 3; }
 // value, would be repeated by each of the N / 2 waves. For the same reason the workgroup's share of them is
 // requested in front of the first W loads, not behind. Rows that do not fit the LDS budget are read
 // from memory as they are needed.
+// U: 16-byte vectors of a W row a lane requests at once (see launch_gemv).
 // EXACT: K = 512 * U, so every lane has exactly U vectors per row and the K loop runs once, without tests.
-template <int MM, bool SILU_LDS, bool EXACT>
+template <int MM, bool SILU_LDS, int U, bool EXACT>
 __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
     const GemmParams p = g.p[blockIdx.y];
-    constexpr int CPW = kGemvCols, U = gemv_depth(MM);  // CPW * U 16-byte loads of W in flight per lane
-    constexpr int PRE = MM <= 4 ? MM + (MM + 1) / 2 : 2;  // activation vectors requested in front: a thread's share at K = 3072
+    constexpr int CPW = kGemvCols;  // CPW * U 16-byte loads of W in flight per lane
+    // Activation vectors a thread requests in front: its share at K = 3072 where a whole such row of W is in flight, one or
+    // two where half of it is (four rows of K = 1536: 5.4 us, 5.6 with two, 6.2 with all six).
+    constexpr int PRE = U == 6 ? MM + (MM + 1) / 2 : (MM <= 4 ? 1 : 2);
     extern __shared__ __attribute__((aligned(16))) char act_lds[];
     const int lane = threadIdx.x & 63;
     const int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * CPW;
@@ -746,11 +746,19 @@ static void launch_gemv(const GemmSet& g, hipStream_t st) {
     const GemmParams& p = g.p[0];
     const dim3 grid((unsigned)((p.N + 4 * kGemvCols - 1) / (4 * kGemvCols)), (unsigned)g.n);
     const size_t act_bytes = static_cast<size_t>(MM) * p.K * 2;
-    const bool lds = act_bytes <= kGemvSiluLds, exact = p.K == 512 * gemv_depth(MM);
-    if (lds && exact) hipLaunchKernelGGL((gemv_small_m_kernel<MM, true, true>), grid, dim3(256), act_bytes, st, g);
-    else if (lds) hipLaunchKernelGGL((gemv_small_m_kernel<MM, true, false>), grid, dim3(256), act_bytes, st, g);
-    else if (exact) hipLaunchKernelGGL((gemv_small_m_kernel<MM, false, true>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((gemv_small_m_kernel<MM, false, false>), grid, dim3(256), 0, st, g);
+    const bool lds = act_bytes <= kGemvSiluLds;   // (at K of 3072 and less always)
+    // Vectors of a W row in flight: what a row has, up to a whole row of 3072; loops over longer rows take half of that from
+    // three activation rows on, whose products need the registers (8 rows of 3072: 33 us, 49 with whole rows).
+    // us with 6 -> 3 vectors, weights in the caches: 1 x 9216 x 1536 7.5 -> 5.6, 2 rows 9.0 -> 6.9, 3 rows 10.6 -> 8.6, 4 x 6144 x 1024
+    // 7.0 -> 6.2, 3 x 24576 x 4096 48.3 -> 41.5; 4 x 3072 x 12288 49.7 -> 50.6.
+    constexpr int WHOLE = MM <= 4 ? 6 : 3, LOOP = MM <= 2 ? 6 : 3;
+#define CALL(LDS, U, EXACT, BYTES) hipLaunchKernelGGL((gemv_small_m_kernel<MM, LDS, U, EXACT>), grid, dim3(256), BYTES, st, g)
+    if (p.K == 512 * WHOLE) CALL(true, WHOLE, true, act_bytes);
+    else if (p.K == 1536) CALL(true, 3, true, act_bytes);
+    else if (p.K < 1536) CALL(true, 3, false, act_bytes);
+    else if (lds) CALL(true, LOOP, false, act_bytes);
+    else CALL(false, LOOP, false, 0);
+#undef CALL
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -518,6 +518,18 @@ def test_linear_row_vector_weight_depths(M, K):
     assert torch.equal(got[:, :9], tk.linear(x, w[:9], b[:9]))
 
 
+@pytest.mark.parametrize("M,K", [(1, 3080), (2, 3080), (4, 3080), (4, 6144), (1, 24576), (8, 15360)])
+def test_line_of_weights_read_past_the_cache(M, K):
+    """Weights of half the cache, and of a column more: the columns of both have the bits of a call with the few of them."""
+    N = (128 << 20) // (2 * K)
+    x = randn(seeded(K), M, K, dtype=torch.bfloat16).to(DEV)
+    w = torch.randn(N + 1, K, generator=torch.Generator(device=DEV).manual_seed(M), device=DEV).bfloat16()
+    few = tk.linear(x, w[N - 100:], None)
+    ref = x.double() @ w[N - 100:].double().T
+    assert ((few.double() - ref).abs() <= ref.abs() * (2.0 ** -8 * 1.01) + (x.double().abs() @ w[N - 100:].double().abs().T) * (K * 2.0 ** -24)).all()
+    assert torch.equal(tk.linear(x, w, None)[:, N - 100:], few) and torch.equal(tk.linear(x, w[:N], None)[:, N - 100:], few[:, :100])
+
+
 @pytest.mark.parametrize("tile_m,tile_n,M,N,K", [(256, 224, 916, 12384, 1024), (256, 224, 1178, 9944, 1032), (224, 256, 880, 12320, 1024), (224, 256, 872, 12376, 1032),
                                                  (224, 288, 1586, 8200, 1024), (224, 288, 1580, 8312, 1032)])
 def test_linear_wide_rectangles(tile_m, tile_n, M, N, K):

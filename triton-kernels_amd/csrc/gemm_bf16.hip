@@ -597,9 +597,9 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_rect_kernel(GemmLaunch L
 // folded with a wave butterfly. The kernel is instantiated per row count, so it has no row tests.
 // Everything a wave needs beside W is requested in front of it: with the activation rows behind the W loads, and the
 // bias behind the sums, each was a wait of its own while all waves of the launch stood at the same place. W is read
-// once, so its loads carry the non-temporal hint (a bare read of 113 MB: 18.4 -> 17.4 us). us, weights from HBM,
+// once, so its loads mostly carry the non-temporal hint (a bare read of 113 MB: 18.4 -> 17.4 us). us, weights from HBM,
 // before -> now: 1 x 9216 x 3072 with SiLU 14.0 -> 11.2 (the bare read 9.5), two such products of 18432 columns in one launch
-// 38.7 -> 33.8 (6.7 TB/s), 3 rows 17.9 -> 15.8, 8 rows 33.6 -> 31.2, 1 x 3072 x 12288 22.3 -> 20.2.
+// 38.7 -> 33.8 (6.7 TB/s), 3 rows 17.9 -> 15.8, 8 rows 33.6 -> 31.2, 1 x 3072 x 12288 22.3 -> 21.4.
 // ------------------------------------------------------------------------------------------------
 constexpr int kGemvCols = 2;  // output columns per wave
 constexpr int kGemvSiluLds = 48 * 1024;  // bytes of LDS for the (activated) input rows (bf16)
@@ -613,7 +613,8 @@ constexpr int kGemvSiluLds = 48 * 1024;  // bytes of LDS for the (activated) inp
 // from memory as they are needed.
 // U: 16-byte vectors of a W row a lane requests at once (see launch_gemv).
 // EXACT: K = 512 * U, so every lane has exactly U vectors per row and the K loop runs once, without tests.
-template <int MM, bool SILU_LDS, int U, bool EXACT>
+// ONCE: W is read with the non-temporal hint (see launch_gemv).
+template <int MM, bool SILU_LDS, int U, bool EXACT, bool ONCE>
 __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
     const GemmParams p = g.p[blockIdx.y];
     constexpr int CPW = kGemvCols;  // CPW * U 16-byte loads of W in flight per lane
@@ -652,7 +653,10 @@ __global__ __launch_bounds__(256) void gemv_small_m_kernel(GemmSet g) {
             const int k = k0 + u * 512;
             // past the end: a harmless re-read, skipped below
 #pragma unroll
-            for (int c = 0; c < CPW; ++c) w[u][c] = ld16_once(wrow[c] + (EXACT || k < p.K ? k : k0));
+            for (int c = 0; c < CPW; ++c) {
+                const bf16_t* const at = wrow[c] + (EXACT || k < p.K ? k : k0);
+                w[u][c] = ONCE ? ld16_once(at) : ld16(at);
+            }
         }
     };
     if (EXACT || lane * 8 < p.K) request_w(lane * 8);
@@ -752,12 +756,23 @@ static void launch_gemv(const GemmSet& g, hipStream_t st) {
     // us with 6 -> 3 vectors, weights in the caches: 1 x 9216 x 1536 7.5 -> 5.6, 2 rows 9.0 -> 6.9, 3 rows 10.6 -> 8.6, 4 x 6144 x 1024
     // 7.0 -> 6.2, 3 x 24576 x 4096 48.3 -> 41.5; 4 x 3072 x 12288 49.7 -> 50.6.
     constexpr int WHOLE = MM <= 4 ? 6 : 3, LOOP = MM <= 2 ? 6 : 3;
-#define CALL(LDS, U, EXACT, BYTES) hipLaunchKernelGGL((gemv_small_m_kernel<MM, LDS, U, EXACT>), grid, dim3(256), BYTES, st, g)
-    if (p.K == 512 * WHOLE) CALL(true, WHOLE, true, act_bytes);
-    else if (p.K == 1536) CALL(true, 3, true, act_bytes);
-    else if (p.K < 1536) CALL(true, 3, false, act_bytes);
-    else if (lds) CALL(true, LOOP, false, act_bytes);
-    else CALL(false, LOOP, false, 0);
+    // The hint gains where W comes from HBM (2 to 9 %), and beside it where the activation rows are read through the cache
+    // that W then leaves to them. Where the same weights are read again at once, it gains at up to 3072 of K too, but
+    // costs 3 to 14 % in the loops over longer rows: us with -> without, 1 x 3072 x 12288 18.3 -> 16.1 (from HBM 20.2 -> 21.4), 3 x 18432
+    // x 6144 50 -> 42 (51 -> 53). So these go without it, but for two rows, where it costs up to 5 % and gains up to 9 from HBM
+    // (2 x 18432 x 6144 44.1 -> 42.1, 45.4 -> 50.1; at 3072 the one loss is 226 MB beside three rows, 42.2 us before these
+    // changes and 46.1 now where they are read again, 50.3 and 46.8 from HBM);
+    // and of the activation rows that do not fit the LDS, those whose weights are more than half of the 256 MiB cache (5 x
+    // 18432 x 6144 109 -> 102; 8 x 3072 x 12288 keeps it, 87.8 against 96.4).
+    const bool once = p.K <= 3072 || (lds ? MM == 2 : static_cast<int64_t>(p.N) * p.K * 2 * g.n <= (int64_t{128} << 20));
+#define CALL(LDS, U, EXACT, ONCE, BYTES) hipLaunchKernelGGL((gemv_small_m_kernel<MM, LDS, U, EXACT, ONCE>), grid, dim3(256), BYTES, st, g)
+    if (p.K == 512 * WHOLE) CALL(true, WHOLE, true, true, act_bytes);
+    else if (p.K == 1536) CALL(true, 3, true, true, act_bytes);
+    else if (p.K < 1536) CALL(true, 3, false, true, act_bytes);
+    else if (lds && once) CALL(true, LOOP, false, true, act_bytes);
+    else if (lds) CALL(true, LOOP, false, false, act_bytes);
+    else if (once) CALL(false, LOOP, false, true, 0);
+    else CALL(false, LOOP, false, false, 0);
 #undef CALL
 }
 

@@ -152,6 +152,31 @@ def test_attention_wide_tile_launch_shapes(B, H, L, D):
 
 
 @pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("B,H", [(1, 2), (2, 65), (1, 257)])   # sums of rounded and of fp32 exponentials, and more workgroups than CUs
+@pytest.mark.parametrize("L", [1, 31, 33, 63, 64, 65, 127, 128, 129])
+def test_attention_of_one_key_tile_and_a_few(B, H, L, D):
+    """Up to 64 rows Q and the output do not go through LDS, up to 128 every (batch, head) is a 128-row workgroup, and the
+    rows past the end are nobody's: packed views in, a head-interleaved output between guard rows out, with lse."""
+    g = seeded(L * 1000 + H + D)
+    qkv = randn(g, B, L, 3, H, D, dtype=torch.bfloat16).to(DEV)
+    q, k, v = qkv.permute(2, 0, 3, 1, 4)
+    wide = torch.full((B, L + 140, H, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    lse = torch.full((B, H, L + 140), float("nan"), device=DEV)
+    flat = lse.view(-1)[:B * H * L].view(B, H, L)
+    tk.attention_into(q, k, v, wide[:, :L].permute(0, 2, 1, 3), lse=flat)
+    # A scaled q is rounded to bf16, 2^-8 of it at most, so no score moves by more than that share of its terms' sizes, and lse by
+    # no more than a score; the output by that share of sum p |v|, twice, by the rounding of p and of its sum, and its own.
+    u = 2.0 ** -8
+    moved = (q.float().abs() @ k.float().abs().transpose(-1, -2)).amax(-1) * (D ** -0.5 * u)
+    assert ((flat - oracle.attention_lse_ref(q, k)).abs() <= 1.4427 * moved + 1e-4).all()
+    ref = oracle.attention_ref_fp32(q, k, v)
+    bound = ref.abs() * u + oracle.attention_ref_fp32(q, k, v.abs()) * (2 * u + 2 * moved[..., None]) + 1e-5
+    assert ((wide[:, :L].permute(0, 2, 1, 3).float() - ref).abs() <= bound).all()
+    assert (wide[:, :L].permute(0, 2, 1, 3).float() - ref).norm() <= 6e-3 * ref.norm()   # (3e-3 measured, four roundings of u / sqrt(12) each)
+    assert torch.isnan(wide[:, L:]).all() and torch.isnan(lse.view(-1)[B * H * L:]).all()
+
+
+@pytest.mark.parametrize("D", [128, 64])
 def test_attention_wide_tile_strided_views(D):
     """The 64-row-per-wave kernels on views of a packed qkv projection (row stride 3 * H * D) with the
     output written head-interleaved, as the blocks pass them, ragged length, with lse."""

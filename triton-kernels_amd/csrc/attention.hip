@@ -132,7 +132,9 @@ constexpr bool attn_units_in_time(int qb_count, int ns, int db_count, int nslot,
 // its rows as fp32 to ws, and attn_combine_kernel adds the parts.
 // FSUM: a row's sum is that of its fp32 exponentials, as in the 64-row kernel; else that of the probabilities
 // rounded to bf16, one instruction for two of them, which round like the numerator they divide.
-template <int D, int QB, int BN, bool SPLIT, bool FSUM>  // BN = keys per tile (32 or 64)
+// DIRECT: Q comes straight into registers and the output leaves from there, for calls of a single key tile, which have
+// nothing to hide the way through LDS behind (see attn_launch_pipe).
+template <int D, int QB, int BN, bool SPLIT, bool FSUM, bool DIRECT>  // BN = keys per tile (32 or 64)
 __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int splits, int part_keys) {
     constexpr int KB = BN / 32;         // 32-key blocks of S^T per tile
     constexpr int PS = BN / 16;         // 16-key steps of P^T per tile
@@ -268,31 +270,44 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
         const u32x4 rk1 = tile_rsrc(kbase, k_row2, BN);
         const bf16_t* const qbase = p.q + b * p.q_sb + h * p.q_sh;
         char* const q_lds = lds + V0 + T_BYTES + wave * (32 * QB * ROWB);
+        // sm_scale*log2(e) goes into Q once (rounded to bf16), so scores leave the MFMA in the
+        // base-2 domain whatever the sign of the scale, and masked keys stay -inf for scale 0
+        auto scaled = [&](u32x4 t) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                t[e] = pack2_bf16(__uint_as_float(t[e] << 16) * p.scale_log2, __uint_as_float(t[e] & 0xffff0000u) * p.scale_log2);
+            return __builtin_bit_cast(bf16x8, t);
+        };
+        if constexpr (DIRECT) {
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) {
+                const bf16_t* const row = qbase + static_cast<int64_t>(min(q0 + qb * 32 + frow, p.L - 1)) * p.q_sl;
+#pragma unroll
+                for (int kk = 0; kk < KSTEPS; ++kk) qf[qb][kk] = scaled(*reinterpret_cast<const u32x4*>(row + (kk * 2 + fhalf) * 8));
+            }
+        }
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) lds_load16_raw(rk0, lds_base + i * 4096, k_voff[i]);
+        if constexpr (!DIRECT) {
 #pragma unroll
-        for (int i = 0; i < 32 * QB / RPW; ++i) {
-            const int r = i * RPW + l_row;
-            lds_load16_global(qbase + static_cast<int64_t>(min(q0 + r, p.L - 1)) * p.q_sl + (l_pos ^ kswz(r)) * 8, lds_addr_of(q_lds) + i * 1024);
+            for (int i = 0; i < 32 * QB / RPW; ++i) {
+                const int r = i * RPW + l_row;
+                lds_load16_global(qbase + static_cast<int64_t>(min(q0 + r, p.L - 1)) * p.q_sl + (l_pos ^ kswz(r)) * 8, lds_addr_of(q_lds) + i * 1024);
+            }
         }
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
             lds_load16_raw(rv0, lds_base + V0 + i * 4096, v_voff[i]);
             lds_load16_raw(rk1, lds_base + T_BYTES + i * 4096, k_voff[i]);
         }
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PASSES) : "memory");   // K(0) and Q have landed; V(0) and K(1) fly on
+        if constexpr (!DIRECT) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PASSES) : "memory");   // K(0) and Q have landed; V(0) and K(1) fly on
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
+            for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-            for (int kk = 0; kk < KSTEPS; ++kk) {
-                u32x4 t = *reinterpret_cast<const u32x4*>(q_lds + (qb * 32 + frow) * ROWB + (((kk * 2 + fhalf) ^ kswz(frow)) * 16));
-                // sm_scale*log2(e) goes into Q once (rounded to bf16), so scores leave the MFMA in the
-                // base-2 domain whatever the sign of the scale, and masked keys stay -inf for scale 0
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    t[e] = pack2_bf16(__uint_as_float(t[e] << 16) * p.scale_log2, __uint_as_float(t[e] & 0xffff0000u) * p.scale_log2);
-                qf[qb][kk] = __builtin_bit_cast(bf16x8, t);
-            }
+                for (int kk = 0; kk < KSTEPS; ++kk)
+                    qf[qb][kk] = scaled(*reinterpret_cast<const u32x4*>(q_lds + (qb * 32 + frow) * ROWB + (((kk * 2 + fhalf) ^ kswz(frow)) * 16)));
+        }
         attn_wait_and_barrier<2 * PASSES>();
     }
     f32x16 sa[QB][KB], sb[QB][KB];  // S^T of the tile in its softmax / of the tile being multiplied
@@ -455,7 +470,7 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
     wait_all_vmem();  // loads of tiles past the end are empty but still count
 
     // ---- finish: fold the two half-waves' partial sums, normalise, store
-    if constexpr (!SPLIT) asm volatile("s_barrier" ::: "memory");   // the buffers are everyone's until here
+    if constexpr (!SPLIT && !DIRECT) asm volatile("s_barrier" ::: "memory");   // the buffers are everyone's until here
     char* const stage = lds + wave * (32 * QB * ROWB);
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -474,6 +489,19 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
                     wblk[(db * 4 + g) * 64] = u32x4{__float_as_uint(acc[qb][db][g * 4 + 0]), __float_as_uint(acc[qb][db][g * 4 + 1]),
                                                     __float_as_uint(acc[qb][db][g * 4 + 2]), __float_as_uint(acc[qb][db][g * 4 + 3])};
             if (fhalf == 0) *reinterpret_cast<f32x2*>(ws + splits * blocks * (32 * D) + (at * 32 + frow) * 2) = f32x2{m_run[qb] * c, l_tot};
+        } else if constexpr (DIRECT) {
+            if (row < p.L) {
+                bf16_t* const orow = p.o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(row) * p.o_sl;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        u32x2 w;
+                        w.x = pack2_bf16(acc[qb][db][g * 4 + 0] * inv, acc[qb][db][g * 4 + 1] * inv);
+                        w.y = pack2_bf16(acc[qb][db][g * 4 + 2] * inv, acc[qb][db][g * 4 + 3] * inv);
+                        *reinterpret_cast<u32x2*>(orow + db * 32 + g * 8 + fhalf * 4) = w;
+                    }
+            }
         } else {
             // 8-byte slot s of row r sits at slot s ^ 2(r mod chunks per row), as in the 64-row kernel
             char* const srow = stage + (qb * 32 + frow) * ROWB;
@@ -486,11 +514,11 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
                     w.y = pack2_bf16(acc[qb][db][g * 4 + 2] * inv, acc[qb][db][g * 4 + 3] * inv);
                     *reinterpret_cast<u32x2*>(srow + (((db * 8 + g * 2 + fhalf) ^ ((frow % CH) * 2)) * 8)) = w;
                 }
-            if (row < p.L && p.lse != nullptr && fhalf == 0)
-                p.lse[static_cast<int64_t>(bh) * p.L + row] = m_run[qb] * c + __builtin_amdgcn_logf(l_tot);
         }
+        if (!SPLIT && row < p.L && p.lse != nullptr && fhalf == 0)
+            p.lse[static_cast<int64_t>(bh) * p.L + row] = m_run[qb] * c + __builtin_amdgcn_logf(l_tot);
     }
-    if constexpr (!SPLIT) {
+    if constexpr (!SPLIT && !DIRECT) {
         // A lane holds runs of four columns of one row, which would leave as 8-byte pieces of 32 rows; through LDS they leave
         // as 16-byte pieces of whole rows.
         __builtin_amdgcn_wave_barrier();   // LDS operations of one wave complete in order
@@ -511,13 +539,13 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
 
 // (The form without parts takes no arguments for them: with some it waits for its arguments twice, which costs up to
 // 2 % of a short call, [1, 24, 1280, 128] 31.6 -> 32.4 us.)
-template <int D, int QB, int BN, bool FSUM>
+template <int D, int QB, int BN, bool FSUM, bool DIRECT>
 __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(AttnParams p) {
-    attn_pipe<D, QB, BN, false, FSUM>(p, nullptr, 1, 0);
+    attn_pipe<D, QB, BN, false, FSUM, DIRECT>(p, nullptr, 1, 0);
 }
 template <int D, int QB, int BN>
 __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_parts_kernel(AttnParams p, float* ws, int splits, int part_keys) {
-    attn_pipe<D, QB, BN, true, false>(p, ws, splits, part_keys);
+    attn_pipe<D, QB, BN, true, false, false>(p, ws, splits, part_keys);
 }
 
 // O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s over the parts of a row, in the order of the keys. A wave
@@ -1382,8 +1410,16 @@ static void attn_launch_pipe(AttnParams& p, int64_t BH, float* ws, int64_t ws_by
     p.total_tiles = static_cast<int>(p.n_qtiles * BH * (split ? splits : 1));
     const int grid = ((p.total_tiles + 7) / 8) * 8;
     if (!split) {
-        if (BH * ((p.L + 255) / 256) >= kFsumTiles) hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, true>), dim3(grid), dim3(256), 0, st, p);
-        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, false>), dim3(grid), dim3(256), 0, st, p);
+        // A single key tile: the way of Q and of the output through LDS is two more waits with nothing beside them. us through LDS
+        // -> direct: [1, 24, 1, 128] 5.7 -> 5.3, [1, 24, 32, 128] 6.1 -> 5.7, [4, 24, 32, 64] 5.0 -> 4.6, [1, 24, 64, 64] 4.7 -> 4.5; from two
+        // tiles on it pays, [4, 24, 93, 128] 8.1 -> 7.6 the other way round.
+        const bool fsum = BH * ((p.L + 255) / 256) >= kFsumTiles, direct = p.L <= 64;
+#define CALL(FSUM, DIRECT) hipLaunchKernelGGL((attn_fwd_pipe_kernel<D, 1, 64, FSUM, DIRECT>), dim3(grid), dim3(256), 0, st, p)
+        if (fsum && direct) CALL(true, true);
+        else if (fsum) CALL(true, false);
+        else if (direct) CALL(false, true);
+        else CALL(false, false);
+#undef CALL
         return;
     }
     hipLaunchKernelGGL((attn_fwd_parts_kernel<D, 1, 64>), dim3(grid), dim3(256), 0, st, p, ws, splits, part_keys);
@@ -1502,8 +1538,10 @@ using namespace flux;
 // Whether 128-row workgroups (32 rows per wave) are few enough for one per CU; then they end sooner than half
 // as many 256-row ones (64 rows per wave), which are faster per row only. us on the 32-row and the 64-row kernel,
 // head dim 128: [1, 24, 1280] (240 workgroups) 29 and 35, [1, 8, 4096] (256) 86 and 89, [1, 24, 1500] (288)
-// 47 and 40; head dim 64: 19 and 24, 52 and 61, 32 and 28.
-static bool attn_short(int64_t BH, int64_t L) { return BH * ((L + 127) / 128) <= kAttnCUs; }
+// 47 and 40; head dim 64: 19 and 24, 52 and 61, 32 and 28. Up to 128 rows a (batch, head) is one workgroup of either
+// kernel, and two of the 32-row one share a CU: [11, 24, 64] 8.4 and 17.0 (head dim 64: 5.6 and 12.3), [16, 24, 128] 14.0 and
+// 21.0 (7.5 and 14.4), [40, 24, 32] 12.9 and 32.5 (9.4 and 24.0).
+static bool attn_short(int64_t BH, int64_t L) { return L <= 128 || BH * ((L + 127) / 128) <= kAttnCUs; }
 // The 64-row kernel reaches the rows of q with 32-bit offsets inside 64 rows; the 32-row one has no such limit.
 static bool attn_q_near(const flux_attn_args* a) { return a->q.sl * 2 * 64 < 0x7fffffffLL; }
 

@@ -1264,10 +1264,11 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     }
     // A workgroup that starts behind this one waits for its first 112 KB to come from HBM with the matrix pipe idle
     // (3.8 us from its start to its first MFMA at head dim 128), so the rows of Q and of the first K and V tile of the
-    // tile 256 blocks on are touched here, a few microseconds ahead. us, with the fetch of Q above, before -> now:
-    // [4, 24, 1024, 128] 58.2 -> 57.2, [4, 24, 800, 128] 45.8 -> 45.2, [2, 24, 2048, 128] 97.8 -> 96.8, [4, 24, 2000, 64]
-    // 112.0 -> 110.6; launches of one round and of many long ones stay as they were.
-    {
+    // tile 256 blocks on are touched here, a few microseconds ahead. us without -> with: [4, 24, 1024, 128] 58.3 -> 58.0, [4, 24,
+    // 700, 128] 40.2 -> 39.5, [8, 24, 1024, 128] 99.1 -> 98.3, [4, 24, 1024, 64] 38.5 -> 38.1, [16, 24, 512, 64] 43.5 -> 42.4; launches of one
+    // round and of many long ones stay as they were. A workgroup of head dim 128 with few key tiles has no few microseconds
+    // left: [83, 24, 256, 128] 146 -> 163, [40, 24, 256, 128] 70 -> 75, [16, 24, 448, 128] 64 -> 67, [16, 24, 640, 128] 99.8 -> 100.5.
+    if (D == 64 || p.L > 640) {
         int nbh, nrow0;
         if (next(nbh, nrow0)) {
             const int nb = nbh / p.H, nh = nbh % p.H;

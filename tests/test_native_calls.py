@@ -9,10 +9,7 @@ import torch.autograd.forward_ad as fwad
 
 import triton_kernels as tk
 from triton_kernels import _native as nv
-from triton_kernels.kernels import attention as attention_mod
-from triton_kernels.kernels import linear as linear_mod
 from triton_kernels.kernels import normalization as norm_mod
-from triton_kernels.kernels import positional_embedding as rope_mod
 from util import DEV, randn, seeded
 
 gpu = pytest.mark.gpu
@@ -159,6 +156,85 @@ def test_rope_linear_attention_forms(monkeypatch):
             for scale in (None, 0.3, 0.0, torch.tensor(0.2)):
                 got, want = tk.scaled_dot_product_attention(q, k, v, scale), launcher(monkeypatch, tk.scaled_dot_product_attention, q, k, v, scale)
                 assert torch.equal(got, want) and got.stride() == want.stride()
+
+
+class _Records:
+    """The native calls, and for each one made whether it served the call."""
+
+    def __init__(self):
+        self.ops, self.served = nv.ops(), []
+
+    def __getattr__(self, name):
+        def call(*args):
+            y = getattr(self.ops, name)(*args)
+            self.served.append((name, y is not None))
+            return y
+        return call
+
+
+@gpu
+def test_which_calls_are_served_in_native_code(monkeypatch):
+    """The forms that programs use are served by the native call itself, with the launcher's bits; the listed others are not."""
+    g = seeded(11)
+
+    def check(op, expected, fn, *args, **kw):
+        records = _Records()
+        with monkeypatch.context() as m:
+            m.setattr(nv, "ops", lambda: records)
+            got = fn(*args, **kw)
+        assert (op, True) in records.served if expected else (op, True) not in records.served, (op, records.served, [getattr(a, "shape", a) for a in args])
+        want = launcher(monkeypatch, fn, *args, **kw)
+        for a, b in zip(got, want) if isinstance(got, tuple) else [(got, want)]:
+            assert torch.equal(a, b) and a.stride() == b.stride() and a.dtype == b.dtype
+
+    def t(*shape, dtype=BF, std=1.0):
+        return randn(g, *shape, dtype=dtype, std=std).to(DEV)
+
+    for dtype, scale_dtype in ((BF, BF), (BF, F32), (F32, F32), (F32, BF)):
+        for x in _views(g, dtype):
+            if x.numel():
+                scale, taken = t(x.shape[-1], dtype=scale_dtype), (dtype, scale_dtype) != (F32, BF) and x.stride(-1) == 1 and x.dim() <= 4
+                check("rms_norm", taken, tk.rms_norm, x, scale)
+                check("rms_norm", taken, tk.rms_norm, x.detach().requires_grad_(True), scale)
+                check("rms_norm", False, tk.rms_norm, x, scale[None])
+    for dtype in (BF, F32):
+        qkv = t(2, 9, 3 * 4 * 128, dtype=dtype).view(2, 9, 3, 4, 128).permute(2, 0, 3, 1, 4)
+        s = t(128, dtype=dtype)
+        with torch.no_grad():
+            check("rms_norm_pair", True, norm_mod.rms_norm_pair, qkv[0], s, qkv[1], s)
+            check("rms_norm_pair", False, norm_mod.rms_norm_pair, qkv[0][..., 1:], s[1:], qkv[1][..., 1:], s[1:])
+        check("rms_norm_pair", False, norm_mod.rms_norm_pair, qkv[0], s, qkv[1], s)
+        pe = t(1, 1, 9, 64, 2, 2, dtype=F32)
+        check("apply_rope", True, tk.apply_rope, qkv[0], qkv[1], pe)
+        check("apply_rope", True, tk.apply_rope, qkv[0].contiguous(), qkv[1].contiguous(), pe.expand(2, 1, 9, 64, 2, 2).contiguous())
+        check("apply_rope", False, tk.apply_rope, qkv[0], qkv[1], pe.double())
+        x, mod = t(2, 7, 256, dtype=dtype), t(2, 1, 3 * 256, dtype=dtype)
+        check("layer_norm_modulation", True, tk.layer_norm_modulation, x, *mod.chunk(3, -1)[:2])
+        check("layer_norm_modulation", True, tk.layer_norm_modulation, x, mod[:, 0, :256].contiguous(), mod[:, 0, 256:512].contiguous())
+        check("layer_norm_modulation", True, tk.layer_norm_modulation, x[:1], mod[:1, :, :256], mod[:1, :, 256:512])
+        check("layer_norm_modulation", False, tk.layer_norm_modulation, x, mod[..., ::3], mod[..., 1::3])
+        check("layer_norm_modulation", False, tk.layer_norm_modulation, x.transpose(0, 1).contiguous().transpose(0, 1), *mod.chunk(3, -1)[:2])
+    for M, N, K in ((1, 64, 64), (8, 40, 72), (300, 136, 3080), (320, 3072, 15360)):
+        x, w, b = t(M, K), t(N, K, std=K ** -0.5), t(N)
+        for act in ("", "GELU"):
+            check("linear", True, tk.linear, x, w, b, activation=act)
+            check("linear", True, tk.linear, x.view(1, M, K), w, None, activation=act)
+        check("linear", False, tk.linear, x, w, b.float())
+        check("linear", False, tk.linear, x, t(K, N, std=K ** -0.5).t(), b)
+        check("linear", False, tk.linear, x, w, b, shared_gpu=True)
+        with monkeypatch.context() as m:
+            m.setattr(sys.modules["triton_kernels.kernels.linear"], "launch_hook", lambda meta: None)
+            check("linear", False, tk.linear, x, w, b)
+    for B, H, L, D in ((1, 2, 1, 64), (2, 3, 77, 128), (1, 2, 2048, 128), (1, 2, 40, 32)):
+        qkv = t(B, L, 3, H, D).permute(2, 0, 3, 1, 4)
+        check("attention", True, tk.scaled_dot_product_attention, *qkv.unbind(0))
+        check("attention", True, tk.scaled_dot_product_attention, *(v.contiguous() for v in qkv), 0.3)
+        check("attention", L == 1, tk.scaled_dot_product_attention, qkv[0], qkv[1].transpose(2, 3).contiguous().transpose(2, 3), qkv[2])
+    assert nv.lib().flux_attention_workspace_bytes(1, 2, 2048, 128) > 0   # (of the calls above: keys in parts, K in parts)
+    a = nv.LinearArgs()
+    a.A = a.W = a.Y = 1 << 20
+    a.M, a.N, a.K, a.lda, a.ldw, a.ldy, a.split_n = 320, 3072, 15360, 15360, 15360, 3072, 3072
+    assert nv.lib().flux_linear_workspace_bytes(nv.byref(a)) > 0
 
 
 @gpu

@@ -361,10 +361,10 @@ def test_qkv_prep_norm_rope_matches_unfused_sequence():
     assert torch.equal(v, torch.cat((tv, iv), 2))
 
 
-@pytest.mark.parametrize("rows", [(136 << 20) // (4 * 3072), (136 << 20) // (4 * 3072) + 1])
+@pytest.mark.parametrize("rows", [(256 << 20) // (3 * 4 * 3072), (256 << 20) // (3 * 4 * 3072) + 1])
 @pytest.mark.parametrize("width", [3072, 3068])
 def test_layer_norm_modulation_inputs_read_once(rows, width):
-    """fp32 inputs of more than 136 MiB are read past the cache: the same bits as a part of them that is read
+    """fp32 inputs of more than a third of the cache are read past it: the same bits as a part of them that is read
     through it, at the size where that begins (3072 values a row) and one row below it."""
     g = torch.Generator(device=DEV).manual_seed(rows + width)
     x = torch.randn(1, rows, width, generator=g, device=DEV)

@@ -668,18 +668,20 @@ static int rms_bwd_launch(const void* dy, const void* x, const void* scale, cons
     return check_launch("flux_rms_norm_bwd");
 }
 
-// fp32 inputs of more than 136 MiB are read with the non-temporal hint: input and output together no longer fit in the
-// 256 MiB cache in front of HBM, so whatever came before the call and comes behind it, much of the input comes from
-// HBM. us, ordinary -> non-temporal, rows of 3072:
-//                                                        96 MiB           128 MiB          132 MiB          144 MiB          192 MiB
-//   input from HBM                                       35.4 -> 34.6     44.6 -> 43.9     46.8 -> 45.1     55.5 -> 49.4     73.7 -> 62.8
-//   the same input again                                 30.1 -> 34.8     40.6 -> 44.0     45.3 -> 45.2     54.1 -> 49.4     73.6 -> 62.9
-//   between additions in place, all three                87.5 -> 90.9    115.5 -> 118.0   124.0 -> 122.3   136.2 -> 132.7   199.2 -> 175.9
-//   between additions from and to other memory          103.1 -> 94.0    134.5 -> 124.9   142.1 -> 130.5   157.4 -> 141.2   208.3 -> 193.8
-// With the line at a third of the cache the last kind gained from 90 MiB on, but the second lost up to 15 % and the
-// third up to 4 % until 128 MiB. bf16 gains a third of what fp32 does. (Stores with the hint make the call faster still, 10.3 us
-// for 13.9 at [1, 4608, 3072] bf16, and the reader of the output slower: the single-stream block at 3 x 4336 tokens 2840 -> 2873.)
-constexpr int64_t kReadPastCache = 136 << 20;
+// fp32 inputs of more than a third of the 256 MiB cache in front of HBM are read with the non-temporal hint: what the
+// operation in front read, the input that it wrote and this output do not fit there together. The hint favours programs
+// whose tensors go through HBM. us, ordinary -> non-temporal, rows of 3072, six inputs and outputs in turn:
+//                                             85.3 MiB       96 MiB         108 MiB        120 MiB          144 MiB
+//   layer norm alone                        37.2 -> 32.6   41.5 -> 36.7   45.5 -> 40.6    48.7 -> 43.8    57.7 -> 52.8
+//   behind an addition to other memory      79.7 -> 72.4   88.8 -> 83.2   99.8 -> 93.5   116.1 -> 104.9  136.9 -> 127.9
+//   the same and a sum that reads y         93.6 -> 89.4  104.6 -> 100.7 119.0 -> 112.2  135.9 -> 123.8  158.4 -> 147.3
+//   behind an addition in place             78.3 -> 73.7   87.3 -> 81.5   98.2 -> 91.5   110.9 -> 102.3  133.8 -> 122.9
+// It costs where one input and one output take turns alone, which do fit: the same call again 30.1 -> 34.8 at 96 MiB, 37.3 -> 41.5 at
+// 120, 45.3 -> 45.2 at 132; between two additions in place 87.5 -> 90.9, 108.1 -> 111.0, 124.0 -> 122.3. Smaller inputs mostly come
+// from that cache (50 MB 15.5 -> 17.0), and bf16 gains a third of what fp32 does. (Stores with the hint make the call faster
+// still, 10.3 us for 13.9 at [1, 4608, 3072] bf16, and the reader of the output slower: the single-stream block at 3 x 4336
+// tokens 2840 -> 2873.)
+constexpr int64_t kCacheBytes = 256 << 20;
 
 template <typename T>
 static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float eps, hipStream_t st) {
@@ -706,7 +708,7 @@ static int ln_mod_launch(const flux_layer_norm_args* a, int count, int n, float 
         return check_launch("flux_layer_norm_modulation");
     }
     if (used == 1) set.t[1] = set.t[0];
-    set.once = bytes > kReadPastCache;
+    set.once = 3 * bytes > kCacheBytes;
 #define CALL(G_, I_)                                                                                        \
     do {                                                                                                    \
         constexpr int RPB_ = kBlock / G_;                                                                    \

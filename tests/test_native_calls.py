@@ -450,3 +450,27 @@ def test_layer_norm_output_is_laid_out_like_its_input(monkeypatch):
     assert x.is_contiguous() and x.stride(0) == 320
     got, want = tk.layer_norm_modulation(x, mod, mod), launcher(monkeypatch, tk.layer_norm_modulation, x, mod, mod)
     assert torch.equal(got, want) and got.stride() == want.stride()
+
+
+@gpu
+def test_the_norms_node_under_hooks_and_a_compiled_backward():
+    """The native backward is a C++ node of the graph: hooks, edges and the engine's compiled mode treat it like any other,
+    with the same gradients."""
+    from torch._dynamo import compiled_autograd
+    g = seeded(12)
+    x0, s0, dy = randn(g, 40, 96, dtype=BF).to(DEV), randn(g, 96, dtype=BF).to(DEV), randn(g, 40, 96, dtype=BF).to(DEV)
+    got = []
+    for compiled in (False, True):
+        x, s = x0.clone().requires_grad_(True), s0.clone().requires_grad_(True)
+        y = tk.rms_norm(x * 2, s)
+        assert [e[0].name() for e in y.grad_fn.next_functions[:2]] == ["MulBackward0", "torch::autograd::AccumulateGrad"]
+        seen = []
+        y.grad_fn.register_hook(lambda grads_in, grads_out: seen.append((grads_in[0].shape, grads_in[1].shape, grads_out[0].shape)))
+        if compiled:
+            with compiled_autograd._enable(torch.compile(backend="eager")):
+                y.backward(dy)
+        else:
+            y.backward(dy)
+        assert seen == [((40, 96), (96,), (40, 96))]
+        got.append((x.grad, s.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*got))

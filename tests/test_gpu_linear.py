@@ -530,6 +530,20 @@ def test_line_of_weights_read_past_the_cache(M, K):
     assert torch.equal(tk.linear(x, w, None)[:, N - 100:], few) and torch.equal(tk.linear(x, w[:N], None)[:, N - 100:], few[:, :100])
 
 
+@pytest.mark.parametrize("M", [2, 3, 4, 5])
+def test_line_of_whole_weight_rows_in_flight(M):
+    """Weights of 80 MiB, up to which three and four activation rows have whole rows of 3072 in flight, and of a column more:
+    every column has the bits of a call with few of them."""
+    K, N = 3072, (80 << 20) // (2 * 3072)
+    x = randn(seeded(M), M, K, dtype=torch.bfloat16).to(DEV)
+    w = torch.randn(N + 1, K, generator=torch.Generator(device=DEV).manual_seed(M), device=DEV).bfloat16()
+    few = tk.linear(x, w[N - 100:], None)
+    ref = x.double() @ w[N - 100:].double().T
+    assert ((few.double() - ref).abs() <= ref.abs() * (2.0 ** -8 * 1.01) + (x.double().abs() @ w[N - 100:].double().abs().T) * (K * 2.0 ** -24)).all()
+    assert torch.equal(tk.linear(x, w, None)[:, N - 100:], few) and torch.equal(tk.linear(x, w[:N], None)[:, N - 100:], few[:, :100])
+    assert torch.equal(tk.linear(x, w, None, activation="GELU")[:, N - 100:], tk.linear(x, w[N - 100:], None, activation="GELU"))
+
+
 @pytest.mark.parametrize("tile_m,tile_n,M,N,K", [(256, 224, 916, 12384, 1024), (256, 224, 1178, 9944, 1032), (224, 256, 880, 12320, 1024), (224, 256, 872, 12376, 1032),
                                                  (224, 288, 1586, 8200, 1024), (224, 288, 1580, 8312, 1032)])
 def test_linear_wide_rectangles(tile_m, tile_n, M, N, K):

@@ -754,19 +754,25 @@ static void launch_gemv(const GemmSet& g, hipStream_t st) {
     // Vectors of a W row in flight: what a row has, up to a whole row of 3072; loops over longer rows take half of that from
     // three activation rows on, whose products need the registers (8 rows of 3072: 33 us, 49 with whole rows).
     // us with 6 -> 3 vectors, weights in the caches: 1 x 9216 x 1536 7.5 -> 5.6, 2 rows 9.0 -> 6.9, 3 rows 10.6 -> 8.6, 4 x 6144 x 1024
-    // 7.0 -> 6.2, 3 x 24576 x 4096 48.3 -> 41.5; 4 x 3072 x 12288 49.7 -> 50.6.
+    // 7.0 -> 6.2, 3 x 24576 x 4096 48.3 -> 41.5; 4 x 3072 x 12288 49.7 -> 50.6. Whole rows of 3072 beside three or four activation
+    // rows pay up to 80 MiB of weights: they take 221 and 246 registers, two waves a SIMD, where half rows take 87 and 101, five
+    // waves, which are worth more once a launch is many rounds of them. us with 6 -> 3, weights in the caches (from HBM): three rows 12288 columns 16.9 -> 17.1 (18.4 -> 18.6),
+    // 14000 19.0 -> 18.4 (20.7 -> 19.8), 36864 45.8 -> 40.7 (45.8 -> 41.8); four rows 14000 20.3 -> 20.2 (21.9 -> 21.9), 36864 48.0 -> 44.9
+    // (48.1 -> 46.3).
     constexpr int WHOLE = MM <= 4 ? 6 : 3, LOOP = MM <= 2 ? 6 : 3;
     // The hint gains where W comes from HBM (2 to 9 %), and beside it where the activation rows are read through the cache
     // that W then leaves to them. Where the same weights are read again at once, it gains at up to 3072 of K too, but
     // costs 3 to 14 % in the loops over longer rows: us with -> without, 1 x 3072 x 12288 18.3 -> 16.1 (from HBM 20.2 -> 21.4), 3 x 18432
     // x 6144 50 -> 42 (51 -> 53). So these go without it, but for two rows, where it costs up to 5 % and gains up to 9 from HBM
-    // (2 x 18432 x 6144 44.1 -> 42.1, 45.4 -> 50.1; at 3072 the one loss is 226 MB beside three rows, 42.2 us before these
-    // changes and 46.1 now where they are read again, 50.3 and 46.8 from HBM);
+    // (2 x 18432 x 6144 44.1 -> 42.1, 45.4 -> 50.1). At 3072 it loses where most of the cache is read again at once, 4 to 8 % of
+    // 226 MB beside three rows and more, which gain 5 to 9 % from HBM (3 x 36864 38.4 us before these changes, 40.7 now; 45.7 and 41.8);
     // and of the activation rows that do not fit the LDS, those whose weights are more than half of the 256 MiB cache (5 x
     // 18432 x 6144 109 -> 102; 8 x 3072 x 12288 keeps it, 87.8 against 96.4).
-    const bool once = p.K <= 3072 || (lds ? MM == 2 : static_cast<int64_t>(p.N) * p.K * 2 * g.n <= (int64_t{128} << 20));
+    const int64_t w_bytes = static_cast<int64_t>(p.N) * p.K * 2 * g.n;
+    const bool once = p.K <= 3072 || (lds ? MM == 2 : w_bytes <= (int64_t{128} << 20));
+    const bool whole = p.K == 512 * WHOLE && (MM <= 2 || MM > 4 || w_bytes <= (int64_t{80} << 20));
 #define CALL(LDS, U, EXACT, ONCE, BYTES) hipLaunchKernelGGL((gemv_small_m_kernel<MM, LDS, U, EXACT, ONCE>), grid, dim3(256), BYTES, st, g)
-    if (p.K == 512 * WHOLE) CALL(true, WHOLE, true, true, act_bytes);
+    if (whole) CALL(true, WHOLE, true, true, act_bytes);
     else if (p.K == 1536) CALL(true, 3, true, true, act_bytes);
     else if (p.K < 1536) CALL(true, 3, false, true, act_bytes);
     else if (lds && once) CALL(true, LOOP, false, true, act_bytes);

@@ -756,9 +756,9 @@ static void launch_gemv(const GemmSet& g, hipStream_t st) {
     // us with 6 -> 3 vectors, weights in the caches: 1 x 9216 x 1536 7.5 -> 5.6, 2 rows 9.0 -> 6.9, 3 rows 10.6 -> 8.6, 4 x 6144 x 1024
     // 7.0 -> 6.2, 3 x 24576 x 4096 48.3 -> 41.5; 4 x 3072 x 12288 49.7 -> 50.6. Whole rows of 3072 beside three or four activation
     // rows pay up to 80 MiB of weights: they take 221 and 246 registers, two waves a SIMD, where half rows take 87 and 101, five
-    // waves, which are worth more once a launch is many rounds of them. us with 6 -> 3, weights in the caches (from HBM): three rows 12288 columns 16.9 -> 17.1 (18.4 -> 18.6),
-    // 14000 19.0 -> 18.4 (20.7 -> 19.8), 36864 45.8 -> 40.7 (45.8 -> 41.8); four rows 14000 20.3 -> 20.2 (21.9 -> 21.9), 36864 48.0 -> 44.9
-    // (48.1 -> 46.3).
+    // waves, which are worth more once a launch is many rounds of them. us with 6 -> 3, weights in the caches (from HBM): three
+    // rows 12288 columns 16.9 -> 17.1 (18.4 -> 18.6), 14000 19.0 -> 18.4 (20.7 -> 19.8), 36864 45.8 -> 40.7 (45.8 -> 41.8); four rows
+    // 14000 20.3 -> 20.2 (21.9 -> 21.9), 36864 48.0 -> 44.9 (48.1 -> 46.3).
     constexpr int WHOLE = MM <= 4 ? 6 : 3, LOOP = MM <= 2 ? 6 : 3;
     // The hint gains where W comes from HBM (2 to 9 %), and beside it where the activation rows are read through the cache
     // that W then leaves to them. Where the same weights are read again at once, it gains at up to 3072 of K too, but

@@ -237,6 +237,86 @@ def test_which_calls_are_served_in_native_code(monkeypatch):
     assert nv.lib().flux_linear_workspace_bytes(nv.byref(a)) > 0
 
 
+def _served(monkeypatch, name, served, fn):
+    """fn() by the native call `name` (or, where served is False, by the launcher behind it) and by the launcher, whose bits it has to have."""
+    answers, real = [], getattr(nv.ops(), name)
+
+    class Spy:
+        def __getattr__(self, other):
+            return getattr(nv_ops, other) if other != name else lambda *a: answers.append(real(*a)) or answers[-1]
+
+    nv_ops = nv.ops()
+    with monkeypatch.context() as m:
+        m.setattr(nv, "ops", lambda: Spy())
+        got = fn()
+    assert answers and (answers[0] is not None) == served
+    want = launcher(monkeypatch, fn)
+    for a, b in zip(got, want):
+        assert (a is None and b is None) or (torch.equal(a, b) and a.stride() == b.stride())
+
+
+@gpu
+def test_calls_of_the_blocks_forms(monkeypatch):
+    """The general linear, two of them, the norm pair, the q/k/v preparation and attention to a given tensor: rows and batches in
+    every order that is read in place, the ones that are copied or refused, each against its launcher bit for bit."""
+    from triton_kernels.kernels.attention import attention_into
+    from triton_kernels.kernels.linear import linear_into, linear_pair_into
+    from triton_kernels.kernels.positional_embedding import qkv_prep
+    g = seeded(11)
+    t = lambda *s, std=1.0, dtype=BF: (randn(g, *s) * std).to(dtype).to(DEV)
+    K, N = 72, 136
+    w, b, wide = t(N, K, std=K ** -0.5), t(N), t(2, 40, 2 * K)
+    into = lambda **kw: lambda: (linear_into(**kw),)
+    for x, served in ((wide[..., :K].contiguous(), True), (wide[..., :K], True), (wide[0, :, :K], True), (wide[:, 3, :K], True), (wide[:, 4:20, :K], False), (wide[..., ::2], False),
+                      (wide[:1, :1, :K], True), (wide[..., :K].transpose(0, 1), False)):
+        M = x.numel() // K
+        _served(monkeypatch, "linear_into", served, into(x=x, w=w, b=b, activation="GELU", act_begin=64))
+        gate, resid = t(1, 1, 3 * N)[..., N:2 * N], t(M, N)
+        _served(monkeypatch, "linear_into", served, into(x=x, w=w, b=None, resid=resid, gate=gate))
+        _served(monkeypatch, "linear_into", served, into(x=x, w=t(N, 2 * K)[:, :K], b=b, resid=resid.view(1, M, N), gate=gate.contiguous()))
+
+        def split():
+            a, c = torch.zeros(M, 64, device=DEV, dtype=BF), torch.zeros(M, N, device=DEV, dtype=BF)
+            return linear_into(x, w, b, out=a, out2=c[:, 8:], split=64), c
+
+        _served(monkeypatch, "linear_into", served, split)
+    x, few = wide[0, :, :K], t(2, K)
+    for kw, served in ((dict(x=few, in_activation="SiLU"), True), (dict(x=x, shared_gpu=True), False), (dict(x=x, b=b.float()), False), (dict(x=x, w=w.t().contiguous().t()), False)):
+        _served(monkeypatch, "linear_into", served, into(**{"w": w, "b": b, **kw}))
+    gates = t(2, 1, 3 * N)[..., :N]
+    for first, second, served in ((wide[:, :30, :K], wide[:, 30:, :K], True), (wide[:1, :30, :K], wide[:1, 30:, :K], True), (few[:1], few[1:], True), (wide[..., ::2], x, False)):
+        calls = [dict(x=v, w=w, b=b) for v in (first, second)]
+        _served(monkeypatch, "linear_pair_into", served, lambda: linear_pair_into(*calls))
+        rows = [v.numel() // K for v in (first, second)]
+        if first.dim() == 3 and served:
+            gated = [dict(c, resid=t(n, N), gate=gates[:v.shape[0]]) for c, n, v in zip(calls, rows, (first, second))]
+            _served(monkeypatch, "linear_pair_into", True, lambda: linear_pair_into(*gated))
+    heads, L = 2, 300
+    hid = heads * 128
+    x, w1, b1, pe = t(2 * L, hid), t(40 * 256, hid, std=hid ** -0.5), t(40 * 256), t(1, 1, L, 64, 2, 2, dtype=F32)
+    scales = t(128).abs() + 0.5, t(128).abs() + 0.5
+    for table, served in ((pe, True), (t(2, 1, L, 64, 2, 2, dtype=F32), True)):
+        def fused():
+            q, k = (torch.zeros(2, heads, L, 128, device=DEV, dtype=BF) for _ in range(2))
+            qk = dict(q_out=q, k_out=k, q_scale=scales[0], k_scale=scales[1], pe=table, heads=heads, seq_len=L)
+            return linear_into(x, w1, b1, activation="GELU", act_begin=2 * hid, out=torch.zeros(2 * L, 40 * 256, device=DEV, dtype=BF), qk=qk), q, k
+        _served(monkeypatch, "linear_into", served, fused)
+    for dtype in (BF, F32):
+        img, txt = (t(2, n, 3 * hid, dtype=dtype).view(2, n, 3, heads, 128).permute(2, 0, 3, 1, 4) for n in (9, 4))
+        s, pe = t(128, dtype=dtype), t(1, 1, 13, 64, 2, 2, dtype=F32)
+        for args, kw, served in (((*img, *txt), dict(pe=pe, q_scale_img=s, k_scale_img=s, q_scale_txt=s, k_scale_txt=s), True), ((*img, *txt), {}, True), ((img[0], img[1], None), dict(pe=pe[:, :, :9].double()), False),
+                                 ((img[0], img[1], None), dict(pe=pe[:, :, :9].contiguous(), q_scale_img=s, k_scale_img=s), True), ((None, img[1], img[2]), {}, False), ((*img, txt[0], txt[1], txt[2].transpose(0, 1).contiguous().transpose(0, 1)), {}, True),
+                                 ((*(v[..., ::2] for v in img),), {}, False)):
+            _served(monkeypatch, "qkv_prep", served, lambda: qkv_prep(*args, **kw))
+        mod = t(2, 1, 6 * 256, dtype=dtype).chunk(6, -1)
+        a, c = t(2, 7, 256, dtype=dtype), t(2, 3, 256, dtype=dtype)
+        for first, second, served in (((a, mod[0], mod[1]), (c, mod[3], mod[4]), True), ((a[:, :5], mod[0], mod[1]), (c, mod[3], mod[4]), False), ((a, mod[0].float(), mod[1]), (c, mod[3], mod[4]), dtype == F32)):
+            _served(monkeypatch, "layer_norm_modulation_pair", served, lambda: norm_mod.layer_norm_modulation_pair(first, second))
+    qkv = t(2, 150, 3, heads, 128).permute(2, 0, 3, 1, 4)
+    for kw, q, served in (({}, qkv[0], True), (dict(sm_scale=0.3), qkv[0].contiguous(), True), ({}, qkv[0].transpose(2, 3).contiguous().transpose(2, 3), False)):
+        _served(monkeypatch, "attention", served, lambda: (attention_into(q, qkv[1], qkv[2], torch.zeros(2, 150, heads, 136, device=DEV, dtype=BF).permute(0, 2, 1, 3)[..., :128], **kw),))
+
+
 @gpu
 def test_refusals_stay_what_they_were(monkeypatch):
     x, w = torch.ones(4, 64, device=DEV, dtype=BF), torch.ones(32, 64, device=DEV, dtype=BF)

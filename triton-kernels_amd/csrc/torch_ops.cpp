@@ -9,7 +9,9 @@
 // turns with runs at half its speed (41 and 43 us, 129 for a step whose kernels take 30). A node of the
 // engine's own kind leaves the interpreter on one core. us a call, before -> now: q/k norm module at 256 tokens 25.5 -> 10.3,
 // training step of the norm at [4, 24, 1024, 128] 107 to 129 -> 57, rotation of short sequences 18.7 -> 6.9, linear at 512 x 3072
-// x 3072 15.8 -> 15.1 (the GPU's own time).
+// x 3072 15.8 -> 15.1 (the GPU's own time). The calls that the fused blocks are made of are here as well: seven of a single-stream
+// block took the host 126 to 132 us a pass (the GPU 131 at 320 tokens), now 67 to 72; ten of a double-stream block 329, now 132; first
+// passes on new weights at 320 tokens 281 -> 241, at 1024 + 256 579 -> 479.
 #include <torch/csrc/python_headers.h>
 #include <ATen/ATen.h>
 #include <torch/csrc/Exceptions.h>
@@ -22,6 +24,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 
@@ -226,17 +229,26 @@ PyObject* py_rms_norm_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 // ---- layer norm + modulation -------------------------------------------------------------------
 
+bool layer_norm_args_ok(const Tensor& x, const Tensor& scale, const Tensor& shift) {
+    if (x.dim() < 2 || type_code(x) < 0 || !same_kind(x, scale) || !same_kind(x, shift) || !x.is_contiguous()) return false;
+    const int64_t batch = x.size(0), n = x.size(-1);
+    auto modulates = [&](const Tensor& m) {
+        return m.dim() >= 2 && m.size(0) == batch && m.size(-1) == n && m.numel() == batch * n && m.stride(-1) == 1 && (batch == 1 || (m.stride(0) == scale.stride(0) && m.stride(0) >= n));
+    };
+    return n <= kMaxRow && modulates(scale) && modulates(shift);
+}
+
+flux_layer_norm_args layer_norm_args(const Tensor& x, const Tensor& scale, const Tensor& shift, const Tensor& y) {
+    const int64_t batch = x.size(0), n = x.size(-1);
+    return {x.data_ptr(), scale.data_ptr(), shift.data_ptr(), y.data_ptr(), batch, x.numel() / n / batch, batch > 1 ? scale.stride(0) : n};
+}
+
 // layer_norm_modulation(x, scale, shift, eps)
 PyObject* py_layer_norm_modulation(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(nargs == 4, "layer_norm_modulation takes 4 arguments");
     const Tensor *x = tensor_of(args[0]), *scale = tensor_of(args[1]), *shift = tensor_of(args[2]);
-    if (!x || !scale || !shift || !quiet() || x->dim() < 2 || type_code(*x) < 0 || !same_kind(*x, *scale) || !same_kind(*x, *shift) || !x->is_contiguous()) Py_RETURN_NONE;
-    const int64_t batch = x->size(0), n = x->size(-1), rows = x->numel() / n;
-    auto modulates = [&](const Tensor& m) {
-        return m.dim() >= 2 && m.size(0) == batch && m.size(-1) == n && m.numel() == batch * n && m.stride(-1) == 1 && (batch == 1 || (m.stride(0) == scale->stride(0) && m.stride(0) >= n));
-    };
-    if (n > kMaxRow || !modulates(*scale) || !modulates(*shift)) Py_RETURN_NONE;
+    if (!x || !scale || !shift || !quiet() || !layer_norm_args_ok(*x, *scale, *shift)) Py_RETURN_NONE;
     double eps;
     if (!number(args[3], eps)) Py_RETURN_NONE;
     Tensor y;
@@ -246,8 +258,8 @@ PyObject* py_layer_norm_modulation(PyObject*, PyObject* const* args, Py_ssize_t 
         const WithoutInterpreter free;
         const c10::DeviceGuard guard(xa.device());
         y = at::empty_like(xa);
-        rc = flux_layer_norm_modulation(xa.data_ptr(), sc.data_ptr(), sh.data_ptr(), y.data_ptr(), batch, rows / batch, static_cast<int32_t>(n),
-                                        batch > 1 ? sc.stride(0) : n, type_code(xa), static_cast<float>(eps), stream_of(xa));
+        const flux_layer_norm_args a = layer_norm_args(xa, sc, sh, y);
+        rc = flux_layer_norm_modulation(a.x, a.scale, a.shift, a.y, a.batch, a.seq, static_cast<int32_t>(xa.size(-1)), a.mod_batch_stride, type_code(xa), static_cast<float>(eps), stream_of(xa));
     }
     if (rc < 0) Py_RETURN_NONE;   // (a refusal: its kind of error is the launcher's)
     check(rc, "flux_layer_norm_modulation");
@@ -255,9 +267,49 @@ PyObject* py_layer_norm_modulation(PyObject*, PyObject* const* args, Py_ssize_t 
     END_HANDLE_TH_ERRORS
 }
 
+// layer_norm_modulation_pair(x0, scale0, shift0, x1, scale1, shift1, eps)
+PyObject* py_layer_norm_modulation_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(nargs == 7, "layer_norm_modulation_pair takes 7 arguments");
+    const Tensor* t[6];
+    for (int i = 0; i < 6; ++i) {
+        t[i] = tensor_of(args[i]);
+        if (!t[i]) Py_RETURN_NONE;
+    }
+    if (!quiet() || !layer_norm_args_ok(*t[0], *t[1], *t[2]) || !layer_norm_args_ok(*t[3], *t[4], *t[5]) || !same_kind(*t[0], *t[3]) || t[0]->size(-1) != t[3]->size(-1)) Py_RETURN_NONE;
+    double eps;
+    if (!number(args[6], eps)) Py_RETURN_NONE;
+    Tensor y0, y1;
+    int rc;
+    {
+        const Tensor x0 = *t[0], s0 = *t[1], h0 = *t[2], x1 = *t[3], s1 = *t[4], h1 = *t[5];
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(x0.device());
+        y0 = at::empty_like(x0);
+        y1 = at::empty_like(x1);
+        const flux_layer_norm_args a0 = layer_norm_args(x0, s0, h0, y0), a1 = layer_norm_args(x1, s1, h1, y1);
+        rc = flux_layer_norm_modulation_pair(&a0, &a1, static_cast<int32_t>(x0.size(-1)), type_code(x0), static_cast<float>(eps), stream_of(x0));
+    }
+    if (rc < 0) Py_RETURN_NONE;
+    check(rc, "flux_layer_norm_modulation_pair");
+    return two(y0, y1);
+    END_HANDLE_TH_ERRORS
+}
+
 // ---- rotation ----------------------------------------------------------------------------------
 
 flux_src4 source(const Tensor& t) { return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)}; }
+
+// A table for all batch elements (stride 0) or one for each, as it lies in memory.
+bool rotation_table(const Tensor& pe, int64_t B, int64_t L, int64_t D, int64_t& batch_stride) {
+    const int64_t lead = pe.dim() - 4;
+    if (D % 2 != 0 || pe.scalar_type() != at::kFloat || !pe.is_contiguous() || lead < 0 || pe.size(lead) != L || pe.size(lead + 1) != D / 2 || pe.size(lead + 2) != 2 ||
+        pe.size(lead + 3) != 2)
+        return false;
+    const int64_t tables = pe.numel() / (L * D * 2);
+    batch_stride = tables == 1 ? 0 : L * D * 2;
+    return tables == 1 || (lead == 2 && pe.size(0) == B && pe.size(1) == 1);
+}
 
 // apply_rope(q, k, table)
 PyObject* py_apply_rope(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -267,12 +319,9 @@ PyObject* py_apply_rope(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!q || !k || !pe || !quiet() || q->dim() != 4 || q->sizes() != k->sizes() || type_code(*q) < 0 || !same_kind(*q, *k) || q->device() != pe->device() ||
         q->stride(3) != 1 || k->stride(3) != 1 || !vector_rows(*q) || !vector_rows(*k))
         Py_RETURN_NONE;
-    const int64_t B = q->size(0), H = q->size(1), L = q->size(2), D = q->size(3), lead = pe->dim() - 4;
-    if (D % 2 != 0 || pe->scalar_type() != at::kFloat || !pe->is_contiguous() || lead < 0 || pe->size(lead) != L || pe->size(lead + 1) != D / 2 || pe->size(lead + 2) != 2 ||
-        pe->size(lead + 3) != 2)
-        Py_RETURN_NONE;
-    const int64_t tables = pe->numel() / (L * D * 2);
-    if (tables != 1 && !(lead == 2 && pe->size(0) == B && pe->size(1) == 1)) Py_RETURN_NONE;
+    const int64_t B = q->size(0), H = q->size(1), L = q->size(2), D = q->size(3);
+    int64_t table_stride;
+    if (!rotation_table(*pe, B, L, D, table_stride)) Py_RETURN_NONE;
     Tensor yq, yk;
     int rc;
     {
@@ -287,7 +336,7 @@ PyObject* py_apply_rope(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         a.q_out = yq.data_ptr();
         a.k_out = yk.data_ptr();
         a.pe = static_cast<const float*>(table.data_ptr());
-        a.pe_batch_stride = tables == 1 ? 0 : L * D * 2;
+        a.pe_batch_stride = table_stride;
         a.B = B; a.H = H; a.Li = L; a.D = static_cast<int32_t>(D);
         a.dtype = a.scale_dtype = type_code(qa);
         a.eps = 1e-6f;
@@ -296,6 +345,85 @@ PyObject* py_apply_rope(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (rc < 0) Py_RETURN_NONE;
     check(rc, "flux_qkv_prep");
     return two(yq, yk);
+    END_HANDLE_TH_ERRORS
+}
+
+// A tensor or None.
+bool optional_tensor(PyObject* o, const Tensor*& t) {
+    t = o == Py_None ? nullptr : tensor_of(o);
+    return t != nullptr || o == Py_None;
+}
+
+PyObject* wrap_or_none(const Tensor& t) {
+    if (t.defined()) return THPVariable_Wrap(t);
+    Py_RETURN_NONE;
+}
+
+// qkv_prep(q_img, k_img, v_img, q_txt, k_txt, v_txt, table, q_scale_img, k_scale_img, q_scale_txt, k_scale_txt, eps): (q, k, v), where
+// q and k are there, v and the three of the text may be None
+PyObject* py_qkv_prep(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(nargs == 12, "qkv_prep takes 12 arguments");
+    const Tensor* t[11];
+    for (int i = 0; i < 11; ++i)
+        if (!optional_tensor(args[i], t[i])) Py_RETURN_NONE;
+    const Tensor *q = t[0], *pe = t[6];
+    if (!q || !t[1] || !quiet() || q->dim() != 4 || type_code(*q) < 0 || (t[3] && t[3]->dim() != 4)) Py_RETURN_NONE;
+    const int64_t B = q->size(0), H = q->size(1), Li = q->size(2), D = q->size(3), Lt = t[3] ? t[3]->size(2) : 0;
+    for (int i = 0; i < 6; ++i) {
+        if (!t[i]) {
+            if (i < 2 || (Lt > 0 && (i < 5 || t[2]))) Py_RETURN_NONE;   // (what one of the sources has, the others have)
+            continue;
+        }
+        if (i >= 3 && (Lt == 0 || !t[i - 3])) Py_RETURN_NONE;
+        if (!same_kind(*q, *t[i]) || t[i]->sizes() != at::IntArrayRef({B, H, i < 3 ? Li : Lt, D}) || t[i]->stride(3) != 1 || !vector_rows(*t[i])) Py_RETURN_NONE;
+    }
+    int64_t table_stride = 0;
+    if (pe && (pe->device() != q->device() || !rotation_table(*pe, B, Lt + Li, D, table_stride))) Py_RETURN_NONE;
+    int scale_type = type_code(*q);
+    bool first = true;
+    for (int i = 7; i < 11; ++i) {
+        if (!t[i]) continue;
+        const int type = type_code(*t[i]);
+        if (type < 0 || (!first && type != scale_type) || (type != type_code(*q) && type_code(*q) != FLUX_BF16) || t[i]->device() != q->device() || t[i]->dim() != 1 ||
+            t[i]->numel() != D || t[i]->stride(0) != 1)
+            Py_RETURN_NONE;
+        scale_type = type;
+        first = false;
+    }
+    double eps;
+    if (!number(args[11], eps)) Py_RETURN_NONE;
+    Tensor out[3];
+    int rc;
+    {
+        Tensor kept[11];   // (the caller's objects are another thread's to drop from here on)
+        for (int i = 0; i < 11; ++i)
+            if (t[i]) kept[i] = *t[i];
+        const WithoutInterpreter free;
+        const c10::DeviceGuard guard(kept[0].device());
+        for (int i = 0; i < 3; ++i)
+            if (kept[i].defined()) out[i] = empty({B, H, Lt + Li, D}, kept[0].scalar_type(), kept[0]);
+        auto at = [&](int i) { return kept[i].defined() ? source(kept[i]) : flux_src4{}; };
+        auto ptr = [](const Tensor& x) -> void* { return x.defined() ? x.data_ptr() : nullptr; };
+        flux_qkv_prep_args a = {};
+        a.q_img = at(0); a.k_img = at(1); a.v_img = at(2);
+        a.q_txt = at(3); a.k_txt = at(4); a.v_txt = at(5);
+        a.q_out = ptr(out[0]); a.k_out = ptr(out[1]); a.v_out = ptr(out[2]);
+        a.pe = static_cast<const float*>(ptr(kept[6]));
+        a.pe_batch_stride = table_stride;
+        a.q_scale_img = ptr(kept[7]); a.k_scale_img = ptr(kept[8]); a.q_scale_txt = ptr(kept[9]); a.k_scale_txt = ptr(kept[10]);
+        a.B = B; a.H = H; a.Lt = Lt; a.Li = Li; a.D = static_cast<int32_t>(D);
+        a.dtype = type_code(kept[0]);
+        a.scale_dtype = scale_type;
+        a.eps = static_cast<float>(eps);
+        rc = flux_qkv_prep(&a, stream_of(kept[0]));
+    }
+    if (rc < 0) Py_RETURN_NONE;
+    check(rc, "flux_qkv_prep");
+    PyObject* const r = PyTuple_New(3);
+    if (!r) return nullptr;
+    for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(r, i, wrap_or_none(out[i]));
+    return r;
     END_HANDLE_TH_ERRORS
 }
 
@@ -340,15 +468,203 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// One product in its general form, and what has to live until it is launched.
+struct Product {
+    flux_linear_args a = {};
+    flux_linear_qk_fusion qk = {};
+    int64_t a_rows = 0, a_batch_stride = 0;
+    Tensor out;
+    c10::SmallVector<Tensor, 12> keep;
+    bool out_given = false;
+};
+
+bool whole_number(PyObject* o, int64_t& value) {
+    value = PyLong_CheckExact(o) ? PyLong_AsLongLong(o) : -1;
+    if (PyLong_CheckExact(o) && !(value == -1 && PyErr_Occurred())) return true;
+    PyErr_Clear();
+    return false;
+}
+
+// x as [rows, n] without copying it.
+bool flat_rows(const Tensor& x, int64_t n, int64_t& rows, int64_t& ld) {
+    if (x.dim() < 1 || x.size(-1) != n || (n > 1 && x.stride(-1) != 1)) return false;
+    rows = 1;
+    ld = n;
+    for (int64_t d = x.dim() - 2; d >= 0; --d) {
+        if (x.size(d) == 1) continue;
+        if (rows == 1) ld = x.stride(d);
+        else if (x.stride(d) != ld * rows) return false;
+        rows *= x.size(d);
+    }
+    return ld >= n;
+}
+
+bool is_bf16(const Tensor& t, const Tensor& beside) { return t.scalar_type() == at::kBFloat16 && t.device() == beside.device(); }
+
+// A matrix of at least `cols` columns to write to.
+bool destination(const Tensor& t, const Tensor& x, int64_t rows, int64_t cols) {
+    return is_bf16(t, x) && t.dim() == 2 && t.size(0) == rows && t.stride(1) == 1 && t.size(1) >= cols;
+}
+
+// call: (x, w, b, activation, act_begin, out, out2, split, resid, gate, qk, in_activation) as linear_into has them, absent ones None;
+// qk: (q_out, k_out, q_scale, k_scale, table, heads, seq_len, pos0, eps) or None. slices: rows of x may lie in batches that are not evenly strided.
+bool read_product(PyObject* call, Product& p, bool slices) {
+    if (!PyTuple_CheckExact(call) || PyTuple_GET_SIZE(call) != 12) return false;
+    auto item = [&](int i) { return PyTuple_GET_ITEM(call, i); };
+    const Tensor *x = tensor_of(item(0)), *w = tensor_of(item(1)), *b, *out, *out2, *resid, *gate;
+    int64_t act, act_begin, in_act, split = -1;
+    if (!x || !w || !optional_tensor(item(2), b) || !optional_tensor(item(5), out) || !optional_tensor(item(6), out2) || !optional_tensor(item(8), resid) ||
+        !optional_tensor(item(9), gate) || !whole_number(item(3), act) || !whole_number(item(4), act_begin) || !whole_number(item(11), in_act) ||
+        (item(7) != Py_None && (!whole_number(item(7), split) || split < 0)))
+        return false;
+    if (act < 0 || in_act < 0 || x->scalar_type() != at::kBFloat16 || !is_bf16(*w, *x) || w->dim() != 2 || x->size(-1) != w->size(1) || (w->size(1) > 1 && w->stride(1) != 1)) return false;
+    const int64_t N = w->size(0), K = w->size(1);
+    if (N > 1 && w->stride(0) < K) return false;
+    int64_t M, ld;
+    if (slices && x->dim() == 3 && x->size(0) > 1 && x->stride(0) != x->size(1) * x->stride(1)) {
+        const int64_t B = x->size(0), L = x->size(1);
+        if (!(B * L > 8 && x->stride(2) == 1 && x->stride(1) >= K && x->stride(0) % 8 == 0 && x->stride(0) >= L * x->stride(1) && x->stride(1) % 8 == 0 && K % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(x->data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w->data_ptr()) % 16 == 0 && w->is_contiguous() && B * x->stride(0) * 2 < (int64_t{1} << 31)))
+            return false;
+        M = B * L;
+        ld = x->stride(1);
+        p.a_rows = L;
+        p.a_batch_stride = x->stride(0);
+    } else if (!flat_rows(*x, K, M, ld)) {
+        return false;
+    }
+    if (in_act != FLUX_ACT_NONE && M > 8) return false;
+    if (b && (!is_bf16(*b, *x) || b->dim() != 1 || b->numel() != N || b->stride(0) != 1)) return false;
+    const bool cut = split >= 0 && split < N;
+    if (out && !destination(*out, *x, M, cut ? split : N)) return false;
+    if (cut && (!out2 || !destination(*out2, *x, M, N - split))) return false;
+    if ((gate == nullptr) != (resid == nullptr)) return false;
+    flux_linear_args& a = p.a;
+    if (gate) {
+        int64_t rows, ldr;
+        if (!is_bf16(*gate, *x) || !is_bf16(*resid, *x) || !flat_rows(*resid, N, rows, ldr) || rows != M) return false;
+        const int64_t nb = gate->is_contiguous() ? gate->numel() / N : gate->size(0);
+        if (gate->dim() < 1 || gate->size(-1) != N || gate->stride(-1) != 1 || gate->numel() != nb * N || nb == 0 || M % nb != 0) return false;
+        a.resid = resid->data_ptr();
+        a.ldresid = ldr;
+        a.gate = gate->data_ptr();
+        a.gate_batch_stride = nb > 1 && !gate->is_contiguous() ? gate->stride(0) : N;
+        a.rows_per_batch = M / nb;
+        p.keep.push_back(*gate);
+        p.keep.push_back(*resid);
+    }
+    if (item(10) != Py_None) {
+        PyObject* const q = item(10);
+        if (!PyTuple_CheckExact(q) || PyTuple_GET_SIZE(q) != 9) return false;
+        const Tensor* t[5];
+        for (int i = 0; i < 5; ++i)
+            if (!(t[i] = tensor_of(PyTuple_GET_ITEM(q, i))) || t[i]->device() != x->device() || !t[i]->is_contiguous()) return false;
+        double eps;
+        flux_linear_qk_fusion& f = p.qk;
+        if (!whole_number(PyTuple_GET_ITEM(q, 5), f.heads) || !whole_number(PyTuple_GET_ITEM(q, 6), f.seq_len) || !whole_number(PyTuple_GET_ITEM(q, 7), f.pos0) ||
+            !number(PyTuple_GET_ITEM(q, 8), eps))
+            return false;
+        if (t[0]->dim() != 4 || t[0]->sizes() != t[1]->sizes() || !is_bf16(*t[0], *x) || !is_bf16(*t[1], *x) || f.seq_len <= 0 || M % f.seq_len != 0 || t[0]->size(0) != M / f.seq_len ||
+            t[0]->size(1) != f.heads || t[0]->size(3) != 128)
+            return false;
+        f.out_len = t[0]->size(2);
+        const int64_t table = f.out_len * 256;
+        if (t[4]->scalar_type() != at::kFloat || t[4]->numel() % table != 0) return false;
+        for (int i = 2; i < 4; ++i)
+            if (!is_bf16(*t[i], *x) || t[i]->numel() != 128) return false;
+        f.q_out = t[0]->data_ptr(); f.k_out = t[1]->data_ptr();
+        f.q_scale = t[2]->data_ptr(); f.k_scale = t[3]->data_ptr();
+        f.pe = static_cast<const float*>(t[4]->data_ptr());
+        f.pe_batch_stride = t[4]->numel() > table ? table : 0;
+        f.eps = static_cast<float>(eps);
+        for (const Tensor* k : t) p.keep.push_back(*k);
+        a.qk = &f;
+    }
+    a.A = x->data_ptr(); a.W = w->data_ptr(); a.bias = b ? b->data_ptr() : nullptr;
+    a.M = M; a.N = N; a.K = K;
+    a.lda = M > 1 ? ld : K;
+    a.ldw = N > 1 ? w->stride(0) : K;
+    a.split_n = cut ? split : N;
+    if (cut) { a.Y2 = out2->data_ptr(); a.ldy2 = out2->stride(0); p.keep.push_back(*out2); }
+    a.act = static_cast<int32_t>(act);
+    a.act_begin = act_begin;
+    a.in_act = static_cast<int32_t>(in_act);
+    p.keep.push_back(*x);
+    p.keep.push_back(*w);
+    if (b) p.keep.push_back(*b);
+    if (out) { p.out = *out; p.out_given = true; }
+    return true;
+}
+
+// The output, where the caller gave none, and its place in the call.
+void place_output(Product& p, const Tensor& beside) {
+    if (!p.out_given) p.out = empty({p.a.M, p.a.split_n}, at::kBFloat16, beside);
+    p.a.Y = p.out.data_ptr();
+    p.a.ldy = p.out.stride(0);
+}
+
+// (K is cut over workgroups beyond 3072 of it only, and up to 256 tiles of 192 x 192)
+bool may_cut_k(int64_t rows, int64_t N, int64_t K) { return K > 3072 && rows > 8 && rows * N <= (int64_t{1} << 24); }
+
+// linear_into(call)
+PyObject* py_linear_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(nargs == 1, "linear_into takes 1 argument");
+    Product p;
+    if (!quiet() || !read_product(args[0], p, false)) Py_RETURN_NONE;
+    int rc;
+    {
+        const WithoutInterpreter free;
+        const Tensor& beside = p.keep.back();
+        const c10::DeviceGuard guard(beside.device());
+        place_output(p, beside);
+        const int64_t need = may_cut_k(p.a.M, p.a.N, p.a.K) ? flux_linear_workspace_bytes(&p.a) : 0;
+        const Tensor ws = need ? empty({need}, at::kByte, beside) : Tensor();
+        rc = flux_linear_bf16_ws(&p.a, need ? ws.data_ptr() : nullptr, need, stream_of(beside));
+    }
+    if (rc < 0) Py_RETURN_NONE;
+    check(rc, "flux_linear_bf16");
+    return THPVariable_Wrap(p.out);
+    END_HANDLE_TH_ERRORS
+}
+
+// linear_pair_into(call, call)
+PyObject* py_linear_pair_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(nargs == 2, "linear_pair_into takes 2 arguments");
+    Product p[2];
+    if (!quiet() || !read_product(args[0], p[0], true) || !read_product(args[1], p[1], true) || p[0].keep.back().device() != p[1].keep.back().device()) Py_RETURN_NONE;
+    int rc;
+    {
+        const WithoutInterpreter free;
+        const Tensor& beside = p[0].keep.back();
+        const c10::DeviceGuard guard(beside.device());
+        flux_linear_pair_args a = {};
+        for (int i = 0; i < 2; ++i) {
+            place_output(p[i], beside);
+            a.product[i] = p[i].a;
+            a.a_rows[i] = p[i].a_rows;
+            a.a_batch_stride[i] = p[i].a_batch_stride;
+        }
+        const int64_t need = may_cut_k(p[0].a.M + p[1].a.M, std::min(p[0].a.N, p[1].a.N), std::max(p[0].a.K, p[1].a.K)) ? flux_linear_pair_workspace_bytes(&a) : 0;
+        const Tensor ws = need ? empty({need}, at::kByte, beside) : Tensor();
+        rc = flux_linear_bf16_pair(&a, need ? ws.data_ptr() : nullptr, need, stream_of(beside));
+    }
+    if (rc < 0) Py_RETURN_NONE;
+    check(rc, "flux_linear_bf16_pair");
+    return two(p[0].out, p[1].out);
+    END_HANDLE_TH_ERRORS
+}
+
 // ---- attention ---------------------------------------------------------------------------------
 
-// attention(q, k, v, scale or None): all of [B, H, L, D]
+// attention(q, k, v, scale or None): all of [B, H, L, D]; attention(q, k, v, scale or None, out): to a tensor that is there
 PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(nargs == 4, "attention takes 4 arguments");
-    const Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]);
-    if (!q || !k || !v || !quiet() || q->dim() != 4 || q->sizes() != k->sizes() || q->sizes() != v->sizes() || q->scalar_type() != at::kBFloat16 || !same_kind(*q, *k) ||
-        !same_kind(*q, *v))
+    TORCH_CHECK(nargs == 4 || nargs == 5, "attention takes 4 or 5 arguments");
+    const Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]), *out = nargs == 5 ? tensor_of(args[4]) : nullptr;
+    if (!q || !k || !v || (nargs == 5 && !out) || !quiet() || q->dim() != 4 || q->sizes() != k->sizes() || q->sizes() != v->sizes() || q->scalar_type() != at::kBFloat16 ||
+        !same_kind(*q, *k) || !same_kind(*q, *v) || (out && (out->sizes() != q->sizes() || !same_kind(*q, *out) || out->stride(3) != 1)))
         Py_RETURN_NONE;
     for (const Tensor* t : {q, k, v})
         if (t->stride(3) != 1 || !vector_rows(*t)) Py_RETURN_NONE;
@@ -358,9 +674,10 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     int rc;
     {
         const Tensor qa = *q, ka = *k, va = *v;
+        if (out) o = *out;
         const WithoutInterpreter free;
         const c10::DeviceGuard guard(qa.device());
-        o = empty(qa.sizes(), at::kBFloat16, qa);
+        if (!out) o = empty(qa.sizes(), at::kBFloat16, qa);
         flux_attn_args a = {};
         a.q = source(qa); a.k = source(ka); a.v = source(va);
         a.o = o.data_ptr();
@@ -378,8 +695,8 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 #define FLUX_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_##name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FLUX_METHOD(rms_norm), FLUX_METHOD(rms_norm_pair), FLUX_METHOD(layer_norm_modulation), FLUX_METHOD(apply_rope), FLUX_METHOD(linear),
-                         FLUX_METHOD(attention), {nullptr, nullptr, 0, nullptr}};
+PyMethodDef methods[] = {FLUX_METHOD(rms_norm), FLUX_METHOD(rms_norm_pair), FLUX_METHOD(layer_norm_modulation), FLUX_METHOD(layer_norm_modulation_pair), FLUX_METHOD(apply_rope),
+                         FLUX_METHOD(qkv_prep), FLUX_METHOD(linear), FLUX_METHOD(linear_into), FLUX_METHOD(linear_pair_into), FLUX_METHOD(attention), {nullptr, nullptr, 0, nullptr}};
 #undef FLUX_METHOD
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_ops", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -27,6 +27,10 @@ def _may_cut_keys(BH: int, L: int) -> bool:
 def attention_into(q: Tensor, k: Tensor, v: Tensor, out: Tensor, sm_scale: float | None = None,
                    lse: Tensor | None = None) -> Tensor:
     """q,k,v,out are [B,H,L,D] views (bf16, last dim contiguous, any other strides)."""
+    if lse is None and not is_compiling():
+        o = nv.ops().attention(q, k, v, sm_scale, out)
+        if o is not None:
+            return o
     D = q.shape[-1]
     assert D == k.shape[-1] == v.shape[-1]
     assert D in {16, 32, 64, 128, 256}

@@ -49,6 +49,16 @@ def _may_cut_k(rows: int, N: int, K: int) -> bool:
     return K > 3072 and rows > 8 and rows * N <= 1 << 24
 
 
+_IN_ACTIVATIONS = {"": nv.ACT_NONE, "SiLU": nv.ACT_SILU}
+
+
+def _positional(x, w, b, *, activation="", act_begin=0, out=None, out2=None, split=None, resid=None, gate=None, qk=None, in_activation="", shared_gpu=False):
+    """A linear_into call as the native calls take it."""
+    if qk is not None:
+        qk = (qk["q_out"], qk["k_out"], qk["q_scale"], qk["k_scale"], qk["pe"], qk["heads"], qk["seq_len"], qk.get("pos0", 0), qk.get("eps", 1e-6))
+    return (x, w, b, -1 if shared_gpu else _ACTIVATIONS.get(activation, -1), act_begin, out, out2, split, resid, gate, qk, _IN_ACTIVATIONS.get(in_activation, -1))
+
+
 def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "", act_begin: int = 0,
                 out: Tensor | None = None, out2: Tensor | None = None, split: int | None = None,
                 resid: Tensor | None = None, gate: Tensor | None = None, qk: dict | None = None,
@@ -68,6 +78,11 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
             that leaves CUs free in its last round instead of one that fills the GPU exactly (same
             result, only the schedule differs); for callers that run streams side by side
     """
+    if launch_hook is None and not is_compiling():
+        y = nv.ops().linear_into(_positional(x, w, b, activation=activation, act_begin=act_begin, out=out, out2=out2, split=split, resid=resid, gate=gate, qk=qk,
+                                             in_activation=in_activation, shared_gpu=shared_gpu))
+        if y is not None:
+            return y
     a = nv.LinearArgs()
     out, dev, M, N, K, _keep = _fill_args(a, x, w, b, activation, act_begin, out, out2, split, resid, gate, qk, in_activation, shared_gpu)
     with nv.on_device(dev):
@@ -85,6 +100,10 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
     """Two linear_into calls (each the keyword arguments of one, `x`, `w` and `b` among them) in one library
     call: products of the same N, K and form of epilogue share a launch. An x of [B, L, K] may be a slice of
     a longer sequence, whose batch elements are not evenly strided rows."""
+    if launch_hook is None and not is_compiling():
+        both = nv.ops().linear_pair_into(_positional(**first), _positional(**second))
+        if both is not None:
+            return both
     args = nv.LinearPairArgs()
     outs, keep, sizes, notes = [], [], [], []
     for i, call in enumerate((first, second)):
@@ -180,7 +199,7 @@ def _fill_args(a: "nv.LinearArgs", x: Tensor, w: Tensor, b: Tensor | None, activ
         a.gate, a.gate_batch_stride, a.rows_per_batch = g2.data_ptr(), (g2.stride(0) if nb > 1 else N), M // nb
     a.act, a.act_begin = act, act_begin
     a.flags = nv.LINEAR_SHARED_GPU if shared_gpu else 0
-    a.in_act = {"": nv.ACT_NONE, "SiLU": nv.ACT_SILU}[in_activation]
+    a.in_act = _IN_ACTIVATIONS[in_activation]
     assert a.in_act == nv.ACT_NONE or M <= 8, "the input activation is fused for at most 8 rows"
     if qk is not None:
         f = nv.LinearQKFusion()

@@ -49,6 +49,10 @@ def qkv_prep(q_img: Tensor | None, k_img: Tensor | None, v_img: Tensor | None,
     """One streaming pass: concat(txt, img) along the sequence, optional per-head RMS norm of q/k,
     optional RoPE of q/k, v copied. Returns (q, k, v) contiguous [B,H,Lt+Li,D]; entries whose inputs
     were None come back as None. All sources are [B,H,L*,D] views (any batch/head/row strides)."""
+    if not is_compiling():
+        outs = nv.ops().qkv_prep(q_img, k_img, v_img, q_txt, k_txt, v_txt, pe, q_scale_img, k_scale_img, q_scale_txt, k_scale_txt, eps)
+        if outs is not None:
+            return outs
     ref = next(t for t in (q_img, k_img, v_img) if t is not None)
     B, H, Li, D = ref.shape
     txt_ref = next((t for t in (q_txt, k_txt, v_txt) if t is not None), None)

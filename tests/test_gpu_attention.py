@@ -361,3 +361,27 @@ def test_attention_keys_in_parts_replayed_from_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(o, eager), i
+
+
+@pytest.mark.parametrize("B,H,L,D", [(1, 2, 65, 128), (1, 24, 129, 128), (1, 24, 1280, 128), (2, 3, 700, 128), (2, 24, 640, 128),   # one launch for both
+                                     (1, 2, 64, 128), (1, 2, 2048, 128), (1, 24, 1300, 128), (1, 24, 300, 64)])                   # the products in front
+@pytest.mark.parametrize("M,K,Ns", [(1, 3072, (9216, 9216)), (1, 2048, (1001, 1001)), (2, 3072, (40,)), (2, 200, (9, 9)), (3, 1536, (333,)), (4, 1544, (8,)), (4, 3072, (100, 100)), (1, 512, (7, 12))])
+def test_attention_beside_row_products(B, H, L, D, M, K, Ns):
+    """Products of a few rows in the attention's launch, where it has one for them, and in front of it elsewhere: the bits of separate
+    launches, with SiLU on the way in, columns and K of every remainder, rows of the output further apart than they are long."""
+    g = seeded(L + K + M)
+    q, k, v = (randn(g, B, H, L, D, dtype=torch.bfloat16).to(DEV) for _ in range(3))
+    x = randn(g, M, K, dtype=torch.bfloat16).to(DEV)
+    calls = []
+    for N in Ns:
+        w, b = randn(g, N, K, dtype=torch.bfloat16).to(DEV) / K ** 0.5, randn(g, N, dtype=torch.bfloat16).to(DEV)
+        calls.append(dict(x=x, w=w, b=b, in_activation="SiLU", out=torch.full((M, N + 3), float("nan"), dtype=torch.bfloat16, device=DEV)[:, :N]))
+    o, lse = torch.empty_like(q), torch.empty(B, H, L, device=DEV)
+    for want_lse in (None, lse):   # (with it the call goes through ctypes)
+        for c in calls:
+            c["out"].fill_(float("nan"))
+        tk.attention_into(q, k, v, o, beside=tuple(calls), lse=want_lse)
+        assert torch.equal(o, tk.scaled_dot_product_attention(q, k, v))
+        for c in calls:
+            assert torch.equal(c["out"], tk.linear_into(x, c["w"], c["b"], in_activation="SiLU"))
+            assert torch.isnan(c["out"].as_strided((M, 3), (c["out"].stride(0), 1), c["out"].storage_offset() + c["w"].shape[0])).all()

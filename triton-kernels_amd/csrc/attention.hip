@@ -29,6 +29,7 @@
 // refilled is the one read a whole iteration earlier.
 #include "common.h"
 #include "attention_params.h"
+#include "gemm_rows.h"
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -135,7 +136,7 @@ constexpr bool attn_units_in_time(int qb_count, int ns, int db_count, int nslot,
 // DIRECT: Q comes straight into registers and the output leaves from there, for calls of a single key tile, which have
 // nothing to hide the way through LDS behind (see attn_launch_pipe).
 template <int D, int QB, int BN, bool SPLIT, bool FSUM, bool DIRECT>  // BN = keys per tile (32 or 64)
-__device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int splits, int part_keys) {
+__device__ __forceinline__ void attn_pipe(const AttnParams& p, char* lds, int nblocks, float* ws, int splits, int part_keys) {
     constexpr int KB = BN / 32;         // 32-key blocks of S^T per tile
     constexpr int PS = BN / 16;         // 16-key steps of P^T per tile
     constexpr int KSTEPS = D / 16;      // contraction steps of S^T = K Q^T
@@ -156,10 +157,9 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
     constexpr int NU = 4 * PS * QB;     // softmax units (two accumulator values each) per tile
     static_assert(NSLOT - KD >= BAR && BAR + 2 * PASSES <= NSLOT && (NKF - 1) * QB - KD < BAR, "slot plan");
     static_assert(attn_units_in_time(QB, NS, DB, NSLOT, PS), "P^T steps must be ready before the MFMAs that take them");
-    __shared__ __attribute__((aligned(1024))) char lds[5 * T_BYTES];  // K: 2 buffers, V: 3 buffers
-    constexpr int V0 = 2 * T_BYTES;
+    constexpr int V0 = 2 * T_BYTES;     // lds: 5 * T_BYTES, K 2 buffers, V 3 buffers
 
-    const int per_xcd = gridDim.x / 8;
+    const int per_xcd = nblocks / 8;
     const int vt = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (vt >= p.total_tiles) return;
     const int bh = SPLIT ? vt / p.n_qtiles / splits : vt / p.n_qtiles, qt = vt % p.n_qtiles;
@@ -539,13 +539,16 @@ __device__ __forceinline__ void attn_pipe(const AttnParams& p, float* ws, int sp
 
 // (The form without parts takes no arguments for them: with some it waits for its arguments twice, which costs up to
 // 2 % of a short call, [1, 24, 1280, 128] 31.6 -> 32.4 us.)
+constexpr int pipe_lds_bytes(int d, int bn) { return 5 * bn * 2 * d; }
 template <int D, int QB, int BN, bool FSUM, bool DIRECT>
 __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_pipe_kernel(AttnParams p) {
-    attn_pipe<D, QB, BN, false, FSUM, DIRECT>(p, nullptr, 1, 0);
+    __shared__ __attribute__((aligned(1024))) char lds[pipe_lds_bytes(D, BN)];
+    attn_pipe<D, QB, BN, false, FSUM, DIRECT>(p, lds, gridDim.x, nullptr, 1, 0);
 }
 template <int D, int QB, int BN>
 __global__ __launch_bounds__(256, (QB == 1 ? 2 : 1)) void attn_fwd_parts_kernel(AttnParams p, float* ws, int splits, int part_keys) {
-    attn_pipe<D, QB, BN, true, false, false>(p, ws, splits, part_keys);
+    __shared__ __attribute__((aligned(1024))) char lds[pipe_lds_bytes(D, BN)];
+    attn_pipe<D, QB, BN, true, false, false>(p, lds, gridDim.x, ws, splits, part_keys);
 }
 
 // O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s over the parts of a row, in the order of the keys. A wave
@@ -1531,6 +1534,58 @@ void attn_launch_w64_d64(AttnParams& p, int64_t BH, hipStream_t st);
 void attn_launch_w64_d64(AttnParams& p, int64_t BH, hipStream_t st) { attn_launch_w64<64>(p, BH, st); }
 #endif
 
+#ifndef FLUX_ATTN_W64_D64_UNIT
+// ------------------------------------------------------------------------------------------------
+// The 32-row kernel of head dim 128 and, in workgroups behind those of the attention, row vectors times weights that have
+// nothing to do with it. Up to 256 workgroups of the attention leave every CU room for a second one, and the memory idle; such a
+// product needs the memory and nothing else. What bounds the launch is a CU's load path, on which the attention's K and V wait
+// behind the weights. us, two launches -> one, beside two products of M x 12288 x 3072 (23.8 and 26.5 us alone): M = 1, [1, 24, 320]
+// 34.6 -> 27.3, [1, 24, 704] 42.8 -> 29.7, [1, 24, 1280] 56.8 -> 39.7; M = 2, [2, 24, 640] 46.8 -> 43.1. Row workgroups of eight columns, whose
+// loads do not overlap their ends, took 47.6 us at [1, 24, 1280]. Beside more than 256 workgroups there is no room: the 64-row
+// kernel fills a CU, and with the rows behind its last tiles [1, 24, 4608] took 38 us more, where the products alone take 20.
+// ------------------------------------------------------------------------------------------------
+constexpr int kRowsLds = 48 * 1024;   // bytes of the activation rows, at most
+static_assert(kRowsLds <= pipe_lds_bytes(128, 64), "the activation rows overlay the attention's LDS");
+
+template <int MM>
+__device__ __forceinline__ void rows_block(const GemmSet& g, int block, int groups, char* lds) {
+    const int all = (g.p[0].N + 4 * kGemvCols - 1) / (4 * kGemvCols), per = (all + groups - 1) / groups;   // groups of columns, and workgroups, of a product
+    const int second = block >= per ? 1 : 0;
+    const GemmParams p = g.p[second];
+    const int first = (block - second * per) * groups;
+    constexpr int U = MM <= 2 ? 6 : 3;   // (two sets of them, and MM activation rows, in the attention's registers)
+    if (p.K % (512 * U) == 0) gemv_groups<MM, U, true>(p, first, min(groups, all - first), lds);
+    else gemv_groups<MM, U, false>(p, first, min(groups, all - first), lds);
+}
+
+template <bool FSUM>
+__global__ __launch_bounds__(256, 2) void attn_fwd_pipe_rows_kernel(AttnParams p, GemmSet g, int attn_blocks, int groups) {
+    __shared__ __attribute__((aligned(1024))) char lds[pipe_lds_bytes(128, 64)];
+    const int block = static_cast<int>(blockIdx.x) - attn_blocks;
+    if (block < 0) attn_pipe<128, 1, 64, false, FSUM, false>(p, lds, attn_blocks, nullptr, 1, 0);
+    else if (g.p[0].M == 1) rows_block<1>(g, block, groups, lds);
+    else if (g.p[0].M == 2) rows_block<2>(g, block, groups, lds);
+    else if (g.p[0].M == 3) rows_block<3>(g, block, groups, lds);
+    else rows_block<4>(g, block, groups, lds);
+}
+
+// Up to four rows in all: more are bound by their arithmetic, which they would share with the attention ([3, 24, 320] beside two
+// products of 3 x 12288 x 3072 49.3 us, 47.3 in two launches).
+static bool rows_fit(const GemmSet& g) { return g.p[0].M * g.n <= 4 && static_cast<int64_t>(g.p[0].M) * g.p[0].K * 2 <= kRowsLds; }
+
+static void attn_launch_rows(AttnParams& p, int64_t BH, const GemmSet& rows, hipStream_t st) {
+    p.n_qtiles = (p.L + 127) / 128;
+    p.total_tiles = static_cast<int>(p.n_qtiles * BH);
+    const int grid = ((p.total_tiles + 7) / 8) * 8;
+    // as many workgroups as there is room for beside the attention's, two to a CU
+    const int all = (rows.p[0].N + 4 * kGemvCols - 1) / (4 * kGemvCols), room = max(2 * kAttnCUs - grid, 64);
+    const int groups = (all * rows.n + room - 1) / room;
+    const int blocks = (all + groups - 1) / groups * rows.n;
+    if (BH * ((p.L + 255) / 256) >= kFsumTiles) hipLaunchKernelGGL(attn_fwd_pipe_rows_kernel<true>, dim3(grid + blocks), dim3(256), 0, st, p, rows, grid, groups);
+    else hipLaunchKernelGGL(attn_fwd_pipe_rows_kernel<false>, dim3(grid + blocks), dim3(256), 0, st, p, rows, grid, groups);
+}
+#endif
+
 }  // namespace flux
 
 #ifndef FLUX_ATTN_W64_D64_UNIT
@@ -1550,20 +1605,22 @@ static bool view_ok(const void* ptr, int64_t sb, int64_t sh, int64_t sl) {
     return ptr != nullptr && aligned16(ptr) && sb % 8 == 0 && sh % 8 == 0 && sl % 8 == 0;
 }
 
-static int attention_launch(const flux_attn_args* a, void* workspace, int64_t workspace_bytes, hipStream_t st) {
+// Checks a call and turns it into the kernels' parameters; `nothing`: there are no rows.
+static int read_attn_args(const flux_attn_args* a, AttnParams& p, bool& nothing) {
+    nothing = false;
     if (!a) return fail(FLUX_E_NULL, "flux_attention_fwd_bf16: null args");
     if (a->B < 0 || a->H <= 0 || a->L < 0) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: bad shape B=%lld H=%lld L=%lld", (long long)a->B, (long long)a->H, (long long)a->L);
     if (a->D != 16 && a->D != 32 && a->D != 64 && a->D != 128 && a->D != 256)
         return fail(FLUX_E_UNSUPPORTED, "flux_attention_fwd_bf16: head dim %d not supported (16, 32, 64, 128, 256)", a->D);
     if (!(a->sm_scale == a->sm_scale)) return fail(FLUX_E_UNSUPPORTED, "flux_attention_fwd_bf16: sm_scale is NaN");
-    if (a->B == 0 || a->L == 0) return FLUX_OK;
+    nothing = a->B == 0 || a->L == 0;
+    if (nothing) return FLUX_OK;
     if (a->L > 0x7fffffff / 64 || a->B * a->H > 0x7fffffff / 64) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: problem too large");
     if (!view_ok(a->q.ptr, a->q.sb, a->q.sh, a->q.sl) || !view_ok(a->k.ptr, a->k.sb, a->k.sh, a->k.sl) ||
         !view_ok(a->v.ptr, a->v.sb, a->v.sh, a->v.sl) || !view_ok(a->o, a->o_sb, a->o_sh, a->o_sl))
         return fail(FLUX_E_ALIGN, "flux_attention_fwd_bf16: q/k/v/o must be non-null, 16-byte aligned, with strides that are multiples of 8");
     if (a->k.sl * 2 * 64 >= 0x7fffffffLL || a->v.sl * 2 * 64 >= 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: row stride too large");
 
-    AttnParams p;
     p.q = static_cast<const bf16_t*>(a->q.ptr); p.k = static_cast<const bf16_t*>(a->k.ptr);
     p.v = static_cast<const bf16_t*>(a->v.ptr); p.o = static_cast<bf16_t*>(a->o); p.lse = a->lse;
     p.q_sb = a->q.sb; p.q_sh = a->q.sh; p.q_sl = a->q.sl;
@@ -1572,11 +1629,18 @@ static int attention_launch(const flux_attn_args* a, void* workspace, int64_t wo
     p.o_sb = a->o_sb; p.o_sh = a->o_sh; p.o_sl = a->o_sl;
     p.H = (int)a->H; p.L = (int)a->L;
     p.scale_log2 = a->sm_scale * 1.4426950408889634f;
+    if (a->D != 64 && a->D != 128 && a->B * a->H * ((a->L + 63) / 64) > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: problem too large");
+    return FLUX_OK;
+}
+
+static int attention_launch(const flux_attn_args* a, void* workspace, int64_t workspace_bytes, hipStream_t st) {
+    AttnParams p;
+    bool nothing;
+    const int rc = read_attn_args(a, p, nothing);
+    if (rc != FLUX_OK || nothing) return rc;
     const int64_t BH = a->B * a->H;
-    if (a->D != 64 && a->D != 128) {
-        if (BH * ((a->L + 63) / 64) > 0x7fffffffLL) return fail(FLUX_E_SHAPE, "flux_attention_fwd_bf16: problem too large");
-        attn_launch_plain(p, BH, a->D, st);
-    } else if (a->D == 128 && !attn_short(BH, a->L) && attn_q_near(a)) attn_launch_w64<128>(p, BH, st);
+    if (a->D != 64 && a->D != 128) attn_launch_plain(p, BH, a->D, st);
+    else if (a->D == 128 && !attn_short(BH, a->L) && attn_q_near(a)) attn_launch_w64<128>(p, BH, st);
     else if (a->D == 128) attn_launch_pipe<128>(p, BH, static_cast<float*>(workspace), workspace_bytes, st);
     else if (!attn_short(BH, a->L) && attn_q_near(a)) attn_launch_w64_d64(p, BH, st);
     else attn_launch_pipe<64>(p, BH, static_cast<float*>(workspace), workspace_bytes, st);
@@ -1599,4 +1663,26 @@ extern "C" int flux_attention_fwd_bf16_ws(const flux_attn_args* a, void* workspa
         return fail(FLUX_E_NULL, "flux_attention_fwd_bf16_ws: workspace must be 16-byte aligned memory");
     return attention_launch(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
-#endif  // FLUX_ATTN_W64_D64_UNIT
+extern "C" int flux_attention_rows_bf16(const flux_attn_args* a, const flux_linear_pair_args* rows, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (!rows) return fail(FLUX_E_NULL, "flux_attention_rows_bf16: null product");
+    if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace))))
+        return fail(FLUX_E_NULL, "flux_attention_rows_bf16: workspace must be 16-byte aligned memory");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    AttnParams p;
+    GemmSet g;
+    bool nothing;
+    int rc = read_attn_args(a, p, nothing);
+    if (rc != FLUX_OK) return rc;
+    const bool together = rows_beside(rows, g, rc);
+    if (rc != FLUX_OK) return rc;
+    const int64_t BH = a->B * a->H;
+    int part_keys;
+    const bool whole = workspace == nullptr || attn_splits(BH, a->L, a->D, part_keys) == 1;
+    if (together && !nothing && a->D == 128 && attn_short(BH, a->L) && a->L > 64 && whole && rows_fit(g)) {
+        attn_launch_rows(p, BH, g, st);
+        return check_launch("flux_attention_rows_bf16");
+    }
+    rc = flux_linear_bf16_pair(rows, nullptr, 0, stream);
+    return rc != FLUX_OK ? rc : attention_launch(a, workspace, workspace_bytes, st);
+}
+#endif

@@ -658,18 +658,24 @@ PyObject* py_linear_pair_into(PyObject*, PyObject* const* args, Py_ssize_t nargs
 
 // ---- attention ---------------------------------------------------------------------------------
 
-// attention(q, k, v, scale or None): all of [B, H, L, D]; attention(q, k, v, scale or None, out): to a tensor that is there
+// attention(q, k, v, scale or None): all of [B, H, L, D]; attention(q, k, v, scale or None, out, calls): to a tensor that is there, beside up to two
+// products (as read_product has them)
 PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(nargs == 4 || nargs == 5, "attention takes 4 or 5 arguments");
-    const Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]), *out = nargs == 5 ? tensor_of(args[4]) : nullptr;
-    if (!q || !k || !v || (nargs == 5 && !out) || !quiet() || q->dim() != 4 || q->sizes() != k->sizes() || q->sizes() != v->sizes() || q->scalar_type() != at::kBFloat16 ||
+    TORCH_CHECK(nargs == 4 || nargs == 6, "attention takes 4 or 6 arguments");
+    const Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]), *out = nargs == 6 ? tensor_of(args[4]) : nullptr;
+    if (!q || !k || !v || (nargs == 6 && !out) || !quiet() || q->dim() != 4 || q->sizes() != k->sizes() || q->sizes() != v->sizes() || q->scalar_type() != at::kBFloat16 ||
         !same_kind(*q, *k) || !same_kind(*q, *v) || (out && (out->sizes() != q->sizes() || !same_kind(*q, *out) || out->stride(3) != 1)))
         Py_RETURN_NONE;
     for (const Tensor* t : {q, k, v})
         if (t->stride(3) != 1 || !vector_rows(*t)) Py_RETURN_NONE;
     double scale = 1.0 / std::sqrt(static_cast<double>(q->size(3)));
     if (args[3] != Py_None && !number(args[3], scale)) Py_RETURN_NONE;
+    Product p[2];
+    const Py_ssize_t products = nargs == 6 && PyTuple_CheckExact(args[5]) ? PyTuple_GET_SIZE(args[5]) : 0;
+    if (products > 2 || (nargs == 6 && !PyTuple_CheckExact(args[5]))) Py_RETURN_NONE;
+    for (Py_ssize_t i = 0; i < products; ++i)
+        if (!read_product(PyTuple_GET_ITEM(args[5], i), p[i], false) || !p[i].out_given || p[i].out.device() != q->device()) Py_RETURN_NONE;
     Tensor o;
     int rc;
     {
@@ -686,7 +692,19 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         a.sm_scale = static_cast<float>(scale);
         const int64_t need = flux_attention_workspace_bytes(a.B, a.H, a.L, a.D);   // keys cut over several workgroups
         const Tensor ws = need ? empty({need}, at::kByte, qa) : Tensor();
-        rc = flux_attention_fwd_bf16_ws(&a, need ? ws.data_ptr() : nullptr, need, stream_of(qa));
+        void* const ws_at = need ? ws.data_ptr() : nullptr;
+        if (products == 0) {
+            rc = flux_attention_fwd_bf16_ws(&a, ws_at, need, stream_of(qa));
+        } else {
+            flux_linear_pair_args rows = {};
+            for (int i = 0; i < 2; ++i) {
+                Product& at = p[i < products ? i : 0];
+                place_output(at, qa);
+                rows.product[i] = at.a;
+            }
+            if (products == 1) rows.product[1].M = 0;
+            rc = flux_attention_rows_bf16(&a, &rows, ws_at, need, stream_of(qa));
+        }
     }
     if (rc < 0) Py_RETURN_NONE;
     check(rc, "flux_attention_fwd_bf16");

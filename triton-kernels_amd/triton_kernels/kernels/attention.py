@@ -9,6 +9,7 @@ from torch import Tensor
 from torch.compiler import is_compiling
 
 from triton_kernels import _native as nv
+from triton_kernels.kernels.linear import hooked, positional, rows_args
 
 
 def _bhld_view(t: Tensor) -> Tensor:
@@ -24,11 +25,19 @@ def _may_cut_keys(BH: int, L: int) -> bool:
     return L > 1024 and BH * ((L + 127) // 128) <= 128
 
 
+def takes_rows(BH: int, L: int, D: int, rows: int, K: int) -> bool:
+    """Whether products of `rows` rows in all with K values each run beside an attention (attention_into's `beside`) and not in
+    front of it (flux_attention_rows_bf16)."""
+    return D == 128 and 64 < L and BH * ((L + 127) // 128) <= 256 and not _may_cut_keys(BH, L) and rows <= 4 and rows * K * 2 <= 48 * 1024
+
+
 def attention_into(q: Tensor, k: Tensor, v: Tensor, out: Tensor, sm_scale: float | None = None,
-                   lse: Tensor | None = None) -> Tensor:
-    """q,k,v,out are [B,H,L,D] views (bf16, last dim contiguous, any other strides)."""
-    if lse is None and not is_compiling():
-        o = nv.ops().attention(q, k, v, sm_scale, out)
+                   lse: Tensor | None = None, beside: tuple[dict, ...] = ()) -> Tensor:
+    """q,k,v,out are [B,H,L,D] views (bf16, last dim contiguous, any other strides).
+    beside: one or two linear_into calls of a few rows (the keyword arguments of each) that have nothing to do with the
+    attention; the library runs them beside it in one launch where it can."""
+    if lse is None and not (beside and hooked()) and not is_compiling():
+        o = nv.ops().attention(q, k, v, sm_scale, out, tuple(positional(**call) for call in beside))
         if o is not None:
             return o
     D = q.shape[-1]
@@ -50,7 +59,11 @@ def attention_into(q: Tensor, k: Tensor, v: Tensor, out: Tensor, sm_scale: float
     a.B, a.H, a.L, a.D, a.sm_scale = B, H, L, D, float(sm_scale)
     with nv.on_device(dev):
         need = nv.lib().flux_attention_workspace_bytes(B, H, L, D) if _may_cut_keys(B * H, L) else 0
-        if need:   # keys cut over several workgroups: partial sums in memory of this launch's stream
+        if beside:
+            rows, _keep = rows_args(beside, dev)
+            ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None
+            rc = nv.lib().flux_attention_rows_bf16(nv.byref(a), nv.byref(rows), nv.ptr(ws), need, nv.stream_ptr(dev))
+        elif need:   # keys cut over several workgroups: partial sums in memory of this launch's stream
             ws = torch.empty((need,), dtype=torch.uint8, device=dev)
             rc = nv.lib().flux_attention_fwd_bf16_ws(nv.byref(a), ws.data_ptr(), need, nv.stream_ptr(dev))
         else:

@@ -23,6 +23,10 @@ _PLANS = {torch.bfloat16: {"tile": (256, 256, 64), "waves": 4, "mfma": "16x16x32
 launch_hook = None
 
 
+def hooked() -> bool:
+    return launch_hook is not None
+
+
 def linear_launch_metadata(M: int, N: int, K: int, elem_bytes: int = 2, epilogue: str = "") -> dict:
     name = f"flux_linear_bf16 [M={M}, N={N}, K={K}]" + (f" {epilogue}" if epilogue else "")
     return {"name": name, f"flops{elem_bytes * 8}": 2.0 * M * N * K, "bytes": elem_bytes * (M * K + N * K + M * N)}
@@ -52,7 +56,7 @@ def _may_cut_k(rows: int, N: int, K: int) -> bool:
 _IN_ACTIVATIONS = {"": nv.ACT_NONE, "SiLU": nv.ACT_SILU}
 
 
-def _positional(x, w, b, *, activation="", act_begin=0, out=None, out2=None, split=None, resid=None, gate=None, qk=None, in_activation="", shared_gpu=False):
+def positional(x, w, b, *, activation="", act_begin=0, out=None, out2=None, split=None, resid=None, gate=None, qk=None, in_activation="", shared_gpu=False):
     """A linear_into call as the native calls take it."""
     if qk is not None:
         qk = (qk["q_out"], qk["k_out"], qk["q_scale"], qk["k_scale"], qk["pe"], qk["heads"], qk["seq_len"], qk.get("pos0", 0), qk.get("eps", 1e-6))
@@ -79,7 +83,7 @@ def linear_into(x: Tensor, w: Tensor, b: Tensor | None, *, activation: str = "",
             result, only the schedule differs); for callers that run streams side by side
     """
     if launch_hook is None and not is_compiling():
-        y = nv.ops().linear_into(_positional(x, w, b, activation=activation, act_begin=act_begin, out=out, out2=out2, split=split, resid=resid, gate=gate, qk=qk,
+        y = nv.ops().linear_into(positional(x, w, b, activation=activation, act_begin=act_begin, out=out, out2=out2, split=split, resid=resid, gate=gate, qk=qk,
                                              in_activation=in_activation, shared_gpu=shared_gpu))
         if y is not None:
             return y
@@ -101,7 +105,7 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
     call: products of the same N, K and form of epilogue share a launch. An x of [B, L, K] may be a slice of
     a longer sequence, whose batch elements are not evenly strided rows."""
     if launch_hook is None and not is_compiling():
-        both = nv.ops().linear_pair_into(_positional(**first), _positional(**second))
+        both = nv.ops().linear_pair_into(positional(**first), positional(**second))
         if both is not None:
             return both
     args = nv.LinearPairArgs()
@@ -137,6 +141,27 @@ def linear_pair_into(first: dict, second: dict) -> tuple[Tensor, Tensor]:
             launch_hook(notes[i])
             _launch_pair(one, sizes[i:i + 1], dev)
     return outs[0], outs[1]
+
+
+def rows_args(calls: tuple[dict, ...], dev: torch.device) -> tuple["nv.LinearPairArgs", list]:
+    """One or two linear_into calls as the library takes them beside an attention, and what has to live until the launch."""
+    args = nv.LinearPairArgs()
+    keep, sizes, notes = [], [], []
+    for i, call in enumerate(calls):
+        out, at, M, N, _, kept = _fill_args(args.product[i], notes=notes, **call)
+        assert at == dev, "tensors on different devices"
+        keep += [out, kept]
+        sizes.append((M, N))
+    if len(calls) == 1:
+        args.product[1] = args.product[0]
+        args.product[1].M = 0
+    if launch_hook is not None:
+        if len(notes) == 2 and sizes[0] == sizes[1]:
+            launch_hook(_pair_launch_metadata(*notes, sizes))
+        else:
+            for n in notes:
+                launch_hook(n)
+    return args, keep
 
 
 def _launch_pair(args: "nv.LinearPairArgs", sizes: list, dev: torch.device) -> None:

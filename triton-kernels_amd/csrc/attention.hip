@@ -694,6 +694,14 @@ template <int R> __device__ __forceinline__ float acc_read() {
     asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(R));
     return v;
 }
+// x of the four lanes of a query row (16 apart), combined, without the LDS: two swaps of register halves.
+template <typename F>
+__device__ __forceinline__ float across_quarters(float x, F&& f) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 // Marks the old value of x as used here, so that its registers stay reserved up to this point.
 template <typename T> __device__ __forceinline__ void keep_regs(T& x) { asm volatile("" : "+v"(x)); }
 // Enough wait states for the newest MFMA result to be readable by the VALU (and the other way round).
@@ -952,32 +960,28 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     }
     load_v(0, 0);
     load_k(1, 1);
-    // The first pass through the loop multiplies P = 0 with whatever the last V buffer holds:
-    // make that finite.
-    {
-        const u32x4 z = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < PP; ++i) *reinterpret_cast<u32x4*>(lds + V0 + 3 * TB + i * (NW * 1024) + tid * 16) = z;
-    }
 
     // Q fragments ("B" operand of S^T): lane holds row q0 + qb*16 + r16, d = ks*32 + g*8 .. +8,
     // scaled by sm_scale*log2(e) and rounded to bf16.
     attn_claim_agprs<(D == 128 ? 48 * QB : 96)>();
     static_for<0, kAccQ>([&](auto i_c) { acc_write<decltype(i_c)::value>(0u); });  // O^T = 0, while the loads are on their way
-    {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PP) : "memory");   // K(0) and Q have landed
-        u32x4 qraw[QB][KS];
+    // In two halves, the first while the second is still on its way: 393 instructions in all, 0.7 us of a wave that has its SIMD to itself.
+    static_for<0, 2>([&](auto h_c) {
+        constexpr int q_lo = decltype(h_c)::value * 2, q_hi = decltype(h_c)::value == 0 ? 2 : QB;
+        // K(0), and the blocks up to q_hi, have landed
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((QB - q_hi) * (16 / RPL) + 2 * PP) : "memory");
+        u32x4 qraw[q_hi - q_lo][KS];
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
+        for (int qb = q_lo; qb < q_hi; ++qb)
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
-                qraw[qb][ks] = *reinterpret_cast<const u32x4*>(q_lds + (qb * 16 + r16) * ROWB + (((ks * 4 + g) ^ k_swz(r16)) * 16));
-        static_for<0, QB * KS * 4>([&](auto i_c) {
+                qraw[qb - q_lo][ks] = *reinterpret_cast<const u32x4*>(q_lds + (qb * 16 + r16) * ROWB + (((ks * 4 + g) ^ k_swz(r16)) * 16));
+        static_for<q_lo * kQRegs, q_hi * kQRegs>([&](auto i_c) {
             constexpr int i = decltype(i_c)::value, qb = i / kQRegs, ks = (i / 4) % KS, e = i % 4;
-            const uint32_t t = qraw[qb][ks][e];
+            const uint32_t t = qraw[qb - q_lo][ks][e];
             acc_write<kAccQ + i>(pack2_bf16(__uint_as_float(t << 16) * c, __uint_as_float(t & 0xffff0000u) * c));
         });
-    }
+    });
 
     // fragment addresses, lane part (the ring offset of the sub-tile is added once per iteration,
     // key-block and second-read offsets are immediates)
@@ -1001,7 +1005,7 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
         seed[qb] = zero4;
         l_run[qb] = 0.0f;
     }
-    const int ntiles = (p.L + 63) / 64;
+    const int nsub = (p.L + 31) / 32;
 
     // Every register an MFMA reads or writes is kept for that purpose through the whole loop
     // (keep_regs in front of each redefinition): see mfma_s_seed.
@@ -1046,19 +1050,23 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     load_k(2, 2);
     load_v(1, 1);
     load_k(3, 3);
+    if (p.L < 32) {   // (a branch of the whole wave: longer sequences are spared 60 instructions)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (kb * 16 + g * 4 + j >= p.L) s0[kb][qb][j] = -INFINITY;
+    }
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         float mx = -INFINITY;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int key = kb * 16 + g * 4 + j;
-                if (key >= p.L) s0[kb][qb][j] = -INFINITY;
-                mx = fmaxf(mx, s0[kb][qb][j]);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s0[kb][qb][j]);
+        mx = across_quarters(mx, [](float x, float y) { return fmaxf(x, y); });
 #pragma unroll
         for (int j = 0; j < 4; ++j) seed[qb][j] = -mx;
 #pragma unroll
@@ -1078,8 +1086,7 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
             constexpr int qb = decltype(qb_c)::value, QBC = qb;
             float mx = fmaxf(fmaxf(sc[0][qb][0], sc[0][qb][1]), fmaxf(sc[0][qb][2], sc[0][qb][3]));
             mx = fmaxf(mx, fmaxf(fmaxf(sc[1][qb][0], sc[1][qb][1]), fmaxf(sc[1][qb][2], sc[1][qb][3])));
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = across_quarters(mx, [](float x, float y) { return fmaxf(x, y); });
             const float d = fmaxf(mx, 0.0f);  // the reference only ever moves up
             const float f = __builtin_amdgcn_exp2f(-d);
             seed[qb] -= d;
@@ -1114,10 +1121,11 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     //         this iteration and the next one.
     //   RAG:  the sub-tile after this one may reach past the last key (the common loop is built
     //         without that test).
+    //   FIRST: there is no P V yet.
     // All offsets are compile-time constants: the body is unrolled over the four ring positions.
-    auto iter = [&](auto bar_c, auto rag_c, auto kc_c, auto kn_c, auto vc_c, auto kld_c, auto vld_c, const u32x4& rk, const u32x4& rv, int u,
+    auto iter = [&](auto first_c, auto bar_c, auto rag_c, auto kc_c, auto kn_c, auto vc_c, auto kld_c, auto vld_c, const u32x4& rk, const u32x4& rv, int u,
                     f32x4 (&sc)[2][QB], f32x4 (&sn)[2][QB], uint32_t (&pc)[QB][4], uint32_t (&pp)[QB][4]) {
-        constexpr bool BAR = decltype(bar_c)::value, RAG = decltype(rag_c)::value;
+        constexpr bool FIRST = decltype(first_c)::value, BAR = decltype(bar_c)::value, RAG = decltype(rag_c)::value;
         constexpr int KC = decltype(kc_c)::value, KN = decltype(kn_c)::value, VC = decltype(vc_c)::value;
         constexpr int KLD = decltype(kld_c)::value, VLD = decltype(vld_c)::value;
         bf16x8 ppf[QB];
@@ -1143,7 +1151,7 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
                 constexpr int n = i / QB, qb = i % QB, kb = n / KS, ks = n % KS;
                 if constexpr (ks == 0) mfma_s_seed<kAccQ + kQRegs * qb>(sn[kb][qb], kf[n % 4], seed[qb]);
                 else mfma_s_acc<kAccQ + kQRegs * qb + 4 * ks>(sn[kb][qb], kf[n % 4]);
-            } else {
+            } else if constexpr (!FIRST) {
                 constexpr int m = (i - NSS) / QB, qb = i % QB;
                 mfma_o_acc<4 * (m * QB + qb)>(vfrag(m % 4), ppf[qb]);
             }
@@ -1154,11 +1162,11 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
                 constexpr int n = decltype(n_c)::value;
                 if constexpr (n < 2 * KS && QB * n - LA == i) read_k(KC, n);
                 if constexpr (n < 2 * KS && NS + QB * n - LA == i) read_k(KN, n);
-                if constexpr (n < DBN && NSS + QB * n - LA == i) {
+                if constexpr (!FIRST && n < DBN && NSS + QB * n - LA == i) {
                     keep_regs(vlo[n % 4]);
                     vlo[n % 4] = lds_read_tr(lds + v_addr[n % DBN] + VC);
                 }
-                if constexpr (n < DBN && NSS + 1 + QB * n - LA == i) {
+                if constexpr (!FIRST && n < DBN && NSS + 1 + QB * n - LA == i) {
                     keep_regs(vhi[n % 4]);
                     vhi[n % 4] = lds_read_tr(lds + v_addr[n % DBN] + (VC + 16 * ROWB));
                 }
@@ -1220,13 +1228,39 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    // Body T: iteration 2T (S^T from the second half of K(T), P V with the second half of V(T-1))
-    // and iteration 2T+1 (first half of K(T+1), first half of V(T)). Tile X sits in ring buffer
-    // X % 4, so four bodies make one trip of the loop. One more body than there are tiles: the last
-    // one only finishes P V. Bodies whose sub-tiles all lie inside the sequence run without the
-    // ragged-tail test; the last few take the variant with it.
-    // Buffer descriptors of the tiles requested by body T: K(T+4) and V(T+2), advanced by one tile
-    // per body; the record count is what is left of the sequence, at most one tile.
+    // What is left behind the last sub-tile's softmax: O^T += V^T P^T alone, with the V sub-tile at offset VC, which has long landed.
+    auto last = [&](int VC, uint32_t (&pp)[QB][4]) {
+        auto read = [&](auto n_c) {
+            constexpr int n = decltype(n_c)::value;
+            if constexpr (n < DBN) {
+                keep_regs(vlo[n % 4]);
+                keep_regs(vhi[n % 4]);
+                vlo[n % 4] = lds_read_tr(lds + v_addr[n] + VC);
+                vhi[n % 4] = lds_read_tr(lds + v_addr[n] + (VC + 16 * ROWB));
+            }
+        };
+        static_for<0, 3>(read);
+        static_for<0, DBN>([&](auto m_c) {
+            constexpr int m = decltype(m_c)::value;
+            static_for<0, QB>([&](auto qb_c) {
+                constexpr int qb = decltype(qb_c)::value;
+                const u32x4 v4 = {pp[qb][0], pp[qb][1], pp[qb][2], pp[qb][3]};
+                mfma_o_acc<4 * (m * QB + qb)>(vfrag(m % 4), __builtin_bit_cast(bf16x8, v4));
+            });
+            read(std::integral_constant<int, m + 3>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+
+    // Iteration 2T takes S^T from the second half of K(T) and P V from the second half of V(T-1), iteration 2T+1 the first
+    // halves of K(T+1) and V(T). Body T is the iterations 2T+1 and 2T+2. Tile X sits in ring buffer X % 4, so four bodies make one trip
+    // of the loop. Iteration 0 comes in front of it, as there is no P V yet, and iteration nsub, one more than there are sub-tiles,
+    // behind it, as P V is all that is left: half an iteration each, and a whole one where the last tile has no second half. (With the
+    // prologue above, which converts the first half of Q while the second is on its way, us before -> now: [4, 24, 300, 128] 18.1 -> 16.8,
+    // [16, 24, 512, 128] 77.8 -> 73.7, [4, 24, 1024, 128] 60.3 -> 58.5, [1, 24, 4608, 128] 208.2 -> 205.2, [2, 24, 1084, 64] 23.2 -> 22.8, [4, 24, 1300,
+    // 64] 67.2 -> 63.2.) Bodies whose sub-tiles all lie inside the sequence run without the ragged-tail test; the last few take the variant with it.
+    // Buffer descriptors of the tiles requested in iterations 2T and 2T+1: K(T+4) and V(T+2), advanced by one tile
+    // each time; the record count is what is left of the sequence, at most one tile.
     uint64_t k_at = reinterpret_cast<uint64_t>(kbase) + static_cast<uint64_t>(4 * 64) * k_row2;
     uint64_t v_at = reinterpret_cast<uint64_t>(vbase) + static_cast<uint64_t>(2 * 64) * v_row2;
     // rows left from the start of the next tile to request; a tile's record count is formed from at most
@@ -1243,21 +1277,26 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
         rows_left -= 64;
         return r;
     };
+    u32x4 rk = next_rsrc(k_at, k_rows, k_row2), rv = next_rsrc(v_at, v_rows, v_row2);
     auto body = [&](auto r_c, auto rag_c, int T) -> bool {
         constexpr int r = decltype(r_c)::value, r0 = r * TB, r1 = ((r + 1) & 3) * TB, r2 = ((r + 2) & 3) * TB, r3 = ((r + 3) & 3) * TB;
-        using ic = std::integral_constant<int, 0>;
-        const u32x4 rk = next_rsrc(k_at, k_rows, k_row2), rv = next_rsrc(v_at, v_rows, v_row2);
-        iter(std::true_type{}, rag_c, std::integral_constant<int, r0 + HALF>{}, std::integral_constant<int, r1>{},
-             std::integral_constant<int, r3 + HALF>{}, std::integral_constant<int, r0>{}, std::integral_constant<int, r2>{},
-             rk, rv, 2 * T, s0, s1, pw0, pw1);
-        if (decltype(rag_c)::value && T == ntiles) return false;
-        iter(std::false_type{}, rag_c, std::integral_constant<int, r1>{}, std::integral_constant<int, r1 + HALF>{},
+        constexpr bool RAG = decltype(rag_c)::value;
+        if (RAG && 2 * T + 1 == nsub) return false;
+        iter(std::false_type{}, std::false_type{}, rag_c, std::integral_constant<int, r1>{}, std::integral_constant<int, r1 + HALF>{},
              std::integral_constant<int, r0>{}, std::integral_constant<int, r0>{}, std::integral_constant<int, r2>{},
              rk, rv, 2 * T + 1, s1, s0, pw1, pw0);
+        if (RAG && 2 * T + 2 == nsub) return false;
+        rk = next_rsrc(k_at, k_rows, k_row2);
+        rv = next_rsrc(v_at, v_rows, v_row2);
+        iter(std::false_type{}, std::true_type{}, rag_c, std::integral_constant<int, r1 + HALF>{}, std::integral_constant<int, r2>{},
+             std::integral_constant<int, r0 + HALF>{}, std::integral_constant<int, r1>{}, std::integral_constant<int, r3>{},
+             rk, rv, 2 * T + 2, s0, s1, pw0, pw1);
         return true;
     };
-    // bodies 0 .. n_plain-1 never look past the last key: (2T + 3) * 32 <= L, in whole trips of four
-    const int n_plain = max(0, (p.L / 32 - 1) / 2) & ~3;
+    iter(std::true_type{}, std::true_type{}, std::true_type{}, std::integral_constant<int, HALF>{}, std::integral_constant<int, TB>{},
+         std::integral_constant<int, 3 * TB + HALF>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 2 * TB>{}, rk, rv, 0, s0, s1, pw0, pw1);
+    // bodies 0 .. n_plain-1 never look past the last key: (2T + 4) * 32 <= L, in whole trips of four
+    const int n_plain = max(0, (p.L / 32 - 2) / 2) & ~3;
     int T = 0;
     for (; T < n_plain; T += 4) {
         body(std::integral_constant<int, 0>{}, std::false_type{}, T);
@@ -1301,6 +1340,11 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
         if (!body(std::integral_constant<int, 2>{}, std::true_type{}, T + 2)) break;
         if (!body(std::integral_constant<int, 3>{}, std::true_type{}, T + 3)) break;
     }
+    {
+        const int at = (nsub - 1) / 2 % 4 * TB + (nsub - 1) % 2 * HALF;
+        if (nsub % 2 != 0) last(at, pw0);
+        else last(at, pw1);
+    }
     wait_all_vmem();
     mfma_settle();
 
@@ -1318,8 +1362,7 @@ __device__ __forceinline__ void attn_w64_tile(const AttnParams& p, char* lds, co
     const int64_t o_step = RPL * p.o_sl;
     static_for<0, QB>([&](auto qb_c) {
         constexpr int qb = decltype(qb_c)::value, QBC = qb;
-        float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 16, 64);
-        l_tot += __shfl_xor(l_tot, 32, 64);
+        const float l_tot = across_quarters(l_run[qb], [](float x, float y) { return x + y; });
         const float inv = 1.0f / l_tot;
         const int row = q0 + qb * 16 + r16;
         char* const srow = stage + (qb * 16 + r16) * ROWB;

@@ -398,6 +398,52 @@ def test_linear_every_tile(family, tile_m, tile_n, whole, tail, parts):
         assert torch.equal(out.view(1, M, N), oracle.gated_residual_ref(x, gate, y.view(1, M, N))), (M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (320, 10920, 4096), (320, 10928, 4096),    # the last W walked in turn and the first one that is not
+    (330, 3072, 15360), (1100, 3072, 15360),   # K in parts, two tile rows; groups of four and of three
+    (900, 3072, 15360),                        # a group of four and a tile row of its own
+    (400, 15000, 3080), (1000, 2920, 15416),   # K tail in a last group of slabs that is shorter and in a whole one
+])
+def test_linear_slabs_out_of_turn(M, N, K):
+    """Eight-wave tiles that walk K in rotated order, against the fp32 product: half a bf16 ulp plus the spread of an fp32 sum in another order."""
+    assert plan_of(linear_args(M, N, K)).family == EIGHT_WAVES
+    g = seeded(M + N + K)
+    a = randn(g, M, K, dtype=torch.bfloat16).to(DEV)
+    w = randn(g, N, K, dtype=torch.bfloat16, std=K ** -0.5).to(DEV)
+    b = randn(g, N, dtype=torch.bfloat16, std=0.5).to(DEV)
+    ref32 = oracle.linear_ref_fp32(a, w, b)
+    assert ((tk.linear(a, w, b).float() - ref32).abs() <= half_ulp_bound(ref32)).all()
+
+
+@pytest.mark.parametrize("L", [320, 257])
+def test_linear_qk_slabs_out_of_turn(L):
+    """The same with QKNorm + RoPE in the epilogue: v and mlp columns against the fp32 product, q and k against the preparation kernel on the plain
+    one. A product on a rounding boundary may go either way: one bf16 ulp, and one for each rounding of norm, scale and rotation."""
+    H, D, mlp = 24, 128, 12288
+    hid = H * D
+    N = 3 * hid + mlp
+    assert plan_of(qk_args(1, L, H, mlp)).family == EIGHT_WAVES
+    g = seeded(L)
+    x = randn(g, L, hid, dtype=torch.bfloat16).to(DEV)
+    w = randn(g, N, hid, dtype=torch.bfloat16, std=hid ** -0.5).to(DEV)
+    qs, ks = [(torch.rand(D, generator=g) + 0.5).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    angle = randn(g, 1, 1, L, D // 2).to(DEV)
+    pe = torch.stack([angle.cos(), -angle.sin(), angle.sin(), angle.cos()], dim=-1).reshape(1, 1, L, D // 2, 2, 2)
+    qkv = torch.zeros(L, 3 * hid, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(L, mlp, dtype=torch.bfloat16, device=DEV)
+    q = torch.empty(1, H, L, D, dtype=torch.bfloat16, device=DEV)
+    k = torch.empty_like(q)
+    tk.linear_into(x, w, None, activation="GELU", act_begin=3 * hid, out=qkv, out2=out, split=3 * hid, qk=dict(q_out=q, k_out=k, q_scale=qs, k_scale=ks, pe=pe, heads=H, seq_len=L, eps=1e-6))
+    ref32, gelu32 = oracle.linear_ref_fp32(x, w, None), oracle.linear_ref_fp32(x, w, None, "GELU")
+    for got, want in ((qkv[:, 2 * hid:], ref32[:, 2 * hid:3 * hid]), (out, gelu32[:, 3 * hid:])):
+        assert ((got.float() - want).abs() <= half_ulp_bound(want)).all()
+    heads = ref32[:, :3 * hid].to(torch.bfloat16).view(1, L, 3, H, D).permute(2, 0, 3, 1, 4)
+    wants = tk.qkv_prep(heads[0], heads[1], None, pe=pe, q_scale_img=qs, k_scale_img=ks)
+    for got, want, raw, scale in ((q, wants[0], heads[0], qs), (k, wants[1], heads[1], ks)):
+        xn = oracle.rms_norm_ref(raw.cpu(), scale.cpu()).to(DEV).float().abs().unflatten(-1, (-1, 2)).sum(-1, keepdim=True).expand(-1, -1, -1, -1, 2).flatten(-2)
+        assert ((got.float() - want.float()).abs() <= 4 * 2.0 ** -7 * xn + 1e-5).all()
+
+
 @pytest.mark.parametrize("B,L,N,K,split,act_begin", [
     (1, 9, 3, 64, None, 0), (1, 65, 97, 128, 50, 33),        # less than a tile; a segment of 8 columns on both sides of the split
     (2, 100, 1001, 72, 1000, 1000), (3, 43, 201, 8192, None, 7),   # K tail; K over several workgroups, batch elements inside a tile

@@ -1,6 +1,8 @@
 // Linear layer on the matrix cores, middle sizes: a few hundred to a few thousand rows.
 #include "gemm_common.h"
 
+#include <climits>
+
 namespace flux {
 
 // ------------------------------------------------------------------------------------------------
@@ -20,10 +22,19 @@ namespace flux {
 // 138 -> 62 us, 1280 x 3072 x 12288 141 -> 93 us, 512 x 3072 x 3072 28 -> 21 us; a four-wave workgroup on the
 // same tiles: 50, 78, 120 and 21 us.
 // ------------------------------------------------------------------------------------------------
+// Slabs out of turn. Tiles that share columns of W run side by side and ask for the same slab at the same time, so each of them waits for it to
+// come from HBM. Where W is too large to be found in the Infinity Cache, the tiles of a column, `turns` of them, take every `turns` slabs of K
+// in an order rotated by their place: each is the first at one slab of such a group and finds the others in the L2, where its neighbours have brought
+// them. The same goes for A among the tiles of a row. us in turn -> rotated, W from HBM: 320 x 21504 x 3072 52.4 -> 46.8, 320 x 3072 x 15360
+// 44.1 -> 42.6, 640 x 3072 x 15360 64.3 -> 62.3; the fused projection of 320 rows 58.9 -> 54.6. W from the Infinity Cache: 41.0 -> 42.1, 40.1 -> 41.1
+// and 59.3 -> 60.7, so a W of up to a third of that cache, which a program may find there, is walked in turn. Two products in a launch gain
+// nothing (1024 + 256 x 3072 x 12288 99.6 and 100.2): the second's one row of tiles has nobody to share with and ends last. Groups of two and
+// four times as many slabs: 48.0 and 49.2 us at the first size. The order is worked out between the slabs: inside one it took 1 % of 512 x 3072 x 3072.
+constexpr int64_t kInfinityCacheBytes = int64_t(256) << 20;
 constexpr int kPairThreads = 512;
 
 template <int FM, int FN, int ST, bool KTAIL, int G>
-__device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, int m0, int n0, int kb, int ke, int w4, int lane, f32x4 (&acc)[FM][FN]) {
+__device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, int m0, int n0, int kb, int ke, int turn, int turns, int w4, int lane, f32x4 (&acc)[FM][FN]) {
     constexpr int BM = 32 * FM, BN = 32 * FN, BK = 64, ROWB = BK * 2;
     constexpr int SLAB = (BM + BN) * ROWB;       // A rows, then W rows
     constexpr int NL = (FM + FN + 1 - G) / 2;    // loads of this wave per slab: passes of 32 rows, every other one
@@ -84,8 +95,27 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
         const int i = idx / FN, j = (i & 1) ? FN - 1 - idx % FN : idx % FN;
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[buf][j], xa[buf][i], acc[i][j], 0, 0, 0);
     };
-    // cur: stage of slab kt (its fragments are in buffer `buf`), nxt: of slab kt + 1
-    auto slab = [&](auto bufc, int kt, int cur, int nxt) {
+    // the slabs in the order of this tile; those of a last, shorter group in turn
+    const bool rotated = turns > 1;
+    int group = kb, at = turn;
+    auto last_group = [&]() {
+        if (group + turns > ke) {
+            at = 0;
+            turn = turns = INT_MAX;
+        }
+    };
+    last_group();
+    auto next_slab = [&]() {
+        const int k = group + at;
+        if (++at == turns) at = 0;
+        if (at == turn) {
+            group += turns;
+            last_group();
+        }
+        return k;
+    };
+    // k: the slab that is requested; cur: stage of the one that is multiplied (its fragments are in buffer `buf`), nxt: of the one behind it
+    auto slab = [&](auto bufc, int k, int cur, int nxt) {
         constexpr int buf = decltype(bufc)::value;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -101,7 +131,7 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
             }
             mfma_one(buf, lo);
             __builtin_amdgcn_sched_barrier(0);
-            if (r >= BS && r - BS < NL) load(cur, r - BS, kt + ST);
+            if (r >= BS && r - BS < NL) load(cur, r - BS, k);
 #pragma unroll
             for (int m = lo + 1; m < hi; ++m) mfma_one(buf, m);
             __builtin_amdgcn_sched_barrier(0);
@@ -109,9 +139,11 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
     };
 
 #pragma unroll
-    for (int s = 0; s < ST; ++s)
+    for (int s = 0; s < ST; ++s) {
+        const int k = rotated ? next_slab() : kb + s;
 #pragma unroll
-        for (int j = 0; j < NL; ++j) load(s * SLAB, j, kb + s);
+        for (int j = 0; j < NL; ++j) load(s * SLAB, j, k);
+    }
     wait_loads_and_barrier<(ST - 1) * NL>();
 #pragma unroll
     for (int r = 0; r < READS; ++r) read_frag(0, 0, r);
@@ -120,8 +152,13 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
     auto after = [](int s) { return s + SLAB == ST * SLAB ? 0 : s + SLAB; };
     for (int kt = kb; kt < ke; kt += 2) {
         const int n1 = after(cur), n2 = after(n1);
-        slab(ic<0>(), kt, cur, n1);
-        if (kt + 1 < ke) slab(ic<1>(), kt + 1, n1, n2);
+        int k0 = kt + ST, k1 = kt + ST + 1;
+        if (rotated) {
+            k0 = next_slab();
+            k1 = next_slab();
+        }
+        slab(ic<0>(), k0, cur, n1);
+        if (kt + 1 < ke) slab(ic<1>(), k1, n1, n2);
         cur = n2;
     }
     wait_vmem_all();
@@ -142,6 +179,11 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
         tile_at(L, t, tm, tn);
     } else {
         if (FN == 8 && L.p[0].qk_cols > 0 ? !tile_of_block_qk(L, BN, tm, tn) : !tile_of_block(L, tm, tn)) return;
+    }
+    int turn = 0, turns = 1;
+    if (L.take_turns) {
+        turns = min(L.tiles_m - tm / L.group_m * L.group_m, L.group_m);
+        turn = (tm % L.group_m + tn) % turns;
     }
     const GemmParams p = L.p[product_of_tile(L, tm)];
     const int m0 = tm * BM, n0 = tn * BN;
@@ -176,10 +218,10 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
     };
     f32x4 acc[FM][FN];
     if (wave < 4) {
-        gemm_pair_slabs<FM, FN, ST, KTAIL, 0>(p, lds, m0, n0, kb, ke, w4, lane, acc);
+        gemm_pair_slabs<FM, FN, ST, KTAIL, 0>(p, lds, m0, n0, kb, ke, turn, turns, w4, lane, acc);
         finish(ic<0>(), acc);
     } else {
-        gemm_pair_slabs<FM, FN, ST, KTAIL, 1>(p, lds, m0, n0, kb, ke, w4, lane, acc);
+        gemm_pair_slabs<FM, FN, ST, KTAIL, 1>(p, lds, m0, n0, kb, ke, turn, turns, w4, lane, acc);
         finish(ic<1>(), acc);
     }
 }
@@ -215,6 +257,7 @@ template <int FM, int FN, int ST>
 static void launch_pair(const GemmSet& g, int splits, float* partial, hipStream_t st) {
     const int K = g.p[0].K;
     GemmLaunch L = make_launch(g, 32 * FM, 32 * FN);
+    L.take_turns = g.n == 1 && static_cast<int64_t>(g.p[0].N) * K * 2 > kInfinityCacheBytes / 3;
     if (splits > 1) {   // (whole slabs only)
         L.slabs_per_split = (K / 64 + splits - 1) / splits;
         L.splits = (K / 64 + L.slabs_per_split - 1) / L.slabs_per_split;

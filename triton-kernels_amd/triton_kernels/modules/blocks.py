@@ -301,16 +301,26 @@ class DoubleStreamBlock(nn.Module):
         img_mod1, img_mod2, txt_mod1, txt_mod2, beside = self._modulations(vec, takes_rows(B * H, Lt + Li, hid // H, 2 * B, hid))
         img_qkv_lin, txt_qkv_lin = self.img_attn.qkv, self.txt_attn.qkv
         img_m, txt_m = layer_norm_modulation_pair((img, img_mod1.scale, img_mod1.shift), (txt, txt_mod1.scale, txt_mod1.shift))
+        qkv = None
         if plain(img_qkv_lin, Linear) and plain(txt_qkv_lin, Linear):
-            img_qkv, txt_qkv = linear_pair_into(dict(x=img_m, w=img_qkv_lin.weight, b=img_qkv_lin.bias),
-                                                dict(x=txt_m, w=txt_qkv_lin.weight, b=txt_qkv_lin.bias))
+            # One batch element: the text's rows and behind them the image's in one buffer, where v is as the attention reads it, and only q and k
+            # are normalised, rotated and joined. qkv_prep at 4096 + 512 tokens 34.7 -> 26.3 us, at 1024 + 256 12.3 -> 10.1.
+            if B == 1:
+                qkv = torch.empty((Lt + Li, 3 * hid), dtype=img.dtype, device=img.device)
+            outs = ({}, {}) if qkv is None else (dict(out=qkv[Lt:]), dict(out=qkv[:Lt]))
+            img_qkv, txt_qkv = linear_pair_into(dict(x=img_m, w=img_qkv_lin.weight, b=img_qkv_lin.bias, **outs[0]),
+                                                dict(x=txt_m, w=txt_qkv_lin.weight, b=txt_qkv_lin.bias, **outs[1]))
         else:
             img_qkv, txt_qkv = img_qkv_lin(img_m), txt_qkv_lin(txt_m)
         img_q, img_k, img_v = _heads(img_qkv.view(B, Li, 3 * hid), H)
         txt_q, txt_k, txt_v = _heads(txt_qkv.view(B, Lt, 3 * hid), H)
+        if qkv is not None:
+            img_v = txt_v = None
         q, k, v = qkv_prep(img_q, img_k, img_v, txt_q, txt_k, txt_v, pe=pe,
                            q_scale_img=self.img_attn.norm.query_norm.scale, k_scale_img=self.img_attn.norm.key_norm.scale,
                            q_scale_txt=self.txt_attn.norm.query_norm.scale, k_scale_txt=self.txt_attn.norm.key_norm.scale)
+        if qkv is not None:
+            v = _heads(qkv.unsqueeze(0), H)[2]
         attn = torch.empty((B, Lt + Li, hid), dtype=img.dtype, device=img.device)
         attention_into(q, k, v, attn.view(B, Lt + Li, H, hid // H).permute(0, 2, 1, 3), beside=beside)
 

@@ -293,7 +293,7 @@ def test_attention_lse_sums_unrounded_probabilities(B, H, L, D):
 
 
 # 128-row workgroups whose keys are cut in parts: equal and shorter last parts, a last tile of one key, ragged rows
-_SPLIT = [(1, 2, 2048), (1, 2, 4096), (2, 1, 2049), (1, 2, 1793), (1, 4, 2500), (1, 1, 3000)]
+_SPLIT = [(1, 2, 2048), (1, 2, 4096), (2, 1, 2049), (1, 2, 1793), (1, 4, 2500), (1, 1, 3000), (4, 2, 2048), (2, 4, 1737)]
 
 
 @pytest.mark.parametrize("D", [128, 64])

@@ -1415,14 +1415,12 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel_pair(AttnParams p4
 // rest of the GPU does; a part costs the traffic of its fp32 results, 0.033 us (0.016) per workgroup, and the
 // second launch about 2 us, both fitted to 46 problems of 2 to 24 heads. More than 256 workgroups would
 // share CUs, which gains nothing (LDS-bound). us before -> after at head dim 128, [1, 2, L]: L 2048
-// 38.7 -> 20.2, 4096 70.6 -> 33.3; [1, 4, 4096] 72.5 -> 51.3; [1, 8, 1500] 31.0 -> 27.3 is
-// not taken: below 6 us the host's part in the second launch can cost what the GPU gains. Nor are calls that take
-// the GPU less than the 22 us that a call in parts takes the host: passes of [1, 2, 1420, 64] 20.7 us in one
-// part and 21.0 to 22.1 in parts, of [1, 2, 1024, 128] 22.2 and 21.2 to 22.4, of [1, 2, 1800, 64] 24.9 and 21.2.
+// 38.7 -> 20.2, 4096 70.6 -> 33.3; [1, 4, 4096] 72.5 -> 51.3; [1, 8, L]: L 1280 25.7 -> 23.6, 1536 29.9 -> 27.5, 2048 39.2 -> 35.1 (head dim 64:
+// 27.1 -> 24.0). The model is off by up to 0.9 us, which a part has to gain at least; calls that take the GPU less than 23 us stay whole.
 static int attn_splits(int64_t BH, int64_t L, int D, int& part_keys) {
     const int64_t groups = BH * ((L + 127) / 128), key_tiles = (L + 63) / 64;
     const double tile_us = D == 128 ? 1.03 : 0.68, fixed_us = D == 128 ? 1.8 : 2.4, group_us = D == 128 ? 0.033 : 0.016;
-    double best = 6.0;
+    double best = 1.5;
     int parts = 1;
     part_keys = static_cast<int>(L);
     if ((D == 128 ? 6.0 : 5.1) + tile_us * static_cast<double>(key_tiles) < 23.0) return parts;

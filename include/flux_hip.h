@@ -242,6 +242,9 @@ typedef struct flux_linear_plan {
     int32_t checked;     /* 1: the tile's epilogue can decide per column and address rows in 64 bits (square tiles always) */
 } flux_linear_plan;
 int flux_linear_plan_of(const flux_linear_args* first, const flux_linear_args* second, int64_t workspace_bytes, flux_linear_plan* plan);
+/* Whether the q/k epilogue of an M x N x K projection of `heads` heads of 128 takes less time than a plain product and
+ * flux_qkv_prep behind it. A matter of speed only: calls with the epilogue are taken either way. */
+int flux_linear_qk_pays(int64_t M, int64_t N, int64_t K, int64_t heads);
 
 /* ---------------------------------------------------------------------------------------------
  * Non-causal attention forward: O = softmax(Q K^T * sm_scale) V, bf16 in/out, fp32 online softmax.

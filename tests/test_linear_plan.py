@@ -181,3 +181,17 @@ def test_calls_beside_another_stream_keep_their_eight_wave_tiles():
     for _ in range(2000):
         M, N, K = round(2 ** rng.uniform(8, 14)), 8 * round(2 ** rng.uniform(7, 11.5)), 64 * rng.randint(16, 240)
         assert plan_of(linear_args(M, N, K, flags=nv.LINEAR_SHARED_GPU)).family != RECT
+
+
+@pytest.mark.parametrize("rows,pays", [(256, 0), (320, 0), (384, 1), (448, 0), (512, 0), (640, 1), (704, 1), (896, 0), (1024, 0), (1280, 1), (1700, 1), (4608, 1), (13008, 1)])
+def test_qk_epilogue_where_it_pays(rows, pays):
+    """Two rounds of the epilogue's tiles at most: on the side that was measured faster; beyond: always."""
+    assert nv.lib().flux_linear_qk_pays(rows, 21504, 3072, 24) == pays
+
+
+def test_qk_epilogue_rule_takes_any_size():
+    for sizes in ((0, 21504, 3072, 24), (320, 0, 3072, 24), (320, 21504, 0, 24), (320, 21504, 3072, 0), (320, 512, 3072, 3), (1 << 40, 21504, 3072, 24), (320, 21504, 3072, 1 << 60), (-1, -1, -1, -1)):
+        assert nv.lib().flux_linear_qk_pays(*sizes) == 1
+    for rows in (1, 255, 2047, 1 << 30):
+        for n, k, heads in ((256, 8, 1), (768, 64, 2), (9216, 3072, 24), (21504, 1 << 20, 24)):
+            assert nv.lib().flux_linear_qk_pays(rows, n, k, heads) in (0, 1)

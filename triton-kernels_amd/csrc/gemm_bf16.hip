@@ -20,6 +20,7 @@
 // more and leaves as full 16-byte row segments, where the optional gated residual is applied.
 #include "gemm_common.h"
 #include "gemm_rows.h"
+#include <limits.h>
 #include <stdlib.h>
 #include <algorithm>
 
@@ -1089,6 +1090,34 @@ extern "C" int64_t flux_linear_pair_workspace_bytes(const flux_linear_pair_args*
 extern "C" int flux_linear_bf16_pair(const flux_linear_pair_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
     if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace)))) return fail(FLUX_E_NULL, "flux_linear_bf16_pair: workspace must be 16-byte aligned memory");
     return linear_pair_launch(a, workspace, workspace_bytes, nullptr, static_cast<hipStream_t>(stream));
+}
+
+// The q/k epilogue needs waves of 128 columns, which leaves three tile shapes. Where those need a round that is mostly empty, or twice the rows,
+// a plain product on a better shape and the preparation kernel behind it take less. Both are priced here: the product as plan_tiles does,
+// the epilogue 1.5 us on eight-wave tiles and 5 on the others, the preparation 4.2 us of launch and latency and 0.83 us per million values of q
+// and k, fitted to passes of the single block of 24 heads and 21504 columns. Passes with the epilogue and with the preparation (us): 320 rows 127.4
+// and 124.1, 384 134.7 135.2, 448 157.5 144.3, 512 161.4 153.2, 640 176.0 178.0, 704 196.0 205.3, 896 258.0 242.3, 1024 272.1 261.6, 1280 303.7
+// 307.4. From three rounds on the prices are off by as much as the two differ: 1700 414.2 and 424.2, priced 2.5 the other way.
+extern "C" int flux_linear_qk_pays(int64_t M, int64_t N, int64_t K, int64_t heads) {
+    if (M <= 0 || N <= 0 || K <= 0 || heads <= 0 || M > INT_MAX || N > INT_MAX || K > INT_MAX || heads > N / 256) return 1;
+    GemmSet g = {};
+    g.n = 1;
+    GemmParams& p = g.p[0];
+    p.M = static_cast<int>(M);
+    p.N = static_cast<int>(N);
+    p.K = static_cast<int>(K);
+    p.lda = p.ldw = K;
+    p.ldy = p.ldy2 = N;
+    p.rows_per_batch = p.M;
+    p.split_n = p.act_begin = static_cast<int>(std::min(N, 3 * heads * 128));
+    p.act = FLUX_ACT_GELU_TANH;
+    p.vec_io = 1;
+    const TilePlan plain = plan_tiles(g, false, 0);
+    p.qk_cols = static_cast<int>(2 * heads * 128);
+    const TilePlan fused = plan_tiles(g, false, 0);
+    if (tile_count(g, {fused.family, fused.fm, fused.fn, 0.0}) > 2 * kGemmCUs) return 1;
+    const double prepared = 4.2 + 0.83e-6 * static_cast<double>(M) * p.qk_cols;
+    return fused.us + (fused.family == kPair ? 1.5 : 5.0) <= plain.us + prepared ? 1 : 0;
 }
 
 extern "C" int flux_linear_plan_of(const flux_linear_args* first, const flux_linear_args* second, int64_t workspace_bytes, flux_linear_plan* plan) {

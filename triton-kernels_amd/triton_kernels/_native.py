@@ -122,6 +122,7 @@ SIGNATURES = {
     "flux_linear_pair_workspace_bytes": (c_int64, [POINTER(LinearPairArgs)]),
     "flux_linear_bf16_pair": (c_int32, [POINTER(LinearPairArgs), c_void_p, c_int64, c_void_p]),
     "flux_linear_plan_of": (c_int32, [POINTER(LinearArgs), POINTER(LinearArgs), c_int64, POINTER(LinearPlan)]),
+    "flux_linear_qk_pays": (c_int32, [c_int64, c_int64, c_int64, c_int64]),
     "flux_attention_fwd_bf16": (c_int32, [POINTER(AttnArgs), c_void_p]),
     "flux_attention_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int32]),
     "flux_attention_fwd_bf16_ws": (c_int32, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p]),

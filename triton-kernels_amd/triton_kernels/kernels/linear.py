@@ -260,6 +260,12 @@ def qk_fusable(x: Tensor, w: Tensor, seq_len: int, head_dim: int) -> bool:
             and N % 256 == 0 and w.shape[1] % 8 == 0 and -(-M // 256) * (N // 256) >= 160)
 
 
+def qk_pays(rows: int, w: Tensor, heads: int) -> bool:
+    """Whether a projection that qk_fusable() names is faster with the epilogue than with qkv_prep behind it: below two rounds of its tiles
+    that depends on how the rows fall on the shapes that either way has."""
+    return nv.lib().flux_linear_qk_pays(rows, w.shape[0], w.shape[1], heads) != 0
+
+
 def linear(x: Tensor, w: Tensor, b: Tensor | None, activation: str = "", shared_gpu: bool = False) -> Tensor:
     act = _ACTIVATIONS.get(activation)
     if act is not None and launch_hook is None and not shared_gpu and not is_compiling():

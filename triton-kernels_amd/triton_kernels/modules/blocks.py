@@ -25,7 +25,7 @@ from torch import Tensor
 
 from triton_kernels import _native as nv
 from triton_kernels.kernels.attention import attention_into, scaled_dot_product_attention, takes_rows
-from triton_kernels.kernels.linear import linear, linear_into, linear_pair_into, qk_fusable
+from triton_kernels.kernels.linear import linear, linear_into, linear_pair_into, qk_fusable, qk_pays
 from triton_kernels.kernels.normalization import layer_norm_modulation, layer_norm_modulation_pair
 from triton_kernels.kernels.positional_embedding import apply_rope, qkv_prep
 from triton_kernels.modules.normalization import QKNorm, plain
@@ -217,7 +217,7 @@ class SingleStreamBlock(nn.Module):
         hook = self.stage_hook or (lambda stage, edge: None)
         hook("linear1", "begin")
         pe_ok = pe.dtype == torch.float32 and pe.is_contiguous() and pe.numel() in (L * D * 2, B * L * D * 2)
-        if self.fuse_qk_epilogue and pe_ok and qk_fusable(x_mod, self.linear1.weight, L, D):
+        if self.fuse_qk_epilogue and pe_ok and qk_fusable(x_mod, self.linear1.weight, L, D) and qk_pays(M, self.linear1.weight, H):
             # linear1: q and k columns -> bias, RMSNorm, RoPE -> q, k [B,H,L,D]; v columns -> qkv;
             # mlp columns -> GELU -> both[:, hid:]
             q = torch.empty((B, H, L, D), dtype=x.dtype, device=x.device)

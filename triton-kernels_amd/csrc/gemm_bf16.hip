@@ -746,12 +746,22 @@ static const double kIdleShare = 0.31;   // a workgroup runs up to this much fas
 static const double kSplitHostUs = 6.0;  // K in parts costs the host this much more, ...
 static const double kSplitCallUs = 20.0; // ... in all about this much
 
+// us per slab of K. The prices were measured with weights in the Infinity Cache. From HBM a CU takes in no more than 55 bytes per ns. The smallest tiles,
+// with the most bytes per product, ask for more, and so does any tile of two products of up to 1024 rows together, where few tiles share a column of W.
+// us by the prices alone -> so: 256 + 64 rows x 3072 x 12288 67.8 (64 x 64 tiles) -> 53.2 (128 x 192 in five parts), 80 + 40 57.1 -> 43.8, 300 + 80
+// 56.8 -> 54.6, 570 + 20 87.1 -> 63.3, 64 x 3072 x 15360 44.7 -> 32.1, 180 x 3072 x 15360 39.4 -> 39.9; 512 + 128 rows and more as before. Applied to every
+// launch it ranks larger tiles worse than their prices: 1536 + 256 rows 135.6 -> 146.8, 512 rows x 3072 x 15360 52.4 -> 54.3.
+static double slab_us(const GemmSet& g, const TileShape& t) {
+    const bool few = t.fm + t.fn <= 6 || (g.n == 2 && g.p[0].M + g.p[1].M <= 1024);
+    return few && weights_from_hbm(g) ? std::max(t.slab_us, (t.fm + t.fn) * 4096 / 55e3) : t.slab_us;
+}
+
 static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
     const int64_t tiles = tile_count(g, t) * splits;
     const int64_t rounds = (tiles + kGemmCUs - 1) / kGemmCUs;
     const double fill = static_cast<double>(tiles) / (rounds * kGemmCUs);
     const int slabs = ((g.p[0].K + 63) / 64 + splits - 1) / splits;
-    const double us = rounds * ((t.family == kPair ? kTilePair : kTileLarge) + slabs * t.slab_us * (1.0 - kIdleShare * (1.0 - fill)));
+    const double us = rounds * ((t.family == kPair ? kTilePair : kTileLarge) + slabs * slab_us(g, t) * (1.0 - kIdleShare * (1.0 - fill)));
     // Below the time the weights take to arrive, shapes would be alike: the one with less of its own to do comes first
     // (12288 columns of 3072 at 64 rows: 64 x 64 tiles 19 us, 96 x 96 23, 192 x 128 30).
     const double weights_us = 2e-3 * g.n * g.p[0].N * g.p[0].K / kWeightGBs;
@@ -760,7 +770,7 @@ static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
 
 // No more than tile_cost_us in `splits` or more parts: the work spread evenly over the CUs, and the traffic of the parts.
 static double split_floor_us(const GemmSet& g, const TileShape& t, int splits) {
-    return kLaunch + kReduce + kTilePair + tile_count(g, t) * (g.p[0].K / 64) * t.slab_us / kGemmCUs + 2e-3 * split_bytes(g, t, splits) / kSplitGBs;
+    return kLaunch + kReduce + kTilePair + tile_count(g, t) * (g.p[0].K / 64) * slab_us(g, t) / kGemmCUs + 2e-3 * split_bytes(g, t, splits) / kSplitGBs;
 }
 
 // The best eight-wave tile for a product whose K is not cut.

@@ -538,6 +538,9 @@ __device__ __forceinline__ void gemm_finish_rect(const GemmParams& p, f32x4 (&ac
     }
 }
 
+// Whether a program is unlikely to find a launch's weights in the Infinity Cache: they are more than a third of it.
+inline bool weights_from_hbm(const GemmSet& g) { return static_cast<int64_t>(g.n) * g.p[0].N * g.p[0].K * 2 > (int64_t{256} << 20) / 3; }
+
 inline GemmLaunch make_launch(const GemmSet& g, int bm, int bn) {
     GemmLaunch L;
     const GemmParams& p = g.p[0];

@@ -30,7 +30,6 @@ namespace flux {
 // and 59.3 -> 60.7, so a W of up to a third of that cache, which a program may find there, is walked in turn. Two products in a launch gain
 // nothing (1024 + 256 x 3072 x 12288 99.6 and 100.2): the second's one row of tiles has nobody to share with and ends last. Groups of two and
 // four times as many slabs: 48.0 and 49.2 us at the first size. The order is worked out between the slabs: inside one it took 1 % of 512 x 3072 x 3072.
-constexpr int64_t kInfinityCacheBytes = int64_t(256) << 20;
 constexpr int kPairThreads = 512;
 
 template <int FM, int FN, int ST, bool KTAIL, int G>
@@ -257,7 +256,7 @@ template <int FM, int FN, int ST>
 static void launch_pair(const GemmSet& g, int splits, float* partial, hipStream_t st) {
     const int K = g.p[0].K;
     GemmLaunch L = make_launch(g, 32 * FM, 32 * FN);
-    L.take_turns = g.n == 1 && static_cast<int64_t>(g.p[0].N) * K * 2 > kInfinityCacheBytes / 3;
+    L.take_turns = g.n == 1 && weights_from_hbm(g);
     if (splits > 1) {   // (whole slabs only)
         L.slabs_per_split = (K / 64 + splits - 1) / splits;
         L.splits = (K / 64 + L.slabs_per_split - 1) / L.slabs_per_split;

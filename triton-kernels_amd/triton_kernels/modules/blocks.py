@@ -7,7 +7,8 @@ passes compute the same function with fewer trips through HBM:
   * linear1 of the single block writes its qkv columns and its GELU'd mlp columns straight into the
     two buffers the rest of the block reads (no split / nn.GELU / torch.cat passes),
   * QK RMSNorm + RoPE (+ the txt/img concat of the double block) is one gather kernel reading the
-    strided qkv projection in place; v is never copied in the single block,
+    strided qkv projection in place, or the projection's epilogue where that is faster; v is not copied in the single
+    block, nor in the double block for one batch element,
   * attention writes its output in "B L (H D)" order into the buffer linear2 / proj consumes,
   * the gated residual x + gate * y is the epilogue of the last linear.
 

@@ -401,7 +401,7 @@ def test_linear_every_tile(family, tile_m, tile_n, whole, tail, parts):
 @pytest.mark.parametrize("M,N,K", [
     (320, 10920, 4096), (320, 10928, 4096),    # the last W walked in turn and the first one that is not
     (330, 3072, 15360), (1100, 3072, 15360),   # K in parts, two tile rows; groups of four and of three
-    (900, 3072, 15360),                        # a group of four and a tile row of its own
+    (940, 3072, 15360), (900, 3072, 15360),    # a group of four and a tile row of its own, full enough and not
     (400, 15000, 3080), (1000, 2920, 15416),   # K tail in a last group of slabs that is shorter and in a whole one
 ])
 def test_linear_slabs_out_of_turn(M, N, K):

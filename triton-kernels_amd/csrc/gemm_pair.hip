@@ -29,7 +29,9 @@ namespace flux {
 // 44.1 -> 42.6, 640 x 3072 x 15360 64.3 -> 62.3; the fused projection of 320 rows 58.9 -> 54.6. W from the Infinity Cache: 41.0 -> 42.1, 40.1 -> 41.1
 // and 59.3 -> 60.7, so a W of up to a third of that cache, which a program may find there, is walked in turn. Two products in a launch gain
 // nothing (1024 + 256 x 3072 x 12288 99.6 and 100.2): the second's one row of tiles has nobody to share with and ends last. Groups of two and
-// four times as many slabs: 48.0 and 49.2 us at the first size. The order is worked out between the slabs: inside one it took 1 % of 512 x 3072 x 3072.
+// four times as many slabs: 48.0 and 49.2 us at the first size. From four tile rows on the last one has to be three quarters full: one of mostly padding
+// runs ahead of its neighbours and is then the first at every slab. K = 15360, full or nearly: 1024 rows 102.8 -> 92.9, 1600 156.0 -> 138.3, 1900 169.3 ->
+// 159.4, 2048 177.8 -> 163.0; hardly filled: 1152 102.8 -> 106.1, 1402 118.4 -> 121.1, 1750 149.0 -> 154.2, 2100 170.8 -> 175.6 (in turn now). The order is worked out between the slabs: inside one it took 1 % of 512 x 3072 x 3072.
 constexpr int kPairThreads = 512;
 
 template <int FM, int FN, int ST, bool KTAIL, int G>
@@ -256,7 +258,7 @@ template <int FM, int FN, int ST>
 static void launch_pair(const GemmSet& g, int splits, float* partial, hipStream_t st) {
     const int K = g.p[0].K;
     GemmLaunch L = make_launch(g, 32 * FM, 32 * FN);
-    L.take_turns = g.n == 1 && weights_from_hbm(g);
+    L.take_turns = g.n == 1 && weights_from_hbm(g) && (L.tiles_m < 4 || 4 * (g.p[0].M - (L.tiles_m - 1) * 32 * FM) >= 3 * 32 * FM);
     if (splits > 1) {   // (whole slabs only)
         L.slabs_per_split = (K / 64 + splits - 1) / splits;
         L.splits = (K / 64 + L.slabs_per_split - 1) / L.slabs_per_split;

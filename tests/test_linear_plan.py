@@ -183,6 +183,19 @@ def test_calls_beside_another_stream_keep_their_eight_wave_tiles():
         assert plan_of(linear_args(M, N, K, flags=nv.LINEAR_SHARED_GPU)).family != RECT
 
 
+@pytest.mark.parametrize("rows,N,K,tile", [
+    # what HBM feeds a CU counts: one row of tiles, two products of few rows
+    ((64,), 3072, 15360, (64, 64, 4)), ((96,), 3072, 15360, (64, 96, 4)), ((90,), 12288, 4096, (64, 96, 1)), ((256, 64), 3072, 12288, (128, 192, 5)), ((570, 20), 3072, 12288, (192, 192, 4)),
+    # and does not: another tile was up to a third slower
+    ((97,), 3072, 15360, (64, 96, 4)), ((180,), 3072, 15360, (96, 96, 4)), ((129,), 12288, 4096, (96, 96, 1)), ((97,), 8192, 8192, (64, 64, 1)),
+    ((168, 488), 9216, 3072, (256, 128, 1)), ((65, 35), 16384, 4096, (160, 128, 1)), ((258, 498), 6144, 6144, (192, 128, 1)), ((150, 10), 4096, 16384, (64, 64, 1)),
+    ((713, 279), 16384, 4096, (192, 128, 1))])
+def test_tiles_of_few_rows_and_weights_from_hbm(rows, N, K, tile):
+    """The faster one of the tiles that the prices alone and the bound by HBM come to, weights from HBM."""
+    p = plan_of(*(linear_args(M, N, K) for M in rows))
+    assert (p.products, p.tile_m, p.tile_n, p.splits) == (len(rows), *tile)
+
+
 @pytest.mark.parametrize("rows,pays", [(256, 0), (320, 0), (384, 1), (448, 0), (512, 0), (640, 1), (704, 1), (896, 0), (1024, 0), (1280, 1), (1700, 1), (4608, 1), (13008, 1)])
 def test_qk_epilogue_where_it_pays(rows, pays):
     """Two rounds of the epilogue's tiles at most: on the side that was measured faster; beyond: always."""

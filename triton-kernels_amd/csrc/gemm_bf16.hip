@@ -746,22 +746,23 @@ static const double kIdleShare = 0.31;   // a workgroup runs up to this much fas
 static const double kSplitHostUs = 6.0;  // K in parts costs the host this much more, ...
 static const double kSplitCallUs = 20.0; // ... in all about this much
 
-// us per slab of K. The prices were measured with weights in the Infinity Cache. From HBM a CU takes in no more than 55 bytes per ns. The smallest tiles,
-// with the most bytes per product, ask for more, and so does any tile of two products of up to 1024 rows together, where few tiles share a column of W.
-// us by the prices alone -> so: 256 + 64 rows x 3072 x 12288 67.8 (64 x 64 tiles) -> 53.2 (128 x 192 in five parts), 80 + 40 57.1 -> 43.8, 300 + 80
-// 56.8 -> 54.6, 570 + 20 87.1 -> 63.3, 64 x 3072 x 15360 44.7 -> 32.1, 180 x 3072 x 15360 39.4 -> 39.9; 512 + 128 rows and more as before. Applied to every
-// launch it ranks larger tiles worse than their prices: 1536 + 256 rows 135.6 -> 146.8, 512 rows x 3072 x 15360 52.4 -> 54.3.
-static double slab_us(const GemmSet& g, const TileShape& t) {
-    const bool few = t.fm + t.fn <= 6 || (g.n == 2 && g.p[0].M + g.p[1].M <= 1024);
-    return few && weights_from_hbm(g) ? std::max(t.slab_us, (t.fm + t.fn) * 4096 / 55e3) : t.slab_us;
+// us per slab of K. The prices were measured with weights in the Infinity Cache. From HBM a CU takes in no more than 55 bytes per ns where nobody else
+// brings its weights in: one product of up to 96 rows in a single row of tiles, or, with `from_hbm`, two products of few rows (see plan_tiles).
+// us, weights from HBM (from the cache), by the prices alone -> so: 64 x 3072 x 15360 44.6 -> 29.1 (27.8 -> 20.8), 90 x 3072 x 15360 37.6 -> 30.3 (24.5 ->
+// 23.0), 90 x 12288 x 4096 34.5 -> 27.5 (20.7 -> 19.8), 90 x 9216 x 6144 51.0 -> 38.7 (28.8 -> 25.4). More rows: tiles of a column share its weights, and
+// a single row of larger tiles is priced well enough. Bounded too, 145 x 3072 x 15360 took 33.7 (27.3) and not 37.5 (26.1), but 129 x 8192 x 8192 49.7 (37.7)
+// and not 50.0 (33.4), 210 x 9216 x 6144 47.9 (36.5) and not 44.2 (34.0).
+static double slab_us(const GemmSet& g, const TileShape& t, bool from_hbm) {
+    const bool bound = g.n == 1 ? g.p[0].M <= std::min(96, 32 * t.fm) : from_hbm;
+    return bound && weights_from_hbm(g) ? std::max(t.slab_us, (t.fm + t.fn) * 4096 / 55e3) : t.slab_us;
 }
 
-static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
+static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits, bool from_hbm = false) {
     const int64_t tiles = tile_count(g, t) * splits;
     const int64_t rounds = (tiles + kGemmCUs - 1) / kGemmCUs;
     const double fill = static_cast<double>(tiles) / (rounds * kGemmCUs);
     const int slabs = ((g.p[0].K + 63) / 64 + splits - 1) / splits;
-    const double us = rounds * ((t.family == kPair ? kTilePair : kTileLarge) + slabs * slab_us(g, t) * (1.0 - kIdleShare * (1.0 - fill)));
+    const double us = rounds * ((t.family == kPair ? kTilePair : kTileLarge) + slabs * slab_us(g, t, from_hbm) * (1.0 - kIdleShare * (1.0 - fill)));
     // Below the time the weights take to arrive, shapes would be alike: the one with less of its own to do comes first
     // (12288 columns of 3072 at 64 rows: 64 x 64 tiles 19 us, 96 x 96 23, 192 x 128 30).
     const double weights_us = 2e-3 * g.n * g.p[0].N * g.p[0].K / kWeightGBs;
@@ -769,8 +770,8 @@ static double tile_cost_us(const GemmSet& g, const TileShape& t, int splits) {
 }
 
 // No more than tile_cost_us in `splits` or more parts: the work spread evenly over the CUs, and the traffic of the parts.
-static double split_floor_us(const GemmSet& g, const TileShape& t, int splits) {
-    return kLaunch + kReduce + kTilePair + tile_count(g, t) * (g.p[0].K / 64) * slab_us(g, t) / kGemmCUs + 2e-3 * split_bytes(g, t, splits) / kSplitGBs;
+static double split_floor_us(const GemmSet& g, const TileShape& t, int splits, bool from_hbm) {
+    return kLaunch + kReduce + kTilePair + tile_count(g, t) * (g.p[0].K / 64) * slab_us(g, t, from_hbm) / kGemmCUs + 2e-3 * split_bytes(g, t, splits) / kSplitGBs;
 }
 
 // The best eight-wave tile for a product whose K is not cut.
@@ -805,7 +806,7 @@ static GemmSet rows_behind(const GemmSet& g, int rows) {
     return tail;
 }
 
-static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_bytes) {
+static TilePlan plan_priced(const GemmSet& g, bool shared_gpu, int64_t workspace_bytes, bool from_hbm) {
     // The branch-free epilogue of the rectangular and eight-wave tiles: 16-byte outputs, a wave's columns on one
     // side of split_n and act_begin, no GELU in front of a gate. The square and the eight-wave tiles have one for
     // anything else as well. (Without it on the eight-wave tiles, calls outside the form ran on square ones: 64 x 3072
@@ -838,7 +839,7 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
         // which replace eight-wave tiles too, would only hide those: 6100 x 9216 x 3072 272 us, 292 on square tiles.
         if (t.family == kRect && t.fn > 6 && p.qk_cols == 0 && (p.K < 1024 || shared_gpu)) continue;
         if ((t.family == kRect || (t.family == kPair && t.fn == 8)) && !columns_ok(t.fn)) continue;
-        const double us = tile_cost_us(g, t, 1);
+        const double us = tile_cost_us(g, t, 1, from_hbm);
         if (us < best.us) best = {t.family, t.fm, t.fn, 1, us, t.family == kPair && !columns_ok(t.fn)};
     }
     // K in parts, where that gains more than the host pays for it: a workspace to allocate and a second launch, 6 us
@@ -851,8 +852,8 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
             if (t.family != kPair || t.fn == 8) continue;
             for (int s = 2; s <= 10; ++s) {
                 if (tile_count(g, t) * s > 2 * kGemmCUs || (p.K / 64) / s < 4 || split_bytes(g, t, s) > workspace_bytes) break;
-                if (split_floor_us(g, t, s) > split.us) break;
-                const double us = tile_cost_us(g, t, s);
+                if (split_floor_us(g, t, s, from_hbm) > split.us) break;
+                const double us = tile_cost_us(g, t, s, from_hbm);
                 if (us < split.us) split = {kPair, t.fm, t.fn, s, us, !columns_ok(t.fn)};
             }
         }
@@ -874,6 +875,25 @@ static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_
     // Beside another stream's work: square tiles leave that work the CUs of their last round.
     if (shared_gpu && best.family == kRect) best = {kSquare, 8, 8, 1, best.us};
     return best;
+}
+
+// Two products of few rows share few columns of weights among their tiles, so what HBM feeds a CU bounds them as well, where the weights come from
+// there. A plan is then made both ways, and the one by that bound is taken where it gains at least 3.5 us by it: smaller gains are within what the
+// model is off by (258 + 498 x 6144 x 6144 72 us by the prices, 81 by the bound, for 1.4 us less in the model; 312 + 35 x 3072 x 12288 49 and 51 for 3.0,
+// 168 + 488 x 9216 x 3072 48 and 53 for 1.2). Up to 768 rows and K = 12288: beyond, either plan may be the worse one (1536 + 256 x 3072 x 12288 136 us by the
+// prices and 147 by the bound, 713 + 279 x 16384 x 4096 142 and 158, 150 + 10 x 4096 x 16384 70 and 78).
+// us, weights from HBM (from the cache), by the prices -> so: 256 + 64 x 3072 x 12288 67.3 -> 48.5 (42.3 -> 38.1), 80 + 40 58.0 -> 43.6 (39.9 -> 30.6), 570 +
+// 20 88.4 -> 63.5 (59.7 -> 55.1), 660 + 60 86.0 -> 70.4 (60.1 -> 65.3), 89 + 272 58.2 -> 49.7 (38.9 -> 41.5), 113 + 53 x 9216 x 3072 37.8 -> 33.5 (25.7 -> 23.7).
+static TilePlan plan_tiles(const GemmSet& g, bool shared_gpu, int64_t workspace_bytes) {
+    const TilePlan plan = plan_priced(g, shared_gpu, workspace_bytes, false);
+    if (g.n == 1 || g.p[0].M + g.p[1].M > 768 || g.p[0].K > 12288 || !weights_from_hbm(g)) return plan;
+    const TilePlan bound = plan_priced(g, shared_gpu, workspace_bytes, true);
+    auto cost = [&](const TilePlan& of) {
+        for (const TileShape& t : kTileShapes)
+            if (t.family == of.family && t.fm == of.fm && t.fn == of.fn) return tile_cost_us(g, t, of.splits, true);
+        return 0.0;
+    };
+    return cost(plan) - cost(bound) >= 3.5 ? bound : plan;
 }
 
 // How a call can be served.

@@ -402,10 +402,11 @@ def test_linear_every_tile(family, tile_m, tile_n, whole, tail, parts):
     (320, 10920, 4096), (320, 10928, 4096),    # the last W walked in turn and the first one that is not
     (330, 3072, 15360), (1100, 3072, 15360),   # K in parts, two tile rows; groups of four and of three
     (940, 3072, 15360), (900, 3072, 15360),    # a group of four and a tile row of its own, full enough and not
+    (470, 3072, 15360), (500, 8200, 6152),     # three tile rows: K in parts, and a K tail in a last group of one slab
     (400, 15000, 3080), (1000, 2920, 15416),   # K tail in a last group of slabs that is shorter and in a whole one
 ])
 def test_linear_slabs_out_of_turn(M, N, K):
-    """Eight-wave tiles that walk K in rotated order, against the fp32 product: half a bf16 ulp plus the spread of an fp32 sum in another order."""
+    """Eight-wave tiles that walk K in orders of their own, against the fp32 product: half a bf16 ulp plus the spread of an fp32 sum in another order."""
     assert plan_of(linear_args(M, N, K)).family == EIGHT_WAVES
     g = seeded(M + N + K)
     a = randn(g, M, K, dtype=torch.bfloat16).to(DEV)

@@ -21,7 +21,7 @@ struct GemmLaunch {
     int tiles_m0;               // tile rows of the first product
     int splits;                 // > 1: every tile's K range is cut into this many parts, each a workgroup of its own
     int slabs_per_split;
-    bool take_turns;            // eight-wave tiles: neighbours walk K in rotated order (gemm_pair.hip)
+    bool take_turns;            // eight-wave tiles: neighbours walk K in orders of their own (gemm_pair.hip)
     float* partial;             // splits > 1: fp32 accumulators, [splits][tiles][4 waves][fragments][64 lanes][4]
 };
 

@@ -23,15 +23,17 @@ namespace flux {
 // same tiles: 50, 78, 120 and 21 us.
 // ------------------------------------------------------------------------------------------------
 // Slabs out of turn. Tiles that share columns of W run side by side and ask for the same slab at the same time, so each of them waits for it to
-// come from HBM. Where W is too large to be found in the Infinity Cache, the tiles of a column, `turns` of them, take every `turns` slabs of K
-// in an order rotated by their place: each is the first at one slab of such a group and finds the others in the L2, where its neighbours have brought
-// them. The same goes for A among the tiles of a row. us in turn -> rotated, W from HBM: 320 x 21504 x 3072 52.4 -> 46.8, 320 x 3072 x 15360
-// 44.1 -> 42.6, 640 x 3072 x 15360 64.3 -> 62.3; the fused projection of 320 rows 58.9 -> 54.6. W from the Infinity Cache: 41.0 -> 42.1, 40.1 -> 41.1
-// and 59.3 -> 60.7, so a W of up to a third of that cache, which a program may find there, is walked in turn. Two products in a launch gain
-// nothing (1024 + 256 x 3072 x 12288 99.6 and 100.2): the second's one row of tiles has nobody to share with and ends last. Groups of two and
-// four times as many slabs: 48.0 and 49.2 us at the first size. From four tile rows on the last one has to be three quarters full: one of mostly padding
-// runs ahead of its neighbours and is then the first at every slab. K = 15360, full or nearly: 1024 rows 102.8 -> 92.9, 1600 156.0 -> 138.3, 1900 169.3 ->
-// 159.4, 2048 177.8 -> 163.0; hardly filled: 1152 102.8 -> 106.1, 1402 118.4 -> 121.1, 1750 149.0 -> 154.2, 2100 170.8 -> 175.6 (in turn now). The order is worked out between the slabs: inside one it took 1 % of 512 x 3072 x 3072.
+// come from HBM. Where W is too large to be found in the Infinity Cache, the tiles of a column take every two or four slabs of K (`turns`, as many as there
+// are tiles, or one more than three) in an order of their own, slab i ^ turn: each is the first at some of a group and finds the others in the L2, where its
+// neighbours have brought them. The same goes for A among the tiles of a row. us, W from HBM, in turn -> so: 320 x 21504 x 3072 50.4 -> 47.3, 320 x 3072 x
+// 15360 45.2 -> 44.5, 640 65.7 -> 63.9, 1024 101.7 -> 92.3, 1600 154.9 -> 135.4, 1900 169.3 -> 154.4, 2048 177.4 -> 158.5. A W of more than a third of
+// that cache that is found there all the same costs 40.0 -> 40.4, 39.9 -> 40.5, 60.0 -> 61.6, 86.9 -> 89.4, 126.8 -> 127.9, 145.1 -> 148.4 and 150.2 -> 153.7 us; a smaller one is walked in turn.
+// The order has to be cheap: rotated by additions, a branch at the end of a group and a division at the head of the kernel, all tiles in turn took 3 % longer at 1600 and 1900
+// rows (130.6 and 148.9 us from the cache; 139.5 and 159.2 rotated, from HBM), and inside a slab instead of between two the order took 1 % of 512 x 3072 x 3072.
+// Two products in a launch gain nothing (1024 + 256 x 3072 x 12288 99.6 and 100.2): the second's one row of tiles has nobody to share with and ends
+// last. Groups of two and four times as many slabs: 48.0 and 49.2 us at the first size, 46.8 so. From four tile rows on the last one has to be three quarters full: one of
+// mostly padding runs ahead of its neighbours and is then the first at every slab (K = 15360, hardly filled: 1152 rows 102.8 -> 106.1, 1402 118.4 -> 121.1, 1750
+// 149.0 -> 154.2, 2100 170.8 -> 175.6, in turn now).
 constexpr int kPairThreads = 512;
 
 template <int FM, int FN, int ST, bool KTAIL, int G>
@@ -96,25 +98,9 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
         const int i = idx / FN, j = (i & 1) ? FN - 1 - idx % FN : idx % FN;
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[buf][j], xa[buf][i], acc[i][j], 0, 0, 0);
     };
-    // the slabs in the order of this tile; those of a last, shorter group in turn
+    // slab number i in the order of this tile; those of a last, shorter group in turn
     const bool rotated = turns > 1;
-    int group = kb, at = turn;
-    auto last_group = [&]() {
-        if (group + turns > ke) {
-            at = 0;
-            turn = turns = INT_MAX;
-        }
-    };
-    last_group();
-    auto next_slab = [&]() {
-        const int k = group + at;
-        if (++at == turns) at = 0;
-        if (at == turn) {
-            group += turns;
-            last_group();
-        }
-        return k;
-    };
+    auto slab_at = [&](int i) { return ((i - kb) | (turns - 1)) < ke - kb ? kb + ((i - kb) ^ turn) : i; };
     // k: the slab that is requested; cur: stage of the one that is multiplied (its fragments are in buffer `buf`), nxt: of the one behind it
     auto slab = [&](auto bufc, int k, int cur, int nxt) {
         constexpr int buf = decltype(bufc)::value;
@@ -141,7 +127,7 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
 
 #pragma unroll
     for (int s = 0; s < ST; ++s) {
-        const int k = rotated ? next_slab() : kb + s;
+        const int k = rotated ? slab_at(kb + s) : kb + s;
 #pragma unroll
         for (int j = 0; j < NL; ++j) load(s * SLAB, j, k);
     }
@@ -155,8 +141,8 @@ __device__ __forceinline__ void gemm_pair_slabs(const GemmParams& p, char* lds, 
         const int n1 = after(cur), n2 = after(n1);
         int k0 = kt + ST, k1 = kt + ST + 1;
         if (rotated) {
-            k0 = next_slab();
-            k1 = next_slab();
+            k0 = slab_at(k0);
+            k1 = slab_at(k1);
         }
         slab(ic<0>(), k0, cur, n1);
         if (kt + 1 < ke) slab(ic<1>(), k1, n1, n2);
@@ -183,8 +169,9 @@ __global__ __launch_bounds__(kPairThreads) void gemm_nt_pair_kernel(GemmLaunch L
     }
     int turn = 0, turns = 1;
     if (L.take_turns) {
-        turns = min(L.tiles_m - tm / L.group_m * L.group_m, L.group_m);
-        turn = (tm % L.group_m + tn) % turns;
+        const int tiles = min(L.tiles_m - tm / L.group_m * L.group_m, L.group_m);
+        turns = tiles > 2 ? 4 : tiles;
+        turn = (tm % L.group_m + tn) & (turns - 1);
     }
     const GemmParams p = L.p[product_of_tile(L, tm)];
     const int m0 = tm * BM, n0 = tn * BN;

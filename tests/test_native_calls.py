@@ -306,6 +306,7 @@ def test_calls_of_the_blocks_forms(monkeypatch):
         s, pe = t(128, dtype=dtype), t(1, 1, 13, 64, 2, 2, dtype=F32)
         for args, kw, served in (((*img, *txt), dict(pe=pe, q_scale_img=s, k_scale_img=s, q_scale_txt=s, k_scale_txt=s), True), ((*img, *txt), {}, True), ((img[0], img[1], None), dict(pe=pe[:, :, :9].double()), False),
                                  ((img[0], img[1], None), dict(pe=pe[:, :, :9].contiguous(), q_scale_img=s, k_scale_img=s), True), ((None, img[1], img[2]), {}, False), ((*img, txt[0], txt[1], txt[2].transpose(0, 1).contiguous().transpose(0, 1)), {}, True),
+                                 ((img[0], img[1], None, txt[0], txt[1], None), dict(pe=pe, q_scale_img=s, k_scale_img=s, q_scale_txt=s, k_scale_txt=s), True), ((img[0], img[1], None, txt[0], txt[1], None), {}, True),
                                  ((*(v[..., ::2] for v in img),), {}, False)):
             _served(monkeypatch, "qkv_prep", served, lambda: qkv_prep(*args, **kw))
         mod = t(2, 1, 6 * 256, dtype=dtype).chunk(6, -1)
@@ -315,6 +316,30 @@ def test_calls_of_the_blocks_forms(monkeypatch):
     qkv = t(2, 150, 3, heads, 128).permute(2, 0, 3, 1, 4)
     for kw, q, served in (({}, qkv[0], True), (dict(sm_scale=0.3), qkv[0].contiguous(), True), ({}, qkv[0].transpose(2, 3).contiguous().transpose(2, 3), False)):
         _served(monkeypatch, "attention", served, lambda: (attention_into(q, qkv[1], qkv[2], torch.zeros(2, 150, heads, 136, device=DEV, dtype=BF).permute(0, 2, 1, 3)[..., :128], **kw),))
+
+
+@gpu
+@pytest.mark.parametrize("kind,batch,tokens", [("single", 1, 96), ("single", 2, 300), ("double", 1, 96), ("double", 2, 96), ("double", 1, 1100), ("double", 5, 40)])
+def test_a_pass_of_a_fused_block_stays_in_native_code(monkeypatch, kind, batch, tokens):
+    """Every call that a fused block makes is served, with a modulation beside the attention or in front, one batch element or several."""
+    g, heads, hid, calls, native = seeded(batch + tokens), 4, 512, [], nv.ops()
+    blk = (tk.SingleStreamBlock(hid, heads) if kind == "single" else tk.DoubleStreamBlock(hid, heads, mlp_ratio=4.0, qkv_bias=True)).to(BF).to(DEV)
+    xs = [randn(g, batch, n, hid, dtype=BF).to(DEV) for n in ((tokens,) if kind == "single" else (tokens, 7))]
+    vec, pe = randn(g, batch, hid, dtype=BF).to(DEV), randn(g, 1, 1, sum(x.shape[1] for x in xs), 64, 2, 2).to(DEV)
+
+    class Spy:
+        def __getattr__(self, name):
+            return lambda *a: calls.append((name, getattr(native, name)(*a))) or calls[-1][1]
+
+    with torch.no_grad():
+        want = launcher(monkeypatch, blk, *xs, vec, pe)
+        with monkeypatch.context() as m:
+            m.setattr(nv, "ops", lambda: Spy())
+            got = blk(*xs, vec, pe)
+    assert [name for name, out in calls if out is None] == []
+    assert len(calls) == (6 if kind == "single" else 9)
+    for a, b in zip((got,) if kind == "single" else got, (want,) if kind == "single" else want):
+        assert torch.equal(a, b)
 
 
 @gpu

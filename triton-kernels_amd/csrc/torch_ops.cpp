@@ -9,9 +9,9 @@
 // turns with runs at half its speed (41 and 43 us, 129 for a step whose kernels take 30). A node of the
 // engine's own kind leaves the interpreter on one core. us a call, before -> now: q/k norm module at 256 tokens 25.5 -> 10.3,
 // training step of the norm at [4, 24, 1024, 128] 107 to 129 -> 57, rotation of short sequences 18.7 -> 6.9, linear at 512 x 3072
-// x 3072 15.8 -> 15.1 (the GPU's own time). The calls that the fused blocks are made of are here as well: seven of a single-stream
-// block took the host 126 to 132 us a pass (the GPU 131 at 320 tokens), now 67 to 72; ten of a double-stream block 329, now 132; first
-// passes on new weights at 320 tokens 281 -> 241, at 1024 + 256 579 -> 479.
+// x 3072 15.8 -> 15.1 (the GPU's own time). The calls that the fused blocks are made of are here as well. Host time of a pass: the six of a single-stream
+// block at 320 tokens 135 -> 78 (the GPU 120 there), the nine of a double-stream block at 1024 + 256 tokens 327 -> 160, of two batch elements
+// at 256 + 64 338 -> 155; first passes on new weights 304 -> 214, 586 -> 474 and 546 -> 396.
 #include <torch/csrc/python_headers.h>
 #include <ATen/ATen.h>
 #include <torch/csrc/Exceptions.h>
@@ -372,7 +372,7 @@ PyObject* py_qkv_prep(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int64_t B = q->size(0), H = q->size(1), Li = q->size(2), D = q->size(3), Lt = t[3] ? t[3]->size(2) : 0;
     for (int i = 0; i < 6; ++i) {
         if (!t[i]) {
-            if (i < 2 || (Lt > 0 && (i < 5 || t[2]))) Py_RETURN_NONE;   // (what one of the sources has, the others have)
+            if (i < 2 || (i >= 3 && Lt > 0 && t[i - 3])) Py_RETURN_NONE;   // (q and k are there; what the image has, the text has)
             continue;
         }
         if (i >= 3 && (Lt == 0 || !t[i - 3])) Py_RETURN_NONE;

@@ -278,11 +278,12 @@ int flux_attention_fwd_bf16(const flux_attn_args* args, void* stream);
 int64_t flux_attention_workspace_bytes(int64_t B, int64_t H, int64_t L, int32_t D);
 int flux_attention_fwd_bf16_ws(const flux_attn_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
-/* The same beside one or two products that neither read what the other writes nor write what it reads (product[1].M == 0: one).
+/* The same beside one or two products that neither read what the other writes nor write what it reads (product[1].M == 0: one, and
+ * nothing else of product[1] is read).
  * Products of up to 4 rows in all (K up to 24576 / M) that could share a launch of their own take workgroups of the attention's
  * launch where that is of head dim 128, of more than 64 rows and of at most 256 workgroups of 128 rows, which leave the memory idle.
- * In all other cases the products run in front of the attention. Results are those of flux_linear_bf16_pair and
- * flux_attention_fwd_bf16_ws. */
+ * In all other cases the products run in front of the attention. The workspace is the attention's: results are those of
+ * flux_linear_bf16_pair without one and of flux_attention_fwd_bf16_ws. */
 int flux_attention_rows_bf16(const flux_attn_args* args, const flux_linear_pair_args* rows, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------------

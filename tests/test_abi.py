@@ -91,6 +91,13 @@ def test_argument_checks_reject_before_launch():
     la.qk = None
     la.M = 0
     assert lib.flux_linear_bf16(ctypes.byref(la), None) == 0                                            # empty
+    a.B, a.D = 0, 128
+    pair = nv.LinearPairArgs()
+    pair.product[0] = la
+    assert lib.flux_attention_rows_bf16(ctypes.byref(a), ctypes.byref(pair), None, 0, None) == 0        # both empty, no second product (all zeros)
+    pair.product[1].M = 1
+    assert lib.flux_attention_rows_bf16(ctypes.byref(a), ctypes.byref(pair), None, 0, None) == -1       # a second product without operands
+    assert lib.flux_attention_rows_bf16(ctypes.byref(a), None, None, 0, None) == -1
     assert lib.flux_silu(p, p, -1, 0, None) == -2
     qa = nv.QkvPrepArgs()
     qa.B, qa.H, qa.Lt, qa.Li, qa.D = 1, 0, 0, 4, 128

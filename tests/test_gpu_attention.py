@@ -385,3 +385,22 @@ def test_attention_beside_row_products(B, H, L, D, M, K, Ns):
         for c in calls:
             assert torch.equal(c["out"], tk.linear_into(x, c["w"], c["b"], in_activation="SiLU"))
             assert torch.isnan(c["out"].as_strided((M, 3), (c["out"].stride(0), 1), c["out"].storage_offset() + c["w"].shape[0])).all()
+
+
+@pytest.mark.parametrize("L", [320, 64])
+def test_attention_beside_one_product(L):
+    """One product through the C entry, the second one's fields all zero, in the attention's launch and in front of it."""
+    g = seeded(L)
+    q, k, v = (randn(g, 1, 4, L, 128, dtype=torch.bfloat16).to(DEV) for _ in range(3))
+    x, w = randn(g, 2, 512, dtype=torch.bfloat16).to(DEV), randn(g, 333, 512, dtype=torch.bfloat16).to(DEV)
+    y, o = torch.full((2, 333), float("nan"), dtype=torch.bfloat16, device=DEV), torch.empty_like(q)
+    pair, a = nv.LinearPairArgs(), nv.AttnArgs()
+    p = pair.product[0]
+    p.A, p.W, p.Y = x.data_ptr(), w.data_ptr(), y.data_ptr()
+    p.M, p.N, p.K, p.lda, p.ldw, p.ldy, p.split_n = 2, 333, 512, 512, 512, 333, 333
+    a.q, a.k, a.v, a.o = nv.src4(q), nv.src4(k), nv.src4(v), o.data_ptr()
+    a.o_sb, a.o_sh, a.o_sl = o.stride()[:3]
+    a.B, a.H, a.L, a.D, a.sm_scale = 1, 4, L, 128, 128 ** -0.5
+    nv.check(nv.lib().flux_attention_rows_bf16(nv.byref(a), nv.byref(pair), None, 0, nv.stream_ptr(q.device)), "flux_attention_rows_bf16")
+    assert torch.equal(y, tk.linear_into(x, w, None))
+    assert torch.equal(o, tk.scaled_dot_product_attention(q, k, v))

@@ -1709,6 +1709,13 @@ extern "C" int flux_attention_rows_bf16(const flux_attn_args* a, const flux_line
     if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace))))
         return fail(FLUX_E_NULL, "flux_attention_rows_bf16: workspace must be 16-byte aligned memory");
     hipStream_t st = static_cast<hipStream_t>(stream);
+    flux_linear_pair_args one;
+    if (rows->product[1].M == 0) {   // (there is no second product: whatever else its fields hold)
+        one = *rows;
+        one.product[1] = one.product[0];
+        one.product[1].M = one.a_rows[1] = one.a_batch_stride[1] = 0;
+        rows = &one;
+    }
     AttnParams p;
     GemmSet g;
     bool nothing;

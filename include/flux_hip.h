@@ -285,6 +285,9 @@ int flux_attention_fwd_bf16_ws(const flux_attn_args* args, void* workspace, int6
  * In all other cases the products run in front of the attention. The workspace is the attention's: results are those of
  * flux_linear_bf16_pair without one and of flux_attention_fwd_bf16_ws. */
 int flux_attention_rows_bf16(const flux_attn_args* args, const flux_linear_pair_args* rows, void* workspace, int64_t workspace_bytes, void* stream);
+/* Whether that call would run everything in one launch (1) or the products in front (0). Launches nothing and needs no GPU; returns what
+ * the call itself would return for its arguments. */
+int flux_attention_rows_together(const flux_attn_args* args, const flux_linear_pair_args* rows, int64_t workspace_bytes, int32_t* together);
 
 /* ---------------------------------------------------------------------------------------------
  * Small element-wise kernels (the reference's inductor-derived `ops`, plus nn.GELU on a view).

@@ -1,6 +1,7 @@
 """HIP flash-attention forward vs the oracle: the reference's grid (tests/test_attention.py: bf16,
 atol 1e-2 vs F.scaled_dot_product_attention), the Flux shape at atol 2e-2 vs an fp32 softmax, ragged
 lengths, strided views, and mathematical invariants at the full size."""
+import ctypes
 import math
 
 import pytest
@@ -10,6 +11,7 @@ import triton_kernels as tk
 from triton_kernels import _native as nv
 from oracle import flux_oracle as oracle
 from triton_kernels import testing as cfg
+from triton_kernels.kernels.linear import rows_args
 from util import DEV, randn, seeded
 
 pytestmark = pytest.mark.gpu
@@ -363,12 +365,24 @@ def test_attention_keys_in_parts_replayed_from_a_graph():
         assert torch.equal(o, eager), i
 
 
-@pytest.mark.parametrize("B,H,L,D", [(1, 2, 65, 128), (1, 24, 129, 128), (1, 24, 1280, 128), (2, 3, 700, 128), (2, 24, 640, 128),   # one launch for both
-                                     (1, 2, 64, 128), (1, 2, 2048, 128), (1, 24, 1300, 128), (1, 24, 300, 64)])                   # the products in front
+def _rows_together(q, k, v, o, calls):
+    """Whether the library takes these calls into the attention's launch."""
+    (B, H, L, D), a, yes = q.shape, nv.AttnArgs(), ctypes.c_int32(-1)
+    a.q, a.k, a.v, a.o = nv.src4(q), nv.src4(k), nv.src4(v), o.data_ptr()
+    a.o_sb, a.o_sh, a.o_sl = o.stride()[:3]
+    a.B, a.H, a.L, a.D, a.sm_scale = B, H, L, D, D ** -0.5
+    rows, _keep = rows_args(calls, q.device)
+    nv.check(nv.lib().flux_attention_rows_together(nv.byref(a), nv.byref(rows), nv.lib().flux_attention_workspace_bytes(B, H, L, D), nv.byref(yes)), "flux_attention_rows_together")
+    return bool(yes.value)
+
+
+@pytest.mark.parametrize("B,H,L,D,together", [(1, 2, 65, 128, True), (1, 24, 129, 128, True), (1, 24, 1280, 128, True), (2, 3, 700, 128, True), (2, 24, 640, 128, True),
+                                              (16, 16, 100, 128, True),   # 256 workgroups
+                                              (1, 2, 64, 128, False), (1, 2, 2048, 128, False), (1, 24, 1300, 128, False), (1, 24, 300, 64, False), (1, 257, 66, 128, False)])
 @pytest.mark.parametrize("M,K,Ns", [(1, 3072, (9216, 9216)), (1, 2048, (1001, 1001)), (2, 3072, (40,)), (2, 200, (9, 9)), (3, 1536, (333,)), (4, 1544, (8,)), (4, 3072, (100, 100)), (1, 512, (7, 12))])
-def test_attention_beside_row_products(B, H, L, D, M, K, Ns):
-    """Products of a few rows in the attention's launch, where it has one for them, and in front of it elsewhere: the bits of separate
-    launches, with SiLU on the way in, columns and K of every remainder, rows of the output further apart than they are long."""
+def test_attention_beside_row_products(B, H, L, D, together, M, K, Ns):
+    """Products of a few rows in the attention's launch, where it has one for them and they are few and alike enough, and in front of it elsewhere: the bits of
+    separate launches, with SiLU on the way in, columns and K of every remainder, rows of the output further apart than they are long."""
     g = seeded(L + K + M)
     q, k, v = (randn(g, B, H, L, D, dtype=torch.bfloat16).to(DEV) for _ in range(3))
     x = randn(g, M, K, dtype=torch.bfloat16).to(DEV)
@@ -377,6 +391,7 @@ def test_attention_beside_row_products(B, H, L, D, M, K, Ns):
         w, b = randn(g, N, K, dtype=torch.bfloat16).to(DEV) / K ** 0.5, randn(g, N, dtype=torch.bfloat16).to(DEV)
         calls.append(dict(x=x, w=w, b=b, in_activation="SiLU", out=torch.full((M, N + 3), float("nan"), dtype=torch.bfloat16, device=DEV)[:, :N]))
     o, lse = torch.empty_like(q), torch.empty(B, H, L, device=DEV)
+    assert _rows_together(q, k, v, o, calls) == (together and M * len(Ns) <= 4 and len(set(Ns)) == 1)
     for want_lse in (None, lse):   # (with it the call goes through ctypes)
         for c in calls:
             c["out"].fill_(float("nan"))

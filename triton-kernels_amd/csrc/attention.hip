@@ -1704,33 +1704,55 @@ extern "C" int flux_attention_fwd_bf16_ws(const flux_attn_args* a, void* workspa
         return fail(FLUX_E_NULL, "flux_attention_fwd_bf16_ws: workspace must be 16-byte aligned memory");
     return attention_launch(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
+// Checks a call with products beside it: the attention's parameters, the products as one launch of row vectors where they can be one, and whether that
+// goes into the attention's launch. At most kAttnCUs workgroups in all cases: with more (up to 128 rows the 32-row kernel takes any number) every CU
+// has two at work, and the products wait for room behind them, in 64 workgroups: beside two products of 1 x 12288 x 3072 [20, 24, 128] took 89.8 us, 40.0 with
+// the products in front, [40, 24, 100] 94.5 and 48.7, [12, 24, 128] 37.5 and 37.1, [11, 24, 100] 33.8 and 35.2.
+static int read_rows_call(const flux_attn_args* a, const flux_linear_pair_args& rows, int64_t workspace_bytes, AttnParams& p, GemmSet& g, bool& together) {
+    bool nothing;
+    int rc = read_attn_args(a, p, nothing), part_keys;
+    if (rc != FLUX_OK) return rc;
+    together = rows_beside(&rows, g, rc) && !nothing && a->D == 128 && a->L > 64 && a->B * a->H * ((a->L + 127) / 128) <= kAttnCUs && rows_fit(g) &&
+               (workspace_bytes == 0 || attn_splits(a->B * a->H, a->L, a->D, part_keys) == 1);
+    return rc;
+}
+
+// product[1].M == 0: there is no second product, whatever else its fields hold.
+static flux_linear_pair_args read_products(const flux_linear_pair_args& rows) {
+    flux_linear_pair_args r = rows;
+    if (r.product[1].M == 0) {
+        r.product[1] = r.product[0];
+        r.product[1].M = r.a_rows[1] = r.a_batch_stride[1] = 0;
+    }
+    return r;
+}
+
 extern "C" int flux_attention_rows_bf16(const flux_attn_args* a, const flux_linear_pair_args* rows, void* workspace, int64_t workspace_bytes, void* stream) {
     if (!rows) return fail(FLUX_E_NULL, "flux_attention_rows_bf16: null product");
     if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !aligned16(workspace))))
         return fail(FLUX_E_NULL, "flux_attention_rows_bf16: workspace must be 16-byte aligned memory");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    flux_linear_pair_args one;
-    if (rows->product[1].M == 0) {   // (there is no second product: whatever else its fields hold)
-        one = *rows;
-        one.product[1] = one.product[0];
-        one.product[1].M = one.a_rows[1] = one.a_batch_stride[1] = 0;
-        rows = &one;
-    }
+    const flux_linear_pair_args products = read_products(*rows);
     AttnParams p;
     GemmSet g;
-    bool nothing;
-    int rc = read_attn_args(a, p, nothing);
+    bool together = false;
+    int rc = read_rows_call(a, products, workspace_bytes, p, g, together);
     if (rc != FLUX_OK) return rc;
-    const bool together = rows_beside(rows, g, rc);
-    if (rc != FLUX_OK) return rc;
-    const int64_t BH = a->B * a->H;
-    int part_keys;
-    const bool whole = workspace == nullptr || attn_splits(BH, a->L, a->D, part_keys) == 1;
-    if (together && !nothing && a->D == 128 && attn_short(BH, a->L) && a->L > 64 && whole && rows_fit(g)) {
-        attn_launch_rows(p, BH, g, st);
+    if (together) {
+        attn_launch_rows(p, a->B * a->H, g, st);
         return check_launch("flux_attention_rows_bf16");
     }
-    rc = flux_linear_bf16_pair(rows, nullptr, 0, stream);
+    rc = flux_linear_bf16_pair(&products, nullptr, 0, stream);
     return rc != FLUX_OK ? rc : attention_launch(a, workspace, workspace_bytes, st);
+}
+
+extern "C" int flux_attention_rows_together(const flux_attn_args* a, const flux_linear_pair_args* rows, int64_t workspace_bytes, int32_t* together) {
+    if (!rows || !together) return fail(FLUX_E_NULL, "flux_attention_rows_together: null argument");
+    AttnParams p;
+    GemmSet g;
+    bool t = false;
+    const int rc = read_rows_call(a, read_products(*rows), workspace_bytes, p, g, t);
+    *together = t ? 1 : 0;
+    return rc;
 }
 #endif

@@ -127,6 +127,7 @@ SIGNATURES = {
     "flux_attention_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int32]),
     "flux_attention_fwd_bf16_ws": (c_int32, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p]),
     "flux_attention_rows_bf16": (c_int32, [POINTER(AttnArgs), POINTER(LinearPairArgs), c_void_p, c_int64, c_void_p]),
+    "flux_attention_rows_together": (c_int32, [POINTER(AttnArgs), POINTER(LinearPairArgs), c_int64, POINTER(c_int32)]),
     "flux_silu": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
     "flux_gelu_tanh": (c_int32, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int32, c_void_p]),
     "flux_modulation_scale_shift": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,

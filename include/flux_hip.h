@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define FLUX_ABI_VERSION 4
+#define FLUX_ABI_VERSION 5
 
 enum flux_dtype { FLUX_BF16 = 0, FLUX_F32 = 1 };
 

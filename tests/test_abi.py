@@ -2,6 +2,7 @@
 structures have the sizes the header's structs have, and argument checks reject bad input before
 any launch (no GPU needed for any of this)."""
 import ctypes
+import hashlib
 import os
 import re
 import subprocess
@@ -31,7 +32,16 @@ def test_every_declared_symbol_is_exported_and_bound():
     for name in names:
         assert hasattr(handle, name), f"{name} is declared in flux_hip.h but not exported"
     assert set(names) == set(nv.SIGNATURES), "ctypes binding table and header disagree"
-    assert nv.lib().flux_abi_version() == 4
+    assert nv.lib().flux_abi_version() == nv.ABI_VERSION == 5
+
+
+def test_the_version_stands_for_what_the_header_declares():
+    """The version is what tells a library and a binding of different builds apart, so functions, structures or constants that
+    come, go or change need another one, and its line here."""
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    version = int(re.search(r"#define FLUX_ABI_VERSION (\d+)", text).group(1))
+    text = re.sub(r"\s+", "", re.sub(r"#define FLUX_ABI_VERSION \d+", "", text))
+    assert (version, hashlib.sha256(text.encode()).hexdigest()[:16]) == (5, "7dafb1aae1f3907a")
 
 
 def test_struct_layouts_match_the_header(tmp_path):

@@ -21,7 +21,7 @@ ACT_NONE, ACT_GELU_TANH, ACT_SILU = 0, 1, 2
 LINEAR_SHARED_GPU = 1
 E_NULL, E_SHAPE, E_DTYPE, E_ALIGN, E_TOO_WIDE, E_UNSUPPORTED = -1, -2, -3, -4, -5, -6
 MAX_ROW = 65536
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _DTYPE_CODE = {torch.bfloat16: FLUX_BF16, torch.float32: FLUX_F32}
 

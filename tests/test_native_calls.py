@@ -281,8 +281,9 @@ def test_calls_of_the_blocks_forms(monkeypatch):
 
         _served(monkeypatch, "linear_into", served, split)
     x, few = wide[0, :, :K], t(2, K)
-    for kw, served in ((dict(x=few, in_activation="SiLU"), True), (dict(x=x, shared_gpu=True), False), (dict(x=x, b=b.float()), False), (dict(x=x, w=w.t().contiguous().t()), False)):
+    for kw, served in ((dict(x=few, in_activation="SiLU"), True), (dict(x=x, shared_gpu=True), False), (dict(x=x, b=b.float()), False), (dict(x=x, w=w.t().contiguous().t()), False), (dict(x=x, split=N), True)):
         _served(monkeypatch, "linear_into", served, into(**{"w": w, "b": b, **kw}))
+    _served(monkeypatch, "linear_into", False, lambda: (linear_into(x, w, b, split=N + 8)[:, :N],))   # (its last eight columns are nobody's)
     gates = t(2, 1, 3 * N)[..., :N]
     for first, second, served in ((wide[:, :30, :K], wide[:, 30:, :K], True), (wide[:1, :30, :K], wide[:1, 30:, :K], True), (few[:1], few[1:], True), (wide[..., ::2], x, False)):
         calls = [dict(x=v, w=w, b=b) for v in (first, second)]

@@ -535,6 +535,7 @@ bool read_product(PyObject* call, Product& p, bool slices) {
     }
     if (in_act != FLUX_ACT_NONE && M > 8) return false;
     if (b && (!is_bf16(*b, *x) || b->dim() != 1 || b->numel() != N || b->stride(0) != 1)) return false;
+    if (split > N) return false;   // (the launcher's output has `split` columns)
     const bool cut = split >= 0 && split < N;
     if (out && !destination(*out, *x, M, cut ? split : N)) return false;
     if (cut && (!out2 || !destination(*out2, *x, M, N - split))) return false;

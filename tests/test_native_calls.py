@@ -352,7 +352,8 @@ def test_refusals_stay_what_they_were(monkeypatch):
              (tk.linear, x, w, None, "RELU"), (tk.linear, x, w, torch.ones(7, device=DEV, dtype=BF)), (tk.scaled_dot_product_attention, h, h, h.float()),
              (tk.scaled_dot_product_attention, h, h, h, float("nan")), (tk.scaled_dot_product_attention, h[..., :24], h[..., :24], h[..., :24]),
              (tk.scaled_dot_product_attention, h, h, h[:, :, :2]), (tk.apply_rope, h, h, torch.ones(1, 1, 5, 32, 2, 2, device=DEV)), (tk.apply_rope, h, h.float(), h), (tk.apply_rope, h[..., :24], h[..., :24], torch.ones(1, 1, 4, 12, 2, 2, device=DEV)),
-             (tk.layer_norm_modulation, h, h[:, :, 0], h[:, :, :1, :32]), (tk.layer_norm_modulation, x, x[:2], x)]
+             (tk.layer_norm_modulation, h, h[:, :, 0], h[:, :, :1, :32]), (tk.layer_norm_modulation, x, x[:2], x),
+             (norm_mod.layer_norm_modulation_pair, (h, h[:, :, 0]), (h, h[:, :, 0], h[:, :, 0])), (norm_mod.layer_norm_modulation_pair, (h, h[:, :, 0]), (h[:, :, 0], h, h[:, :, 0], h[:, :, 0]))]
     for fn, *args in calls:
         errors = []
         for call in (lambda: fn(*args), lambda: launcher(monkeypatch, fn, *args)):

@@ -159,7 +159,7 @@ def layer_norm_modulation(x: torch.Tensor, weight: torch.Tensor, bias: torch.Ten
 
 def layer_norm_modulation_pair(first: tuple, second: tuple, eps=1e-5) -> tuple[torch.Tensor, torch.Tensor]:
     """layer_norm_modulation of two (x, weight, bias) triples of the same width and type in one launch."""
-    y = None if is_compiling() else nv.ops().layer_norm_modulation_pair(*first, *second, eps)
+    y = nv.ops().layer_norm_modulation_pair(*first, *second, eps) if len(first) == len(second) == 3 and not is_compiling() else None
     if y is not None:
         return y
     a0, y0, _keep0 = _layer_norm_args(*first)

@@ -41,7 +41,8 @@ def _pair(kind, seed):
 
 @pytest.mark.parametrize("batch_size", [1, 2])
 @pytest.mark.parametrize("seq_len", [256, 1024])
-def test_single_stream_block(batch_size, seq_len):
+def test_single_stream_block(batch_size, seq_len, monkeypatch):
+    from triton_kernels.modules import blocks
     ref, hip = _pair("single", seq_len + batch_size)
     g = seeded(seq_len)
     x = randn(g, batch_size, seq_len, HID, dtype=torch.bfloat16).to(DEV)
@@ -49,7 +50,13 @@ def test_single_stream_block(batch_size, seq_len):
     pe = randn(g, 1, 1, seq_len, HEAD_DIM // 2, 2, 2).to(DEV)
     with torch.no_grad():
         y_ref = ref(x=x, vec=vec, pe=pe)
-        y_hip = hip(x=x, vec=vec, pe=pe)              # fused, QKNorm + RoPE in linear1's epilogue
+        y_hip = hip(x=x, vec=vec, pe=pe)              # fused, QKNorm + RoPE wherever that is the faster way at this size
+        with monkeypatch.context() as m:              # fused, QKNorm + RoPE in linear1's epilogue wherever that is possible
+            calls = []
+            m.setattr(blocks, "qk_pays", lambda *a: True)
+            m.setattr(blocks, "linear_into", lambda *a, **kw: calls.append(kw.get("qk") is not None) or tk.linear_into(*a, **kw))
+            y_epilogue = hip(x=x, vec=vec, pe=pe)
+        assert any(calls) == blocks.qk_fusable(x, hip.linear1.weight, seq_len, HEAD_DIM) == (batch_size * seq_len > 256)
         hip.fuse_qk_epilogue = False
         y_prep = hip(x=x, vec=vec, pe=pe)             # fused, QKNorm + RoPE as one kernel behind linear1
         hip.fused = False
@@ -59,6 +66,9 @@ def test_single_stream_block(batch_size, seq_len):
     _close(y_unfused, y_ref)
     _close(y_hip, y_unfused, atol=0.05)
     _close(y_hip, y_prep, atol=0.05)
+    _close(y_epilogue, y_ref)
+    _close(y_epilogue, y_unfused, atol=0.05)
+    _close(y_epilogue, y_prep, atol=0.05)
 
 
 @pytest.mark.parametrize("batch_size", [1, 2])

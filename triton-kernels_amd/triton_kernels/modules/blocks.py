@@ -167,7 +167,7 @@ class SingleStreamBlock(nn.Module):
 
     fused = True
     # QKNorm + RoPE inside linear1's epilogue when the shapes allow (heads of 128, sequences of at least
-    # 256 tokens); otherwise, or with this switched off, one preparation kernel behind linear1
+    # 256 tokens) and that is the faster way (qk_pays); otherwise, or with this switched off, one preparation kernel behind linear1
     fuse_qk_epilogue = True
     # Optional callable(stage, edge), invoked on the launching thread right before (edge "begin") and
     # right after ("end") the launch of a stage of the forward: "modulation", "layer_norm" and, in the

@@ -1416,7 +1416,9 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel_pair(AttnParams p4
 // second launch about 2 us, both fitted to 46 problems of 2 to 24 heads. More than 256 workgroups would
 // share CUs, which gains nothing (LDS-bound). us before -> after at head dim 128, [1, 2, L]: L 2048
 // 38.7 -> 20.2, 4096 70.6 -> 33.3; [1, 4, 4096] 72.5 -> 51.3; [1, 8, L]: L 1280 25.7 -> 23.6, 1536 29.9 -> 27.5, 2048 39.2 -> 35.1 (head dim 64:
-// 27.1 -> 24.0). The model is off by up to 0.9 us, which a part has to gain at least; calls that take the GPU less than 23 us stay whole.
+// 27.1 -> 24.0). The model is off by up to 1.6 us, so parts have to gain 1.5 us by it: of 70 calls that are cut for less than 6, the least gained [1, 10, 1530] 29.9 ->
+// 30.0 and [3, 3, 1146] 23.7 -> 23.8. Calls that one part takes the GPU less than 23 us for stay whole. That line comes from the time when a call in parts took the
+// host 22 us; since it takes 10, parts would gain there too where calls follow one another ([1, 2, 1024] 21.6 -> 14.0 in four).
 static int attn_splits(int64_t BH, int64_t L, int D, int& part_keys) {
     const int64_t groups = BH * ((L + 127) / 128), key_tiles = (L + 63) / 64;
     const double tile_us = D == 128 ? 1.03 : 0.68, fixed_us = D == 128 ? 1.8 : 2.4, group_us = D == 128 ? 0.033 : 0.016;
